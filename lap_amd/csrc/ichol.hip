@@ -288,6 +288,7 @@ const IcPlan *ic_factor(int n, int nnzA, const int *ia, const int *ja, double *a
   }
   tri_ell_build(*P.lplan, P.lja->as<int>(), P.lval->as<double>(), P.lell);
   tri_ell_build(*P.uplan, P.uja->as<int>(), P.uval->as<double>(), P.uell);
+  P.comp = tri_compose(*P.lplan, *P.uplan);
   std::vector<int> h_bad = dev_download(bad->as<int>(), 2);
   if (h_bad[0]) {
     P.ok = false;
@@ -303,6 +304,7 @@ const IcPlan *ic_factor(int n, int nnzA, const int *ia, const int *ja, double *a
 
 void ic_apply_launch(const IcPlan &p, const double *x, double *y, double *aux,
                      const int *done) {
+  if (tri_solve_two_launch(*p.lplan, p.lell, *p.uplan, p.uell, p.comp, x, y, done)) return;
   tri_solve_launch(*p.lplan, p.lia->as<int>(), p.lja->as<int>(), p.lval->as<double>(), nullptr,
                    x, aux, done, &p.lell);
   tri_solve_launch(*p.uplan, p.uia->as<int>(), p.uja->as<int>(), p.uval->as<double>(), nullptr,

@@ -336,23 +336,25 @@ struct TriPlan {
   std::vector<int> level_seg;  // host, nlevels + 1
   DevBufPtr segd, seg_part, seg_tick;
   bool has_diag = true;        // every row holds its pivot
-  // Chunked schedule (one persistent workgroup per chunk of consecutive rows
-  // in solve order; built when every row holds at most 8 entries).  Chunk c
-  // runs its rows level by level ("steps"); before a step it waits until
-  // each earlier chunk it depends on has published the level it needs.
+  // Chunked schedule (four chunks of rows per workgroup; built when every row
+  // holds at most 4 entries beside its pivot).  Chunk c runs its rows level by
+  // level in steps of at most 64 rows, padded to that; a dependency on
+  // another workgroup (or on a row too many steps back) is one entry of the
+  // chunk's inbox, filled by the chunk that solves the row.
   struct Chunks {
-    int nchunks = 0, nsteps = 0, nwaits = 0;
+    int nchunks = 0, nrec = 0;  // nrec: 64 records per step, padding included
     DevBufPtr cstep;  // int[nchunks + 1]: first step of each chunk
-    DevBufPtr sptr;   // int[nsteps + 1]: first position of each step
-    DevBufPtr slev;   // int[nsteps]: the step's level
-    DevBufPtr wptr;   // int[nsteps + 1]: first wait of each step
-    DevBufPtr wchk;   // int[nwaits]: chunk waited on
-    DevBufPtr wlev;   // int[nwaits]: level it must have published
-    DevBufPtr crow;   // int[n]: rows in (chunk, level, row) order
-    DevBufPtr cmap;   // int[n]: level-order position (into desc) of crow[t]
-    DevBufPtr code;   // int[n * w]: each record's dependencies (see sptrsv.hip)
-    int w = 0;        // record width
-    long long cost = 0;  // simulated pipeline length (steps)
+    DevBufPtr crow;   // int[nrec]: row of each record, -1: padding
+    DevBufPtr pos;    // int[n]: record of each row
+    DevBufPtr cmap;   // int[nrec]: its level-order position (into desc)
+    DevBufPtr code;   // int2[nrec]: four 16-bit LDS entries (see sptrsv.hip)
+    DevBufPtr need;   // int2[steps]: what a step waits for (see sptrsv.hip)
+    DevBufPtr lstep;  // int[steps]: its number within its chunk
+    DevBufPtr hbase;  // int[nchunks + 1]: first inbox entry of each chunk
+    DevBufPtr ebase;  // int[nchunks + 1]: first export of each chunk
+    DevBufPtr exps;   // int2[exports]: {record within the chunk, inbox entry}
+    DevBufPtr inbox;  // values between chunks, each half tagged with the solve
+    DevBufPtr epoch;  // unsigned: the solve's tag
   } ch;
 };
 // Rows longer than this many entries (pivot included) are solved by a
@@ -399,7 +401,18 @@ void tri_ch_pack32(const TriPlan &p, const int *ja, const float *a, TriChunks32 
 void tri_solve32_launch(const TriPlan &p, const int *ja, const float *a, const float *x, float *y,
                         const int *done, const TriChunks32 *c = nullptr);
 int tri_launches32(const TriPlan &p, const TriChunks32 *c);
-// Sync-free mode: nonzero once a dependency wait ran out (the result is then
+// Two chunked solves in a row, y = T2^{-1} T1^{-1} x: the second one takes its
+// right-hand sides straight from the first one's results in schedule order
+// (comp = tri_compose of the two), one pass over the vector less.  False when
+// either triangle has no chunked schedule (nothing is launched).
+DevBufPtr tri_compose(const TriPlan &first, const TriPlan &second);
+bool tri_solve_two_launch(const TriPlan &p1, const TriEll &e1, const TriPlan &p2,
+                          const TriEll &e2, const DevBufPtr &comp, const double *x, double *y,
+                          const int *done);
+bool tri_solve32_two_launch(const TriPlan &p1, const TriChunks32 &c1, const TriPlan &p2,
+                            const TriChunks32 &c2, const DevBufPtr &comp, const float *x,
+                            float *y, const int *done);
+// Chunked solves: nonzero once a dependency wait ran out (the result is then
 // invalid); reset by tri_clear_error.
 int tri_error();
 void tri_clear_error();
@@ -412,6 +425,7 @@ struct IcPlan {
   DevBufPtr uia, uja, uval;  // U = L^T (diagonal first)
   const TriPlan *lplan = nullptr, *uplan = nullptr;
   TriEll lell, uell;  // the factors' rows packed in level order
+  DevBufPtr comp;     // tri_compose of the two plans (null: not both chunked)
   bool ok = true;
 };
 const IcPlan *ic_plan_find(const double *vals);

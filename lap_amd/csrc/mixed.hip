@@ -834,6 +834,7 @@ const double *inner_d_r<double>(MixPlan *, const double *d_r, int) {
 // rounding costs iterations on badly conditioned systems.
 inline void ic_inner(const IcPlan &P, const MixPlan &M, const float *l32, const float *u32,
                      const float *x, float *y, float *aux, const int *done) {
+  if (tri_solve32_two_launch(*P.lplan, M.lch, *P.uplan, M.uch, P.comp, x, y, done)) return;
   tri_solve32_launch(*P.lplan, P.lja->as<int>(), l32, x, aux, done, &M.lch);
   tri_solve32_launch(*P.uplan, P.uja->as<int>(), u32, aux, y, done, &M.uch);
 }

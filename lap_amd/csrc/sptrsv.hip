@@ -9,23 +9,15 @@
 // computed with exactly the reference's sequential arithmetic
 // (simple_blas.c:46-85) and the result equals the sequential solve bitwise.
 //
-// Chunked mode (option sptrsv_mode 3, the default): one persistent launch
-// per solve, one workgroup per chunk of rows (all workgroups resident: at
-// most one per CU).  A chunk runs its rows level by level; a level of a chunk
-// is a "step", one lane per row, the rows packed as fixed-size records.
-// Every dependency of a step lies in an earlier step of its own chunk (LDS
-// ring or y) or in another chunk, at a lower level; before a step, compute
-// wave 0 makes sure every chunk the step depends on has published (in its
-// progress counter) the highest level the step needs from it --
-// point-to-point waits, listed per step by the analysis and pruned to the
-// ones not already implied by an earlier wait of the chunk.  y is stored with
-// agent-scope stores and dependencies are read with agent-scope loads (both
-// coherent across the XCDs' L2s without cache write-backs); a step's stores
-// are complete (s_waitcnt) before its level is published.  Every wait is
-// bounded and raises the shared error flag when it runs out, so the kernel
-// always ends.  Same row arithmetic as the level launches: bitwise
-// identical.  Triangles whose rows do not fit a record keep the level
-// launches (option sptrsv_mode 0 forces them everywhere).
+// Chunked mode (option sptrsv_mode 3, the default): one launch per solve over
+// chunks of rows that are all resident, values between chunks passed as
+// tagged words through memory (k_tri_flow).  Same row arithmetic as the level
+// launches: bitwise identical.  Triangles whose rows do not fit a record keep
+// the level launches (option sptrsv_mode 0 forces them everywhere).  Measured
+// against the level launches and against one workgroup of 256-row steps per
+// chunk with progress counters, which it replaced, per IC0 / GS_std PCG
+// iteration (us): 128^3 434 / 480 against 1840 / 2100; 256^3 2100 / 2690
+// against 4460 / 4970; level launches at 256^3 7780 / 8310.
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
@@ -335,325 +327,534 @@ __global__ __launch_bounds__(kBlock) void k_tri_level_ell(
 }
 
 // ---------------------------------------------------------- chunked mode
-constexpr int kChMinRows = 2048;  // rows per chunk at least
-constexpr int kChMax = 1024;      // chunks at most (the kernel's LDS table)
-constexpr int kChStepRows = kBlock;  // rows per step of a chunk at most (one per lane)
-constexpr int kChRing = 4;        // steps of results kept in LDS
-constexpr int kChSteps = 512;     // steps of a chunk at most (LDS table)
-constexpr int kChWaits = 1024;    // waits of a chunk at most (LDS table)
-constexpr unsigned kChSpinLimit = 1u << 22;  // polls of one wait before the solve fails
+constexpr int kFlRing = 16;       // steps of results kept in LDS
+constexpr int kFlHalo = 512;      // values from other chunks kept in LDS (>= 256 = one step's)
+constexpr int kFlGroup = 4;       // steps per unrolled group (chunks are padded to it)
+constexpr int kFlTeam = 2;        // chunks per workgroup
+constexpr int kFlPerCu = 2;       // workgroups per CU at most
+constexpr int kFlAhead = 4;       // windows of the export list read ahead
+constexpr int kFlMaxSteps = 1 << 18;  // of a chunk: its records stay below 2^31 bytes
+// LDS entries per chunk: ring, halo buffer, a zero
+constexpr int kFlLds = kFlRing * kWave + kFlHalo + 8;
+constexpr int kFlZero = kFlLds - 8;
+constexpr unsigned kFlSpins = 1u << 22;  // polls of one wait before the solve fails
 
-__global__ __launch_bounds__(kBlock) void k_ch_reset(int nchunks, int *progress,
-                                                     const int *__restrict__ done) {
-  if (done && *done) return;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < nchunks; i += gridDim.x * kBlock)
-    __hip_atomic_store(&progress[i], -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// The schedule's records, one block per step of kWave rows, each field
+// stored for the 64 rows together so that every load of the compute wave is
+// contiguous (bytes, l = lane):
+//   [0, 1024)     int4: the LDS byte offsets of the row's four dependencies in
+//                 CSR order, 16 bits each (.x, .y; padding: a zero entry,
+//                 value 0), the step's word for lane l (.z, see FlLane) and
+//                 the base of the row's range test (.w, see fl_out)
+//   then W = 4 off-diagonal values per row (FP64: two double2 planes, FP32:
+//   one float4 plane), then double2 {pivot, 1/pivot}.
+typedef __attribute__((ext_vector_type(4))) unsigned fl_u4;
+typedef __attribute__((ext_vector_type(2))) unsigned fl_u2;
+__device__ __forceinline__ double fl_f64(unsigned lo, unsigned hi) {
+  return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
-
-// Workgroup barrier for LDS traffic only: waits for this wave's LDS
-// operations, not for its outstanding global loads (__syncthreads would wait
-// for every memory operation of the wave).  The signal fences keep the
-// compiler from moving memory accesses across it.
-__device__ __forceinline__ void lds_barrier() {
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
-// s_waitcnt encoding (gfx9) for vmcnt(N) alone: lgkmcnt and expcnt at their
-// maxima.
-constexpr unsigned vmcnt_only(unsigned n) {
-  return (n & 15u) | ((n >> 4) << 14) | (7u << 4) | (15u << 8);
-}
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef __attribute__((address_space(1))) void global_void_t;
-
-// The chunked schedule's records, one per row in schedule order (bytes):
-// [0, 4W) the off-diagonal dependency codes in CSR order (-1 padding, >= 0 a
-// row of y, <= -2 the LDS ring slot -(code + 2)); [4W, 4W + 4) the row; then
-// the off-diagonal values and the pivot: FP64 values at [4W + 16, 12W + 16)
-// and [12W + 16, 12W + 24), FP32 values at [4W + 8, 8W + 8) and
-// [8W + 8, 8W + 12).  The size is a multiple of 16 bytes.
-template <int W, class AT>
-struct ChRec;
-template <int W>
-struct ChRec<W, double> {
-  static constexpr int bytes = 12 * W + 32;
-  static constexpr int row = W;                  // int index
-  static constexpr int val = (4 * W + 16) / 8;   // value index
-  static constexpr int piv = (12 * W + 16) / 8;  // value index
-  static constexpr int dma = bytes / 4;          // 16-byte loads of 64 lanes per kBlock records
+template <class AT>
+struct FlRec;
+template <>
+struct FlRec<double> {
+  static constexpr int bytes = kWave * 64;
+  fl_u4 c, v0, v1, pv;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, int lane16, int off) {
+    c = __builtin_amdgcn_raw_buffer_load_b128(b, lane16, off, 0);
+    v0 = __builtin_amdgcn_raw_buffer_load_b128(b, lane16 + 1024, off, 0);
+    v1 = __builtin_amdgcn_raw_buffer_load_b128(b, lane16 + 2048, off, 0);
+    pv = __builtin_amdgcn_raw_buffer_load_b128(b, lane16 + 3072, off, 0);
+  }
+  __device__ __forceinline__ double val(int j) const {
+    return j == 0   ? fl_f64(v0.x, v0.y)
+           : j == 1 ? fl_f64(v0.z, v0.w)
+           : j == 2 ? fl_f64(v1.x, v1.y)
+                    : fl_f64(v1.z, v1.w);
+  }
 };
-template <int W>
-struct ChRec<W, float> {
-  static constexpr int bytes = (8 * W + 12 + 15) / 16 * 16;
-  static constexpr int row = W;          // int index
-  static constexpr int val = W + 2;      // value index
-  static constexpr int piv = 2 * W + 2;  // value index
-  static constexpr int dma = bytes / 4;
+template <>
+struct FlRec<float> {
+  static constexpr int bytes = kWave * 48;
+  fl_u4 c, v, pv;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, int lane16, int off) {
+    c = __builtin_amdgcn_raw_buffer_load_b128(b, lane16, off, 0);
+    v = __builtin_amdgcn_raw_buffer_load_b128(b, lane16 + 1024, off, 0);
+    pv = __builtin_amdgcn_raw_buffer_load_b128(b, lane16 + 2048, off, 0);
+  }
+  __device__ __forceinline__ double val(int j) const {
+    return (double)__uint_as_float(j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w);
+  }
+};
+__device__ __forceinline__ void fl_load_x(__amdgpu_buffer_rsrc_t b, int lane, int step, double *x) {
+  const fl_u2 u = __builtin_amdgcn_raw_buffer_load_b64(b, lane * 8, step * (kWave * 8), 0);
+  *x = fl_f64(u.x, u.y);
+}
+__device__ __forceinline__ void fl_load_x(__amdgpu_buffer_rsrc_t b, int lane, int step, float *x) {
+  *x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, lane * 4, step * (kWave * 4), 0));
+}
+// a buffer of `bytes` from p (gfx9 word 3: raw data, 32-bit)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t fl_buffer(const void *p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00027000);
+}
+
+// Whether x lies outside [2^-400, 2^400): inside it (and with the pivot in
+// it) the refined division below neither overflows nor loses bits to
+// underflow in any step.  `base` is kFlBase, or kFlNever where the pivot is
+// outside, which makes every x fail.
+constexpr unsigned kFlBase = 623u << 20, kFlSpan = 800u << 20, kFlNever = 0x80000000u;
+__device__ __forceinline__ bool fl_out(double x, unsigned base) {
+  const unsigned h = (unsigned)((unsigned long long)__double_as_longlong(x) >> 32) & 0x7fffffffu;
+  return h - base >= kFlSpan;
+}
+
+// a / b correctly rounded, from y = 1/b correctly rounded: two residual
+// corrections of a*y by fused multiply-adds.  The first leaves the quotient
+// within one unit in the last place, and Markstein's theorem (P. W.
+// Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", IBM J. Res. Dev. 34, 1990) makes the second's result the
+// rounded quotient, so the bits are the divide instruction sequence's at less
+// than half its dependent latency (five operations).  a and b not fl_out.
+__device__ __forceinline__ double fl_div(double a, double b, double y) {
+  double q = a * y;
+  q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
+// One value of another chunk in an inbox: its 32-bit halves (FP32: the whole)
+// each beside the solve's tag in one aligned 8-byte word.  Such a word is
+// written and read whole, so a matching tag means the half is this solve's: no
+// flag, fence or store order is involved.  Stores and loads are agent-scope
+// (sc1): past the CU's cache and the XCD's L2.
+constexpr int kFlAgent = 16;
+__device__ __forceinline__ void fl_put(__amdgpu_buffer_rsrc_t box, int i, unsigned tag, double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  __builtin_amdgcn_raw_buffer_store_b128(fl_u4{(unsigned)b, tag, (unsigned)(b >> 32), tag}, box,
+                                         i * 16, 0, kFlAgent);
+}
+__device__ __forceinline__ void fl_put(__amdgpu_buffer_rsrc_t box, int i, unsigned tag, float v) {
+  __builtin_amdgcn_raw_buffer_store_b64(fl_u2{__float_as_uint(v), tag}, box, i * 8, 0, kFlAgent);
+}
+template <class VT>
+struct FlBoxed;
+template <>
+struct FlBoxed<double> {
+  fl_u4 w;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t box, int i) {
+    w = __builtin_amdgcn_raw_buffer_load_b128(box, i * 16, 0, kFlAgent);
+  }
+  __device__ __forceinline__ bool is(unsigned tag) const { return w.y == tag && w.w == tag; }
+  __device__ __forceinline__ double value() const { return fl_f64(w.x, w.z); }
+};
+template <>
+struct FlBoxed<float> {
+  fl_u2 w;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t box, int i) {
+    w = __builtin_amdgcn_raw_buffer_load_b64(box, i * 8, 0, kFlAgent);
+  }
+  __device__ __forceinline__ bool is(unsigned tag) const { return w.y == tag; }
+  __device__ __forceinline__ float value() const { return __uint_as_float(w.x); }
 };
 
-// One workgroup per chunk: kBlock compute lanes (one row each per step) and
-// one prefetch wave.  progress[c]: highest level of chunk c whose rows are
-// all complete and visible; state[1]: error flag (a wait ran out).
-//  * the prefetch wave copies each step's records and right-hand sides (xc:
-//    x in schedule order, gathered beforehand by k_ch_gather) into an LDS
-//    slot D steps ahead with direct global-to-LDS loads; before each step
-//    ends it waits, by count, for the next step's slot only (its loads are
-//    all of one kind and complete in order).  No compute lane ever waits on
-//    a copy;
-//  * a step starts with compute wave 0 checking its waits against a table
-//    of the levels already seen published, which that wave refreshes by
-//    polling the next step's producers while the current step runs.  Only
-//    when a wait is not covered does the chunk block: it first publishes
-//    everything it has completed, so that no chunk waits on finished but
-//    unpublished work, and polls until the levels it needs are published;
-//  * each row reads rows of this chunk from the last kChRing steps out of
-//    the LDS ring and the others from y (agent-scope loads), and writes its
-//    result to the ring and to y (agent-scope store).  A step ends with the
-//    lanes waiting, by count, for the previous step's store only and a
-//    barrier, after which the previous step's level is published: one step
-//    behind, so that no lane waits on a store it has just issued.
+// The compiler may not move memory accesses across this (LDS operations of a
+// wave execute in issue order, so no wait is needed between them).
+__device__ __forceinline__ void fl_fence() { __atomic_signal_fence(__ATOMIC_SEQ_CST); }
+
+// LDS progress words of a chunk, each written by one wave.
+struct FlProg {
+  int hready;        // halo: values in LDS so far
+  int xdone, ydone;  // export / store: steps whose results they no longer need
+  int failed;        // 0, or -1
+  int cdone, hcons;  // compute: steps finished, halo values consumed
+};
+__device__ __forceinline__ int fl_ld(const int *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void fl_st(int *p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// What a step waits for, one word per lane of the compute wave: lane l of the
+// step's record holds the least value that the progress word of lane l must
+// have, and the wave keeps the words as last seen in one register, so the
+// test is one comparison, and one LDS read when it fails.  Lanes 0 and 7 of
+// the record are also what the wave publishes when the step is done.
+enum FlLane {
+  FL_HALO = 0,   // hready >= halo values the step uses (published to hcons)
+  FL_SIB = 1,    // cdone of the workgroup's other chunk
+  FL_X = 2,      // xdone and ydone: the step's ring entries are free
+  FL_Y = 3,
+  FL_FAILED = 4, // failed >= 0
+  FL_DONE = 5,   // nothing to wait for (published to cdone)
+};
+
+// Two chunks per workgroup, four waves per chunk.  A chunk runs its rows
+// level by level in steps of at most 64 rows; each of its waves has one job
+// and they hand over through LDS words, with no barrier and no wait on global
+// memory between a step and the next:
+//   wave 0, compute: a row per lane; dependencies come from the LDS rings (the
+//     last kFlRing steps of each chunk of the workgroup) or from the chunk's
+//     LDS halo buffer, the result goes into its own ring.  Records and
+//     right-hand sides are loaded kFlGroup steps ahead into registers.
+//   wave 1, halo: takes the values other workgroups put into this chunk's
+//     inbox, in the order the steps use them, into the halo buffer.  It never
+//     waits for a later value while an earlier one is there, so a chunk's
+//     progress depends only on values it needs next.
+//   wave 2, export: puts results other workgroups use into their inboxes.
+//   wave 3, store: writes results over the right-hand sides they came from
+//     (schedule order, contiguous).  Scattered to their rows from here they
+//     cost 64 write requests a step, which held up the CU's loads;
+//     k_fl_spread does it afterwards with the whole chip.
+// What bounds it: the chain of levels.  A step costs the LDS round trip of
+// the previous step's results, four dependent subtractions and the division,
+// 0.16 us.  Crossing into another workgroup costs a trip through memory, about
+// 3 us, but only once per boundary on the longest path: a chunk runs behind
+// its neighbours by that much and then at their pace.  Two chunks per
+// workgroup save a third of the boundaries; four saved half, but a CU reads
+// records at no more than about 57 GB/s, which four chunks' steps exceed.
+// (Before: a workgroup took a step of 256 rows between two barriers, loaded
+// its neighbours' values inside the step and published a counter after it:
+// about 2.2 us per level.)  Every wait is bounded; one that runs out raises
+// state[1] and ends the workgroup, and the others follow.
 // AT: the values' type, VT: the vectors' (FP32 values and vectors are
 // summed in FP64 and the result rounded once, as the FP32 level launches do).
-template <class AT, class VT, int W, int D, int NS>
-__global__ __launch_bounds__(kBlock + kWave) void k_tri_chunks(
-    const int *__restrict__ cstep, const int *__restrict__ sptr, const int *__restrict__ slev,
-    const int *__restrict__ wptr, const int *__restrict__ wchk, const int *__restrict__ wlev,
-    const char *__restrict__ rec, const VT *xc, VT *y,
-    int *progress, int *state, const int *__restrict__ done) {
+template <class AT, class VT>
+__global__ __launch_bounds__(4 * kFlTeam * kWave, 4) void k_tri_flow(
+    const int *__restrict__ cstep, const char *__restrict__ rec, VT *xc, const int *__restrict__ hbase,
+    const int *__restrict__ ebase, const int2 *__restrict__ exps, void *inbox, int inbox_bytes,
+    const unsigned *epoch, int *state, const int *__restrict__ done) {
   if (done && *done) return;
-  using R = ChRec<W, AT>;
-  constexpr int XB = kBlock * (int)sizeof(VT);  // the step's right-hand sides
-  constexpr int SLOT = kBlock * R::bytes + XB;
-  constexpr int PER = R::dma + XB / (kWave * 4);  // loads per step: records, right-hand sides
-  static_assert((D - 1) * PER <= 63, "vmcnt range");
-  static_assert(D < NS, "a slot in use is never refilled");
-  __shared__ __attribute__((aligned(16))) char slots[NS * SLOT];
-  __shared__ int seen[kChMax];  // highest level seen published, per chunk
-  __shared__ VT ring[kChRing * kBlock];
-  __shared__ int tsptr[kChSteps + 1], tslev[kChSteps], twptr[kChSteps + 1];
-  __shared__ int twchk[kChWaits], twlev[kChWaits];
-  __shared__ int failed, must_wait;
-  const int c = blockIdx.x;
-  const bool pf = threadIdx.x >= kBlock;  // the prefetch wave
-  const int p = threadIdx.x;              // a compute lane's row position in a step
+  __shared__ VT all[kFlTeam * kFlLds];  // per chunk: ring, halo buffer, a zero
+  __shared__ FlProg progs[kFlTeam];
+  __shared__ int free_word, spare[kFlTeam * kWave];
+  // a workgroup's waves are dealt to the CU's four SIMDs in turn: each chunk's
+  // jobs are rotated by one against the last's, so that every SIMD gets one
+  // compute wave
+  const int team = __builtin_amdgcn_readfirstlane((int)threadIdx.x / (4 * kWave));
+  const int wave = (__builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave) - team) & 3;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int c = blockIdx.x * kFlTeam + team;
   const int k0 = __builtin_amdgcn_readfirstlane(cstep[c]);
-  const int ns = __builtin_amdgcn_readfirstlane(cstep[c + 1]) - k0;
-  const int q0 = wptr[k0];
-  const int nw = wptr[k0 + ns] - q0;
-  constexpr int nt = kBlock + kWave;
-  for (int i = threadIdx.x; i < (int)gridDim.x; i += nt) seen[i] = -1;
-  for (int i = threadIdx.x; i <= ns; i += nt) {
-    tsptr[i] = sptr[k0 + i];
-    twptr[i] = wptr[k0 + i] - q0;
-    if (i < ns) tslev[i] = slev[k0 + i];
+  const int ns = __builtin_amdgcn_readfirstlane(cstep[c + 1]) - k0;  // a multiple of kFlGroup
+  const unsigned tag = (unsigned)__builtin_amdgcn_readfirstlane((int)*epoch);
+  VT *vals = all + team * kFlLds;
+  FlProg &prog = progs[team];
+  if (threadIdx.x < kFlTeam) {
+    progs[threadIdx.x] = FlProg{0, 0, 0, 0, 0, 0};
+    all[threadIdx.x * kFlLds + kFlZero] = VT(0);
   }
-  for (int i = threadIdx.x; i < nw; i += nt) {
-    twchk[i] = wchk[q0 + i];
-    twlev[i] = wlev[q0 + i];
-  }
-  if (threadIdx.x == 0) {
-    failed = 0;
-    must_wait = 0;
-  }
+  if (threadIdx.x == 0) free_word = 0x7fffffff;
   __syncthreads();
-  const int tfirst = tsptr[0];
-  const int lane = (int)threadIdx.x - kBlock;  // prefetch wave lane
-  // prefetch wave: step rel's records into its slot (for rel >= ns a
-  // harmless copy of the chunk's first ones, so every step issues as many)
-  auto copy_records = [&](int rel) {
-    const int t0 = rel < ns ? tsptr[rel] : tfirst;
-    char *slot = slots + (rel % NS) * SLOT;
-    const char *src = rec + (size_t)t0 * R::bytes + lane * 16;
-#pragma unroll
-    for (int i = 0; i < R::dma; ++i)
-      __builtin_amdgcn_global_load_lds((global_void_t *)(src + i * 1024),
-                                       (lds_void_t *)(slot + i * 1024), 16, 0, 0);
-    const char *xs = reinterpret_cast<const char *>(xc + t0) + lane * 4;
-#pragma unroll
-    for (int i = 0; i < XB / (kWave * 4); ++i)
-      __builtin_amdgcn_global_load_lds((global_void_t *)(xs + i * 256),
-                                       (lds_void_t *)(slot + kBlock * R::bytes + i * 256), 4, 0,
-                                       0);
+  auto fail = [&]() {
+    if (lane < kFlTeam) fl_st(&progs[lane].failed, -1);
+    if (lane == 0)
+      __hip_atomic_store(&state[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
-  if (pf) {
+  VT *const xk = xc + (size_t)k0 * kWave;
+  const __amdgpu_buffer_rsrc_t box = fl_buffer(inbox, inbox_bytes);
+  if (wave == 0) {
+    __builtin_amdgcn_s_setprio(3);
+    const __amdgpu_buffer_rsrc_t rb =
+        fl_buffer(rec + (size_t)k0 * FlRec<AT>::bytes, (ns + kFlGroup) * FlRec<AT>::bytes);
+    const __amdgpu_buffer_rsrc_t xb =
+        fl_buffer(xk, (ns + kFlGroup) * kWave * (int)sizeof(VT));
+    // this lane's progress word (see FlLane) and where it publishes
+    const int *word = lane == FL_HALO     ? &prog.hready
+                      : lane == FL_SIB    ? &progs[team ^ 1].cdone
+                      : lane == FL_X      ? &prog.xdone
+                      : lane == FL_Y      ? &prog.ydone
+                      : lane == FL_FAILED ? &prog.failed
+                                          : &free_word;
+    int *const out = lane == FL_HALO   ? &prog.hcons
+                     : lane == FL_DONE ? &prog.cdone
+                                       : &spare[team * kWave + lane];
+    FlRec<AT> R[kFlGroup];
+    VT X[kFlGroup];
 #pragma unroll
-    for (int r = 0; r < D; ++r) copy_records(r);
-    __builtin_amdgcn_s_waitcnt(vmcnt_only((D - 1) * PER));  // step 0's slot
-  }
-  for (int rel = 0; rel < ns; ++rel) {
-    if (threadIdx.x < kWave) {  // compute wave 0: are the step's waits already satisfied?
-      bool ready = true;
-      for (int q = twptr[rel] + (int)threadIdx.x; q < twptr[rel + 1]; q += kWave)
-        ready = ready && seen[twchk[q]] >= twlev[q];
-      const bool all = __builtin_amdgcn_ballot_w64(!ready) == 0;
-      if (threadIdx.x == 0) must_wait = !all;
+    for (int j = 0; j < kFlGroup; ++j) {
+      R[j].load(rb, lane * 16, j * FlRec<AT>::bytes);
+      fl_load_x(xb, lane, j, &X[j]);
     }
-    lds_barrier();  // must_wait set; the previous step's ring entries and slot done
-    if (__builtin_amdgcn_readfirstlane(must_wait)) {
-      // about to block: first publish the previous step (its stores complete),
-      // so that no chunk ever waits on work that is done but unpublished
-      if (!pf) __builtin_amdgcn_s_waitcnt(0);
-      lds_barrier();
-      if (threadIdx.x == 0 && rel > 0)
-        __hip_atomic_store(&progress[c], tslev[rel - 1], __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-      if (threadIdx.x < kWave) {  // wave 0: the step's waits, one lane per producer
-        int ok = 1;
-        const int qe = twptr[rel + 1];
-        for (int q = twptr[rel] + (int)threadIdx.x; q < qe; q += kWave) {
-          const int pc = twchk[q], need = twlev[q];
-          if (seen[pc] >= need) continue;
+    // every load complete here, so that the waits inside the loop (which count
+    // loads in flight) follow the loop's own order and leave the other steps'
+    // loads in flight
+#pragma unroll
+    for (int j = 0; j < kFlGroup; ++j) {
+      asm volatile("" ::"v"(R[j].c), "v"(R[j].pv), "v"(X[j]));
+#pragma unroll
+      for (int d = 0; d < 4; ++d) asm volatile("" ::"v"(R[j].val(d)));
+    }
+    int seen = lane < FL_DONE ? 0 : 0x7fffffff;  // the lane's progress word, as last seen
+    // (a failed wait ends the loop with its group: leaving it inside would
+    // merge the steps' load counts and make every wait a full one)
+    int dead = 0;
+    for (int k = 0; k < ns && !dead; k += kFlGroup) {
+#pragma unroll
+      for (int j = 0; j < kFlGroup; ++j) {
+        const int need = (int)R[j].c.z;
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(seen < need) != 0, 0)) {
           unsigned spins = 0;
-          int v = __hip_atomic_load(&progress[pc], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          while (v < need) {
-            if (++spins > kChSpinLimit ||
-                __hip_atomic_load(&state[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-              ok = 0;
-              break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-            v = __hip_atomic_load(&progress[pc], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          do {
+            seen = fl_ld(word);
+            dead |= __builtin_amdgcn_readlane(seen, FL_FAILED) | (++spins > 4 * kFlSpins);
+          } while (!dead && __builtin_amdgcn_ballot_w64(seen < need) != 0);
+        }
+        fl_fence();
+        const char *const lds = reinterpret_cast<const char *>(all);
+        auto at = [&](unsigned o) { return *reinterpret_cast<const VT *>(lds + o); };
+        VT yv[4];
+        yv[0] = at(R[j].c.x & 0xffffu);
+        yv[1] = at(R[j].c.x >> 16);
+        yv[2] = at(R[j].c.y & 0xffffu);
+        yv[3] = at(R[j].c.y >> 16);
+        double acc = (double)X[j];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) acc -= R[j].val(d) * (double)yv[d];
+        const double piv = fl_f64(R[j].pv.x, R[j].pv.y);
+        double q = fl_div(acc, piv, fl_f64(R[j].pv.z, R[j].pv.w));
+        // outside the refined division's range (a zero among them): divide
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(fl_out(acc, R[j].c.w)) != 0, 0)) {
+          fl_fence();  // (kept a branch)
+          q = acc / piv;
+        }
+        vals[k % kFlRing * kWave + j * kWave + lane] = (VT)q;
+        fl_fence();
+        fl_st(out, need);
+        // (past the chunk's end: the following blocks, which are allocated)
+        __builtin_amdgcn_sched_barrier(0);
+        R[j].load(rb, lane * 16, (k + j + kFlGroup) * FlRec<AT>::bytes);
+        fl_load_x(xb, lane, k + j + kFlGroup, &X[j]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (dead) fail();
+  } else if (wave == 1) {
+    const int h0 = __builtin_amdgcn_readfirstlane(hbase[c]);
+    const int nh = __builtin_amdgcn_readfirstlane(hbase[c + 1]) - h0;
+    // Two looks at the inbox are in flight at a time, each at the two windows
+    // of 64 entries from the first one missing when it was issued: a value is
+    // seen half a round trip after it can be, not up to a whole one.
+    int base = 0, at[2];
+    FlBoxed<VT> w[2][2];
+    auto look = [&](int s) {
+      at[s] = base;
+      // (past the inbox's end the buffer reads as zero, which is no tag)
+      w[s][0].load(box, h0 + base + lane);
+      w[s][1].load(box, h0 + base + kWave + lane);
+    };
+    if (nh > 0) {
+      look(0);
+      look(1);
+    }
+    unsigned spins = 0;
+    while (base < nh) {
+      bool stop = false;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int lim = min(nh, __builtin_amdgcn_readfirstlane(fl_ld(&prog.hcons)) + kFlHalo);
+        const int i = at[s] + lane, i2 = i + kWave;
+        const bool got = i < base || (i < lim && w[s][0].is(tag));
+        const bool got2 = i2 < base || (i2 < lim && w[s][1].is(tag));
+        const unsigned long long m = ~__builtin_amdgcn_ballot_w64(got);
+        const unsigned long long m2 = ~__builtin_amdgcn_ballot_w64(got2);
+        const int to = at[s] + (m ? __builtin_ctzll(m) : m2 ? kWave + __builtin_ctzll(m2) : 2 * kWave);
+        if (to > base) {  // the leading run of values that are there
+          VT *const buf = vals + kFlRing * kWave;
+          if (i >= base && i < to) buf[i % kFlHalo] = w[s][0].value();
+          if (i2 >= base && i2 < to) buf[i2 % kFlHalo] = w[s][1].value();
+          fl_fence();
+          base = to;
+          if (lane == 0) fl_st(&prog.hready, base);
+          spins = 0;
+        } else {
+          // (a chunk that the solve has not reached yet leaves the memory to
+          // the others)
+          if (spins > 8) __builtin_amdgcn_s_sleep(12);
+          if (fl_ld(&prog.failed)) stop = true;
+          if (++spins > kFlSpins) {
+            fail();
+            stop = true;
+          } else if ((spins & 63u) == 0 &&
+                     __hip_atomic_load(&state[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+            if (lane < kFlTeam) fl_st(&progs[lane].failed, -1);
+            stop = true;
           }
-          seen[pc] = v;
-          if (!ok) break;
         }
-        if (!ok) {
-          __hip_atomic_store(&state[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          failed = 1;
-        }
+        look(s);
       }
-      lds_barrier();
-      if (__builtin_amdgcn_readfirstlane(failed)) break;
+      if (__builtin_amdgcn_readfirstlane((int)stop)) break;
     }
-    if (pf) {
-      copy_records(rel + D);
-      // the next step's slot is complete; later ones may still be in flight
-      __builtin_amdgcn_s_waitcnt(vmcnt_only((D - 1) * PER));
-    } else {
-      // wave 0: poll a producer of the next step not yet seen far enough,
-      // issued before this step's loads and read after them
-      int poll_pc = -1, poll_v = 0;
-      if (threadIdx.x < kWave && rel + 1 < ns) {
-        const int q = twptr[rel + 1] + (int)threadIdx.x;
-        if (q < twptr[rel + 2] && seen[twchk[q]] < twlev[q]) {
-          poll_pc = twchk[q];
-          poll_v = __hip_atomic_load(&progress[poll_pc], __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
+  } else if (wave == 2) {
+    const int e0 = __builtin_amdgcn_readfirstlane(ebase[c]);
+    const int ne = __builtin_amdgcn_readfirstlane(ebase[c + 1]) - e0;
+    const int2 none{0x7fffffff, 0};
+    // the list is read kFlAhead windows ahead (a window is a few steps long,
+    // less than a trip to memory)
+    int2 win[kFlAhead];
+#pragma unroll
+    for (int w = 0; w < kFlAhead; ++w)
+      win[w] = w * kWave + lane < ne ? exps[e0 + w * kWave + lane] : none;
+    if (ne == 0 && lane == 0) fl_st(&prog.xdone, 0x3fffffff);
+    unsigned spins = 0;
+    bool stop = false;
+    for (int b = 0; b < ne && !stop; b += kWave) {
+      const int2 e = win[0];  // {local record, inbox entry}, ascending records
+#pragma unroll
+      for (int w = 0; w + 1 < kFlAhead; ++w) win[w] = win[w + 1];
+      const int nb = b + kFlAhead * kWave + lane;
+      win[kFlAhead - 1] = nb < ne ? exps[e0 + nb] : none;
+      bool pending = e.x != none.x;
+      for (;;) {
+        const int cd = __builtin_amdgcn_readfirstlane(fl_ld(&prog.cdone));
+        fl_fence();
+        const bool now = pending && e.x < cd * kWave;
+        const unsigned long long any = __builtin_amdgcn_ballot_w64(now);
+        if (now) {
+          fl_put(box, e.y, tag, vals[e.x % (kFlRing * kWave)]);
+          pending = false;
+        }
+        const unsigned long long left = __builtin_amdgcn_ballot_w64(pending);
+        // the first record still to be exported (of this window or the next)
+        const int t = left ? __builtin_amdgcn_readlane(e.x, __builtin_ctzll(left))
+                           : __builtin_amdgcn_readfirstlane(win[0].x);
+        fl_fence();
+        if (lane == 0) fl_st(&prog.xdone, t == none.x ? 0x3fffffff : t / kWave);
+        if (!left) break;
+        if (any) {
+          spins = 0;
+        } else {
+          if (fl_ld(&prog.failed)) stop = true;
+          if (++spins > 4 * kFlSpins) {
+            fail();
+            stop = true;
+          }
+          if (__builtin_amdgcn_readfirstlane((int)stop)) break;
+          __builtin_amdgcn_s_sleep(1);
         }
       }
-      const bool has_row = tsptr[rel] + p < tsptr[rel + 1];
-      int row = 0;
-      VT r = VT(0);
-      if (has_row) {
-        const char *slot = slots + (rel % NS) * SLOT;
-        const int *ri = reinterpret_cast<const int *>(slot + p * R::bytes);
-        const AT *rd = reinterpret_cast<const AT *>(slot + p * R::bytes);
-        int cc[W];
-        VT yv[W];
-#pragma unroll
-        for (int j = 0; j < W; ++j) cc[j] = ri[j];
-#pragma unroll
-        for (int j = 0; j < W; ++j)  // the dependencies on y first: one wait for all
-          yv[j] = cc[j] >= 0 ? sf_load(y + cc[j]) : VT(0);
-        row = ri[R::row];
-        const VT xr = reinterpret_cast<const VT *>(slot + kBlock * R::bytes)[p];
-        const double piv = (double)rd[R::piv];
-#pragma unroll
-        for (int j = 0; j < W; ++j)
-          if (cc[j] < -1) yv[j] = ring[-(cc[j] + 2)];
-        double acc = (double)xr;
-#pragma unroll
-        for (int j = 0; j < W; ++j) {
-          if (cc[j] == -1) break;
-          acc -= (double)rd[R::val + j] * (double)yv[j];
-        }
-        r = (VT)(acc / piv);
-        ring[(rel % kChRing) * kBlock + p] = r;
-      }
-      if (poll_pc >= 0) atomicMax(&seen[poll_pc], poll_v);
-      if (has_row) {
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        sf_store(y + row, r);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      }
-      // The loads of this step were consumed above, so only stores are in
-      // flight, and stores complete in order: all but this step's store
-      // (present when one of the wave's lanes has a row) are complete, the
-      // previous step's included.
-      if (__builtin_amdgcn_ballot_w64(has_row) != 0)
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(1));
-      else
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
     }
-    lds_barrier();  // ring entries written; every wave's previous-step stores complete
-    if (threadIdx.x == 0 && rel > 0)
-      __hip_atomic_store(&progress[c], tslev[rel - 1], __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    bool stop = false;
+    for (int k = 0; k < ns; k += kFlGroup) {
+      unsigned spins = 0;
+      while (__builtin_amdgcn_readfirstlane(fl_ld(&prog.cdone)) < k + kFlGroup) {
+        if (fl_ld(&prog.failed)) stop = true;
+        if (++spins > 4 * kFlSpins) {
+          fail();
+          stop = true;
+        }
+        if (__builtin_amdgcn_readfirstlane((int)stop)) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      if (__builtin_amdgcn_readfirstlane((int)stop)) break;
+      fl_fence();
+      VT v[kFlGroup];
+#pragma unroll
+      for (int j = 0; j < kFlGroup; ++j) v[j] = vals[k % kFlRing * kWave + j * kWave + lane];
+      fl_fence();
+      if (lane == 0) fl_st(&prog.ydone, k + kFlGroup);
+#pragma unroll
+      for (int j = 0; j < kFlGroup; ++j) st_nt(xk + (k + j) * kWave + lane, v[j]);
+    }
   }
-  // the last step: its stores complete, then its level published
-  if (!pf) __builtin_amdgcn_s_waitcnt(0);
-  lds_barrier();
-  if (threadIdx.x == 0 && ns > 0 && !__builtin_amdgcn_readfirstlane(failed))
-    __hip_atomic_store(&progress[c], tslev[ns - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (pf) __builtin_amdgcn_s_waitcnt(0);  // no copy into LDS outlives the workgroup
 }
 
-// xc[t] = x[row of schedule position t]: the right-hand side in the chunked
-// schedule's order, for k_tri_chunks' prefetch.
+// xc[t] = x[map[t]]: the right-hand side in the order the compute waves read
+// it (padding, map < 0, keeps the 1.0 it was given), and the next solve's tag.
 // The rows of neighbouring schedule positions share lines of x, so each XCD
 // (workgroups are dealt to the 8 XCDs round-robin) sweeps one contiguous
 // eighth of the positions: its workgroups then read the same lines out of
 // their own L2.  The grid is a multiple of 8.
 template <class VT>
-__global__ __launch_bounds__(kBlock) void k_ch_gather(int n, const int *__restrict__ crow,
+__global__ __launch_bounds__(kBlock) void k_fl_gather(int n, const int *__restrict__ map,
                                                       const VT *__restrict__ x,
-                                                      VT *__restrict__ xc,
+                                                      VT *__restrict__ xc, unsigned *epoch,
+                                                      const int *__restrict__ done) {
+  if (done && *done) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *epoch += 1u;
+  const int xcd = blockIdx.x & 7, per = gridDim.x >> 3;
+  const long long lo = (long long)n * xcd / 8, hi = (long long)n * (xcd + 1) / 8;
+  for (long long t = lo + (long long)(blockIdx.x >> 3) * kBlock + threadIdx.x; t < hi;
+       t += (long long)per * kBlock) {
+    const int row = ld_nt(map + t);  // the map and xc are streamed; x lines are reused
+    if (row >= 0) st_nt(xc + t, x[row]);
+  }
+}
+
+// y[i] = xc[pos[i]]: a solve's results in row order (the same walk).
+template <class VT>
+__global__ __launch_bounds__(kBlock) void k_fl_spread(int n, const int *__restrict__ pos,
+                                                      const VT *__restrict__ xc,
+                                                      VT *__restrict__ y,
                                                       const int *__restrict__ done) {
   if (done && *done) return;
   const int xcd = blockIdx.x & 7, per = gridDim.x >> 3;
   const long long lo = (long long)n * xcd / 8, hi = (long long)n * (xcd + 1) / 8;
-  for (long long t = lo + (long long)(blockIdx.x >> 3) * kBlock + threadIdx.x; t < hi;
-       t += (long long)per * kBlock)
-    st_nt(xc + t, x[ld_nt(crow + t)]);  // the map and xc are streamed; x lines are reused
+  for (long long i = lo + (long long)(blockIdx.x >> 3) * kBlock + threadIdx.x; i < hi;
+       i += (long long)per * kBlock)
+    st_nt(y + i, xc[ld_nt(pos + i)]);
 }
 
-// The records of the chunked schedule for one set of values (k_tri_chunks).
-template <int W, class AT>
-__global__ __launch_bounds__(kBlock) void k_ch_pack(int n, const int *__restrict__ cmap,
+// comp[t] = pos[map[t]]: a schedule's right-hand sides taken from another
+// schedule's results.
+__global__ __launch_bounds__(kBlock) void k_fl_compose(int n, const int *__restrict__ map,
+                                                       const int *__restrict__ pos,
+                                                       int *__restrict__ comp) {
+  for (int t = blockIdx.x * kBlock + threadIdx.x; t < n; t += gridDim.x * kBlock)
+    comp[t] = map[t] < 0 ? -1 : pos[map[t]];
+}
+
+// The records for one set of values, and xc's padding.
+template <class AT, class VT>
+__global__ __launch_bounds__(kBlock) void k_fl_pack(int n, const int *__restrict__ cmap,
                                                     const int4 *__restrict__ desc,
                                                     const int *__restrict__ ja,
                                                     const AT *__restrict__ a,
-                                                    const int *__restrict__ code,
-                                                    char *__restrict__ rec) {
-  using R = ChRec<W, AT>;
+                                                    const int2 *__restrict__ code,
+                                                    const int2 *__restrict__ need,
+                                                    const int *__restrict__ step_in_chunk,
+                                                    char *__restrict__ rec,
+                                                    VT *__restrict__ xc) {
   for (int t = blockIdx.x * kBlock + threadIdx.x; t < n; t += gridDim.x * kBlock) {
-    int *ri = reinterpret_cast<int *>(rec + (size_t)t * R::bytes);
-    AT *rd = reinterpret_cast<AT *>(rec + (size_t)t * R::bytes);
-    const int4 d = desc[cmap[t]];
-#pragma unroll
-    for (int j = 0; j < W; ++j) ri[j] = code[(size_t)t * W + j];
-    ri[R::row] = d.x;
-    int k = 0;
-    AT piv = AT(0);
-    for (int e = d.y; e < d.z; ++e) {
-      if (ja[e] == d.x)
-        piv = a[e];
-      else if (k < W)
-        rd[R::val + k++] = a[e];
+    const int k = t / kWave, l = t % kWave;
+    char *blk = rec + (size_t)k * FlRec<AT>::bytes;
+    AT v[4] = {AT(0), AT(0), AT(0), AT(0)};
+    AT piv = AT(1);
+    const int m = cmap[t];
+    if (m >= 0) {
+      const int4 d = desc[m];
+      int j = 0;
+      for (int e = d.y; e < d.z; ++e) {
+        if (ja[e] == d.x)
+          piv = a[e];
+        else if (j < 4)
+          v[j++] = a[e];
+      }
     }
-    for (; k < W; ++k) rd[R::val + k] = AT(0);
-    rd[R::piv] = piv;
+    if (m < 0) xc[t] = VT(1);
+    const int2 ce = code[t];  // LDS entries -> byte offsets
+    const int2 cd{(int)((unsigned)ce.x * sizeof(VT)), (int)((unsigned)ce.y * sizeof(VT))};
+    const int2 nd = need[k];
+    const int low = -0x7fffffff;
+    const int step = step_in_chunk[k];
+    const int word = l == FL_HALO             ? nd.x
+                     : l == FL_SIB            ? nd.y
+                     : l == FL_X || l == FL_Y ? step - kFlRing + 1
+                     : l == FL_FAILED         ? 0
+                     : l == FL_DONE           ? step + 1
+                                              : low;
+    const double dp = (double)piv;
+    const bool out = fl_out(dp, kFlBase);
+    reinterpret_cast<int4 *>(blk)[l] = int4{cd.x, cd.y, word, (int)(out ? kFlNever : kFlBase)};
+    const double2 pv{dp, out ? 0.0 : 1.0 / dp};
+    if constexpr (sizeof(AT) == 8) {
+      double2 *p = reinterpret_cast<double2 *>(blk + kWave * 16);
+      p[l] = double2{v[0], v[1]};
+      p[kWave + l] = double2{v[2], v[3]};
+      p[2 * kWave + l] = pv;
+    } else {
+      reinterpret_cast<float4 *>(blk + kWave * 16)[l] = float4{v[0], v[1], v[2], v[3]};
+      reinterpret_cast<double2 *>(blk + kWave * 32)[l] = pv;
+    }
   }
-}
-
-int *ch_progress() {
-  static DevBufPtr buf;
-  if (!buf) buf = dev_alloc(kChMax * sizeof(int));
-  return buf && buf->p ? buf->as<int>() : nullptr;
 }
 
 int *sf_state() {  // [unused, error flag, unused, unused]
@@ -685,21 +886,22 @@ void forget_tri_plans(const void *p) {
 
 // ------------------------------------------------ chunked schedule (host)
 //
-// A partition of the rows into at most one chunk per CU is chosen among a few
-// candidates by simulating the pipeline: every step of a chunk costs one unit
-// and every wait on another chunk kHopCost more (a value crossing between
-// workgroups goes through memory).  Candidates: contiguous ranges in solve
-// order, and for matrices whose column offsets take few values (grids in
-// lexicographic order) tiles over two of the offset strides, which keep the
-// long dependency chains inside one chunk (e.g. the 256^3 grid's chains along
-// z: 16 x 16 x 256 tiles cross 30 chunk boundaries on the critical path
-// against 255 for z-slabs).
-constexpr int kHopCost = 6;
+// A partition of the rows into at most kFlTeam chunks per CU is chosen among
+// a few candidates by simulating the pipeline: every step of a chunk costs
+// one unit, a value from another chunk of the workgroup kSibCost more, one
+// from another workgroup kHopCost more (it goes through memory).  Candidates:
+// contiguous ranges in solve order, and for matrices whose column offsets
+// take few values (grids in lexicographic order) tiles over two of the offset
+// strides, which keep the long dependency chains inside one chunk (e.g. the
+// 256^3 grid's chains along z: 8 x 8 x 256 tiles, whose levels fill a step of
+// 64 rows, 2 x 2 tiles to a workgroup).
+constexpr int kHopCost = 18;
+constexpr int kSibCost = 1;
 
 // f(t0, t1) over contiguous ranges covering [0, n), one per host thread.
 template <class F>
-static void host_ranges(int n, F f) {
-  const int T = std::max(1, std::min(host_threads(), n / 65536 + 1));
+static void host_ranges(int n, F f, int grain = 65536) {
+  const int T = std::max(1, std::min(host_threads(), n / grain + 1));
   std::vector<std::thread> th;
   for (int k = 1; k < T; ++k)
     th.emplace_back(f, (int)((long)n * k / T), (int)((long)n * (k + 1) / T));
@@ -708,105 +910,113 @@ static void host_ranges(int n, F f) {
 }
 
 struct ChunkSched {
-  int G = 0;
-  std::vector<int> cbase, crow, cmap;  // rows in (chunk, level, row) order
-  std::vector<int> cstep, sptr, slev, wptr, wchk, wlev;
+  int G = 0;  // chunks, a multiple of kFlTeam; kFlTeam consecutive ones share a workgroup
+  std::vector<int> cstep;        // first step of each chunk (+ end), multiples of kFlGroup
+  std::vector<int> crow, cmap;   // row and level-order position of each record, -1: padding
+  std::vector<int> pos;          // record of each row (64 * step + lane)
+  std::vector<int> slev;         // level of each step, kFlPadLevel: padding
+  std::vector<int> owner;        // chunk of each step
   long long cost = -1;
+  // How step k of chunk c gets the result of step kd: 0 through c's inbox, 1
+  // from its own ring, 2 from the ring of another chunk of the workgroup.  The
+  // step that overwrites kd's ring entries waits for step k (see need below);
+  // that step has a higher level than k here, so all waits, like the
+  // dependencies, lead from lower to higher levels and none can close a cycle.
+  int how(int c, int k, int kd) const {
+    const int cd = owner[(size_t)kd];
+    if (cd == c) return k - kd < kFlRing ? 1 : 0;
+    if (cd / kFlTeam != c / kFlTeam) return 0;
+    const int over = kd + kFlRing;
+    return over >= cstep[(size_t)cd + 1] || slev[(size_t)k] < slev[(size_t)over] ? 2 : 0;
+  }
 };
+constexpr int kFlPadLevel = 0x7fffffff;
 
-// Steps and pruned waits of a partition; false when a chunk's step holds
-// more than max_step rows.
+// The steps of a partition (each chunk's rows level by level, at most 64 rows
+// a step) and its simulated length; false when padding would more than
+// quadruple the records.
 static bool sched_build(ChunkSched &S, const std::vector<int> &chunk_of, int G,
                         const std::vector<int> &ia, const std::vector<int> &ja,
-                        const std::vector<int> &level, const std::vector<int> &order,
-                        int max_step) {
+                        const std::vector<int> &level, const std::vector<int> &order) {
   const int n = (int)chunk_of.size();
   S.G = G;
-  S.cbase.assign((size_t)G + 1, 0);
-  for (int i = 0; i < n; ++i) S.cbase[(size_t)chunk_of[(size_t)i] + 1]++;
-  for (int c = 0; c < G; ++c) S.cbase[(size_t)c + 1] += S.cbase[(size_t)c];
-  S.crow.assign((size_t)n, 0);
-  S.cmap.assign((size_t)n, 0);
-  std::vector<int> fill(S.cbase.begin(), S.cbase.end() - 1);
-  for (int t = 0; t < n; ++t) {  // order is (level, row): bucket stably by chunk
-    const int i = order[(size_t)t];
-    const int pos = fill[(size_t)chunk_of[(size_t)i]]++;
-    S.crow[(size_t)pos] = i;
-    S.cmap[(size_t)pos] = t;
+  std::vector<int> cbase((size_t)G + 1, 0);
+  for (int i = 0; i < n; ++i) cbase[(size_t)chunk_of[(size_t)i] + 1]++;
+  for (int c = 0; c < G; ++c) cbase[(size_t)c + 1] += cbase[(size_t)c];
+  std::vector<int> at((size_t)n);  // level-order positions by (chunk, level, row)
+  {
+    std::vector<int> fill(cbase.begin(), cbase.end() - 1);
+    for (int t = 0; t < n; ++t)
+      at[(size_t)fill[(size_t)chunk_of[(size_t)order[(size_t)t]]]++] = t;
   }
+  const long long most = 4ll * n + 65536;
   S.cstep.assign((size_t)G + 1, 0);
-  S.sptr.clear();
   S.slev.clear();
-  S.wptr.clear();
-  S.wchk.clear();
-  S.wlev.clear();
-  std::vector<int> running((size_t)G, -1), req((size_t)G, -1), touched, prod;
+  S.crow.clear();
+  S.cmap.clear();
+  S.crow.reserve((size_t)n + (size_t)n / 8);
+  S.cmap.reserve((size_t)n + (size_t)n / 8);
+  S.pos.assign((size_t)n, 0);
+  auto pad = [&](int upto) {
+    S.crow.resize((size_t)upto, -1);
+    S.cmap.resize((size_t)upto, -1);
+  };
   for (int c = 0; c < G; ++c) {
     S.cstep[(size_t)c] = (int)S.slev.size();
-    prod.clear();
-    for (int t = S.cbase[(size_t)c]; t < S.cbase[(size_t)c + 1];) {
-      const int lv = level[(size_t)S.crow[(size_t)t]];
-      int u = t;
-      touched.clear();
-      while (u < S.cbase[(size_t)c + 1] && level[(size_t)S.crow[(size_t)u]] == lv) {
-        const int i = S.crow[(size_t)u];
-        for (int e = ia[i]; e < ia[i + 1]; ++e) {
-          const int d = ja[e];
-          if (d == i) continue;
-          const int cd = chunk_of[(size_t)d];
-          if (cd == c) continue;
-          if (req[(size_t)cd] < 0) touched.push_back(cd);
-          req[(size_t)cd] = std::max(req[(size_t)cd], level[(size_t)d]);
-        }
-        ++u;
+    for (int t = cbase[(size_t)c]; t < cbase[(size_t)c + 1];) {
+      const int lv = level[(size_t)order[(size_t)at[(size_t)t]]];
+      const int p0 = (int)S.slev.size() * kWave;
+      int l = 0;
+      for (; l < kWave && t < cbase[(size_t)c + 1]; ++l, ++t) {
+        const int m = at[(size_t)t], i = order[(size_t)m];
+        if (level[(size_t)i] != lv) break;
+        S.crow.push_back(i);
+        S.cmap.push_back(m);
+        S.pos[(size_t)i] = p0 + l;
       }
-      if (u - t > max_step) return false;
-      S.sptr.push_back(t);
       S.slev.push_back(lv);
-      S.wptr.push_back((int)S.wchk.size());
-      std::sort(touched.begin(), touched.end());
-      for (int cd : touched) {
-        if (req[(size_t)cd] > running[(size_t)cd]) {
-          if (running[(size_t)cd] < 0) prod.push_back(cd);
-          running[(size_t)cd] = req[(size_t)cd];
-          S.wchk.push_back(cd);
-          S.wlev.push_back(req[(size_t)cd]);
-        }
-        req[(size_t)cd] = -1;
-      }
-      t = u;
+      pad(p0 + kWave);
     }
-    for (int cd : prod) running[(size_t)cd] = -1;
+    while (S.slev.size() % kFlGroup) {
+      S.slev.push_back(kFlPadLevel);
+      pad((int)S.slev.size() * kWave);
+    }
+    if ((long long)S.crow.size() > most ||
+        (int)S.slev.size() - S.cstep[(size_t)c] > kFlMaxSteps)
+      return false;
   }
   const int nsteps = (int)S.slev.size();
   S.cstep[(size_t)G] = nsteps;
-  S.sptr.push_back(n);
-  S.wptr.push_back((int)S.wchk.size());
-  for (int c = 0; c < G; ++c) {  // the kernel's LDS tables
-    const int k0 = S.cstep[(size_t)c], k1 = S.cstep[(size_t)c + 1];
-    if (k1 - k0 > kChSteps || S.wptr[(size_t)k1] - S.wptr[(size_t)k0] > kChWaits) return false;
-  }
-  // pipeline simulation, steps taken in level order (every wait refers to a
-  // lower level, so its producer step is already timed)
-  int nlev = 0;
-  for (int v : S.slev) nlev = std::max(nlev, v + 1);
-  std::vector<int> lcnt((size_t)nlev + 1, 0), byl((size_t)nsteps), owner((size_t)nsteps);
+  S.owner.resize((size_t)nsteps);
   for (int c = 0; c < G; ++c)
-    for (int k = S.cstep[(size_t)c]; k < S.cstep[(size_t)c + 1]; ++k) owner[(size_t)k] = c;
-  for (int k = 0; k < nsteps; ++k) lcnt[(size_t)S.slev[(size_t)k] + 1]++;
+    for (int k = S.cstep[(size_t)c]; k < S.cstep[(size_t)c + 1]; ++k) S.owner[(size_t)k] = c;
+  // pipeline simulation, steps taken in level order (a dependency has a lower
+  // level, so its step is already timed)
+  int nlev = 0;
+  for (int v : S.slev)
+    if (v != kFlPadLevel) nlev = std::max(nlev, v + 1);
+  std::vector<int> lcnt((size_t)nlev + 1, 0), byl;
+  int real = 0;
+  for (int v : S.slev)
+    if (v != kFlPadLevel) lcnt[(size_t)v + 1]++, ++real;
   for (int l = 0; l < nlev; ++l) lcnt[(size_t)l + 1] += lcnt[(size_t)l];
-  for (int k = 0; k < nsteps; ++k) byl[(size_t)lcnt[(size_t)S.slev[(size_t)k]]++] = k;
-  std::vector<long long> tdone((size_t)nsteps, 0);
-  long long cost = 0;
+  byl.resize((size_t)real);
+  for (int k = 0; k < nsteps; ++k)
+    if (S.slev[(size_t)k] != kFlPadLevel) byl[(size_t)lcnt[(size_t)S.slev[(size_t)k]]++] = k;
+  std::vector<int> tdone((size_t)nsteps, 0);
+  const int extra[3] = {kHopCost, 0, kSibCost};
+  int cost = 0;
   for (int k : byl) {
-    const int c = owner[(size_t)k];
-    long long t0 = k > S.cstep[(size_t)c] ? tdone[(size_t)k - 1] : 0;
-    for (int q = S.wptr[(size_t)k]; q < S.wptr[(size_t)k + 1]; ++q) {
-      const int cd = S.wchk[(size_t)q], L = S.wlev[(size_t)q];
-      // the producer's first step at a level >= L
-      const int *b0 = S.slev.data() + S.cstep[(size_t)cd], *b1 = S.slev.data() + S.cstep[(size_t)cd + 1];
-      const int kk = (int)(std::lower_bound(b0, b1, L) - S.slev.data());
-      t0 = std::max(t0, tdone[(size_t)kk] + kHopCost);
+    const int c = S.owner[(size_t)k];
+    int t0 = k > S.cstep[(size_t)c] ? tdone[(size_t)k - 1] : 0;
+    for (int l = 0; l < kWave; ++l) {
+      const int i = S.crow[(size_t)k * kWave + l];
+      if (i < 0) break;
+      for (int e = ia[i]; e < ia[i + 1]; ++e) {
+        if (ja[e] == i) continue;
+        const int kd = S.pos[(size_t)ja[e]] / kWave;
+        t0 = std::max(t0, tdone[(size_t)kd] + extra[S.how(c, k, kd)]);
+      }
     }
     tdone[(size_t)k] = t0 + 1;
     cost = std::max(cost, t0 + 1);
@@ -815,54 +1025,103 @@ static bool sched_build(ChunkSched &S, const std::vector<int> &chunk_of, int G,
   return true;
 }
 
-// The chunked schedule of a triangle whose rows hold at most 8 entries.
+// The chunked schedule of a triangle whose rows hold at most 4 entries beside
+// the pivot (a record's dependencies).
 static void tri_chunks_build(TriPlan &p, const std::vector<int> &ia, const std::vector<int> &ja,
                              const std::vector<int> &level, const std::vector<int> &order) {
   const int n = p.n;
-  if (n <= 0 || p.max_row > 5 || !p.has_diag) return;
-  const int Gmax = std::min({device_cus(), kChMax, std::max(1, n / kChMinRows)});
+  if (n <= 0 || p.max_row > 5 || !p.has_diag || !sf_state()) return;
+  const int Gmax = std::max(1, device_cus() * kFlPerCu) * kFlTeam;
   const bool lower = p.lower;
   auto pos_of = [&](int i) { return lower ? i : n - 1 - i; };
-  std::vector<std::pair<std::vector<int>, int>> cands;
-  {  // contiguous ranges in solve order
-    int C = (n + Gmax - 1) / Gmax;
-    C = (C + 63) / 64 * 64;
-    const int G = (n + C - 1) / C;
-    std::vector<int> co((size_t)n);
-    for (int i = 0; i < n; ++i) co[(size_t)i] = pos_of(i) / C;
-    cands.emplace_back(std::move(co), G);
-  }
-  {  // tiles over two offset strides
-    std::vector<int> offs;
-    for (int i = 0; i < n && offs.size() <= 16; ++i)
-      for (int e = ia[i]; e < ia[i + 1]; ++e) {
-        const int d = ja[e];
-        if (d == i) continue;
-        const int o = std::abs(i - d);
-        if (std::find(offs.begin(), offs.end(), o) == offs.end()) offs.push_back(o);
-      }
-    if (offs.size() <= 16) {
-      std::sort(offs.begin(), offs.end());
-      for (size_t x = 0; x < offs.size(); ++x)
-        for (size_t y = x + 1; y < offs.size(); ++y) {
-          const int Oa = offs[x], Ob = offs[y];
-          if (Oa < 2 || Ob % Oa || n % Ob) continue;
-          const int nb = Ob / Oa;  // extent of the second coordinate
-          for (int nI = 1; nI <= Gmax; nI *= 2) {
-            const int nJ = Gmax / nI;
-            if (nI > Oa || nJ > nb || nI * nJ < 2) continue;
-            const int Ti = (Oa + nI - 1) / nI, Tj = (nb + nJ - 1) / nJ;
-            const int gi = (Oa + Ti - 1) / Ti, gj = (nb + Tj - 1) / Tj;
-            std::vector<int> co((size_t)n);
-            for (int r = 0; r < n; ++r) {
-              const int ps = pos_of(r);
-              co[(size_t)r] = ((ps / Oa) % nb / Tj) * gi + (ps % Oa) / Ti;
+  // candidate partitions: {chunk rows of a contiguous range} or {strides and
+  // tile of a tiling}
+  struct Cand {
+    int C = 0, Oa = 0, nb = 0, Ti = 0, Tj = 0, gi = 0, gj = 0;
+    int wi = 1, wj = 1, hi = 0, hj = 0;
+    long est = 0;
+  };
+  std::vector<Cand> tiles, cands;
+  std::vector<int> offs;
+  for (int i = 0; i < n && offs.size() <= 16; ++i)
+    for (int e = ia[i]; e < ia[i + 1]; ++e) {
+      const int d = ja[e];
+      if (d == i) continue;
+      const int o = std::abs(i - d);
+      if (std::find(offs.begin(), offs.end(), o) == offs.end()) offs.push_back(o);
+    }
+  int line = 0;  // the longest offset that divides n: ranges aligned to it
+  if (offs.size() <= 16) {
+    std::sort(offs.begin(), offs.end());
+    for (size_t x = 0; x < offs.size(); ++x) {
+      if (offs[x] >= 2 && n % offs[x] == 0) line = offs[x];
+      for (size_t y = x + 1; y < offs.size(); ++y) {
+        const int Oa = offs[x], Ob = offs[y];
+        if (Oa < 2 || Ob % Oa || n % Ob) continue;
+        const int nb = Ob / Oa;  // extent of the second coordinate
+        for (int Ti = 2; Ti <= 64; Ti *= 2)
+          for (int Tj = 2; Tj <= 64; Tj *= 2) {
+            Cand t;
+            t.Oa = Oa;
+            t.nb = nb;
+            t.Ti = std::min(Ti, Oa);
+            t.Tj = std::min(Tj, nb);
+            t.gi = (Oa + t.Ti - 1) / t.Ti;
+            t.gj = (nb + t.Tj - 1) / t.Tj;
+            if ((Ti > 2 * Oa) || (Tj > 2 * nb)) continue;
+            const long sub = ((long)t.Ti * t.Tj + kWave - 1) / kWave;
+            for (int wi = 1; wi <= kFlTeam; wi *= 2) {  // tiles of a workgroup
+              t.wi = wi;
+              t.wj = kFlTeam / wi;
+              t.hi = (t.gi + t.wi - 1) / t.wi;
+              t.hj = (t.gj + t.wj - 1) / t.wj;
+              if ((long)t.hi * t.hj * kFlTeam > Gmax) continue;
+              t.est = (Oa + nb + n / Ob) * sub + (long)(t.hi + t.hj - 2) * kHopCost +
+                      (long)(t.gi - t.hi + t.gj - t.hj) * kSibCost;
+              tiles.push_back(t);
             }
-            cands.emplace_back(std::move(co), gi * gj);
           }
-        }
+      }
     }
   }
+  std::stable_sort(tiles.begin(), tiles.end(),
+                   [](const Cand &u, const Cand &v) { return u.est < v.est; });
+  if (tiles.size() > 3) tiles.resize(3);
+  auto ranges = [&](long C) {
+    C = std::max(1l, std::min(C, (long)n));
+    if ((n + C - 1) / C > Gmax) return;
+    for (const Cand &o : cands)
+      if (o.C == (int)C) return;
+    Cand t;
+    t.C = (int)C;
+    cands.push_back(t);
+  };
+  auto round64 = [](long v) { return (v + 63) / 64 * 64; };
+  ranges(round64((n + Gmax - 1) / Gmax));
+  if (tiles.empty()) {
+    for (int G = Gmax / 4; G >= 1; G /= 4) ranges(round64((n + G - 1) / G));
+    if (line)
+      for (long q = 16; q <= 64; q *= 2) ranges(q * line);
+    const size_t most = n > 2000000 ? 3 : 8;
+    if (cands.size() > most) cands.resize(most);
+  }
+  cands.insert(cands.end(), tiles.begin(), tiles.end());
+  auto chunk_fn = [&](const Cand &t, std::vector<int> &co) {
+    co.resize((size_t)n);
+    for (int r = 0; r < n; ++r) {
+      const int ps = pos_of(r);
+      if (t.C) {
+        co[(size_t)r] = ps / t.C;
+        continue;
+      }
+      const int ti = (ps % t.Oa) / t.Ti, tj = (ps / t.Oa) % t.nb / t.Tj;
+      co[(size_t)r] = ((tj / t.wj) * t.hi + ti / t.wi) * kFlTeam + tj % t.wj * t.wi + ti % t.wi;
+    }
+  };
+  auto chunks_of = [&](const Cand &t) {
+    return t.C ? ((n + t.C - 1) / t.C + kFlTeam - 1) / kFlTeam * kFlTeam
+               : t.hi * t.hj * kFlTeam;
+  };
   // the candidates are independent: one host thread each (the lowest cost
   // wins, ties to the earlier candidate, so the choice does not depend on
   // thread timing)
@@ -870,10 +1129,12 @@ static void tri_chunks_build(TriPlan &p, const std::vector<int> &ia, const std::
   {
     std::atomic<size_t> next{0};
     auto work = [&]() {
-      for (size_t ci; (ci = next.fetch_add(1)) < cands.size();)
-        if (!sched_build(built[ci], cands[ci].first, cands[ci].second, ia, ja, level, order,
-                         kChStepRows))
+      std::vector<int> co;
+      for (size_t ci; (ci = next.fetch_add(1)) < cands.size();) {
+        chunk_fn(cands[ci], co);
+        if (!sched_build(built[ci], co, chunks_of(cands[ci]), ia, ja, level, order))
           built[ci] = ChunkSched();
+      }
     };
     const int T = std::max(1, std::min(host_threads(), (int)cands.size()));
     std::vector<std::thread> th;
@@ -888,62 +1149,132 @@ static void tri_chunks_build(TriPlan &p, const std::vector<int> &ia, const std::
   if (cands.empty() || built[best_i].cost < 0) return;
   ChunkSched best = std::move(built[best_i]);
   built.clear();
-  if (getenv("LAP_SCHED_LOG"))
-    fprintf(stderr, "[lapgfx] %s triangle n=%d: chunked schedule %zu of %zu, %d chunks, %zu steps, "
-            "%zu waits, simulated length %lld (one launch per level: %d)\n",
-            lower ? "lower" : "upper", n, best_i, cands.size(), best.G, best.slev.size(),
-            best.wchk.size(), best.cost, p.nlevels);
-  const std::vector<int> &chunk_of = cands[best_i].first;
-  const int G = best.G;
-  // dependency codes of the off-diagonal entries, records in schedule order:
-  // -1 padding, >= 0 a row read from y, <= -2 the LDS ring slot -(code + 2)
-  // of a row of this chunk solved fewer than kChRing steps earlier
-  const int W = 4;  // off-diagonal entries per record
-  std::vector<int> lstep((size_t)n), lpos((size_t)n);  // local step and position of each row
-  for (int c = 0; c < G; ++c)
-    for (int k = best.cstep[(size_t)c]; k < best.cstep[(size_t)c + 1]; ++k)
-      for (int t = best.sptr[(size_t)k]; t < best.sptr[(size_t)k + 1]; ++t) {
-        lstep[(size_t)best.crow[(size_t)t]] = k - best.cstep[(size_t)c];
-        lpos[(size_t)best.crow[(size_t)t]] = t - best.sptr[(size_t)k];
-      }
-  std::vector<int> code((size_t)n * W, -1);
-  host_ranges(n, [&](int t0, int t1) {  // records are independent: contiguous ranges per thread
-    for (int t = t0; t < t1; ++t) {
-      const int i = best.crow[(size_t)t];
-      int k = 0;
-      for (int e = ia[i]; e < ia[i + 1]; ++e) {
-        const int d = ja[e];
-        if (d == i) continue;  // the pivot is kept apart
-        int cd = d;
-        if (chunk_of[(size_t)d] == chunk_of[(size_t)i] &&
-            lstep[(size_t)i] - lstep[(size_t)d] < kChRing)
-          cd = -(2 + (lstep[(size_t)d] % kChRing) * kChStepRows + lpos[(size_t)d]);
-        code[(size_t)t * W + k++] = cd;
+  const int G = best.G, nsteps = (int)best.slev.size();
+  // LDS entries of the dependencies: results in a ring of the workgroup are
+  // read there, any other one comes through the chunk's inbox, one entry per
+  // use, in the order the steps use them
+  std::vector<int> hcnt((size_t)G + 1, 0);
+  auto in_ring = [&](int c, int k, int d) {
+    return best.how(c, k, best.pos[(size_t)d] / kWave) != 0;
+  };
+  host_ranges(G, [&](int c0, int c1) {
+    for (int c = c0; c < c1; ++c) {
+      int h = 0;
+      for (int k = best.cstep[(size_t)c]; k < best.cstep[(size_t)c + 1]; ++k)
+        for (int l = 0; l < kWave; ++l) {
+          const int i = best.crow[(size_t)k * kWave + l];
+          if (i < 0) break;
+          for (int e = ia[i]; e < ia[i + 1]; ++e)
+            if (ja[e] != i && !in_ring(c, k, ja[e])) ++h;
+        }
+      hcnt[(size_t)c + 1] = h;
+    }
+  }, 8);
+  long long total = 0;
+  for (int c = 0; c < G; ++c) total += hcnt[(size_t)c + 1];
+  if (total > 0x7fffffell) return;  // the inbox stays below 2^31 bytes
+  for (int c = 0; c < G; ++c) hcnt[(size_t)c + 1] += hcnt[(size_t)c];
+  const size_t T = (size_t)nsteps * kWave;
+  std::vector<unsigned> code(2 * T);
+  std::vector<int> need(2 * (size_t)nsteps, 0), src((size_t)total);  // src: feeds an entry
+  host_ranges(G, [&](int c0, int c1) {
+    for (int c = c0; c < c1; ++c) {
+      int h = 0;
+      for (int k = best.cstep[(size_t)c]; k < best.cstep[(size_t)c + 1]; ++k) {
+        for (int l = 0; l < kWave; ++l) {
+          const size_t t = (size_t)k * kWave + l;
+          unsigned cd[4] = {kFlZero, kFlZero, kFlZero, kFlZero};
+          const int i = best.crow[t];
+          if (i >= 0) {
+            int j = 0;
+            for (int e = ia[i]; e < ia[i + 1]; ++e) {
+              const int d = ja[e];
+              if (d == i) continue;
+              const int pd = best.pos[(size_t)d];
+              const int kd = pd / kWave, oc = best.owner[(size_t)kd];
+              if (in_ring(c, k, d)) {
+                cd[j++] = (unsigned)(oc % kFlTeam * kFlLds +
+                                     (kd - best.cstep[(size_t)oc]) % kFlRing * kWave + pd % kWave);
+                if (oc != c) {
+                  int &nd = need[2 * (size_t)k + 1];
+                  nd = std::max(nd, kd - best.cstep[(size_t)oc] + 1);
+                }
+              } else {
+                src[(size_t)hcnt[(size_t)c] + h] = pd;
+                cd[j++] = (unsigned)(c % kFlTeam * kFlLds + kFlRing * kWave + h % kFlHalo);
+                ++h;
+              }
+            }
+          }
+          code[2 * t] = cd[0] | cd[1] << 16;
+          code[2 * t + 1] = cd[2] | cd[3] << 16;
+        }
+        need[2 * (size_t)k] = h;
       }
     }
-  });
-  // the progress counters and the error flag, allocated here (never inside
-  // a graph capture of the solve)
-  if (!ch_progress() || !sf_state()) return;
-  if (best.wchk.empty()) {  // keep the device arrays non-empty
-    best.wchk.push_back(0);
-    best.wlev.push_back(-1);
+  }, 8);
+  // a step that overwrites ring entries waits for their readers in the
+  // workgroup's other chunks (one host thread per workgroup: its chunks only)
+  host_ranges(G / kFlTeam, [&](int w0, int w1) {
+    for (int c = w0 * kFlTeam; c < w1 * kFlTeam; ++c)
+      for (int k = best.cstep[(size_t)c]; k < best.cstep[(size_t)c + 1]; ++k)
+        for (int l = 0; l < kWave; ++l) {
+          const int i = best.crow[(size_t)k * kWave + l];
+          if (i < 0) break;
+          for (int e = ia[i]; e < ia[i + 1]; ++e) {
+            const int kd = best.pos[(size_t)ja[e]] / kWave, oc = best.owner[(size_t)kd];
+            if (oc == c || best.how(c, k, kd) != 2) continue;
+            const int over = kd + kFlRing;
+            if (over >= best.cstep[(size_t)oc + 1]) continue;
+            int &nd = need[2 * (size_t)over + 1];
+            nd = std::max(nd, k - best.cstep[(size_t)c] + 1);
+          }
+        }
+  }, 8);
+  // exports by producing record: a chunk's are consecutive and in the order
+  // its steps make them
+  std::vector<int> first((size_t)nsteps + 1, 0), ebase((size_t)G + 1, 0);
+  for (int t : src) first[(size_t)(t / kWave) + 1]++;
+  for (int k = 0; k < nsteps; ++k) first[(size_t)k + 1] += first[(size_t)k];
+  for (int c = 0; c <= G; ++c) ebase[(size_t)c] = first[(size_t)best.cstep[(size_t)c]];
+  std::vector<int> exps(2 * (size_t)total + 2, 0);
+  {
+    std::vector<int> fill(first.begin(), first.end() - 1);
+    for (size_t h = 0; h < src.size(); ++h) {
+      const int k = src[h] / kWave, s = fill[(size_t)k]++;
+      exps[2 * (size_t)s] = src[h] - best.cstep[(size_t)best.owner[(size_t)k]] * kWave;
+      exps[2 * (size_t)s + 1] = (int)h;
+    }
   }
   TriPlan::Chunks &ch = p.ch;
-  ch.nchunks = G;
-  ch.nsteps = (int)best.slev.size();
-  ch.nwaits = best.wptr.back();
-  ch.w = W;
-  ch.cost = best.cost;
+  ch.inbox = dev_alloc(16 * ((size_t)total + 1));
+  ch.epoch = dev_alloc(16);
+  if (!ch.inbox->p || !ch.epoch->p) return;
+  LAP_HIP(hipMemsetAsync(ch.inbox->p, 0, 16 * ((size_t)total + 1), stream()));
+  LAP_HIP(hipMemsetAsync(ch.epoch->p, 0, 16, stream()));
+  std::vector<int> lstep((size_t)nsteps);
+  for (int k = 0; k < nsteps; ++k)
+    lstep[(size_t)k] = k - best.cstep[(size_t)best.owner[(size_t)k]];
   ch.cstep = dev_upload(best.cstep);
-  ch.sptr = dev_upload(best.sptr);
-  ch.slev = dev_upload(best.slev);
-  ch.wptr = dev_upload(best.wptr);
-  ch.wchk = dev_upload(best.wchk);
-  ch.wlev = dev_upload(best.wlev);
   ch.crow = dev_upload(best.crow);
   ch.cmap = dev_upload(best.cmap);
   ch.code = dev_upload(code);
+  ch.need = dev_upload(need);
+  ch.lstep = dev_upload(lstep);
+  ch.pos = dev_upload(best.pos);
+  ch.hbase = dev_upload(hcnt);
+  ch.ebase = dev_upload(ebase);
+  ch.exps = dev_upload(exps);
+  for (const DevBufPtr &b : {ch.cstep, ch.crow, ch.cmap, ch.code, ch.need, ch.lstep, ch.pos, ch.hbase, ch.ebase,
+                             ch.exps})
+    if (!b->p) return;
+  ch.nrec = (int)T;
+  ch.nchunks = G;
+  if (getenv("LAP_SCHED_LOG"))
+    fprintf(stderr, "[lapgfx] %s triangle n=%d: chunked schedule %zu of %zu, %d chunks, %d steps, "
+            "%lld values between chunks, simulated length %lld (one launch per level: %d)\n",
+            lower ? "lower" : "upper", n, best_i, cands.size(), G, nsteps, total, best.cost,
+            p.nlevels);
 }
 
 // Host-side level analysis of a triangular CSR pattern.
@@ -1071,7 +1402,6 @@ std::pair<std::unique_ptr<TriPlan>, std::unique_ptr<TriPlan>> tri_analyse_pair(
     int n, const std::vector<int> &lia, const std::vector<int> &lja,
     const std::vector<int> &uia, const std::vector<int> &uja) {
   // the shared device buffers are allocated lazily: before the threads
-  ch_progress();
   sf_state();
   std::unique_ptr<TriPlan> up;
   std::thread tu([&] { up = tri_analyse_host(n, uia, uja, false); });
@@ -1089,7 +1419,6 @@ void tri_plan_pair(int n, int nnzL, const int *lia, const int *lja, int nnzU, co
     tri_plan(n, nnzU, uia, uja, false);
     return;
   }
-  ch_progress();
   sf_state();
   std::unique_ptr<TriPlan> up;
   std::thread tu([&] { up = tri_plan_make(n, nnzU, uia, uja, false); });
@@ -1112,6 +1441,44 @@ void tri_clear_error() {
   if (st) LAP_HIP(hipMemsetAsync(st, 0, 4 * sizeof(int), stream()));
 }
 
+// The chunked schedule's records for one set of values, and its right-hand
+// side buffer, each with kFlGroup steps of room past the end.
+template <class AT, class VT>
+static bool tri_fl_pack(const TriPlan &p, const int *ja, const AT *a, DevBufPtr &rec,
+                        DevBufPtr &xc) {
+  const size_t steps = (size_t)p.ch.nrec / kWave + kFlGroup;
+  const size_t rb = steps * FlRec<AT>::bytes, xb = steps * kWave * sizeof(VT);
+  if (!rec || rec->bytes < rb) rec = dev_alloc(rb);
+  if (!xc || xc->bytes < xb) xc = dev_alloc(xb);
+  if (!rec->p || !xc->p) return false;
+  const unsigned g = grid_for((size_t)p.ch.nrec, 1, kBlock, 65536);
+  k_fl_pack<AT, VT><<<g, kBlock, 0, stream()>>>(
+      p.ch.nrec, p.ch.cmap->as<int>(), p.desc->as<int4>(), ja, a, p.ch.code->as<int2>(),
+      p.ch.need->as<int2>(), p.ch.lstep->as<int>(), rec->as<char>(), xc->as<VT>());
+  return true;
+}
+
+// One solve over the chunks: the right-hand sides x[map[t]] (x in row order
+// and map = crow, or another schedule's results and the composed map) into
+// schedule order, then the chunks, which leave the results there.
+template <class AT, class VT>
+static void tri_fl_launch(const TriPlan &p, const DevBufPtr &rec, const DevBufPtr &xc,
+                          const VT *x, const int *map, const int *done) {
+  const TriPlan::Chunks &ch = p.ch;
+  const unsigned g = std::min(2048u, 8u * ((unsigned)ch.nrec / (8u * kBlock) + 1u));
+  k_fl_gather<VT><<<g, kBlock, 0, stream()>>>(ch.nrec, map, x, xc->as<VT>(),
+                                              ch.epoch->as<unsigned>(), done);
+  k_tri_flow<AT, VT><<<ch.nchunks / kFlTeam, 4 * kFlTeam * kWave, 0, stream()>>>(
+      ch.cstep->as<int>(), rec->as<char>(), xc->as<VT>(), ch.hbase->as<int>(),
+      ch.ebase->as<int>(), ch.exps->as<int2>(), ch.inbox->p, (int)ch.inbox->bytes,
+      ch.epoch->as<unsigned>(), sf_state(), done);
+}
+template <class VT>
+static void tri_fl_spread(const TriPlan &p, const DevBufPtr &xc, VT *y, const int *done) {
+  const unsigned g = std::min(2048u, 8u * ((unsigned)p.n / (8u * kBlock) + 1u));
+  k_fl_spread<VT><<<g, kBlock, 0, stream()>>>(p.n, p.ch.pos->as<int>(), xc->as<VT>(), y, done);
+}
+
 void tri_ell_build(const TriPlan &p, const int *ja, const double *a, TriEll &e) {
   e.w = 0;
   if (p.n <= 0 || p.max_row > 8) return;
@@ -1127,30 +1494,11 @@ void tri_ell_build(const TriPlan &p, const int *ja, const double *a, TriEll &e) 
     k_ell_pack<8><<<g, kBlock, 0, stream()>>>(p.n, p.desc->as<int4>(), ja, a, e.ja->as<int>(),
                                               e.a->as<double>());
   e.w = w;
-  if (p.ch.nchunks > 0 && p.ch.w == 4) {  // the chunked schedule's records for these values
-    // kBlock records of padding: the prefetch copies whole slots
-    e.crec = dev_alloc((size_t)ChRec<4, double>::bytes * ((size_t)p.n + kBlock));
-    e.xc = dev_alloc(sizeof(double) * ((size_t)p.n + kBlock));
-    if (!e.crec || !e.crec->p || !e.xc || !e.xc->p) return;
-    k_ch_pack<4, double><<<g, kBlock, 0, stream()>>>(p.n, p.ch.cmap->as<int>(),
-                                                     p.desc->as<int4>(), ja, a,
-                                                     p.ch.code->as<int>(), e.crec->as<char>());
-  }
+  if (p.ch.nchunks > 0) tri_fl_pack<double, double>(p, ja, a, e.crec, e.xc);
 }
 
 void tri_ch_pack32(const TriPlan &p, const int *ja, const float *a, TriChunks32 &c) {
-  c.ok = false;
-  if (p.n <= 0 || p.ch.nchunks <= 0 || p.ch.w != 4) return;
-  const size_t bytes = (size_t)ChRec<4, float>::bytes * ((size_t)p.n + kBlock);
-  if (!c.rec || c.rec->bytes < bytes) c.rec = dev_alloc(bytes);
-  const size_t xb = sizeof(float) * ((size_t)p.n + kBlock);
-  if (!c.xc || c.xc->bytes < xb) c.xc = dev_alloc(xb);
-  if (!c.rec || !c.rec->p || !c.xc || !c.xc->p) return;
-  const unsigned g = grid_for((size_t)p.n, 1, kBlock, 65536);
-  k_ch_pack<4, float><<<g, kBlock, 0, stream()>>>(p.n, p.ch.cmap->as<int>(), p.desc->as<int4>(),
-                                                  ja, a, p.ch.code->as<int>(),
-                                                  c.rec->as<char>());
-  c.ok = true;
+  c.ok = p.n > 0 && p.ch.nchunks > 0 && tri_fl_pack<float, float>(p, ja, a, c.rec, c.xc);
 }
 
 // One launch per level: a lane per short row, then a workgroup per long row
@@ -1185,8 +1533,7 @@ enum TriPath { TRI_CHUNKS, TRI_LEVELS_ELL, TRI_LEVELS };
 
 static TriPath tri_path(const TriPlan &p, const TriEll *ell, bool in_place) {
   const int mode = options().sptrsv_mode;
-  if (mode == 3 && ell && ell->w && ell->crec && ell->xc && p.ch.nchunks > 0 && p.ch.w == 4 &&
-      sf_state() && ch_progress())
+  if (mode == 3 && ell && ell->w && ell->crec && ell->xc && p.ch.nchunks > 0 && sf_state())
     return TRI_CHUNKS;
   (void)in_place;  // the chunked kernel reads x from its own gathered copy
   if (ell && ell->w) return TRI_LEVELS_ELL;
@@ -1207,22 +1554,9 @@ void tri_solve_launch(const TriPlan &p, const int *ia, const int *ja, const doub
   const int *order = p.order->as<int>();
   const TriPath path = tri_path(p, ell, x == y);
   if (path == TRI_CHUNKS) {
-    int *st = sf_state(), *prog = ch_progress();
-    {
-      const TriPlan::Chunks &ch = p.ch;
-      k_ch_reset<<<(ch.nchunks + kBlock - 1) / kBlock, kBlock, 0, stream()>>>(ch.nchunks, prog,
-                                                                             done);
-      k_ch_gather<double><<<2048, kBlock, 0, stream()>>>(
-          p.n, ch.crow->as<int>(), x, ell->xc->as<double>(), done);
-#define LAP_CH_ARGS                                                                            \
-  ch.cstep->as<int>(), ch.sptr->as<int>(), ch.slev->as<int>(), ch.wptr->as<int>(),             \
-      ch.wchk->as<int>(), ch.wlev->as<int>(), ell->crec->as<char>(),                           \
-      ell->xc->as<double>(), y, prog, st, done
-      k_tri_chunks<double, double, 4, 3, 4><<<ch.nchunks, kBlock + kWave, 0, stream()>>>(
-          LAP_CH_ARGS);
-#undef LAP_CH_ARGS
-      return;
-    }
+    tri_fl_launch<double, double>(p, ell->crec, ell->xc, x, p.ch.crow->as<int>(), done);
+    tri_fl_spread(p, ell->xc, y, done);
+    return;
   }
   if (path == TRI_LEVELS_ELL) {
     for (int l = 0; l < p.nlevels; ++l) {
@@ -1243,6 +1577,26 @@ void tri_solve_launch(const TriPlan &p, const int *ia, const int *ja, const doub
   tri_level_launch<double, double>(p, ja, a, diag, x, y, done);
 }
 
+DevBufPtr tri_compose(const TriPlan &first, const TriPlan &second) {
+  if (first.ch.nchunks <= 0 || second.ch.nchunks <= 0) return nullptr;
+  DevBufPtr m = dev_alloc(sizeof(int) * (size_t)second.ch.nrec);
+  if (!m->p) return nullptr;
+  k_fl_compose<<<grid_for((size_t)second.ch.nrec, 4, kBlock, 4096), kBlock, 0, stream()>>>(
+      second.ch.nrec, second.ch.crow->as<int>(), first.ch.pos->as<int>(), m->as<int>());
+  return m;
+}
+
+bool tri_solve_two_launch(const TriPlan &p1, const TriEll &e1, const TriPlan &p2,
+                          const TriEll &e2, const DevBufPtr &comp, const double *x, double *y,
+                          const int *done) {
+  if (!comp || tri_path(p1, &e1, false) != TRI_CHUNKS || tri_path(p2, &e2, false) != TRI_CHUNKS)
+    return false;
+  tri_fl_launch<double, double>(p1, e1.crec, e1.xc, x, p1.ch.crow->as<int>(), done);
+  tri_fl_launch<double, double>(p2, e2.crec, e2.xc, e1.xc->as<double>(), comp->as<int>(), done);
+  tri_fl_spread(p2, e2.xc, y, done);
+  return true;
+}
+
 template <class VT>
 static void tri_mixed_launch(const TriPlan &p, const int *ja, const float *a, const VT *x, VT *y,
                              const int *done) {
@@ -1250,27 +1604,28 @@ static void tri_mixed_launch(const TriPlan &p, const int *ja, const float *a, co
 }
 
 static bool tri_chunks32_ready(const TriPlan &p, const TriChunks32 *c) {
-  return c && c->ok && options().sptrsv_mode == 3 && p.ch.nchunks > 0 && p.ch.w == 4 &&
-         sf_state() && ch_progress();
+  return c && c->ok && options().sptrsv_mode == 3 && p.ch.nchunks > 0 && sf_state();
 }
 
 int tri_launches32(const TriPlan &p, const TriChunks32 *c) {
   return tri_chunks32_ready(p, c) ? 3 : p.nlevels;
 }
 
+bool tri_solve32_two_launch(const TriPlan &p1, const TriChunks32 &c1, const TriPlan &p2,
+                            const TriChunks32 &c2, const DevBufPtr &comp, const float *x,
+                            float *y, const int *done) {
+  if (!comp || !tri_chunks32_ready(p1, &c1) || !tri_chunks32_ready(p2, &c2)) return false;
+  tri_fl_launch<float, float>(p1, c1.rec, c1.xc, x, p1.ch.crow->as<int>(), done);
+  tri_fl_launch<float, float>(p2, c2.rec, c2.xc, c1.xc->as<float>(), comp->as<int>(), done);
+  tri_fl_spread(p2, c2.xc, y, done);
+  return true;
+}
+
 void tri_solve32_launch(const TriPlan &p, const int *ja, const float *a, const float *x, float *y,
                         const int *done, const TriChunks32 *c) {
   if (tri_chunks32_ready(p, c)) {
-    const TriPlan::Chunks &ch = p.ch;
-    int *st = sf_state(), *prog = ch_progress();
-    k_ch_reset<<<(ch.nchunks + kBlock - 1) / kBlock, kBlock, 0, stream()>>>(ch.nchunks, prog,
-                                                                           done);
-    k_ch_gather<float><<<2048, kBlock, 0, stream()>>>(p.n, ch.crow->as<int>(), x,
-                                                      c->xc->as<float>(), done);
-    k_tri_chunks<float, float, 4, 3, 4><<<ch.nchunks, kBlock + kWave, 0, stream()>>>(
-        ch.cstep->as<int>(), ch.sptr->as<int>(), ch.slev->as<int>(), ch.wptr->as<int>(),
-        ch.wchk->as<int>(), ch.wlev->as<int>(), c->rec->as<char>(), c->xc->as<float>(), y, prog,
-        st, done);
+    tri_fl_launch<float, float>(p, c->rec, c->xc, x, p.ch.crow->as<int>(), done);
+    tri_fl_spread(p, c->xc, y, done);
     return;
   }
   tri_mixed_launch<float>(p, ja, a, x, y, done);
