@@ -262,11 +262,15 @@ long long scan_exclusive(const int *in, long long n, int *out, long long *ws);
 void forget_plans(const void *p);
 
 // ------------------------------------------------------------- SpMV plan
+struct ResPlan;
 struct SpmvPlan {
   int n = 0, nnz = 0;
   int nblocks = 0;        // row blocks
   DevBufPtr rowblk;       // int[nblocks + 1]: first row of each block
   int max_row = 0;
+  // the resident Jacobi PCG's analysis of the same matrix, made at its first
+  // solve (null: none yet)
+  mutable std::shared_ptr<ResPlan> res;
 };
 // Finds or builds the plan for (ia, ja, n, nnz) (device arrays).
 const SpmvPlan *spmv_plan(int n, int nnz, const int *ia, const int *ja);
@@ -277,6 +281,19 @@ void spmv_launch(const SpmvPlan &p, const int *ia, const int *ja, const double *
                  const int *done = nullptr);
 // Persistent SpMV grid: min(row blocks, 8 workgroups per CU).
 unsigned spmv_grid(const SpmvPlan &p);
+
+// ------------------------------------------------- resident Jacobi PCG
+struct ResOut {
+  int iterations, flag;
+  double res0, res;
+};
+// The whole Jacobi PCG solve as one launch with the system in registers and
+// LDS (resident.hip).  hist: device, maxit + 2 entries; r, p: n-vectors of
+// scratch.  1: done (out filled), 0: the matrix does not fit (nothing was
+// launched that touches x), -1: an error was recorded.
+int pcg_resident(const SpmvPlan &A, const int *ia, const int *ja, const double *a,
+                 const double *d_r, double *x, const double *b, double tol, int maxit,
+                 double *hist, double *r, double *p, ResOut &out);
 
 // ------------------------------------------------- value-indexed CSR
 // Encodes a[0..nnz) as one-byte indices into a table of its distinct values

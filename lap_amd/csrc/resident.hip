@@ -1,0 +1,571 @@
+// resident.hip -- Jacobi PCG of small and medium systems as one launch, the
+// whole system on the chip.
+//
+// Why: three launches per iteration cost 12 us whatever the system's size
+// (n = 16,384: 13.5 us per iteration for 0.7 MB of traffic), and a system of
+// up to a few hundred thousand rows fits the registers and LDS of the 256
+// CUs: 2^17 rows of 11 entries are 15 MB of matrix against 128 MiB of
+// registers.
+//
+// How: a workgroup of 1024 threads owns a contiguous range of rows, R rows per
+// thread, for the whole solve.  A thread keeps its rows' values, column slots,
+// x, r, p and 1/diag in registers; the LDS holds the p of the workgroup's rows
+// and of the other rows they refer to (its halo).  What crosses between
+// workgroups per iteration:
+//   1. p.q, one partial sum per workgroup, read by all of them;
+//   2. r.w and r.r likewise, and w = d_r r of the rows others refer to: the
+//      owner of a halo entry keeps p = beta p + w itself, from the same
+//      operands, so p is never sent.
+// They travel as tagged words (boxed.hpp), two trips through memory per
+// iteration and no barrier between workgroups.  A place is written again only
+// after every reader has taken the value it held: the writer is then past a
+// sum to which each reader contributed after reading.
+//
+// Arithmetic: the recurrence of k_jac_update_nx / k_jac_px (pcg.hip), each row
+// summed in CSR order and each vector entry updated by the same operations;
+// the three dot products are summed in another fixed order (rows of a thread,
+// lanes of a wave, waves, workgroups).
+//
+// All workgroups must run at once: at most one per CU.  Waits are bounded and
+// one that runs out ends every workgroup with an error.
+#include <algorithm>
+#include <cmath>
+
+#include "boxed.hpp"
+#include "lap_core.hpp"
+
+namespace lap {
+
+namespace {
+
+constexpr int kResThreads = 1024;
+constexpr int kResWaves = kResThreads / kWave;
+constexpr int kResHalo = 8192;     // halo entries of a workgroup at most
+constexpr int kResMaxWg = 256;     // workgroups at most (partials: one per thread of 4 waves)
+// Rows per workgroup at least: fewer workgroups have fewer partial sums to
+// exchange, until the LDS reads of a thread's rows take longer than that
+// saves.  us per iteration with 512 / 1024 / 2048 rows: 128^2 4.66 / 4.44 /
+// 3.89, 512^2 9.05 / 9.08 / 6.86, 40^3 7.15 / 6.66 / 6.70, 64^3 9.4 / 9.4 /
+// 11.1, 97 x 90 x 31 8.7 / 8.7 / 10.6: 2048 for rows of up to 5 entries.
+constexpr int kResRows = 1024, kResRowsShort = 2048, kResShort = 5;
+constexpr int kResMaxN = 1 << 19;  // rows at most (the analysis' bitmap in LDS)
+constexpr int kResIters = 8192;    // iterations per launch
+constexpr unsigned kResSpins = 1u << 22;
+
+struct ResState {
+  double rho, tolrel, res0, res;
+  int iter, flag;  // flag: -1 not finished
+  int error;       // a wait ran out
+  unsigned tag;    // last tag used
+};
+
+struct ResArgs {
+  int n, nr, nwg, nhmax;  // nr: rows per workgroup
+  const int *ia;
+  const double *a;
+  const unsigned short *lcol;
+  const int *hcnt, *hcol;
+  const unsigned char *sent;
+  const double *d_r, *b;
+  double *x, *r, *p;
+  double tol;
+  int maxit, resume, iters;
+  unsigned tag0;
+  double *hist;
+  void *box_a, *box_b, *box_w;
+  ResState *st;
+};
+
+// Sum over the wave's first 16 (W16) or all 64 lanes, valid in the last of
+// them; fixed order.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + fl_f64((unsigned)lo, (unsigned)hi);
+}
+__device__ __forceinline__ double row_sum_dpp(double v) {  // lane 15 of each row of 16
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  return dpp_add<0x118, 0xf>(v);
+}
+__device__ __forceinline__ double wave_sum_dpp(double v) {  // lane 63
+  v = row_sum_dpp(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+}
+
+// The launch.  R rows per thread, rows of at most L entries.
+template <int R, int L>
+__global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
+  extern __shared__ double ps[];  // own rows, halo, a zero; the halo's rows
+  __shared__ double red[2][kResWaves], tot[2][4];
+  __shared__ int dead;
+  const int t = threadIdx.x, lane = t & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int w = blockIdx.x;
+  const int base = w * g.nr, rows = min(g.nr, g.n - base);
+  const int nh = g.hcnt[w];
+  double *const halo = ps + R * kResThreads;
+  const int zero = R * kResThreads + g.nhmax;
+  int *const hcol = reinterpret_cast<int *>(ps + zero + 1);  // the halo's rows
+  const __amdgpu_buffer_rsrc_t box_a = fl_buffer(g.box_a, g.nwg * 16);
+  const __amdgpu_buffer_rsrc_t box_b = fl_buffer(g.box_b, g.nwg * 32);
+  const __amdgpu_buffer_rsrc_t box_w = fl_buffer(g.box_w, g.n * 16);
+  if (t == 0) {
+    dead = 0;
+    ps[zero] = 0.0;
+  }
+  for (int h = t; h < nh; h += kResThreads) hcol[h] = g.hcol[(size_t)w * kResHalo + h];
+  __syncthreads();
+  // the thread's rows
+  double val[R][L], x[R], r[R], p[R], d[R];
+  unsigned slot[R][L / 2];
+  bool have[R], sent[R];
+  int longest[R];  // of the wave's rows
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int l = t + k * kResThreads, row = base + l;
+    have[k] = l < rows;
+    const int e0 = have[k] ? g.ia[row] : 0, len = have[k] ? g.ia[row + 1] - e0 : 0;
+#pragma unroll
+    for (int j = 0; j < L; ++j) {
+      val[k][j] = j < len ? g.a[e0 + j] : 0.0;
+      const unsigned s = j < len ? g.lcol[e0 + j] : (unsigned)zero;
+      if (j & 1)
+        slot[k][j / 2] |= s << 16;
+      else
+        slot[k][j / 2] = s;
+    }
+    d[k] = have[k] ? g.d_r[row] : 0.0;
+    x[k] = have[k] ? g.x[row] : 0.0;
+    r[k] = p[k] = 0.0;
+    sent[k] = have[k] && g.sent[row];
+    int m = len;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
+    longest[k] = __builtin_amdgcn_readfirstlane(m);
+  }
+  auto row_sums = [&](double(&s)[R]) {  // CSR order; padding adds 0 * 0
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      s[k] = 0.0;
+#pragma unroll
+      for (int j = 0; j < L; j += 4) {
+        if (j >= longest[k]) break;
+        double v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          v[i] = ps[(i & 1) ? slot[k][(j + i) / 2] >> 16 : slot[k][(j + i) / 2] & 0xffffu];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[k] += val[k][j + i] * v[i];
+      }
+    }
+  };
+  // One wait of this wave (every lane that still misses something): false
+  // once it has to be given up.
+  auto again = [&](unsigned &spins) {
+    if (++spins > kResSpins ||
+        ((spins & 63u) == 0 && __hip_atomic_load(&g.st->error, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))) {
+      if (lane == 0) {
+        dead = 1;
+        __hip_atomic_store(&g.st->error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      return false;
+    }
+    return true;
+  };
+  // Sums of v over all workgroups (N = 1: box_a, 2: box_b), to every thread;
+  // `between` runs while they are on their way.
+  auto all_sums = [&](auto &v, unsigned tag, auto &&between) {
+    constexpr int N = sizeof(v) / sizeof(v[0]);
+    const __amdgpu_buffer_rsrc_t box = N == 1 ? box_a : box_b;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const double s = wave_sum_dpp(v[i]);
+      if (lane == kWave - 1) red[i][wave] = s;
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const double s = row_sum_dpp(lane < kResWaves ? red[i][lane] : 0.0);
+        if (lane == kResWaves - 1) fl_put(box, w * N + i, tag, s);
+      }
+    }
+    between();
+    if (wave < 4) {
+      double got[N];
+      if (wave * kWave < g.nwg) {
+        FlBoxed<double> f[N];
+        unsigned spins = 0;
+        for (;;) {
+          bool ok = true;
+#pragma unroll
+          for (int i = 0; i < N; ++i) f[i].load(box, t * N + i);
+#pragma unroll
+          for (int i = 0; i < N; ++i) ok = ok && f[i].is(tag);
+          fl_fence();
+          if (__builtin_amdgcn_ballot_w64(!ok && t < g.nwg) == 0) break;
+          if (!again(spins)) break;
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) got[i] = t < g.nwg ? f[i].value() : 0.0;
+      } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) got[i] = 0.0;
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const double s = wave_sum_dpp(got[i]);
+        if (lane == kWave - 1) tot[i][wave] = s;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = ((tot[i][0] + tot[i][1]) + tot[i][2]) + tot[i][3];
+  };
+  // halo entries: p = w (first) or beta p + w, w as its owner sent it.  The
+  // first entry of each thread is asked for ahead (halo_ask).
+  FlBoxed<double> ahead;
+  auto halo_ask = [&] { ahead.load(box_w, t < nh ? hcol[t] : 0); };
+  auto halo_update = [&](unsigned tag, bool first, double beta) {
+    for (int h0 = wave * kWave; h0 < nh; h0 += kResThreads) {
+      const int h = h0 + lane;
+      const int c = h < nh ? hcol[h] : 0;
+      FlBoxed<double> f;
+      if (h0 < kResThreads)
+        f = ahead;
+      else
+        f.load(box_w, c);
+      unsigned spins = 0;
+      while (__builtin_amdgcn_ballot_w64(h < nh && !f.is(tag)) != 0) {
+        if (!again(spins)) break;
+        f.load(box_w, c);
+        fl_fence();
+      }
+      if (h < nh) halo[h] = first ? f.value() : halo[h] * beta + f.value();
+    }
+  };
+  auto own_update = [&]() {
+#pragma unroll
+    for (int k = 0; k < R; ++k) ps[t + k * kResThreads] = p[k];
+  };
+  auto nothing = [] {};
+
+  double rho, tolrel, res0, res;
+  int it, flag = -1;
+  unsigned tag = g.tag0;
+  if (g.resume) {
+    rho = g.st->rho;
+    tolrel = g.st->tolrel;
+    res0 = g.st->res0;
+    res = g.st->res;
+    it = g.st->iter;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int row = base + t + k * kResThreads;
+      r[k] = have[k] ? g.r[row] : 0.0;
+      p[k] = have[k] ? g.p[row] : 0.0;
+    }
+    for (int h = t; h < nh; h += kResThreads) halo[h] = g.p[hcol[h]];
+    own_update();
+    __syncthreads();
+  } else {
+    // r = -(A x - b) (cg.c:48-55), w = d_r r, p = w
+#pragma unroll
+    for (int k = 0; k < R; ++k) ps[t + k * kResThreads] = x[k];
+    for (int h = t; h < nh; h += kResThreads) halo[h] = g.x[hcol[h]];
+    __syncthreads();
+    double s[R], v[2] = {0.0, 0.0};
+    row_sums(s);
+    ++tag;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int row = base + t + k * kResThreads;
+      r[k] = have[k] ? -(s[k] - g.b[row]) : 0.0;
+      p[k] = d[k] * r[k];
+      if (sent[k]) fl_put(box_w, row, tag, p[k]);
+      v[0] += r[k] * p[k];
+      v[1] += r[k] * r[k];
+    }
+    all_sums(v, tag, halo_ask);
+    rho = v[0];
+    res0 = res = sqrt(v[1]);
+    tolrel = g.tol * res0;
+    it = 0;
+    if (w == 0 && t == 0) g.hist[0] = res0;
+    if (!isfinite(res0)) flag = 2;
+    if (res0 == 0.0) flag = 0;  // x0 solves the system
+    flag = __builtin_amdgcn_readfirstlane(flag);
+    if (flag < 0) {
+      own_update();
+      halo_update(tag, true, 0.0);
+    }
+    __syncthreads();
+  }
+  const int stop = it + g.iters;
+  while (flag < 0 && it < stop && !__builtin_amdgcn_readfirstlane(dead)) {
+    ++it;
+    // q = A p, p.q, alpha
+    double q[R], v1[1] = {0.0};
+    row_sums(q);
+#pragma unroll
+    for (int k = 0; k < R; ++k) v1[0] += p[k] * q[k];
+    all_sums(v1, ++tag, nothing);
+    const double alpha = rho / v1[0], nalpha = -1.0 * alpha;
+    // r -= alpha q, w = d_r r, r.w, r.r; x += alpha p on the way
+    double wv[R], v[2] = {0.0, 0.0};
+    ++tag;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      r[k] = r[k] + nalpha * q[k];
+      wv[k] = d[k] * r[k];
+      if (sent[k]) fl_put(box_w, base + t + k * kResThreads, tag, wv[k]);
+      v[0] += r[k] * wv[k];
+      v[1] += r[k] * r[k];
+    }
+    all_sums(v, tag, [&] {
+#pragma unroll
+      for (int k = 0; k < R; ++k) x[k] += alpha * p[k];
+      halo_ask();
+    });
+    // convergence test (cg.c:106-123) and beta
+    res = sqrt(v[1]);
+    if (w == 0 && t == 0) g.hist[it] = res;
+    if (!isfinite(res)) flag = 2;
+    else if (res < tolrel) flag = 0;
+    else if (it > g.maxit) flag = 1;
+    flag = __builtin_amdgcn_readfirstlane(flag);
+    if (flag >= 0) break;
+    const double beta = v[0] / rho;
+    rho = v[0];
+#pragma unroll
+    for (int k = 0; k < R; ++k) p[k] = p[k] * beta + wv[k];
+    own_update();
+    halo_update(tag, false, beta);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int row = base + t + k * kResThreads;
+    if (!have[k]) continue;
+    g.x[row] = x[k];
+    if (flag < 0) {
+      g.r[row] = r[k];
+      g.p[row] = p[k];
+    }
+  }
+  if (w == 0 && t == 0) {
+    g.st->rho = rho;
+    g.st->tolrel = tolrel;
+    g.st->res0 = res0;
+    g.st->res = res;
+    g.st->iter = it;
+    g.st->flag = flag;
+    g.st->tag = tag;
+  }
+}
+
+// The analysis: workgroup w lists the rows outside its own that its rows refer
+// to (ascending), marks them as sent, and gives every nonzero its slot: own
+// rows first, then the halo.  cnt[w]: the halo's length (more than kResHalo:
+// nothing else is written).  Dynamic LDS: a bitmap of the n rows and the rank
+// of each of its words.
+__global__ __launch_bounds__(kResThreads) void k_res_plan(int n, int nr, int own,
+                                                          const int *__restrict__ ia,
+                                                          const int *__restrict__ ja,
+                                                          int *__restrict__ cnt,
+                                                          int *__restrict__ hcol,
+                                                          unsigned char *__restrict__ sent,
+                                                          unsigned short *__restrict__ lcol) {
+  extern __shared__ unsigned bits[];
+  __shared__ int scan[kResThreads];
+  const int words = (n + 31) / 32;
+  unsigned short *rank = reinterpret_cast<unsigned short *>(bits + words);
+  const int w = blockIdx.x, t = threadIdx.x;
+  const int base = w * nr, end = min(n, base + nr);
+  const int e0 = ia[base], e1 = ia[end];
+  for (int i = t; i < words; i += kResThreads) bits[i] = 0;
+  __syncthreads();
+  for (int e = e0 + t; e < e1; e += kResThreads) {
+    const int c = ja[e];
+    if (c < base || c >= end) atomicOr(&bits[c >> 5], 1u << (c & 31));
+  }
+  __syncthreads();
+  // ranks of the words: each thread a run of them
+  const int per = (words + kResThreads - 1) / kResThreads;
+  const int i0 = min(words, t * per), i1 = min(words, i0 + per);
+  int c = 0;
+  for (int i = i0; i < i1; ++i) c += __popc(bits[i]);
+  scan[t] = c;
+  __syncthreads();
+  for (int o = 1; o < kResThreads; o <<= 1) {
+    const int v = t >= o ? scan[t - o] : 0;
+    __syncthreads();
+    scan[t] += v;
+    __syncthreads();
+  }
+  const int total = scan[kResThreads - 1];
+  if (t == 0) cnt[w] = total;
+  if (total > kResHalo) return;
+  int at = scan[t] - c;
+  for (int i = i0; i < i1; ++i) {
+    rank[i] = (unsigned short)at;
+    for (unsigned m = bits[i]; m; m &= m - 1) {
+      const int col = i * 32 + __ffs((int)m) - 1;
+      hcol[(size_t)w * kResHalo + at++] = col;
+      sent[col] = 1;
+    }
+  }
+  __syncthreads();
+  for (int e = e0 + t; e < e1; e += kResThreads) {
+    const int col = ja[e];
+    lcol[e] = (unsigned short)(col >= base && col < end
+                                   ? col - base
+                                   : own + rank[col >> 5] +
+                                         __popc(bits[col >> 5] & ((1u << (col & 31)) - 1u)));
+  }
+}
+
+__global__ void k_res_zero(long long n, unsigned *p) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x)
+    p[i] = 0;
+}
+
+using ResKernel = void (*)(ResArgs);
+struct ResShape {
+  int r, l;
+  ResKernel fn;
+};
+// A thread's registers hold R (2.5 L + 8) words beside the work of a row: 128
+// registers per thread at 1024 threads allow these.
+const ResShape kShapes[] = {{1, 8, k_resident<1, 8>},   {2, 8, k_resident<2, 8>},
+                            {1, 16, k_resident<1, 16>}, {1, 24, k_resident<1, 24>},
+                            {1, 32, k_resident<1, 32>}};
+
+}  // namespace
+
+struct ResPlan {
+  bool ok = false;
+  int nr = 0, nwg = 0, nhmax = 0, lds = 0;
+  ResKernel fn = nullptr;
+  DevBufPtr hcnt, hcol, sent, lcol, boxes, state;
+  size_t box_words = 0;
+  unsigned tag = 0;
+};
+
+// Built at a matrix's first resident solve and kept with its SpMV plan.
+static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const int *ja) {
+  auto P = std::make_shared<ResPlan>();
+  const int n = A.n, cus = std::min(device_cus(), kResMaxWg);
+  if (n < 1 || n > kResMaxN || A.max_row > 32) return P;
+  const ResShape *s = nullptr;
+  int nr = 0;
+  const int least = A.max_row <= kResShort ? kResRowsShort : kResRows;
+  for (const ResShape &c : kShapes) {
+    if (A.max_row > c.l) continue;
+    nr = std::max(least, ((n + cus - 1) / cus + kWave - 1) / kWave * kWave);
+    if (nr <= c.r * kResThreads) {
+      s = &c;
+      break;
+    }
+  }
+  if (!s) return P;
+  P->nr = nr;
+  P->nwg = (n + nr - 1) / nr;
+  P->fn = s->fn;
+  const size_t words = ((size_t)n + 31) / 32;
+  P->hcnt = dev_alloc(sizeof(int) * (size_t)P->nwg);
+  P->hcol = dev_alloc(sizeof(int) * (size_t)P->nwg * kResHalo);
+  P->sent = dev_alloc(((size_t)n + 3) / 4 * 4);
+  P->lcol = dev_alloc(sizeof(unsigned short) * (size_t)std::max(A.nnz, 1));
+  P->state = dev_alloc(sizeof(ResState));
+  P->box_words = 4 * ((size_t)n + 3 * (size_t)P->nwg);
+  P->boxes = dev_alloc(sizeof(unsigned) * P->box_words);
+  for (const DevBufPtr &b : {P->hcnt, P->hcol, P->sent, P->lcol, P->state, P->boxes})
+    if (!b->p) return P;
+  const int plan_lds = (int)(words * 4 + (words + 1) / 2 * 4);
+  if (!LAP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_res_plan),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, plan_lds)))
+    return P;
+  k_res_zero<<<256, kBlock, 0, stream()>>>(((long long)n + 3) / 4, P->sent->as<unsigned>());
+  k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P->box_words, P->boxes->as<unsigned>());
+  k_res_plan<<<P->nwg, kResThreads, plan_lds, stream()>>>(
+      n, nr, s->r * kResThreads, ia, ja, P->hcnt->as<int>(), P->hcol->as<int>(),
+      P->sent->as<unsigned char>(), P->lcol->as<unsigned short>());
+  for (int c : dev_download(P->hcnt->as<int>(), (size_t)P->nwg)) P->nhmax = std::max(P->nhmax, c);
+  if (lap_last_status() == LAP_ERR_HIP || P->nhmax > kResHalo) return P;
+  P->lds = (int)sizeof(double) * (s->r * kResThreads + P->nhmax + 1) + 4 * P->nhmax;
+  if (!LAP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(P->fn),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, P->lds)))
+    return P;
+  P->ok = true;
+  return P;
+}
+
+int pcg_resident(const SpmvPlan &A, const int *ia, const int *ja, const double *a,
+                 const double *d_r, double *x, const double *b, double tol, int maxit,
+                 double *hist, double *r, double *p, ResOut &out) {
+  if (!A.res) A.res = res_plan_build(A, ia, ja);
+  ResPlan &P = *A.res;
+  if (!P.ok) return 0;
+  char *box = P.boxes->as<char>();
+  ResArgs g{};
+  g.n = A.n;
+  g.nr = P.nr;
+  g.nwg = P.nwg;
+  g.nhmax = P.nhmax;
+  g.ia = ia;
+  g.a = a;
+  g.lcol = P.lcol->as<unsigned short>();
+  g.hcnt = P.hcnt->as<int>();
+  g.hcol = P.hcol->as<int>();
+  g.sent = P.sent->as<unsigned char>();
+  g.d_r = d_r;
+  g.b = b;
+  g.x = x;
+  g.r = r;
+  g.p = p;
+  g.tol = tol;
+  g.maxit = maxit;
+  g.iters = kResIters;
+  g.hist = hist;
+  g.box_a = box;
+  g.box_b = box + 16 * (size_t)P.nwg;
+  g.box_w = box + 48 * (size_t)P.nwg;
+  g.st = P.state->as<ResState>();
+  k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResState) / 4), P.state->as<unsigned>());
+  ResState h{};
+  // iter <= maxit + 1, so this many launches always finish
+  for (long k = 0; k <= (long)(maxit + 1) / kResIters + 1; ++k) {
+    g.resume = k > 0;
+    g.tag0 = P.tag;
+    P.fn<<<P.nwg, kResThreads, P.lds, stream()>>>(g);
+    if (!LAP_HIP(hipGetLastError()) ||
+        !LAP_HIP(hipMemcpyAsync(&h, g.st, sizeof h, hipMemcpyDeviceToHost, stream())))
+      return -1;
+    sync();
+    if (lap_last_status() == LAP_ERR_HIP) return -1;
+    if (h.error) {  // start over with unused tags next time
+      k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P.box_words,
+                                               P.boxes->as<unsigned>());
+      P.tag = 0;
+      set_error(LAP_ERR_NUMERIC, "pcg: a wait between workgroups ran out");
+      return -1;
+    }
+    P.tag = h.tag;
+    if (h.flag >= 0) break;
+  }
+  out.iterations = h.iter;
+  out.flag = h.flag < 0 ? 2 : h.flag;
+  out.res0 = h.res0;
+  out.res = h.res;
+  return 1;
+}
+
+}  // namespace lap

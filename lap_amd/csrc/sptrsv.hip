@@ -23,6 +23,7 @@
 #include <cstdlib>
 #include <thread>
 
+#include "boxed.hpp"
 #include "lap_core.hpp"
 
 namespace lap {
@@ -348,11 +349,6 @@ constexpr unsigned kFlSpins = 1u << 22;  // polls of one wait before the solve f
 //                 the base of the row's range test (.w, see fl_out)
 //   then W = 4 off-diagonal values per row (FP64: two double2 planes, FP32:
 //   one float4 plane), then double2 {pivot, 1/pivot}.
-typedef __attribute__((ext_vector_type(4))) unsigned fl_u4;
-typedef __attribute__((ext_vector_type(2))) unsigned fl_u2;
-__device__ __forceinline__ double fl_f64(unsigned lo, unsigned hi) {
-  return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
-}
 template <class AT>
 struct FlRec;
 template <>
@@ -392,11 +388,6 @@ __device__ __forceinline__ void fl_load_x(__amdgpu_buffer_rsrc_t b, int lane, in
 __device__ __forceinline__ void fl_load_x(__amdgpu_buffer_rsrc_t b, int lane, int step, float *x) {
   *x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, lane * 4, step * (kWave * 4), 0));
 }
-// a buffer of `bytes` from p (gfx9 word 3: raw data, 32-bit)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t fl_buffer(const void *p, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00027000);
-}
-
 // Whether x lies outside [2^-400, 2^400): inside it (and with the pivot in
 // it) the refined division below neither overflows nor loses bits to
 // underflow in any step.  `base` is kFlBase, or kFlNever where the pivot is
@@ -420,44 +411,9 @@ __device__ __forceinline__ double fl_div(double a, double b, double y) {
   return __builtin_fma(__builtin_fma(-b, q, a), y, q);
 }
 
-// One value of another chunk in an inbox: its 32-bit halves (FP32: the whole)
-// each beside the solve's tag in one aligned 8-byte word.  Such a word is
-// written and read whole, so a matching tag means the half is this solve's: no
-// flag, fence or store order is involved.  Stores and loads are agent-scope
-// (sc1): past the CU's cache and the XCD's L2.
-constexpr int kFlAgent = 16;
-__device__ __forceinline__ void fl_put(__amdgpu_buffer_rsrc_t box, int i, unsigned tag, double v) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  __builtin_amdgcn_raw_buffer_store_b128(fl_u4{(unsigned)b, tag, (unsigned)(b >> 32), tag}, box,
-                                         i * 16, 0, kFlAgent);
-}
-__device__ __forceinline__ void fl_put(__amdgpu_buffer_rsrc_t box, int i, unsigned tag, float v) {
-  __builtin_amdgcn_raw_buffer_store_b64(fl_u2{__float_as_uint(v), tag}, box, i * 8, 0, kFlAgent);
-}
-template <class VT>
-struct FlBoxed;
-template <>
-struct FlBoxed<double> {
-  fl_u4 w;
-  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t box, int i) {
-    w = __builtin_amdgcn_raw_buffer_load_b128(box, i * 16, 0, kFlAgent);
-  }
-  __device__ __forceinline__ bool is(unsigned tag) const { return w.y == tag && w.w == tag; }
-  __device__ __forceinline__ double value() const { return fl_f64(w.x, w.z); }
-};
-template <>
-struct FlBoxed<float> {
-  fl_u2 w;
-  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t box, int i) {
-    w = __builtin_amdgcn_raw_buffer_load_b64(box, i * 8, 0, kFlAgent);
-  }
-  __device__ __forceinline__ bool is(unsigned tag) const { return w.y == tag; }
-  __device__ __forceinline__ float value() const { return __uint_as_float(w.x); }
-};
-
-// The compiler may not move memory accesses across this (LDS operations of a
-// wave execute in issue order, so no wait is needed between them).
-__device__ __forceinline__ void fl_fence() { __atomic_signal_fence(__ATOMIC_SEQ_CST); }
+// (Values between workgroups: boxed.hpp.  A chunk's inbox is one box per use,
+// the tag is the solve's number.  LDS operations of a wave execute in issue
+// order, so between them fl_fence, which binds only the compiler, is enough.)
 
 // LDS progress words of a chunk, each written by one wave.
 struct FlProg {
