@@ -268,9 +268,9 @@ struct SpmvPlan {
   int nblocks = 0;        // row blocks
   DevBufPtr rowblk;       // int[nblocks + 1]: first row of each block
   int max_row = 0;
-  // the resident Jacobi PCG's analysis of the same matrix, made at its first
-  // solve (null: none yet)
-  mutable std::shared_ptr<ResPlan> res;
+  // the resident Jacobi PCG's analyses of the same matrix, made at its first
+  // solve as one system and as a batch (null: none yet)
+  mutable std::shared_ptr<ResPlan> res, res_batch;
 };
 // Finds or builds the plan for (ia, ja, n, nnz) (device arrays).
 const SpmvPlan *spmv_plan(int n, int nnz, const int *ia, const int *ja);
@@ -287,13 +287,19 @@ struct ResOut {
   int iterations, flag;
   double res0, res;
 };
-// The whole Jacobi PCG solve as one launch with the system in registers and
-// LDS (resident.hip).  hist: device, maxit + 2 entries; r, p: n-vectors of
-// scratch.  1: done (out filled), 0: the matrix does not fit (nothing was
-// launched that touches x), -1: an error was recorded.
-int pcg_resident(const SpmvPlan &A, const int *ia, const int *ja, const double *a,
-                 const double *d_r, double *x, const double *b, double tol, int maxit,
-                 double *hist, double *r, double *p, ResOut &out);
+// Jacobi PCG solves as one launch with the systems in registers and LDS
+// (resident.hip).  off: the systems' row offsets within the block-diagonal
+// matrix A (0, n: one system).  The plan may turn out not to fit (res_plan_ok
+// false).
+std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const int *ja,
+                                        const std::vector<int> &off);
+bool res_plan_ok(const ResPlan &P);
+bool res_plan_for(const ResPlan &P, const std::vector<int> &off);  // built for these systems
+// Solves; out: one per system.  hist: device, maxit + 2 entries (one system;
+// null: none); r, p: n-vectors of scratch.  1: done, -1: an error was recorded.
+int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double *d_r, double *x,
+                 const double *b, double tol, int maxit, double *hist, double *r, double *p,
+                 ResOut *out);
 
 // ------------------------------------------------- value-indexed CSR
 // Encodes a[0..nnz) as one-byte indices into a table of its distinct values

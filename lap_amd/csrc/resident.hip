@@ -26,10 +26,15 @@
 // the three dot products are summed in another fixed order (rows of a thread,
 // lanes of a wave, waves, workgroups).
 //
-// All workgroups must run at once: at most one per CU.  Waits are bounded and
-// one that runs out ends every workgroup with an error.
+// Several systems (lap_pcg_batched's lockstep mode) run in one launch, each by a
+// team of consecutive workgroups of its own, the largest first: as teams end,
+// the next ones take their CUs.  A team waits for its own workgroups only, and
+// workgroups start in order, so the first team still running always has all of
+// its workgroups.  A team is at most one workgroup per CU.  Waits are bounded
+// and one that runs out ends every workgroup with an error.
 #include <algorithm>
 #include <cmath>
+#include <numeric>
 
 #include "boxed.hpp"
 #include "lap_core.hpp"
@@ -48,19 +53,28 @@ constexpr int kResMaxWg = 256;     // workgroups at most (partials: one per thre
 // 3.89, 512^2 9.05 / 9.08 / 6.86, 40^3 7.15 / 6.66 / 6.70, 64^3 9.4 / 9.4 /
 // 11.1, 97 x 90 x 31 8.7 / 8.7 / 10.6: 2048 for rows of up to 5 entries.
 constexpr int kResRows = 1024, kResRowsShort = 2048, kResShort = 5;
-constexpr int kResMaxN = 1 << 19;  // rows at most (the analysis' bitmap in LDS)
+constexpr int kResMaxN = 1 << 19;  // rows of a system at most (the analysis' bitmap in LDS)
+constexpr int kResMaxRows = 1 << 26;  // rows of all systems at most (box_w stays below 2^31 bytes)
 constexpr int kResIters = 8192;    // iterations per launch
 constexpr unsigned kResSpins = 1u << 22;
 
 struct ResState {
   double rho, tolrel, res0, res;
   int iter, flag;  // flag: -1 not finished
-  int error;       // a wait ran out
-  unsigned tag;    // last tag used
+};
+struct ResShared {
+  int error;     // a wait ran out
+  unsigned tag;  // highest tag used
+};
+// A workgroup: its first row and row count, its team's first workgroup and
+// workgroup count, its system and that system's rows.
+struct ResWg {
+  int base, rows, team, size, sys, s0, s1, pad;
 };
 
 struct ResArgs {
-  int n, nr, nwg, nhmax;  // nr: rows per workgroup
+  int nhmax;
+  const ResWg *wg;
   const int *ia;
   const double *a;
   const unsigned short *lcol;
@@ -71,9 +85,11 @@ struct ResArgs {
   double tol;
   int maxit, resume, iters;
   unsigned tag0;
-  double *hist;
+  double *hist;  // of a single system (may be null)
   void *box_a, *box_b, *box_w;
-  ResState *st;
+  int n, nwg;
+  ResState *st;  // per system
+  ResShared *sh;
 };
 
 // Sum over the wave's first 16 (W16) or all 64 lanes, valid in the last of
@@ -101,12 +117,14 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {  // lane 63
 template <int R, int L>
 __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
   extern __shared__ double ps[];  // own rows, halo, a zero; the halo's rows
-  __shared__ double red[2][kResWaves], tot[2][4];
+  __shared__ double red[2][kResWaves], tot[2][4], one[2];
   __shared__ int dead;
   const int t = threadIdx.x, lane = t & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int w = blockIdx.x;
-  const int base = w * g.nr, rows = min(g.nr, g.n - base);
+  const ResWg wg = g.wg[w];
+  const int base = wg.base, rows = wg.rows, team = wg.team, size = wg.size;
+  ResState *const st = g.st + wg.sys;
   const int nh = g.hcnt[w];
   double *const halo = ps + R * kResThreads;
   const int zero = R * kResThreads + g.nhmax;
@@ -168,17 +186,17 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
   // once it has to be given up.
   auto again = [&](unsigned &spins) {
     if (++spins > kResSpins ||
-        ((spins & 63u) == 0 && __hip_atomic_load(&g.st->error, __ATOMIC_RELAXED,
+        ((spins & 63u) == 0 && __hip_atomic_load(&g.sh->error, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT))) {
       if (lane == 0) {
         dead = 1;
-        __hip_atomic_store(&g.st->error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&g.sh->error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       return false;
     }
     return true;
   };
-  // Sums of v over all workgroups (N = 1: box_a, 2: box_b), to every thread;
+  // Sums of v over the team (N = 1: box_a, 2: box_b), to every thread;
   // `between` runs while they are on their way.
   auto all_sums = [&](auto &v, unsigned tag, auto &&between) {
     constexpr int N = sizeof(v) / sizeof(v[0]);
@@ -193,27 +211,32 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         const double s = row_sum_dpp(lane < kResWaves ? red[i][lane] : 0.0);
-        if (lane == kResWaves - 1) fl_put(box, w * N + i, tag, s);
+        if (lane == kResWaves - 1) {
+          if (size > 1)
+            fl_put(box, w * N + i, tag, s);
+          else
+            one[i] = s;
+        }
       }
     }
     between();
-    if (wave < 4) {
+    if (wave < 4 && size > 1) {
       double got[N];
-      if (wave * kWave < g.nwg) {
+      if (wave * kWave < size) {
         FlBoxed<double> f[N];
         unsigned spins = 0;
         for (;;) {
           bool ok = true;
 #pragma unroll
-          for (int i = 0; i < N; ++i) f[i].load(box, t * N + i);
+          for (int i = 0; i < N; ++i) f[i].load(box, (team + t) * N + i);
 #pragma unroll
           for (int i = 0; i < N; ++i) ok = ok && f[i].is(tag);
           fl_fence();
-          if (__builtin_amdgcn_ballot_w64(!ok && t < g.nwg) == 0) break;
+          if (__builtin_amdgcn_ballot_w64(!ok && t < size) == 0) break;
           if (!again(spins)) break;
         }
 #pragma unroll
-        for (int i = 0; i < N; ++i) got[i] = t < g.nwg ? f[i].value() : 0.0;
+        for (int i = 0; i < N; ++i) got[i] = t < size ? f[i].value() : 0.0;
       } else {
 #pragma unroll
         for (int i = 0; i < N; ++i) got[i] = 0.0;
@@ -226,7 +249,8 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = ((tot[i][0] + tot[i][1]) + tot[i][2]) + tot[i][3];
+    for (int i = 0; i < N; ++i)
+      v[i] = size > 1 ? ((tot[i][0] + tot[i][1]) + tot[i][2]) + tot[i][3] : one[i];
   };
   // halo entries: p = w (first) or beta p + w, w as its owner sent it.  The
   // first entry of each thread is asked for ahead (halo_ask).
@@ -260,11 +284,11 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
   int it, flag = -1;
   unsigned tag = g.tag0;
   if (g.resume) {
-    rho = g.st->rho;
-    tolrel = g.st->tolrel;
-    res0 = g.st->res0;
-    res = g.st->res;
-    it = g.st->iter;
+    rho = st->rho;
+    tolrel = st->tolrel;
+    res0 = st->res0;
+    res = st->res;
+    it = st->iter;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
       const int row = base + t + k * kResThreads;
@@ -297,7 +321,7 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
     res0 = res = sqrt(v[1]);
     tolrel = g.tol * res0;
     it = 0;
-    if (w == 0 && t == 0) g.hist[0] = res0;
+    if (g.hist && w == 0 && t == 0) g.hist[0] = res0;
     if (!isfinite(res0)) flag = 2;
     if (res0 == 0.0) flag = 0;  // x0 solves the system
     flag = __builtin_amdgcn_readfirstlane(flag);
@@ -307,7 +331,7 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
     }
     __syncthreads();
   }
-  const int stop = it + g.iters;
+  const long long stop = (long long)it + g.iters;
   while (flag < 0 && it < stop && !__builtin_amdgcn_readfirstlane(dead)) {
     ++it;
     // q = A p, p.q, alpha
@@ -335,7 +359,7 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
     });
     // convergence test (cg.c:106-123) and beta
     res = sqrt(v[1]);
-    if (w == 0 && t == 0) g.hist[it] = res;
+    if (g.hist && w == 0 && t == 0) g.hist[it] = res;
     if (!isfinite(res)) flag = 2;
     else if (res < tolrel) flag = 0;
     else if (it > g.maxit) flag = 1;
@@ -359,23 +383,18 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
       g.p[row] = p[k];
     }
   }
-  if (w == 0 && t == 0) {
-    g.st->rho = rho;
-    g.st->tolrel = tolrel;
-    g.st->res0 = res0;
-    g.st->res = res;
-    g.st->iter = it;
-    g.st->flag = flag;
-    g.st->tag = tag;
+  if (w == team && t == 0) {
+    *st = ResState{rho, tolrel, res0, res, it, flag};
+    atomicMax(&g.sh->tag, tag);
   }
 }
 
 // The analysis: workgroup w lists the rows outside its own that its rows refer
 // to (ascending), marks them as sent, and gives every nonzero its slot: own
-// rows first, then the halo.  cnt[w]: the halo's length (more than kResHalo:
-// nothing else is written).  Dynamic LDS: a bitmap of the n rows and the rank
-// of each of its words.
-__global__ __launch_bounds__(kResThreads) void k_res_plan(int n, int nr, int own,
+// rows first, then the halo.  cnt[w]: the halo's length (more than kResHalo, or
+// a column outside the system: nothing else is written).  Dynamic LDS: a bitmap
+// of the system's rows and the rank of each of its words.
+__global__ __launch_bounds__(kResThreads) void k_res_plan(const ResWg *__restrict__ wgs, int own,
                                                           const int *__restrict__ ia,
                                                           const int *__restrict__ ja,
                                                           int *__restrict__ cnt,
@@ -384,16 +403,22 @@ __global__ __launch_bounds__(kResThreads) void k_res_plan(int n, int nr, int own
                                                           unsigned short *__restrict__ lcol) {
   extern __shared__ unsigned bits[];
   __shared__ int scan[kResThreads];
-  const int words = (n + 31) / 32;
-  unsigned short *rank = reinterpret_cast<unsigned short *>(bits + words);
+  __shared__ int bad;
   const int w = blockIdx.x, t = threadIdx.x;
-  const int base = w * nr, end = min(n, base + nr);
+  const ResWg wg = wgs[w];
+  const int words = (wg.s1 - wg.s0 + 31) / 32;
+  unsigned short *rank = reinterpret_cast<unsigned short *>(bits + words);
+  const int base = wg.base, end = wg.base + wg.rows;
   const int e0 = ia[base], e1 = ia[end];
+  if (t == 0) bad = 0;
   for (int i = t; i < words; i += kResThreads) bits[i] = 0;
   __syncthreads();
   for (int e = e0 + t; e < e1; e += kResThreads) {
-    const int c = ja[e];
-    if (c < base || c >= end) atomicOr(&bits[c >> 5], 1u << (c & 31));
+    const int c = ja[e], i = c - wg.s0;
+    if (c < wg.s0 || c >= wg.s1)
+      bad = 1;
+    else if (c < base || c >= end)
+      atomicOr(&bits[i >> 5], 1u << (i & 31));
   }
   __syncthreads();
   // ranks of the words: each thread a run of them
@@ -410,24 +435,24 @@ __global__ __launch_bounds__(kResThreads) void k_res_plan(int n, int nr, int own
     __syncthreads();
   }
   const int total = scan[kResThreads - 1];
-  if (t == 0) cnt[w] = total;
-  if (total > kResHalo) return;
+  if (t == 0) cnt[w] = bad ? kResHalo + 1 : total;
+  if (total > kResHalo || bad) return;
   int at = scan[t] - c;
   for (int i = i0; i < i1; ++i) {
     rank[i] = (unsigned short)at;
     for (unsigned m = bits[i]; m; m &= m - 1) {
-      const int col = i * 32 + __ffs((int)m) - 1;
+      const int col = wg.s0 + i * 32 + __ffs((int)m) - 1;
       hcol[(size_t)w * kResHalo + at++] = col;
       sent[col] = 1;
     }
   }
   __syncthreads();
   for (int e = e0 + t; e < e1; e += kResThreads) {
-    const int col = ja[e];
+    const int col = ja[e], i = col - wg.s0;
     lcol[e] = (unsigned short)(col >= base && col < end
                                    ? col - base
-                                   : own + rank[col >> 5] +
-                                         __popc(bits[col >> 5] & ((1u << (col & 31)) - 1u)));
+                                   : own + rank[i >> 5] +
+                                         __popc(bits[i >> 5] & ((1u << (i & 31)) - 1u)));
   }
 }
 
@@ -452,51 +477,76 @@ const ResShape kShapes[] = {{1, 8, k_resident<1, 8>},   {2, 8, k_resident<2, 8>}
 
 struct ResPlan {
   bool ok = false;
-  int nr = 0, nwg = 0, nhmax = 0, lds = 0;
+  std::vector<int> off;
+  int nsys = 0, nwg = 0, nhmax = 0, lds = 0;
   ResKernel fn = nullptr;
-  DevBufPtr hcnt, hcol, sent, lcol, boxes, state;
+  DevBufPtr wg, hcnt, hcol, sent, lcol, boxes, state, shared;
   size_t box_words = 0;
   unsigned tag = 0;
 };
 
-// Built at a matrix's first resident solve and kept with its SpMV plan.
-static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const int *ja) {
+std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const int *ja,
+                                        const std::vector<int> &off) {
   auto P = std::make_shared<ResPlan>();
-  const int n = A.n, cus = std::min(device_cus(), kResMaxWg);
-  if (n < 1 || n > kResMaxN || A.max_row > 32) return P;
+  P->off = off;
+  const int n = A.n, cus = std::min(device_cus(), kResMaxWg), ns = (int)off.size() - 1;
+  int big = 0;
+  for (int s = 0; s < ns; ++s) big = std::max(big, off[(size_t)s + 1] - off[(size_t)s]);
+  if (big < 1 || big > kResMaxN || n > kResMaxRows || A.max_row > 32) return P;
   const ResShape *s = nullptr;
-  int nr = 0;
   const int least = A.max_row <= kResShort ? kResRowsShort : kResRows;
+  auto rows_per = [&](int rows) {
+    return std::max(least, ((rows + cus - 1) / cus + kWave - 1) / kWave * kWave);
+  };
   for (const ResShape &c : kShapes) {
     if (A.max_row > c.l) continue;
-    nr = std::max(least, ((n + cus - 1) / cus + kWave - 1) / kWave * kWave);
-    if (nr <= c.r * kResThreads) {
+    if (rows_per(big) <= c.r * kResThreads) {
       s = &c;
       break;
     }
   }
   if (!s) return P;
-  P->nr = nr;
-  P->nwg = (n + nr - 1) / nr;
+  // teams, the largest system first
+  std::vector<int> ord((size_t)ns);
+  std::iota(ord.begin(), ord.end(), 0);
+  std::stable_sort(ord.begin(), ord.end(), [&](int u, int v) {
+    return off[(size_t)u + 1] - off[(size_t)u] > off[(size_t)v + 1] - off[(size_t)v];
+  });
+  std::vector<ResWg> wgs;
+  for (int q : ord) {
+    const int s0 = off[(size_t)q], s1 = off[(size_t)q + 1], rows = s1 - s0;
+    if (!rows) continue;
+    // as few workgroups as hold the rows, of about equal size
+    const int k = (rows + rows_per(rows) - 1) / rows_per(rows), team = (int)wgs.size();
+    const int nr = std::min(rows_per(rows), ((rows + k - 1) / k + kWave - 1) / kWave * kWave);
+    const int size = (rows + nr - 1) / nr;
+    for (int i = 0; i < size; ++i)
+      wgs.push_back(ResWg{s0 + i * nr, std::min(nr, rows - i * nr), team, size, q, s0, s1, 0});
+  }
+  P->nsys = ns;
+  P->nwg = (int)wgs.size();
   P->fn = s->fn;
-  const size_t words = ((size_t)n + 31) / 32;
+  P->wg = dev_upload(wgs);
   P->hcnt = dev_alloc(sizeof(int) * (size_t)P->nwg);
   P->hcol = dev_alloc(sizeof(int) * (size_t)P->nwg * kResHalo);
   P->sent = dev_alloc(((size_t)n + 3) / 4 * 4);
   P->lcol = dev_alloc(sizeof(unsigned short) * (size_t)std::max(A.nnz, 1));
-  P->state = dev_alloc(sizeof(ResState));
+  P->state = dev_alloc(sizeof(ResState) * (size_t)ns);
+  P->shared = dev_alloc(sizeof(ResShared));
   P->box_words = 4 * ((size_t)n + 3 * (size_t)P->nwg);
   P->boxes = dev_alloc(sizeof(unsigned) * P->box_words);
-  for (const DevBufPtr &b : {P->hcnt, P->hcol, P->sent, P->lcol, P->state, P->boxes})
+  for (const DevBufPtr &b : {P->wg, P->hcnt, P->hcol, P->sent, P->lcol, P->state, P->shared,
+                             P->boxes})
     if (!b->p) return P;
-  const int plan_lds = (int)(words * 4 + (words + 1) / 2 * 4);
+  const int words = (big + 31) / 32;
+  const int plan_lds = words * 4 + (words + 1) / 2 * 4;
   if (!LAP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_res_plan),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, plan_lds)))
     return P;
   k_res_zero<<<256, kBlock, 0, stream()>>>(((long long)n + 3) / 4, P->sent->as<unsigned>());
   k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P->box_words, P->boxes->as<unsigned>());
   k_res_plan<<<P->nwg, kResThreads, plan_lds, stream()>>>(
-      n, nr, s->r * kResThreads, ia, ja, P->hcnt->as<int>(), P->hcol->as<int>(),
+      P->wg->as<ResWg>(), s->r * kResThreads, ia, ja, P->hcnt->as<int>(), P->hcol->as<int>(),
       P->sent->as<unsigned char>(), P->lcol->as<unsigned short>());
   for (int c : dev_download(P->hcnt->as<int>(), (size_t)P->nwg)) P->nhmax = std::max(P->nhmax, c);
   if (lap_last_status() == LAP_ERR_HIP || P->nhmax > kResHalo) return P;
@@ -508,17 +558,17 @@ static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia,
   return P;
 }
 
-int pcg_resident(const SpmvPlan &A, const int *ia, const int *ja, const double *a,
-                 const double *d_r, double *x, const double *b, double tol, int maxit,
-                 double *hist, double *r, double *p, ResOut &out) {
-  if (!A.res) A.res = res_plan_build(A, ia, ja);
-  ResPlan &P = *A.res;
-  if (!P.ok) return 0;
+bool res_plan_ok(const ResPlan &P) { return P.ok; }
+bool res_plan_for(const ResPlan &P, const std::vector<int> &off) { return P.off == off; }
+
+int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double *d_r, double *x,
+                 const double *b, double tol, int maxit, double *hist, double *r, double *p,
+                 ResOut *out) {
   char *box = P.boxes->as<char>();
   ResArgs g{};
-  g.n = A.n;
-  g.nr = P.nr;
+  g.n = n;
   g.nwg = P.nwg;
+  g.wg = P.wg->as<ResWg>();
   g.nhmax = P.nhmax;
   g.ia = ia;
   g.a = a;
@@ -533,38 +583,49 @@ int pcg_resident(const SpmvPlan &A, const int *ia, const int *ja, const double *
   g.p = p;
   g.tol = tol;
   g.maxit = maxit;
-  g.iters = kResIters;
+  // one system: launches of kResIters iterations; several: one launch, so that
+  // a team's CUs go to the next one when it ends
+  g.iters = P.nsys == 1 ? kResIters : 0x7fffffff;
   g.hist = hist;
   g.box_a = box;
   g.box_b = box + 16 * (size_t)P.nwg;
   g.box_w = box + 48 * (size_t)P.nwg;
   g.st = P.state->as<ResState>();
-  k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResState) / 4), P.state->as<unsigned>());
-  ResState h{};
+  g.sh = P.shared->as<ResShared>();
+  std::vector<ResState> h((size_t)P.nsys);
+  auto clear_boxes = [&] {
+    k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P.box_words, P.boxes->as<unsigned>());
+    P.tag = 0;
+  };
+  if (P.tag > 0xf0000000u) clear_boxes();  // tags only grow
+  k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResState) / 4 * P.nsys),
+                                        P.state->as<unsigned>());
+  k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResShared) / 4),
+                                        P.shared->as<unsigned>());
   // iter <= maxit + 1, so this many launches always finish
   for (long k = 0; k <= (long)(maxit + 1) / kResIters + 1; ++k) {
     g.resume = k > 0;
     g.tag0 = P.tag;
     P.fn<<<P.nwg, kResThreads, P.lds, stream()>>>(g);
+    ResShared sh{};
     if (!LAP_HIP(hipGetLastError()) ||
-        !LAP_HIP(hipMemcpyAsync(&h, g.st, sizeof h, hipMemcpyDeviceToHost, stream())))
+        !LAP_HIP(hipMemcpyAsync(h.data(), g.st, sizeof(ResState) * h.size(),
+                                hipMemcpyDeviceToHost, stream())) ||
+        !LAP_HIP(hipMemcpyAsync(&sh, g.sh, sizeof sh, hipMemcpyDeviceToHost, stream())))
       return -1;
     sync();
     if (lap_last_status() == LAP_ERR_HIP) return -1;
-    if (h.error) {  // start over with unused tags next time
-      k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P.box_words,
-                                               P.boxes->as<unsigned>());
-      P.tag = 0;
+    if (sh.error) {  // start over with unused tags next time
+      clear_boxes();
       set_error(LAP_ERR_NUMERIC, "pcg: a wait between workgroups ran out");
       return -1;
     }
-    P.tag = h.tag;
-    if (h.flag >= 0) break;
+    P.tag = sh.tag;
+    if (P.nsys > 1 || h[0].flag >= 0) break;
   }
-  out.iterations = h.iter;
-  out.flag = h.flag < 0 ? 2 : h.flag;
-  out.res0 = h.res0;
-  out.res = h.res;
+  for (int s = 0; s < P.nsys; ++s)
+    out[s] = ResOut{h[(size_t)s].iter, h[(size_t)s].flag < 0 ? 2 : h[(size_t)s].flag,
+                    h[(size_t)s].res0, h[(size_t)s].res};
   return 1;
 }
 

@@ -100,3 +100,26 @@ def test_solve_longer_than_one_launch():
     assert abs(res.true_res - res.history[-1]) <= 9001 * 1e-16 * 100 * res.history.max()
     first = S.pcg(A, b, P, tol=0.0, maxit=8300)
     assert np.array_equal(res.history[:8302], first.history)
+
+
+def test_batch_of_uneven_systems_equals_single_solves():
+    """One launch over systems of one row to several workgroups: each system's
+    team has the workgroups its own solve would have, so x, iteration count
+    and flag are the single solves' bit for bit, whatever shares the launch."""
+    dims = [[1], [2048], [64, 32], [2049], [7, 9], [70, 90], [3], [130, 101], [61, 67]]
+    dims += [[5, 5 + k % 7] for k in range(300)]  # more teams than the chip has CUs
+    systems = [grid_laplacian(d, 0.05) for d in dims]
+    rng = np.random.default_rng(11)
+    rhs = [rng.standard_normal(A.n) for A in systems]
+    rhs[4][:] = 0.0
+    B = S.Batch.from_systems(systems, rhs)
+    x, it, fl, r0, rs, _ = S.pcg_batched(B, tol=1e-10, block=-1)
+    again, *_ = S.pcg_batched(B, tol=1e-10, block=-1)
+    assert torch.equal(x, again)
+    for k in list(range(9)) + [9, 100, 308]:
+        A = S.DeviceCSR.from_csr(systems[k])
+        P = S.make_preconditioner(A, systems[k], "line_jacobi")
+        one = S.pcg(A, S.to_dev(rhs[k]), P, tol=1e-10)
+        assert (it[k], fl[k], r0[k]) == (one.iterations, one.flag, one.res0), k
+        assert torch.equal(B.split(x)[k], one.x), k
+    assert it[4] == 0 and fl[4] == 0
