@@ -238,7 +238,8 @@ struct Options {
   int mixed_vectors = 0;   // lap_pcg_mixed inner vectors: 0 FP32, 1 FP64
   int sptrsv_long = 0;     // level solves' rows > kTriLongRow entries: 0 summed
                            // in CSR order (bitwise), 1 as a workgroup tree
-  int spmv_format = 0;     // PCG SpMV: 0 CSR values, 1 value-indexed when the
+  int spmv_format = 0;     // PCG SpMV: 0 CSR values, or row classes (cls.hpp) in
+                           // large systems; 1 value-indexed when the
                            // matrix has at most 255 distinct values, 2 also
                            // the columns as offset indices (<= 255 distinct
                            // col - row, rows <= 64 entries), else as 1

@@ -26,6 +26,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "cls.hpp"
 #include "lap_core.hpp"
 #include "spmv_core.hpp"
 
@@ -294,9 +295,81 @@ __global__ __launch_bounds__(BS) void k_spmv_pq_dvi(int nblk, const int *__restr
   if (threadIdx.x == 0) partials[blockIdx.x] = t;
 }
 
+// K_A over row classes (cls.hpp): a byte per row instead of its entries.  Same
+// row blocks, one lane per row, same products and order: bitwise the CSR
+// kernel.  Bound by the latency of its loads, so a workgroup has two row blocks
+// in flight (one of wide rows) and loads the next ones' bounds and classes
+// meanwhile, in the 64 registers that let all 8 workgroups of a CU run at once
+// (with 68 the grid's last eighth ran alone).
+template <int BS, int W>
+__global__ __launch_bounds__(BS, 8) void k_spmv_pq_cls(int nblk, const int *__restrict__ rowblk,
+                                                    const unsigned char *__restrict__ cls,
+                                                    int ncls, const int *__restrict__ off,
+                                                    const double *__restrict__ val,
+                                                    const int *__restrict__ len,
+                                                    const double *__restrict__ p,
+                                                    double *__restrict__ q, PcgCtl *ctl,
+                                                    double *partials, int xcd, int group) {
+  if (ctl->done) return;
+  if (ctl->pend_done) {  // the previous kernel stopped the solve: commit it
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->done = 1;
+    return;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0 && ctl->pend_valid) {
+    ctl->iter = ctl->pend_iter;
+    ctl->rho = ctl->pend_rho;
+    ctl->pend_valid = 0;
+  }
+  __shared__ double red[BS / kWave];
+  extern __shared__ double cls_lds[];
+  ClsLds<W> tab;
+  PqEpi epi{q, p, 0.0};
+  BlockWalk w = block_walk(nblk, xcd);
+  const int me = xcd == 0 ? cls_block(blockIdx.x, group) : (int)blockIdx.x;
+  if (xcd == 0) w.begin = me;
+  const int t = threadIdx.x;
+  struct Blk {
+    int r0, r1, c;
+  };
+  constexpr int K = W > 8 ? 1 : 2;
+  Blk cur[K], nxt[K];
+  auto ask = [&](int s) {
+    Blk k;
+    const int b = s < w.end ? w.block(s) : nblk;
+    k.r0 = b < nblk ? rowblk[b] : 0;
+    k.r1 = b < nblk ? rowblk[b + 1] : 0;
+    k.c = k.r0 + t < k.r1 ? cls[k.r0 + t] : 0;
+    return k;
+  };
+#pragma unroll
+  for (int u = 0; u < K; ++u) cur[u] = ask(w.begin + u * w.step);
+  tab.init(reinterpret_cast<char *>(cls_lds), ncls, off, val, len);
+  for (int s = w.begin; s < w.end; s += K * w.step) {
+    double xv[K][W];
+#pragma unroll
+    for (int u = 0; u < K; ++u) nxt[u] = ask(s + (K + u) * w.step);
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+      if (cur[u].r0 + t < cur[u].r1) tab.load(cur[u].c, p + (cur[u].r0 + t), xv[u]);
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      if (cur[u].r0 + t < cur[u].r1) epi.store(cur[u].r0 + t, tab.sum(cur[u].c, xv[u]));
+      for (int row = cur[u].r0 + BS + t; row < cur[u].r1; row += BS) {  // (spmv_rows > BS)
+        const int c = cls[row];
+        tab.load(c, p + row, xv[u]);
+        epi.store(row, tab.sum(c, xv[u]));
+      }
+      cur[u] = nxt[u];
+    }
+  }
+  const double t_pq = block_sum<BS>(epi.acc, red);
+  if (t == 0) partials[me] = t_pq;
+}
+
 // A value-indexed copy of the matrix for one solve (vi == nullptr and
-// code == nullptr: the CSR arrays are used).
+// code == nullptr and no classes: the CSR arrays are used).
 struct ViVals {
+  ClsMat cls;  // row classes
   const unsigned char *vi = nullptr;
   const double *dict = nullptr;
   int nd = 0;
@@ -307,9 +380,13 @@ struct ViVals {
 
 constexpr int kDviMaxRow = 64;
 
-// Encodes the matrix when options().spmv_format asks for it and it fits:
-// format 2 tries the delta-indexed form first, then (like format 1) the
-// value-indexed one.
+// Systems of fewer rows keep the CSR arrays in format 0: their matrix is in the
+// Infinity Cache and an iteration is mostly launches (at 10^6 rows of 7 entries
+// an iteration takes 45 us with the CSR arrays and 35 with classes).
+constexpr int kClsMinRows = 1 << 19;
+
+// Encodes the matrix as options().spmv_format asks and it fits: format 2 tries
+// the delta-indexed form first, then (like format 1) the value-indexed one.
 static ViVals vi_prepare(int nnz, const double *a, int n = 0, const int *ia = nullptr,
                          const int *ja = nullptr) {
   ViVals v;
@@ -361,15 +438,36 @@ __device__ __forceinline__ int stop_flag(double res, int it, const PcgCtl *ctl) 
 // can skip its rows' x update by seeing `done` early.  Same operations on the
 // same values as cg.c's order of updates.
 
+// 1/diag of row i: from the vector, or (row classes) one byte and a table in
+// LDS, 7 of 8 bytes less to read
+struct JacD {
+  const double *d_r;
+  __device__ __forceinline__ void init() {}
+  __device__ __forceinline__ double at(size_t i) const { return ld_nt(d_r + i); }
+};
+struct JacDCls {
+  const unsigned char *cls;
+  const double *d;
+  int ncls;
+  double *lds;
+  __device__ __forceinline__ void init() {
+    __shared__ double t[kClsMax + 1];
+    lds = t;
+    for (int i = threadIdx.x; i < ncls; i += blockDim.x) t[i] = d[i];
+    __syncthreads();
+  }
+  __device__ __forceinline__ double at(size_t i) const { return lds[ld_nt(cls + i)]; }
+};
+
 // K_B: alpha = rho/(p.q); r -= alpha q; partials of r.(d_r r) and r.r
-template <int BS>
+template <int BS, class D>
 __global__ __launch_bounds__(BS) void k_jac_update_nx(int n, double *__restrict__ r,
-                                                      const double *__restrict__ q,
-                                                      const double *__restrict__ d_r,
+                                                      const double *__restrict__ q, D d_r,
                                                       PcgCtl *ctl, const double *pq_part,
                                                       int pq_cnt, double *partials) {
   if (ctl->done) return;
   __shared__ double red[BS / kWave];
+  d_r.init();
   const double pq = sum_partials<BS>(pq_part, pq_cnt, 1, red);
   const double alpha = ctl->rho / pq, nalpha = -1.0 * alpha;
   double rz = 0.0, rr = 0.0;
@@ -379,7 +477,7 @@ __global__ __launch_bounds__(BS) void k_jac_update_nx(int n, double *__restrict_
   for (size_t i = (size_t)blockIdx.x * BS + threadIdx.x; i < (size_t)n; i += stride) {
     const double ri = ld_nt(r + i) + nalpha * ld_nt(q + i);
     st_nt(r + i, ri);
-    const double wi = ld_nt(d_r + i) * ri;
+    const double wi = d_r.at(i) * ri;
     rz += ri * wi;
     rr += ri * ri;
   }
@@ -393,14 +491,14 @@ __global__ __launch_bounds__(BS) void k_jac_update_nx(int n, double *__restrict_
 }
 
 // K_C: convergence test and beta; x += alpha p, then p = beta p + d_r r
-template <int BS>
+template <int BS, class D>
 __global__ __launch_bounds__(BS) void k_jac_px(int n, double *__restrict__ x,
-                                               const double *__restrict__ r,
-                                               const double *__restrict__ d_r,
+                                               const double *__restrict__ r, D d_r,
                                                double *__restrict__ p, PcgCtl *ctl,
                                                double *hist, const double *part, int cnt) {
   if (ctl->done) return;
   __shared__ double red[BS / kWave];
+  d_r.init();
   const double rz = sum_partials<BS>(part, cnt, 2, red);
   const double rr = sum_partials<BS>(part + 1, cnt, 2, red);
   const int it = ctl->iter + 1;
@@ -431,7 +529,7 @@ __global__ __launch_bounds__(BS) void k_jac_px(int n, double *__restrict__ x,
   for (size_t i = (size_t)blockIdx.x * BS + threadIdx.x; i < (size_t)n; i += stride) {
     const double pi = ld_nt(p + i);
     st_nt(x + i, ld_nt(x + i) + alpha * pi);
-    st_nt(p + i, pi * beta + ld_nt(d_r + i) * ld_nt(r + i));
+    st_nt(p + i, pi * beta + d_r.at(i) * ld_nt(r + i));
   }
 }
 
@@ -530,6 +628,19 @@ static void launch_spmv_pq(unsigned g, const SpmvPlan &A, const int *ia, const i
                            double *part, const ViVals &vv = ViVals()) {
   const int xcd = options().spmv_walk;
   const int *rb = A.rowblk->as<int>();
+  if (vv.cls.cls) {
+    const int group = cls_group(vv.cls.offsets, options().spmv_rows, g);
+    auto go = [&](auto *k, int rec) {
+      k<<<g, kBlock, vv.cls.ncls * rec, stream()>>>(A.nblocks, rb, vv.cls.cls, vv.cls.ncls,
+                                                    vv.cls.off, vv.cls.val, vv.cls.len, p, q, ctl,
+                                                    part, xcd, group);
+    };
+    if (vv.cls.width == 8)
+      go(k_spmv_pq_cls<kBlock, 8>, ClsLds<8>::kRec);
+    else
+      go(k_spmv_pq_cls<kBlock, 16>, ClsLds<16>::kRec);
+    return;
+  }
   if (vv.code) {
     k_spmv_pq_dvi<kBlock><<<g, kBlock, 0, stream()>>>(A.nblocks, rb, ia, vv.code, vv.dict, vv.nd,
                                                       vv.ddict, vv.ndl, p, q, ctl, part, xcd);
@@ -913,7 +1024,7 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
   LAP_HIP(hipEventRecord(ev0, stream()));
   launch_init(gA, A, ia, ja, a, x, b, r, R0);
   const bool jac = o.kind == P_JACOBI;
-  const ViVals vv = vi_prepare(nnz, a, n, ia, ja);
+  ViVals vv = vi_prepare(nnz, a, n, ia, ja);
   if (jac) {
     k_start<kBlock, true><<<gV, kBlock, 0, stream()>>>(n, R0, (int)gA, tol, r, pd->d_r, p, ctl,
                                                        hist, R1);
@@ -925,9 +1036,14 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
   auto iteration = [&]() {
     if (jac) {
       launch_spmv_pq(gA, A, ia, ja, a, p, q, ctl, R2, vv);
-      k_jac_update_nx<kBlock><<<gV, kBlock, 0, stream()>>>(n, r, q, pd->d_r, ctl, R2, (int)gA,
-                                                           R3);
-      k_jac_px<kBlock><<<gV, kBlock, 0, stream()>>>(n, x, r, pd->d_r, p, ctl, hist, R3, (int)gV);
+      auto vectors = [&](auto d) {
+        k_jac_update_nx<kBlock><<<gV, kBlock, 0, stream()>>>(n, r, q, d, ctl, R2, (int)gA, R3);
+        k_jac_px<kBlock><<<gV, kBlock, 0, stream()>>>(n, x, r, d, p, ctl, hist, R3, (int)gV);
+      };
+      if (vv.cls.cls)
+        vectors(JacDCls{vv.cls.cls, vv.cls.d, vv.cls.ncls, nullptr});
+      else
+        vectors(JacD{pd->d_r});
     } else {
       prec_launch(o, r, w, done);
       k_rw<kBlock><<<gV, kBlock, 0, stream()>>>(n, r, w, ctl, R1);
@@ -956,7 +1072,10 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
   int *flags = pinned_flags();
   if (!flags) status = LAP_ERR_HIP;
   hipGraphExec_t gexec = nullptr;
-  if (options().use_graph) {
+  auto capture = [&]() {
+    if (gexec) (void)hipGraphExecDestroy(gexec);
+    gexec = nullptr;
+    if (!options().use_graph) return true;
     hipGraph_t graph = nullptr;
     bool ok = LAP_HIP(hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal));
     if (ok) {
@@ -965,11 +1084,15 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
     }
     if (ok) ok = LAP_HIP(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
     if (graph) (void)hipGraphDestroy(graph);
-    if (!ok) {
-      gexec = nullptr;
-      status = LAP_ERR_HIP;
-    }
-  }
+    if (!ok) gexec = nullptr;
+    return ok;
+  };
+  if (!capture()) status = LAP_ERR_HIP;
+  // Row classes come in after the first batch of iterations: encoding (0.15 ms
+  // at 10^6 rows, 1.5 ms at 1.7 * 10^7, 0.08 ms to find too many) takes as long
+  // as 6 to 15 iterations win, which a solve that ends in the first batch would
+  // not get back.
+  const bool classes = options().spmv_format == 0 && n >= kClsMinRows;
   if (status == LAP_OK) {
     hipEvent_t pe[2];
     LAP_HIP(hipEventCreateWithFlags(&pe[0], hipEventDisableTiming));
@@ -978,6 +1101,13 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
     const long max_batches = (long)(maxit + 1) / G + 3;
     bool finished = false;
     for (long k = 0; k < max_batches + 1 && !finished; ++k) {
+      if (k == 1 && classes && LAP_HIP(hipEventSynchronize(pe[0])) && !flags[0]) {
+        vv.cls = cls_encode("a", n, nnz, ia, ja, a, jac ? pd->d_r : nullptr, A.max_row);
+        if (vv.cls.cls && !capture()) {
+          status = LAP_ERR_HIP;
+          break;
+        }
+      }
       if (k < max_batches) {
         if (gexec) {
           if (!LAP_HIP(hipGraphLaunch(gexec, stream()))) break;
@@ -1101,7 +1231,7 @@ double lap_pcg_spmv_timed(int n, int nnz, const int *ia, const int *ja, const do
   PcgCtl *ctl = reinterpret_cast<PcgCtl *>(scratch_vec("timed_ctl", sizeof(PcgCtl) / 8 + 1));
   LAP_HIP(hipMemcpyAsync(ctl, &h, sizeof h, hipMemcpyHostToDevice, stream()));
   const unsigned g = spmv_grid(*A);
-  const ViVals vv = vi_prepare(nnz, a, n, ia, ja);  // the kernel the solve would run
+  const ViVals vv = vi_prepare(nnz, a, n, ia, ja);  // (format 0: the CSR kernel)
   auto launch = [&]() { launch_spmv_pq(g, *A, ia, ja, a, p, q, ctl, ws.partials + kR2, vv); };
   launch();
   hipEvent_t e0, e1;

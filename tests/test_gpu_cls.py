@@ -1,0 +1,123 @@
+"""PCG with the matrix as row classes (the default for large systems with few
+distinct rows) against the CSR path: every product and sum is the same, so
+solutions, histories and flags are equal bit for bit.  Rows of 1 to 17 entries,
+few and too many classes, the first size that is encoded, ragged last row
+blocks, an inverse diagonal that does not follow from the row, and infinities.
+
+The CSR path is the one that option spmv_format 1 falls back to when the matrix
+has more than 255 distinct values, or the value-indexed one, which is bitwise
+the CSR one."""
+import numpy as np
+import pytest
+import torch
+
+from lap_amd import solver as S
+from lap_amd.problems import CSR, grid_laplacian
+
+pytestmark = pytest.mark.gpu
+
+MIN_ROWS = 1 << 19
+
+
+def band(n, offs, weights=None, shift=0.05):
+    """Graph Laplacian + shift of the graph i -- i + o (o in offs), by columns."""
+    i = np.arange(n, dtype=np.int64)
+    rows, cols, vals = [i], [i], [np.full(n, shift)]
+    for k, o in enumerate(offs):
+        w = np.ones(n - o) if weights is None else weights(i[: n - o], k)
+        lo, hi = i[: n - o], i[o:]
+        rows += [lo, hi]
+        cols += [hi, lo]
+        vals += [-w, -w]
+        vals[0][:n - o] += w
+        vals[0][o:] += w
+    rows, cols, vals = map(np.concatenate, (rows, cols, vals))
+    order = np.lexsort((cols, rows))
+    ia = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    return CSR(n, ia, cols[order].astype(np.int32), vals[order])
+
+
+def both(Ah, kind, b, maxit=40, d=None, x0=None, **opts):
+    A = S.DeviceCSR.from_csr(Ah)
+    P = S.make_preconditioner(A, Ah, kind)
+    if d is not None:
+        P.keep["d_r"].copy_(S.to_dev(d))
+    out = []
+    old = {k: S.set_option(k, v) for k, v in opts.items()}
+    try:
+        for fmt in (0, 1):
+            prev = S.set_option("spmv_format", fmt)
+            try:
+                kw = {} if x0 is None else {"x0": S.to_dev(x0)}
+                out.append(S.pcg(A, S.to_dev(b), P, tol=0.0, maxit=maxit, **kw))
+            finally:
+                S.set_option("spmv_format", prev)
+    finally:
+        for k, v in old.items():
+            S.set_option(k, v)
+    return out
+
+
+def same(r, s):
+    assert (r.iterations, r.flag) == (s.iterations, s.flag)
+    assert np.array_equal(r.history, s.history, equal_nan=True)
+    assert torch.equal(r.x.view(torch.int64), s.x.view(torch.int64))
+
+
+CASES = {
+    "first_encoded": lambda: band(MIN_ROWS, [1, 777]),
+    "last_csr": lambda: band(MIN_ROWS - 1, [1, 777]),
+    "cube_odd": lambda: grid_laplacian([83, 79, 89], 0.05),
+    "plane": lambda: grid_laplacian([1023, 517], 0.05),
+    "diagonal": lambda: CSR(MIN_ROWS + 5, np.arange(MIN_ROWS + 6, dtype=np.int32),
+                            np.arange(MIN_ROWS + 5, dtype=np.int32),
+                            1.0 + np.arange(MIN_ROWS + 5) % 3),
+    "row_9": lambda: band(MIN_ROWS + 257, [1, 2, 900, 901]),
+    "row_15": lambda: band(MIN_ROWS + 1, [1, 2, 3, 4, 5, 6, 1000]),
+    "row_17": lambda: band(MIN_ROWS + 1, [1, 2, 3, 4, 5, 6, 7, 1000]),  # too wide
+    "mixed_classes": lambda: band(MIN_ROWS + 99, [1, 512],  # many classes in every wave
+                                  lambda i, k: 1.0 + (i * 2654435761 % 97 % 2)),
+    "too_many": lambda: band(MIN_ROWS + 99, [1, 512], lambda i, k: 1.0 + (i * 37 + k) % 509),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_bitwise_the_csr_solve(name):
+    Ah = CASES[name]()
+    b = np.random.default_rng(3).standard_normal(Ah.n)
+    same(*both(Ah, "line_jacobi", b))
+
+
+@pytest.mark.parametrize("kind", ["none", "it_jacobi", "GS_it2", "ichol"])
+def test_other_preconditioners(kind):
+    Ah = grid_laplacian([91, 73, 83], 0.05)
+    b = np.random.default_rng(4).standard_normal(Ah.n)
+    same(*both(Ah, kind, b, maxit=20))
+
+
+@pytest.mark.parametrize("rows,walk", [(512, 0), (100, 0), (256, 3)])
+def test_row_blocks_and_walks(rows, walk):
+    Ah = grid_laplacian([81, 83, 85], 0.05)
+    b = np.random.default_rng(5).standard_normal(Ah.n)
+    same(*both(Ah, "line_jacobi", b, spmv_rows=rows, spmv_walk=walk))
+
+
+def test_inverse_diagonal_of_its_own():
+    """d_r with few values that do not follow the matrix's rows, and with many."""
+    Ah = grid_laplacian([90, 80, 85], 0.05)
+    rng = np.random.default_rng(6)
+    b = rng.standard_normal(Ah.n)
+    for d in (0.1 + 0.05 * (np.arange(Ah.n) % 7), rng.uniform(0.1, 0.2, Ah.n)):
+        same(*both(Ah, "line_jacobi", b, d=d))
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_not_finite(bad):
+    Ah = grid_laplacian([90, 80, 85], 0.05)
+    b = np.random.default_rng(7).standard_normal(Ah.n)
+    x0 = np.zeros(Ah.n)
+    x0[[0, 4321]] = bad
+    r, s = both(Ah, "line_jacobi", b, x0=x0, maxit=40)
+    assert (r.iterations, r.flag) == (s.iterations, s.flag)
+    assert np.array_equal(r.history, s.history, equal_nan=True)
+    assert torch.equal(torch.isnan(r.x), torch.isnan(s.x))
