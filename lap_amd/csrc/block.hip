@@ -8,31 +8,47 @@
 // i*k + j), so a row of P is one contiguous 8k-byte run and a CSR column
 // index addresses a whole run.
 //
-// SpMM: one column per lane; a wave holds G = 64/k row groups of k lanes.
-// Each group takes RU rows per step and, for each row, issues the loads of
-// EU nonzeros (column index, value, the P entries) before summing them, so a
-// lane keeps RU*EU gathers in flight; the sums themselves run in CSR order,
-// one per column, which is the reference's simple_csr_matvec sum
-// (simple_blas.c:24-44) bit for bit whatever RU is.  RU (1, 2, 4) is picked
-// per (matrix, k) by timing the candidates once.
+// SpMM: one column per lane; a wave holds G = 64/k row groups of k lanes and
+// takes kRW consecutive rows (a chunk) at a time, whose row pointers, column
+// indices and values it loads into LDS while it works on the chunk before: the
+// gathers of P then wait for nothing but P.  (Loading index, value and P one
+// after the other left 2/3 of the time to the index's latency.)  A gather past
+// a row's end reads +0.0 by the buffer's bounds check, which saves the compares
+// and selects of 8 nonzeros per row.  Each group takes RU rows per step
+// and issues the gathers of EU nonzeros of each before summing them; the sums
+// themselves run in CSR order, one per column, which is the reference's
+// simple_csr_matvec sum (simple_blas.c:24-44) bit for bit whatever RU is.  RU
+// (1, 2, 4) is picked per (matrix, k) by timing the candidates once.  A chunk
+// with too many nonzeros for its LDS reads them from memory as it goes.
+//
+// Workgroups are dealt to the 8 XCDs in turn, each with an L2 of its own, so
+// the chunks are handed out such that a row's neighbours are mostly worked on
+// by the same XCD (spmm_shape).
+//
+// Measured at 96^3, k = 32: 418 -> 200 us, the whole iteration 785 -> 505.  It
+// moves 347 MB in and 228 out of memory (the least is 300 and 226), and 1.4 GB
+// from the L2s to the CUs: 6 of the 8 rows of P that a row reads are not in the
+// CU's L1, and that is what bounds it now (RU, 2 to 8 workgroups per CU and
+// fewer instructions change little).
 //
 // Per-column scalars (rho, alpha, beta, tolrel, flags) live in a device
 // control block.  One iteration is five launches, graph-replayed:
 //   spmm    Q = A P, per-workgroup per-column partials of P.Q
-//   alpha   one workgroup: alpha_j = rho_j / (p.q)_j
+//   alpha   a workgroup per column: alpha_j = rho_j / (p.q)_j
 //   update  R -= alpha Q; partials of R.W (W = d_r R) and R.R
-//   conv    one workgroup: per-column convergence test (cg.c:106-123), beta
+//   conv    a workgroup per column: convergence test (cg.c:106-123), beta
 //   dir     X += alpha P for the columns live in this iteration, then
 //           P = beta P + d_r R for the columns still live
 // Moving x += alpha p from `update` into `dir` reads P once per iteration
 // instead of twice; the x of a column that stops is still updated in the
-// iteration it stops, as in cg.c (a final launch covers the last iteration,
-// whose `dir` is skipped once every column has stopped).  A stopped column
-// keeps its x, iteration count and residual, as a single-RHS solve does.
+// iteration it stops, as in cg.c.  A stopped column keeps its x, iteration
+// count and residual, as a single-RHS solve does.
 #include <algorithm>
 #include <climits>
 #include <cmath>
 
+#include "boxed.hpp"
+#include "cls.hpp"
 #include "lap_core.hpp"
 
 namespace lap {
@@ -40,92 +56,186 @@ namespace lap {
 namespace {
 
 constexpr int kMaxK = 64;         // columns per block solve
-constexpr int kRedThreads = 1024; // one-workgroup column reductions
 
 struct BlkCtl {
   double rho[kMaxK], alpha[kMaxK], beta[kMaxK], tolrel[kMaxK], res0[kMaxK], res[kMaxK];
   int done[kMaxK];  // column stopped (converged / maxit / non-finite)
   int xup[kMaxK];   // column was live in the last finished iteration
   int flag[kMaxK], iters[kMaxK];
-  int iter, maxit, all_done, pad;
+  int maxit, all_done;  // all_done: every column has stopped
+  int left, pad;        // columns that have not
 };
 
 // ---------------------------------------------------------------- SpMM
 
+// The rows a wave works on at a time, and the nonzeros of them it has room for
+// (a lane's loads of each).
+template <int K>
+struct Chunk {
+  static constexpr int G = 64 / K;
+  static constexpr int kRW = G > 16 ? G : 16;
+  static constexpr int kEPL = G > 16 ? 8 : 4;
+  static constexpr int kCap = kEPL * 64;
+};
+
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Q = A P for K columns.  MODE 0: plain (lap_csr_matmat); 1: partials of
 // P.Q per column; 2: Q = -(A P - B) (initial residual) with partials of
-// Q.Q.  Partials: part[blockIdx.x * K + col].
-template <int BS, int K, int RU, int EU, int MODE>
+// Q.Q.  Partials: part[col * gridDim.x + blockIdx.x].
+// FAR: P has 4 GB or more, beyond the 32-bit offsets of a buffer load.
+template <int BS, int K, int RU, int EU, int MODE, bool FAR>
 __global__ __launch_bounds__(BS) void k_spmm(int n, const int *__restrict__ ia,
                                              const int *__restrict__ ja,
                                              const double *__restrict__ a,
                                              const double *__restrict__ P, double *__restrict__ Q,
                                              const double *__restrict__ Bm, double *part,
-                                             const BlkCtl *ctl) {
+                                             const BlkCtl *ctl, int group) {
   if (MODE == 1 && ctl->all_done) return;
-  constexpr int G = 64 / K, NW = BS / 64;
+  using C = Chunk<K>;
+  constexpr int G = C::G, RW = C::kRW, EPL = C::kEPL, NW = BS / 64;
+  static_assert(RW % (G * RU) == 0 && RW <= 64, "whole steps per chunk");
+  // a nonzero: its value and the byte offset (FAR: the number) of its row of P;
+  // the last one stands for none
+  struct __align__(16) Nz {
+    double v;
+    unsigned at, pad;
+  };
+  __shared__ Nz s_nz[NW][C::kCap + 1];
+  __shared__ int s_ptr[NW][RW + 1];
   __shared__ double lds[K * NW];
   const int lane = threadIdx.x & 63;
-  // wave-uniform: with K = 64 every row index below is uniform, so the row
-  // pointers, column indices and values are scalar loads
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int g = lane / K, c = lane % K;
-  const int wave_id = (int)blockIdx.x * NW + wave, nwaves = (int)gridDim.x * NW;
+  Nz *const nz = s_nz[wave];
+  int *const ptr = s_ptr[wave];
+  constexpr unsigned kRowBytes = FAR ? 1 : K * 8, kNone = 0xffffffffu;
+  if (lane == 0) nz[C::kCap] = Nz{0.0, kNone, 0};
+  const __amdgpu_buffer_rsrc_t pb = fl_buffer(P, FAR ? 0 : (unsigned)((size_t)n * K * 8));
+  // P at a nonzero's row; +0.0 where there is none, which with the value 0
+  // leaves a sum as it is (it started at +0.0, so it is never -0.0)
+  auto gather = [&](unsigned at) {
+    if constexpr (FAR) return at != kNone ? P[(size_t)at * K + c] : 0.0;
+    // (no row at kNone: the load's bounds check gives 0)
+    const fl_u2 u = __builtin_amdgcn_raw_buffer_load_b64(pb, at | (unsigned)(c * 8), 0, 0);
+    return fl_f64(u.x, u.y);
+  };
+  const int nblk = (n - 1) / (RW * NW) + 1;
+
+  // a chunk's row pointers (lane l: rows l and l + 1), then its entries
+  struct Ptr {
+    int row0, p0, p1;
+  };
+  struct Ent {
+    int row0, p0, e0, cnt;
+    int j[EPL];
+    double v[EPL];
+  };
+  auto ask_ptr = [&](int blk) {
+    Ptr p;
+    p.row0 = blk < nblk ? (blk * NW + wave) * RW : n;
+    p.p0 = p.p1 = 0;
+    if (lane < RW) {
+      p.p0 = ia[p.row0 + min(lane, n - p.row0)];
+      p.p1 = ia[p.row0 + min(lane + 1, n - p.row0)];
+    }
+    return p;
+  };
+  auto ask_ent = [&](const Ptr &p) {
+    Ent e;
+    e.row0 = p.row0;
+    e.e0 = __builtin_amdgcn_readfirstlane(p.p0);
+    e.cnt = __builtin_amdgcn_readlane(p.p1, RW - 1) - e.e0;
+    e.p0 = p.p0 - e.e0;
+    if (e.cnt <= C::kCap) {
+#pragma unroll
+      for (int u = 0; u < EPL; ++u) {
+        const int i = u * 64 + lane;
+        e.j[u] = i < e.cnt ? ja[e.e0 + i] : 0;
+        e.v[u] = i < e.cnt ? a[e.e0 + i] : 0.0;
+      }
+    }
+    return e;
+  };
   double acc = 0.0;
-  for (long base = (long)wave_id * G * RU; base < n; base += (long)nwaves * G * RU) {
-    int e0[RU], e1[RU];
+  // the rows of a chunk; entry(e, end): its e-th nonzero, or none from end on
+  auto work = [&](int row0, auto entry) {
+    for (int base = 0; base < RW && base < n - row0; base += G * RU) {
+      int e0[RU], e1[RU];
+      double s[RU], own[RU];
 #pragma unroll
-    for (int j = 0; j < RU; ++j) {
-      const long row = base + (long)j * G + g;
-      e0[j] = row < n ? ia[row] : 0;
-      e1[j] = row < n ? ia[row + 1] : 0;
-    }
-    double s[RU];
+      for (int j = 0; j < RU; ++j) {
+        const int r = base + j * G + g;
+        e0[j] = ptr[r];
+        e1[j] = ptr[r + 1];
+        s[j] = 0.0;
+        if (MODE == 1) own[j] = r < n - row0 ? P[(size_t)(row0 + r) * K + c] : 0.0;
+      }
+      for (int off = 0;; off += EU) {
+        bool any = false;
 #pragma unroll
-    for (int j = 0; j < RU; ++j) s[j] = 0.0;
-    for (int off = 0;; off += EU) {
-      bool any = false;
+        for (int j = 0; j < RU; ++j) any |= e0[j] + off < e1[j];
+        if (!any) break;
+        double av[RU][EU], v[RU][EU];
 #pragma unroll
-      for (int j = 0; j < RU; ++j) any |= e0[j] + off < e1[j];
-      if (!any) break;
-      bool ok[RU][EU];
-      int col[RU][EU];
-      double av[RU][EU], v[RU][EU];
+        for (int j = 0; j < RU; ++j)
 #pragma unroll
-      for (int j = 0; j < RU; ++j)
+          for (int t = 0; t < EU; ++t) {
+            const Nz x = entry(e0[j] + off + t, e1[j]);
+            av[j][t] = x.v;
+            v[j][t] = gather(x.at);
+          }
 #pragma unroll
-        for (int t = 0; t < EU; ++t) {
-          const int e = e0[j] + off + t;
-          ok[j][t] = e < e1[j];
-          col[j][t] = ok[j][t] ? ja[e] : 0;
-          av[j][t] = ok[j][t] ? a[e] : 0.0;
-        }
+        for (int j = 0; j < RU; ++j)
 #pragma unroll
-      for (int j = 0; j < RU; ++j)
+          for (int t = 0; t < EU; ++t) s[j] += av[j][t] * v[j][t];
+      }
 #pragma unroll
-        for (int t = 0; t < EU; ++t)
-          v[j][t] = ok[j][t] ? P[(size_t)col[j][t] * K + c] : 0.0;
-#pragma unroll
-      for (int j = 0; j < RU; ++j)
-#pragma unroll
-        for (int t = 0; t < EU; ++t)
-          if (ok[j][t]) s[j] += av[j][t] * v[j][t];
-    }
-#pragma unroll
-    for (int j = 0; j < RU; ++j) {
-      const long row = base + (long)j * G + g;
-      if (row < n) {
-        const size_t o = (size_t)row * K + c;
-        if (MODE == 2) {
-          const double r = -(s[j] - Bm[o]);  // r = A x; r += -1*b; r *= -1
-          Q[o] = r;
-          acc += r * r;
-        } else {
-          Q[o] = s[j];
-          if (MODE == 1) acc += P[o] * s[j];
+      for (int j = 0; j < RU; ++j) {
+        const int row = row0 + base + j * G + g;
+        if (row < n) {
+          const size_t o = (size_t)row * K + c;
+          if (MODE == 2) {
+            const double r = -(s[j] - Bm[o]);  // r = A x; r += -1*b; r *= -1
+            Q[o] = r;
+            acc += r * r;
+          } else {
+            st_nt(Q + o, s[j]);
+            if (MODE == 1) acc += own[j] * s[j];
+          }
         }
       }
     }
+  };
+
+  const int first = cls_block(blockIdx.x, group), step = (int)gridDim.x;
+  Ptr p = ask_ptr(first);
+  Ent e = ask_ent(p);
+  p = ask_ptr(first + step);
+  for (int blk = first; blk < nblk; blk += step) {
+    const int row0 = e.row0, cnt = e.cnt, eb = e.e0;
+    wave_sync();  // (the last chunk's reads are done)
+    if (lane < RW) ptr[lane] = e.p0;
+    if (lane == 0) ptr[RW] = cnt;
+    if (cnt <= C::kCap) {
+#pragma unroll
+      for (int u = 0; u < EPL; ++u) {
+        nz[u * 64 + lane] = Nz{e.v[u], (unsigned)e.j[u] * kRowBytes, 0};
+      }
+    }
+    wave_sync();
+    e = ask_ent(p);
+    p = ask_ptr(blk + 2 * step);
+    if (cnt <= C::kCap)
+      work(row0, [&](int i, int end) { return nz[i < end ? i : C::kCap]; });
+    else
+      work(row0, [&](int i, int end) {
+        if (i >= end) return Nz{0.0, kNone, 0};
+        return Nz{a[eb + i], (unsigned)ja[eb + i] * kRowBytes, 0};
+      });
   }
   if (MODE == 0) return;
   // fixed-order reduction: butterfly over the row groups of a wave, then
@@ -136,157 +246,35 @@ __global__ __launch_bounds__(BS) void k_spmm(int n, const int *__restrict__ ia,
   for (int cc = threadIdx.x; cc < K; cc += BS) {
     double t = 0.0;
     for (int w = 0; w < NW; ++w) t += lds[cc * NW + w];
-    part[(size_t)blockIdx.x * K + cc] = t;
-  }
-}
-
-// K = 64, wave-cooperative: one wave = the 64 columns of a row; a step takes
-// RU consecutive rows, whose nonzeros are contiguous in CSR, so their
-// column indices and values arrive in one coalesced load per 64 entries and
-// v_readlane hands each entry to the whole wave.  The gathers of up to 16
-// entries are issued before they are summed; rows are summed in CSR order
-// and written as soon as they end.  Control flow is wave-uniform.
-__device__ __forceinline__ double readlane_f64(double v, int l) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), l);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
-template <int BS, int RU, int MODE>
-__global__ __launch_bounds__(BS) void k_spmm64(int n, const int *__restrict__ ia,
-                                               const int *__restrict__ ja,
-                                               const double *__restrict__ a,
-                                               const double *__restrict__ P,
-                                               double *__restrict__ Q,
-                                               const double *__restrict__ Bm, double *part,
-                                               const BlkCtl *ctl) {
-  static_assert(RU < 64, "row pointers of a step fit one wave");
-  if (MODE == 1 && ctl->all_done) return;
-  constexpr int K = 64, NW = BS / 64, EB = 16;
-  __shared__ double lds[K * NW];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int wave_id = (int)blockIdx.x * NW + wave, nwaves = (int)gridDim.x * NW;
-  double acc = 0.0;
-  // P's own row for the p.q epilogue: the diagonal entry's gather already
-  // holds it (loaded only for a row without a stored diagonal)
-  double pown = 0.0;
-  bool have_own = false;
-  auto finish = [&](int row, double sum) {
-    const size_t o = (size_t)row * K + lane;
-    if (MODE == 2) {
-      const double r = -(sum - Bm[o]);  // r = A x; r += -1*b; r *= -1
-      Q[o] = r;
-      acc += r * r;
-    } else {
-      Q[o] = sum;
-      if (MODE == 1) acc += (have_own ? pown : P[o]) * sum;
-    }
-    have_own = false;
-  };
-  for (int base = wave_id * RU; base < n; base += nwaves * RU) {
-    const int nrows = min(RU, n - base);
-    const int ptr_l = lane <= nrows ? ia[base + lane] : 0;
-    const int e_begin = __builtin_amdgcn_readlane(ptr_l, 0);
-    const int e_end = __builtin_amdgcn_readlane(ptr_l, nrows);
-    int j = 0;                                             // row within the step
-    int next = __builtin_amdgcn_readlane(ptr_l, 1);        // end of row j
-    double cur = 0.0;
-    for (int c0 = e_begin; c0 < e_end; c0 += 64) {
-      const int cnt = min(64, e_end - c0);
-      const int jl = lane < cnt ? ja[c0 + lane] : 0;
-      const double al = lane < cnt ? a[c0 + lane] : 0.0;
-      for (int t0 = 0; t0 < cnt; t0 += EB) {
-        double v[EB];
-#pragma unroll
-        for (int u = 0; u < EB; ++u)
-          if (t0 + u < cnt)
-            v[u] = P[(size_t)__builtin_amdgcn_readlane(jl, t0 + u) * K + lane];
-#pragma unroll
-        for (int u = 0; u < EB; ++u) {
-          if (t0 + u < cnt) {
-            const int e = c0 + t0 + u;
-            while (e >= next) {  // row j ends before entry e
-              finish(base + j, cur);
-              cur = 0.0;
-              ++j;
-              next = __builtin_amdgcn_readlane(ptr_l, j + 1);
-            }
-            if (MODE == 1 && __builtin_amdgcn_readlane(jl, t0 + u) == base + j) {
-              pown = v[u];
-              have_own = true;
-            }
-            cur += readlane_f64(al, t0 + u) * v[u];
-          }
-        }
-      }
-    }
-    while (j < nrows) {  // the last row with entries, then empty rows
-      finish(base + j, cur);
-      cur = 0.0;
-      ++j;
-    }
-  }
-  if (MODE == 0) return;
-  lds[lane * NW + wave] = acc;
-  __syncthreads();
-  for (int cc = threadIdx.x; cc < K; cc += BS) {
-    double t = 0.0;
-    for (int w = 0; w < NW; ++w) t += lds[cc * NW + w];
-    part[(size_t)blockIdx.x * K + cc] = t;
+    part[(size_t)cc * gridDim.x + blockIdx.x] = t;
   }
 }
 
 // --------------------------------------------------- column reductions
+// A workgroup per column (blockIdx.x): its partial sums lie together.
 
-// One workgroup of kRedThreads: out[j] = sum over b < nparts of
-// part[b * stride + j], j < k, in a fixed order.
-__device__ __forceinline__ void column_sums(const double *part, int nparts, int stride, int k,
-                                            double *lds, double *out) {
-  const int nchunk = kRedThreads / k;  // k | 1024
-  const int col = threadIdx.x % k, chunk = threadIdx.x / k;
-  double s = 0.0;
-  for (int b = chunk; b < nparts; b += nchunk) s += part[(size_t)b * stride + col];
-  lds[threadIdx.x] = s;
-  __syncthreads();
-  if (threadIdx.x < k) {
-    double t = 0.0;
-    for (int ch = 0; ch < nchunk; ++ch) t += lds[ch * k + threadIdx.x];
-    out[threadIdx.x] = t;
-  }
-  __syncthreads();
+// column `j` stops; the last one ends the solve
+__device__ __forceinline__ void stop_column(BlkCtl *ctl, int j) {
+  ctl->done[j] = 1;
+  if (atomicSub(&ctl->left, 1) == 1) ctl->all_done = 1;
 }
 
-// start: ||r0||, tolrel and the stop state of every column
-__global__ __launch_bounds__(kRedThreads) void k_blk_res0(const double *part, int nparts, int k,
-                                                          double tol, int maxit, BlkCtl *ctl,
-                                                          double *hist) {
-  __shared__ double lds[kRedThreads];
-  __shared__ double sums[kMaxK];
-  __shared__ int any_live;
-  if (threadIdx.x == 0) any_live = 0;
-  column_sums(part, nparts, k, k, lds, sums);
-  if (threadIdx.x < k) {
-    const int j = threadIdx.x;
-    const double r0 = sqrt(sums[j]);
-    const bool stop = !isfinite(r0) || r0 == 0.0;  // r0 == 0: x0 solves column j
-    ctl->res0[j] = r0;
-    ctl->res[j] = r0;
-    ctl->tolrel[j] = tol * r0;
-    ctl->iters[j] = 0;
-    ctl->flag[j] = isfinite(r0) ? 0 : 2;
-    ctl->done[j] = stop ? 1 : 0;
-    ctl->xup[j] = 0;
-    if (hist) hist[j] = r0;
-    if (!stop) atomicOr(&any_live, 1);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    ctl->iter = 0;
-    ctl->maxit = maxit;
-    ctl->all_done = any_live ? 0 : 1;
-  }
+// start: ||r0||, tolrel and the stop state of the column
+template <int BS>
+__global__ __launch_bounds__(BS) void k_blk_res0(const double *part, int nparts, double tol,
+                                                 BlkCtl *ctl, double *hist) {
+  __shared__ double red[BS / kWave];
+  const int j = blockIdx.x;
+  const double sum = sum_partials<BS>(part + (size_t)j * nparts, nparts, 1, red);
+  if (threadIdx.x != 0) return;
+  const double r0 = sqrt(sum);
+  const bool stop = !isfinite(r0) || r0 == 0.0;  // r0 == 0: x0 solves column j
+  ctl->res0[j] = r0;
+  ctl->res[j] = r0;
+  ctl->tolrel[j] = tol * r0;
+  ctl->flag[j] = isfinite(r0) ? 0 : 2;
+  if (hist) hist[j] = r0;
+  if (stop) stop_column(ctl, j);
 }
 
 // W = d_r R; P = W; per-workgroup partials of R.W
@@ -309,31 +297,31 @@ __global__ __launch_bounds__(BS) void k_blk_start(int n, int k, int lk,
   for (int col = threadIdx.x; col < k; col += BS) {
     double s = 0.0;
     for (int t = col; t < BS; t += k) s += lds[t];
-    part[(size_t)blockIdx.x * k + col] = s;
+    part[(size_t)col * gridDim.x + blockIdx.x] = s;
   }
 }
 
 // rho_j from the R.W partials
-__global__ __launch_bounds__(kRedThreads) void k_blk_rho(const double *part, int nparts, int k,
-                                                         BlkCtl *ctl) {
-  __shared__ double lds[kRedThreads];
-  __shared__ double sums[kMaxK];
-  column_sums(part, nparts, k, k, lds, sums);
-  if (threadIdx.x < k) ctl->rho[threadIdx.x] = sums[threadIdx.x];
+template <int BS>
+__global__ __launch_bounds__(BS) void k_blk_rho(const double *part, int nparts, BlkCtl *ctl) {
+  __shared__ double red[BS / kWave];
+  const int j = blockIdx.x;
+  const double sum = sum_partials<BS>(part + (size_t)j * nparts, nparts, 1, red);
+  if (threadIdx.x == 0) ctl->rho[j] = sum;
 }
 
 // alpha_j = rho_j / (p.q)_j
-__global__ __launch_bounds__(kRedThreads) void k_blk_alpha(const double *part, int nparts, int k,
-                                                           BlkCtl *ctl) {
-  if (ctl->all_done) return;
-  __shared__ double lds[kRedThreads];
-  __shared__ double sums[kMaxK];
-  column_sums(part, nparts, k, k, lds, sums);
-  if (threadIdx.x < k) ctl->alpha[threadIdx.x] = ctl->rho[threadIdx.x] / sums[threadIdx.x];
+template <int BS>
+__global__ __launch_bounds__(BS) void k_blk_alpha(const double *part, int nparts, BlkCtl *ctl) {
+  __shared__ double red[BS / kWave];
+  const int j = blockIdx.x;
+  if (ctl->done[j]) return;
+  const double sum = sum_partials<BS>(part + (size_t)j * nparts, nparts, 1, red);
+  if (threadIdx.x == 0) ctl->alpha[j] = ctl->rho[j] / sum;
 }
 
 // R -= alpha Q for the live columns; per-workgroup partials of R.W and R.R
-// (part[b*2k + j] and part[b*2k + k + j])
+// (part[j * gridDim.x + b] and part[(k + j) * gridDim.x + b])
 template <int BS>
 __global__ __launch_bounds__(BS) void k_blk_update(int n, int k, int lk, double *__restrict__ R,
                                                    const double *__restrict__ Q,
@@ -364,101 +352,105 @@ __global__ __launch_bounds__(BS) void k_blk_update(int n, int k, int lk, double 
       s1 += lds[t];
       s2 += lds[BS + t];
     }
-    part[(size_t)blockIdx.x * 2 * k + cc] = s1;
-    part[(size_t)blockIdx.x * 2 * k + k + cc] = s2;
+    part[(size_t)cc * gridDim.x + blockIdx.x] = s1;
+    part[(size_t)(k + cc) * gridDim.x + blockIdx.x] = s2;
   }
 }
 
-// per-column convergence test (cg.c:106-123) and beta; hist[it*k + j]
-__global__ __launch_bounds__(kRedThreads) void k_blk_conv(const double *part, int nparts, int k,
-                                                          double *hist, BlkCtl *ctl) {
-  if (ctl->all_done) return;
-  __shared__ double lds[kRedThreads];
-  __shared__ double rz[kMaxK], rr[kMaxK];
-  __shared__ int any_live;
-  if (threadIdx.x == 0) any_live = 0;
-  column_sums(part, nparts, 2 * k, k, lds, rz);
-  column_sums(part + k, nparts, 2 * k, k, lds, rr);
-  const int it = ctl->iter + 1;
-  if (threadIdx.x < k) {
-    const int j = threadIdx.x;
-    const bool live = !ctl->done[j];
-    ctl->xup[j] = live ? 1 : 0;
-    if (live) {
-      const double res = sqrt(rr[j]);
-      ctl->res[j] = res;
-      ctl->iters[j] = it;
-      if (hist) hist[(size_t)it * k + j] = res;
-      int flag = -1;
-      if (!isfinite(res))
-        flag = 2;
-      else if (res < ctl->tolrel[j])
-        flag = 0;
-      else if (it > ctl->maxit)
-        flag = 1;
-      if (flag >= 0) {
-        ctl->flag[j] = flag;
-        ctl->done[j] = 1;
-      } else {
-        ctl->beta[j] = rz[j] / ctl->rho[j];
-        ctl->rho[j] = rz[j];
-        atomicOr(&any_live, 1);
-      }
-    }
+// convergence test of the column (cg.c:106-123) and beta; hist[it*k + j]
+template <int BS>
+__global__ __launch_bounds__(BS) void k_blk_conv(const double *part, int nparts, double *hist,
+                                                 BlkCtl *ctl) {
+  __shared__ double red[BS / kWave];
+  const int j = blockIdx.x, k = gridDim.x;
+  if (ctl->done[j]) {  // its x has had its last update
+    if (threadIdx.x == 0) ctl->xup[j] = 0;
+    return;
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    ctl->iter = it;
-    ctl->all_done = any_live ? 0 : 1;
+  const double rz = sum_partials<BS>(part + (size_t)j * nparts, nparts, 1, red);
+  const double rr = sum_partials<BS>(part + (size_t)(k + j) * nparts, nparts, 1, red);
+  if (threadIdx.x != 0) return;
+  const int it = ctl->iters[j] + 1;
+  const double res = sqrt(rr);
+  ctl->xup[j] = 1;
+  ctl->res[j] = res;
+  ctl->iters[j] = it;
+  if (hist) hist[(size_t)it * k + j] = res;
+  int flag = -1;
+  if (!isfinite(res))
+    flag = 2;
+  else if (res < ctl->tolrel[j])
+    flag = 0;
+  else if (it > ctl->maxit)
+    flag = 1;
+  if (flag >= 0) {
+    ctl->flag[j] = flag;
+    stop_column(ctl, j);
+  } else {
+    ctl->beta[j] = rz / ctl->rho[j];
+    ctl->rho[j] = rz;
   }
 }
 
 // X += alpha P (columns live in this iteration); P = beta P + d_r R
-// (columns still live).  FINAL: the X update of the last iteration only.
-template <int BS, bool FINAL>
+// (columns still live).  Four elements' loads in flight per thread: 177 us for
+// 1.13 GB at 96^3, k = 32 (one: 208).
+constexpr int kVU = 4;
+template <int BS>
 __global__ __launch_bounds__(BS) void k_blk_dir(int n, int k, int lk, double *__restrict__ X,
                                                 const double *__restrict__ R,
                                                 const double *__restrict__ d_r,
                                                 double *__restrict__ P, const BlkCtl *ctl) {
-  if (!FINAL && ctl->all_done) return;
   const int col = (int)threadIdx.x & (k - 1);
-  const bool xup = ctl->xup[col], live = !FINAL && !ctl->done[col];
+  const bool xup = ctl->xup[col], live = !ctl->done[col];
   if (!xup && !live) return;
   const double alpha = ctl->alpha[col], beta = ctl->beta[col];
   const size_t total = (size_t)n * k, stride = (size_t)gridDim.x * BS;
-  for (size_t o = (size_t)blockIdx.x * BS + threadIdx.x; o < total; o += stride) {
-    const double pv = ld_nt(P + o);
-    if (xup) st_nt(X + o, ld_nt(X + o) + alpha * pv);                    // x += alpha*p
-    if (live) st_nt(P + o, pv * beta + d_r[o >> lk] * ld_nt(R + o));  // p = beta p + w
+  for (size_t o0 = (size_t)blockIdx.x * BS + threadIdx.x; o0 < total; o0 += kVU * stride) {
+    double p[kVU], x[kVU], r[kVU], d[kVU];
+#pragma unroll
+    for (int u = 0; u < kVU; ++u) {
+      const size_t o = o0 + u * stride;
+      if (o >= total) continue;
+      p[u] = ld_nt(P + o);
+      x[u] = xup ? ld_nt(X + o) : 0.0;
+      r[u] = live ? ld_nt(R + o) : 0.0;
+      d[u] = live ? d_r[o >> lk] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < kVU; ++u) {
+      const size_t o = o0 + u * stride;
+      if (o >= total) continue;
+      if (xup) st_nt(X + o, x[u] + alpha * p[u]);             // x += alpha*p
+      if (live) st_nt(P + o, p[u] * beta + d[u] * r[u]);  // p = beta p + w
+    }
   }
 }
 
-using SpmmFn = void (*)(unsigned, int, const int *, const int *, const double *, const double *,
+// The workgroups of an SpMM and how they are dealt to the XCDs (cls_block).
+struct SpmmShape {
+  unsigned grid;
+  int group;
+};
+
+using SpmmFn = void (*)(SpmmShape, int, const int *, const int *, const double *, const double *,
                         double *, const double *, double *, const BlkCtl *, int);
 
-template <int K, int RU>
-void spmm_launch(unsigned g, int n, const int *ia, const int *ja, const double *a,
+template <int K, int RU0>
+void spmm_launch(SpmmShape g, int n, const int *ia, const int *ja, const double *a,
                  const double *P, double *Q, const double *Bm, double *part, const BlkCtl *ctl,
                  int mode) {
-  constexpr int EU = RU == 1 ? 8 : 4;
-  if (mode == 2)
-    k_spmm<kBlock, K, RU, EU, 2><<<g, kBlock, 0, stream()>>>(n, ia, ja, a, P, Q, Bm, part, ctl);
-  else if (mode == 1)
-    k_spmm<kBlock, K, RU, EU, 1><<<g, kBlock, 0, stream()>>>(n, ia, ja, a, P, Q, Bm, part, ctl);
-  else
-    k_spmm<kBlock, K, RU, EU, 0><<<g, kBlock, 0, stream()>>>(n, ia, ja, a, P, Q, Bm, part, ctl);
-}
-
-template <int RU>
-void spmm64_launch(unsigned g, int n, const int *ia, const int *ja, const double *a,
-                   const double *P, double *Q, const double *Bm, double *part, const BlkCtl *ctl,
-                   int mode) {
-  if (mode == 2)
-    k_spmm64<kBlock, RU, 2><<<g, kBlock, 0, stream()>>>(n, ia, ja, a, P, Q, Bm, part, ctl);
-  else if (mode == 1)
-    k_spmm64<kBlock, RU, 1><<<g, kBlock, 0, stream()>>>(n, ia, ja, a, P, Q, Bm, part, ctl);
-  else
-    k_spmm64<kBlock, RU, 0><<<g, kBlock, 0, stream()>>>(n, ia, ja, a, P, Q, Bm, part, ctl);
+  constexpr int kMost = Chunk<K>::kRW / Chunk<K>::G;  // rows per group in a chunk
+  constexpr int RU = RU0 < kMost ? RU0 : kMost, EU = RU == 4 ? 4 : 8;
+  auto pick = [&](auto far) {
+    constexpr bool F = decltype(far)::value;
+    return mode == 2   ? k_spmm<kBlock, K, RU, EU, 2, F>
+           : mode == 1 ? k_spmm<kBlock, K, RU, EU, 1, F>
+                       : k_spmm<kBlock, K, RU, EU, 0, F>;
+  };
+  const bool far = (size_t)n * K * 8 > 0xfffffff0u;
+  auto *f = far ? pick(std::true_type{}) : pick(std::false_type{});
+  f<<<g.grid, kBlock, 0, stream()>>>(n, ia, ja, a, P, Q, Bm, part, ctl, g.group);
 }
 
 template <int K>
@@ -466,8 +458,7 @@ SpmmFn spmm_for_k(int ru) {
   switch (ru) {
     case 1: return spmm_launch<K, 1>;
     case 2: return spmm_launch<K, 2>;
-    case 4: return spmm_launch<K, 4>;
-    default: return nullptr;
+    default: return spmm_launch<K, 4>;
   }
 }
 
@@ -479,16 +470,12 @@ SpmmFn spmm_for(int k, int ru) {
     case 8: return spmm_for_k<8>(ru);
     case 16: return spmm_for_k<16>(ru);
     case 32: return spmm_for_k<32>(ru);
-    case 64:
-      if (ru == 8) return spmm64_launch<8>;
-      if (ru == 16) return spmm64_launch<16>;
-      return spmm_for_k<64>(ru);
+    case 64: return spmm_for_k<64>(ru);
     default: return nullptr;
   }
 }
 
-// 1, 2, 4: rows per lane group; 8, 16 (k = 64): rows per wave step with
-// wave-cooperative index loads
+// 1, 2, 4: rows per lane group at a time; 8, 16 (k = 64) as 4
 bool tile_ok(int k, int ru) {
   return ru == 1 || ru == 2 || ru == 4 || (k == 64 && (ru == 8 || ru == 16));
 }
@@ -502,9 +489,31 @@ int log2i(int k) {
 // (ia, ja, a, n, k, mode) -> chosen tile
 std::map<std::tuple<const void *, const void *, const void *, int, int, int>, int> g_tile;
 
-unsigned spmm_grid() {
+// The grid: spmm_wg_per_cu workgroups per CU, less what makes it a multiple of
+// 8 groups.  The group: as cls_group, the one with the fewest rows of P read by
+// several XCDs, from the plan's sample of column offsets (at most a 64th of the
+// row blocks, so that no XCD is left without work; a matrix without locality
+// has no better group than 1).
+SpmmShape spmm_shape(const SpmvPlan &A, int k) {
   const int per_cu = std::max(1, std::min(16, options().spmm_wg_per_cu));
-  return (unsigned)std::max(1, per_cu * device_cus());
+  const int grid = std::max(8, per_cu * device_cus());
+  const int rows = std::max(64 / k, 16) * (kBlock / kWave);
+  const long nblk = ((long)A.n + rows - 1) / rows;
+  const auto known = A.spmm_shapes.find({rows, grid});
+  if (known != A.spmm_shapes.end()) return {known->second.first, known->second.second};
+  SpmmShape best{(unsigned)grid, 1};
+  double least = 1e30;
+  for (int g = 1; g * 8 <= grid && (g == 1 || (long)g * 64 <= nblk); ++g) {
+    const int used = grid / (8 * g) * (8 * g);
+    if (used < 0.9 * grid) continue;
+    const double cost = xcd_cost(A.offsets, rows, g);
+    if (cost < 0.97 * least) {
+      least = cost;
+      best = {(unsigned)used, g};
+    }
+  }
+  A.spmm_shapes[{rows, grid}] = {best.grid, best.group};
+  return best;
 }
 
 unsigned vec_grid(size_t elems) {
@@ -514,22 +523,20 @@ unsigned vec_grid(size_t elems) {
 
 // Times every rows-per-group choice on Y = A X (three runs each, after a
 // warm-up).
-int pick_tile(int n, const int *ia, const int *ja, const double *a, int k, const double *X,
-              double *Y, int mode = 0, double *part = nullptr, const BlkCtl *ctl = nullptr) {
+int pick_tile(SpmmShape g, int n, const int *ia, const int *ja, const double *a, int k,
+              const double *X, double *Y, int mode = 0, double *part = nullptr, const BlkCtl *ctl = nullptr) {
   auto key = std::make_tuple((const void *)ia, (const void *)ja, (const void *)a, n, k, mode);
   auto it = g_tile.find(key);
   if (it != g_tile.end()) return it->second;
   int best_ru = 0;
   float best = 1e30f;
-  const unsigned g = spmm_grid();
   hipEvent_t e0, e1;
   if (!LAP_HIP(hipEventCreate(&e0))) return 0;
   if (!LAP_HIP(hipEventCreate(&e1))) {
     (void)hipEventDestroy(e0);
     return 0;
   }
-  for (int ru = 1; ru <= 16; ru *= 2) {
-    if (!tile_ok(k, ru)) continue;
+  for (int ru = 1; ru <= 4; ru *= 2) {
     SpmmFn fn = spmm_for(k, ru);
     fn(g, n, ia, ja, a, X, Y, nullptr, part, ctl, mode);
     LAP_HIP(hipEventRecord(e0, stream()));
@@ -588,10 +595,12 @@ extern "C" int lap_csr_matmat(int n, int nnz, const int *ia, const int *ja, cons
   if (!block_args("csr_matmat", n, nnz, ia, ja, a, k, tile)) return lap_last_status();
   const size_t nk = sizeof(double) * (size_t)n * (size_t)k;
   if (!check_device("csr_matmat", {{X, "X", nk}, {Y, "Y", nk}})) return lap_last_status();
-  if (!spmv_plan(n, nnz, ia, ja)) return lap_last_status();  // validates ia / ja
-  if (!tile) tile = pick_tile(n, ia, ja, a, k, X, Y);
+  const SpmvPlan *A = spmv_plan(n, nnz, ia, ja);  // validates ia / ja
+  if (!A) return lap_last_status();
+  const SpmmShape g = spmm_shape(*A, k);
+  if (!tile) tile = pick_tile(g, n, ia, ja, a, k, X, Y);
   if (!tile) return LAP_ERR_HIP;
-  spmm_for(k, tile)(spmm_grid(), n, ia, ja, a, X, Y, nullptr, nullptr, nullptr, 0);
+  spmm_for(k, tile)(g, n, ia, ja, a, X, Y, nullptr, nullptr, nullptr, 0);
   if (!LAP_HIP(hipGetLastError())) return LAP_ERR_HIP;
   sync();
   return LAP_OK;
@@ -611,13 +620,15 @@ extern "C" int lap_pcg_block(int n, int nnz, const int *ia, const int *ja, const
                                   {X, "X", nk},
                                   {Bm, "B", nk}}))
     return lap_last_status();
-  if (!spmv_plan(n, nnz, ia, ja)) return lap_last_status();  // validates ia / ja
+  const SpmvPlan *A = spmv_plan(n, nnz, ia, ja);  // validates ia / ja
+  if (!A) return lap_last_status();
   double *R = scratch_vec("blk_r", (size_t)n * k), *P = scratch_vec("blk_p", (size_t)n * k),
          *Q = scratch_vec("blk_q", (size_t)n * k);
   BlkCtl *ctl =
       reinterpret_cast<BlkCtl *>(scratch_vec("blk_ctl", sizeof(BlkCtl) / sizeof(double) + 1));
-  const unsigned g = spmm_grid(), gv = vec_grid((size_t)n * k);
-  double *part = scratch_vec("blk_part", (size_t)2 * kMaxK * std::max(g, gv));
+  const SpmmShape g = spmm_shape(*A, k);
+  const unsigned gv = vec_grid((size_t)n * k);
+  double *part = scratch_vec("blk_part", (size_t)2 * kMaxK * std::max(g.grid, gv));
   const size_t hist_len = ((size_t)maxit + 2) * (size_t)k;
   if (h_hist && hist_len > (size_t)INT_MAX) {
     set_error(LAP_ERR_ARG, "pcg_block: history of (maxit+2)*k entries is too long");
@@ -627,11 +638,12 @@ extern "C" int lap_pcg_block(int n, int nnz, const int *ia, const int *ja, const
   if (!R || !P || !Q || !ctl || !part || (h_hist && !hist)) return lap_last_status();
   // rows past a column's own stop stay 0
   if (hist) launch_fill((int)hist_len, 0.0, hist);
-  if (!tile) {  // timed in the solve's own mode (q = A p with the p.q epilogue)
-    const int live = 0;
-    LAP_HIP(hipMemcpyAsync(&ctl->all_done, &live, sizeof(int), hipMemcpyHostToDevice, stream()));
-    tile = pick_tile(n, ia, ja, a, k, Bm, Q, 1, part, ctl);
-  }
+  BlkCtl h{};
+  h.maxit = maxit;
+  h.left = k;
+  LAP_HIP(hipMemcpyAsync(ctl, &h, sizeof h, hipMemcpyHostToDevice, stream()));
+  // timed in the solve's own mode (q = A p with the p.q epilogue)
+  if (!tile) tile = pick_tile(g, n, ia, ja, a, k, Bm, Q, 1, part, ctl);
   if (!tile) return LAP_ERR_HIP;
   SpmmFn spmm = spmm_for(k, tile);
   const int lk = log2i(k);
@@ -644,15 +656,15 @@ extern "C" int lap_pcg_block(int n, int nnz, const int *ia, const int *ja, const
   }
   LAP_HIP(hipEventRecord(ev0, stream()));
   spmm(g, n, ia, ja, a, X, R, Bm, part, ctl, 2);
-  k_blk_res0<<<1, kRedThreads, 0, stream()>>>(part, (int)g, k, tol, maxit, ctl, hist);
+  k_blk_res0<kBlock><<<k, kBlock, 0, stream()>>>(part, (int)g.grid, tol, ctl, hist);
   k_blk_start<kBlock><<<gv, kBlock, 0, stream()>>>(n, k, lk, R, d_r, P, part);
-  k_blk_rho<<<1, kRedThreads, 0, stream()>>>(part, (int)gv, k, ctl);
+  k_blk_rho<kBlock><<<k, kBlock, 0, stream()>>>(part, (int)gv, ctl);
   auto iteration = [&]() {
     spmm(g, n, ia, ja, a, P, Q, nullptr, part, ctl, 1);
-    k_blk_alpha<<<1, kRedThreads, 0, stream()>>>(part, (int)g, k, ctl);
+    k_blk_alpha<kBlock><<<k, kBlock, 0, stream()>>>(part, (int)g.grid, ctl);
     k_blk_update<kBlock><<<gv, kBlock, 0, stream()>>>(n, k, lk, R, Q, d_r, ctl, part);
-    k_blk_conv<<<1, kRedThreads, 0, stream()>>>(part, (int)gv, k, hist, ctl);
-    k_blk_dir<kBlock, false><<<gv, kBlock, 0, stream()>>>(n, k, lk, X, R, d_r, P, ctl);
+    k_blk_conv<kBlock><<<k, kBlock, 0, stream()>>>(part, (int)gv, hist, ctl);
+    k_blk_dir<kBlock><<<gv, kBlock, 0, stream()>>>(n, k, lk, X, R, d_r, P, ctl);
   };
   // iter <= maxit + 1 for every column, so G * max_batches iterations
   // always reach all_done
@@ -690,7 +702,6 @@ extern "C" int lap_pcg_block(int n, int nnz, const int *ia, const int *ja, const
       set_error(LAP_ERR_NUMERIC, "pcg_block: stop flags never set");
       status = LAP_ERR_NUMERIC;
     }
-    k_blk_dir<kBlock, true><<<gv, kBlock, 0, stream()>>>(n, k, lk, X, R, d_r, P, ctl);
   }
   LAP_HIP(hipEventRecord(ev1, stream()));
   sync();
@@ -700,16 +711,17 @@ extern "C" int lap_pcg_block(int n, int nnz, const int *ia, const int *ja, const
   (void)hipEventDestroy(ev1);
   if (gexec) (void)hipGraphExecDestroy(gexec);
   if (gpu_ms) *gpu_ms = ms;
-  BlkCtl h{};
   LAP_HIP(hipMemcpy(&h, ctl, sizeof h, hipMemcpyDeviceToHost));
+  int last = 0;
   for (int j = 0; j < k; ++j) {
+    last = std::max(last, h.iters[j]);
     if (iters) iters[j] = h.iters[j];
     if (flags) flags[j] = h.flag[j];
     if (res0) res0[j] = h.res0[j];
     if (res) res[j] = h.res[j];
   }
   if (h_hist && hist)
-    LAP_HIP(hipMemcpy(h_hist, hist, sizeof(double) * ((size_t)h.iter + 1) * k,
+    LAP_HIP(hipMemcpy(h_hist, hist, sizeof(double) * ((size_t)last + 1) * k,
                       hipMemcpyDeviceToHost));
   if (status == LAP_OK && lap_last_status() == LAP_ERR_HIP) status = LAP_ERR_HIP;
   return status;

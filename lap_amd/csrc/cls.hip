@@ -172,15 +172,20 @@ __global__ __launch_bounds__(kBlock) void k_cls_assign(
 
 }  // namespace
 
+double xcd_cost(const std::vector<int> &offsets, int rows, int group) {
+  double cost = 0.0;
+  for (int o : offsets) {
+    const double d = std::fmod(std::abs((double)o) / rows, 8.0 * group);
+    cost += std::min(1.0, std::min(d, 8.0 * group - d) / group);
+  }
+  return cost;
+}
+
 int cls_group(const std::vector<int> &offsets, int rows, unsigned grid) {
   int best = 1;
   double least = 1e30;
   for (int g = 1; g <= 256 && grid % (8u * (unsigned)g) == 0; g *= 2) {
-    double cost = 0.0;
-    for (int o : offsets) {  // the share of blocks whose neighbour o rows on is another XCD's
-      const double d = std::fmod(std::abs((double)o) / rows, 8.0 * g);
-      cost += std::min(1.0, std::min(d, 8.0 * g - d) / g);
-    }
+    const double cost = xcd_cost(offsets, rows, g);
     if (cost < least - 1e-9) {
       least = cost;
       best = g;

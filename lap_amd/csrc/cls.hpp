@@ -46,6 +46,9 @@ __host__ __device__ __forceinline__ int cls_block(int wg, int group) {
   const int x = wg & 7, s = wg >> 3;
   return s / group * (8 * group) + x * group + s % group;
 }
+// How many of the column offsets lead to a row block of another XCD, for row
+// blocks of `rows` rows.
+double xcd_cost(const std::vector<int> &offsets, int rows, int group);
 // The group for row blocks of `rows` rows and a grid of `grid` workgroups: the
 // power of two with the fewest lines of x read by several XCDs, by the
 // matrix's column offsets.
