@@ -170,7 +170,56 @@ __global__ __launch_bounds__(kBlock) void k_cls_assign(
   }
 }
 
+// one workgroup, a thread per class: cls_inner's table, from the entries in
+// k_mx_values's order
+__global__ __launch_bounds__(kBlock) void k_cls_inner(int ncls, int width, int width_o,
+                                                      const int *__restrict__ off,
+                                                      const double *__restrict__ val,
+                                                      const int *__restrict__ len,
+                                                      int *__restrict__ off_o,
+                                                      double *__restrict__ val_o,
+                                                      int *__restrict__ len_o) {
+  const int c = threadIdx.x;
+  if (c >= ncls) return;
+  double d = 0.0, comp = 0.0;
+  int m = 1;
+  for (int j = 0; j < len[c]; ++j) {
+    const double v = val[c * width + j];
+    if (off[c * width + j] == 0) {
+      d += v;
+      continue;
+    }
+    const float f = (float)v;
+    comp += v - (double)f;
+    off_o[c * width_o + m] = off[c * width + j];
+    val_o[c * width_o + m] = (double)f;
+    ++m;
+  }
+  off_o[c * width_o] = 0;
+  val_o[c * width_o] = d + comp;
+  len_o[c] = m;
+  for (; m < width_o; ++m) {
+    off_o[c * width_o + m] = 0;
+    val_o[c * width_o + m] = 0.0;
+  }
+}
+
 }  // namespace
+
+ClsMat cls_inner(const ClsMat &A, int max_row) {
+  ClsMat m = A;
+  m.width = (max_row + 8) / 8 * 8;
+  double *val = scratch_vec("cls_inner_val", (size_t)kClsMax * kClsRow);
+  int *off = reinterpret_cast<int *>(
+      scratch_vec("cls_inner_off", kClsMax * (kClsRow + 1) / 2 + 1));
+  if (!A.cls || m.width > kClsRow || !val || !off) return ClsMat();
+  m.off = off;
+  m.val = val;
+  m.len = off + kClsMax * kClsRow;
+  k_cls_inner<<<1, kBlock, 0, stream()>>>(A.ncls, A.width, m.width, A.off, A.val, A.len, off, val,
+                                          off + kClsMax * kClsRow);
+  return m;
+}
 
 double xcd_cost(const std::vector<int> &offsets, int rows, int group) {
   double cost = 0.0;

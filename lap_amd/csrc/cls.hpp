@@ -22,6 +22,11 @@ namespace lap {
 constexpr int kClsMax = 255;   // classes
 constexpr int kClsRow = 16;    // entries of a row at most
 
+// Systems of fewer rows keep the CSR arrays: their matrix is in the Infinity
+// Cache and an iteration is mostly launches (at 10^6 rows of 7 entries an
+// iteration of Jacobi PCG takes 45 us with the CSR arrays and 35 with classes).
+constexpr int kClsMinRows = 1 << 19;
+
 // A row-class matrix on the device; cls == nullptr: the matrix has too many
 // distinct rows (or none was asked for).  Class c's entries are off / val
 // [c * width .. + width), padded with offset 0 (the row itself) and value +0.0.
@@ -60,6 +65,12 @@ int cls_group(const std::vector<int> &offsets, int rows, unsigned grid);
 // thousand rows.
 ClsMat cls_encode(const char *tag, int n, int nnz, const int *ia, const int *ja, const double *a,
                   const double *d_r, int max_row);
+
+// The mixed solver's inner operator of the same rows: per class first the
+// diagonal (with what rounding took from the row's off-diagonals), then the
+// off-diagonals rounded to FP32, in CSR order.  Wide enough for
+// max_row + 1 entries; cls == nullptr where that is too many.
+ClsMat cls_inner(const ClsMat &A, int max_row);
 
 // The table in LDS, a record per class: W values, W offsets, the number of
 // entries, and 12 bytes so that the records of different classes start in
@@ -100,6 +111,42 @@ struct ClsLds {
     }
     return s;
   }
+  // the same for cls_inner's tables: the sum starts with the diagonal's product
+  template <class XT>
+  __device__ __forceinline__ double sum_inner(int c, const XT (&xv)[W]) const {
+    const double *v = reinterpret_cast<const double *>(t + c * kRec);
+    const int len = reinterpret_cast<const int *>(t + c * kRec + W * 12)[0];
+    double s = v[0] * (double)xv[0];
+#pragma unroll
+    for (int i = 1; i < W; ++i) {
+      const double e = s + (1.0 * v[i]) * (double)xv[i];
+      s = i < len ? e : s;
+    }
+    return s;
+  }
+};
+
+// 1/diag of row i: from the vector, or (row classes) one byte and a table in
+// LDS, 7 of 8 bytes (FP32: 3 of 4) less to read
+template <class T>
+struct JacD {
+  const T *d_r;
+  __device__ __forceinline__ void init() {}
+  __device__ __forceinline__ T at(size_t i) const { return ld_nt(d_r + i); }
+};
+template <class T>
+struct JacDCls {
+  const unsigned char *cls;
+  const double *d;
+  int ncls;
+  T *lds;
+  __device__ __forceinline__ void init() {
+    __shared__ T t[kClsMax + 1];
+    lds = t;
+    for (int i = threadIdx.x; i < ncls; i += blockDim.x) t[i] = (T)d[i];
+    __syncthreads();
+  }
+  __device__ __forceinline__ T at(size_t i) const { return lds[ld_nt(cls + i)]; }
 };
 
 }  // namespace lap

@@ -35,6 +35,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "cls.hpp"
 #include "lap_core.hpp"
 #include "spmv_core.hpp"
 
@@ -299,19 +300,87 @@ __global__ __launch_bounds__(BS) void k_mx_spmv_pq_dvi(int nblk, const int *__re
   if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
+// The same over row classes (cls_inner's table): one byte per row, bitwise the
+// CSR kernel's rows.  As k_spmv_pq_cls, two row blocks of a workgroup are in
+// flight.  At 190 x 203 x 171 it takes 29 us where the CSR kernel takes 92, and
+// with 1/diag by class the update 30 (33) and the direction 21 (22).
+template <int BS, int W, class VT>
+__global__ __launch_bounds__(BS, 8) void k_mx_spmv_pq_cls(int nblk,
+                                                          const int *__restrict__ rowblk,
+                                                          const unsigned char *__restrict__ cls,
+                                                          int ncls, const int *__restrict__ off,
+                                                          const double *__restrict__ val,
+                                                          const int *__restrict__ len,
+                                                          const VT *__restrict__ p,
+                                                          VT *__restrict__ q, MixCtl *ctl,
+                                                          double *part, int walk, int group) {
+  if (ctl->done) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && ctl->pend_valid) {
+    ctl->iter = ctl->pend_iter;
+    ctl->rho = ctl->pend_rho;
+    ctl->maxr2 = ctl->pend_maxr2;
+    ctl->refinements = ctl->pend_refinements;
+    ctl->pend_valid = 0;
+  }
+  __shared__ double red[BS / kWave];
+  extern __shared__ double cls_lds[];
+  ClsLds<W> tab;
+  PqMxEpi<VT> epi{q, p, nullptr, 0.0};
+  BlockWalk w = block_walk(nblk, walk);
+  const int me = walk == 0 ? cls_block(blockIdx.x, group) : (int)blockIdx.x;
+  if (walk == 0) w.begin = me;
+  const int t = threadIdx.x;
+  struct Blk {
+    int r0, r1, c;
+  };
+  constexpr int K = W > 8 ? 1 : 2;
+  Blk cur[K], nxt[K];
+  auto ask = [&](int s) {
+    Blk k;
+    const int b = s < w.end ? w.block(s) : nblk;
+    k.r0 = b < nblk ? rowblk[b] : 0;
+    k.r1 = b < nblk ? rowblk[b + 1] : 0;
+    k.c = k.r0 + t < k.r1 ? cls[k.r0 + t] : 0;
+    return k;
+  };
+#pragma unroll
+  for (int u = 0; u < K; ++u) cur[u] = ask(w.begin + u * w.step);
+  tab.init(reinterpret_cast<char *>(cls_lds), ncls, off, val, len);
+  for (int s = w.begin; s < w.end; s += K * w.step) {
+    VT xv[K][W];
+#pragma unroll
+    for (int u = 0; u < K; ++u) nxt[u] = ask(s + (K + u) * w.step);
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+      if (cur[u].r0 + t < cur[u].r1) tab.load(cur[u].c, p + (cur[u].r0 + t), xv[u]);
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      if (cur[u].r0 + t < cur[u].r1) epi.store(cur[u].r0 + t, tab.sum_inner(cur[u].c, xv[u]));
+      for (int row = cur[u].r0 + BS + t; row < cur[u].r1; row += BS) {  // (spmv_rows > BS)
+        const int c = cls[row];
+        tab.load(c, p + row, xv[u]);
+        epi.store(row, tab.sum_inner(c, xv[u]));
+      }
+      cur[u] = nxt[u];
+    }
+  }
+  const double t_pq = block_sum<BS>(epi.acc, red);
+  if (t == 0) part[me] = t_pq;
+}
+
 // alpha = rho/(p.q); x32 += alpha p; r32 -= alpha q (each rounded once from
 // FP64 to VT); partials of r.r and, with Jacobi, r.w for w = d_r r (stride
 // 2: [rz, rr]).
-template <int BS, bool JAC, class VT>
+template <int BS, bool JAC, class VT, class D>
 __global__ __launch_bounds__(BS) void k_mx_update(int n, VT *__restrict__ x32,
                                                   VT *__restrict__ r32,
                                                   const VT *__restrict__ p,
                                                   const VT *__restrict__ q,
-                                                  const VT *__restrict__ d_r,
-                                                  const MixCtl *ctl, const double *pq_part,
+                                                  D d_r, const MixCtl *ctl, const double *pq_part,
                                                   int pq_cnt, double *part) {
   if (ctl->done) return;
   __shared__ double red[BS / kWave];
+  if (JAC) d_r.init();
   const double pq = sum_partials<BS>(pq_part, pq_cnt, 1, red);
   const double alpha = ctl->rho / pq;
   double rz = 0.0, rr = 0.0;
@@ -323,7 +392,7 @@ __global__ __launch_bounds__(BS) void k_mx_update(int n, VT *__restrict__ x32,
     st_nt(r32 + i, rf);
     rr += (double)rf * (double)rf;
     if (JAC) {
-      const VT wf = ld_nt(d_r + i) * rf;
+      const VT wf = d_r.at(i) * rf;
       rz += (double)rf * (double)wf;
     }
   }
@@ -427,16 +496,16 @@ __device__ __forceinline__ MxStep mx_step(const MixCtl *ctl, const double *upd_p
 
 // Jacobi: convergence bookkeeping, the refinement's fold (x += x32, x32 = 0,
 // after k_mx_resid has used x + x32), beta, p = beta p + d_r r
-template <int BS, class VT>
+template <int BS, class VT, class D>
 __global__ __launch_bounds__(BS) void k_mx_jac_p(int n, const VT *__restrict__ r32,
-                                                 const VT *__restrict__ d_r,
-                                                 VT *__restrict__ p, double *__restrict__ x,
+                                                 D d_r, VT *__restrict__ p, double *__restrict__ x,
                                                  VT *__restrict__ x32, MixCtl *ctl,
                                                  double *hist, const double *upd_part,
                                                  int upd_cnt, const double *ref_part,
                                                  int ref_cnt) {
   if (ctl->done) return;
   __shared__ double red[BS / kWave];
+  d_r.init();
   const MxStep s = mx_step<BS>(ctl, upd_part, upd_cnt, ref_part, ref_cnt, red);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     hist[s.it] = s.res;
@@ -463,7 +532,7 @@ __global__ __launch_bounds__(BS) void k_mx_jac_p(int n, const VT *__restrict__ r
   if (s.flag >= 0) return;
   const double beta = s.rz / ctl->rho;
   for (size_t i = (size_t)blockIdx.x * BS + threadIdx.x; i < (size_t)n; i += stride) {
-    const VT wf = ld_nt(d_r + i) * ld_nt(r32 + i);
+    const VT wf = d_r.at(i) * ld_nt(r32 + i);
     st_nt(p + i, (VT)((double)ld_nt(p + i) * beta + (double)wf));
   }
 }
@@ -973,8 +1042,20 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
   // value-indexed inner SpMV when spmv_format asks for it and the table fits
   const bool dvi32 = options().spmv_format == 2 && M->ndl > 0;
   const bool vi32 = !dvi32 && options().spmv_format >= 1 && M->nd > 0;
+  ClsMat cls;  // row classes, from the second batch of iterations on
   auto spmv32 = [&]() {
-    if (dvi32)
+    if (cls.cls) {
+      const int group = walk == 0 ? cls_group(cls.offsets, options().spmv_rows, gO) : 1;
+      auto go = [&](auto *k, int rec) {
+        k<<<gO, kBlock, cls.ncls * rec, stream()>>>(M->off->nblocks, rb_o, cls.cls, cls.ncls,
+                                                    cls.off, cls.val, cls.len, p32, q32, ctl, Q1,
+                                                    walk, group);
+      };
+      if (cls.width == 8)
+        go(k_mx_spmv_pq_cls<kBlock, 8, VT>, ClsLds<8>::kRec);
+      else
+        go(k_mx_spmv_pq_cls<kBlock, 16, VT>, ClsLds<16>::kRec);
+    } else if (dvi32)
       k_mx_spmv_pq_dvi<kBlock, VT><<<gO, kBlock, 0, stream()>>>(
           M->off->nblocks, rb_o, io, M->code_o->as<unsigned short>(), M->dict_o->as<float>(),
           M->nd, M->ddict_o->as<int>(), M->ndl, dg, p32, q32, ctl, Q1, walk);
@@ -987,15 +1068,21 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
                                                                    jo, ao, dg, p32, q32, ctl,
                                                                    Q1, walk);
   };
+  auto jacobi = [&](auto d) {
+    spmv32();
+    k_mx_update<kBlock, true, VT><<<gV, kBlock, 0, stream()>>>(n, x32, r32, p32, q32, d, ctl,
+                                                               Q1, (int)gO, Q2);
+    k_mx_resid<kBlock, kSpmvTile, VT><<<gA, kBlock, 0, stream()>>>(
+        A64->nblocks, rb_a, ia, ja, a, x, x32, b, r32, d_r32, ctl, Q2, (int)gV, Q3, walk);
+    k_mx_jac_p<kBlock, VT><<<gV, kBlock, 0, stream()>>>(n, r32, d, p32, x, x32, ctl, hist, Q2,
+                                                        (int)gV, Q3, (int)gA);
+  };
   auto iteration = [&]() {
     if (jac) {
-      spmv32();
-      k_mx_update<kBlock, true, VT><<<gV, kBlock, 0, stream()>>>(n, x32, r32, p32, q32, d_r32,
-                                                                 ctl, Q1, (int)gO, Q2);
-      k_mx_resid<kBlock, kSpmvTile, VT><<<gA, kBlock, 0, stream()>>>(
-          A64->nblocks, rb_a, ia, ja, a, x, x32, b, r32, d_r32, ctl, Q2, (int)gV, Q3, walk);
-      k_mx_jac_p<kBlock, VT><<<gV, kBlock, 0, stream()>>>(n, r32, d_r32, p32, x, x32, ctl, hist,
-                                                          Q2, (int)gV, Q3, (int)gA);
+      if (cls.cls)
+        jacobi(JacDCls<VT>{cls.cls, cls.d, cls.ncls, nullptr});
+      else
+        jacobi(JacD<VT>{d_r32});
     } else {
       if (ic) {
         ic_inner(*icp, *M, l32, u32, r32, w32, aux32, done);
@@ -1013,7 +1100,8 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
       }
       spmv32();
       k_mx_update<kBlock, false, VT><<<gV, kBlock, 0, stream()>>>(n, x32, r32, p32, q32,
-                                                                  nullptr, ctl, Q1, (int)gO, Q2);
+                                                                  JacD<VT>{nullptr}, ctl, Q1,
+                                                                  (int)gO, Q2);
       k_mx_fold<kBlock, VT><<<gV, kBlock, 0, stream()>>>(n, x, x32, ctl, Q2, (int)gV,
                                                          defl ? Q3 : nullptr);
       if (defl)
@@ -1036,7 +1124,10 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
 
   int status = LAP_OK;
   hipGraphExec_t gexec = nullptr;
-  if (options().use_graph) {
+  auto capture = [&]() {
+    if (gexec) (void)hipGraphExecDestroy(gexec);
+    gexec = nullptr;
+    if (!options().use_graph) return true;
     hipGraph_t graph = nullptr;
     bool ok = LAP_HIP(hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal));
     if (ok) {
@@ -1045,11 +1136,12 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
     }
     if (ok) ok = LAP_HIP(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
     if (graph) (void)hipGraphDestroy(graph);
-    if (!ok) {
-      gexec = nullptr;
-      status = LAP_ERR_HIP;
-    }
-  }
+    if (!ok) gexec = nullptr;
+    return ok;
+  };
+  if (!capture()) status = LAP_ERR_HIP;
+  // as in lap_pcg: a solve that ends in its first batch does not pay for them
+  const bool classes = options().spmv_format == 0 && n >= kClsMinRows;
   int *flags = pinned_flags();
   if (!flags) status = LAP_ERR_HIP;
   if (status == LAP_OK) {
@@ -1059,6 +1151,14 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
     const long max_batches = (long)(maxit + 1) / G + 3;
     bool finished = false;
     for (long k = 0; k < max_batches + 1 && !finished; ++k) {
+      if (k == 1 && classes && LAP_HIP(hipEventSynchronize(pe[0])) && !flags[0]) {
+        cls = cls_inner(cls_encode("a", n, nnz, ia, ja, a, jac ? pd->d_r : nullptr, A64->max_row),
+                        A64->max_row);
+        if (cls.cls && !capture()) {
+          status = LAP_ERR_HIP;
+          break;
+        }
+      }
       if (k < max_batches) {
         if (gexec) {
           if (!LAP_HIP(hipGraphLaunch(gexec, stream()))) break;

@@ -380,11 +380,6 @@ struct ViVals {
 
 constexpr int kDviMaxRow = 64;
 
-// Systems of fewer rows keep the CSR arrays in format 0: their matrix is in the
-// Infinity Cache and an iteration is mostly launches (at 10^6 rows of 7 entries
-// an iteration takes 45 us with the CSR arrays and 35 with classes).
-constexpr int kClsMinRows = 1 << 19;
-
 // Encodes the matrix as options().spmv_format asks and it fits: format 2 tries
 // the delta-indexed form first, then (like format 1) the value-indexed one.
 static ViVals vi_prepare(int nnz, const double *a, int n = 0, const int *ia = nullptr,
@@ -437,27 +432,6 @@ __device__ __forceinline__ int stop_flag(double res, int it, const PcgCtl *ctl) 
 // pend_done (committed to done by the next K_A), so that no workgroup of K_C
 // can skip its rows' x update by seeing `done` early.  Same operations on the
 // same values as cg.c's order of updates.
-
-// 1/diag of row i: from the vector, or (row classes) one byte and a table in
-// LDS, 7 of 8 bytes less to read
-struct JacD {
-  const double *d_r;
-  __device__ __forceinline__ void init() {}
-  __device__ __forceinline__ double at(size_t i) const { return ld_nt(d_r + i); }
-};
-struct JacDCls {
-  const unsigned char *cls;
-  const double *d;
-  int ncls;
-  double *lds;
-  __device__ __forceinline__ void init() {
-    __shared__ double t[kClsMax + 1];
-    lds = t;
-    for (int i = threadIdx.x; i < ncls; i += blockDim.x) t[i] = d[i];
-    __syncthreads();
-  }
-  __device__ __forceinline__ double at(size_t i) const { return lds[ld_nt(cls + i)]; }
-};
 
 // K_B: alpha = rho/(p.q); r -= alpha q; partials of r.(d_r r) and r.r
 template <int BS, class D>
@@ -1041,9 +1015,9 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
         k_jac_px<kBlock><<<gV, kBlock, 0, stream()>>>(n, x, r, d, p, ctl, hist, R3, (int)gV);
       };
       if (vv.cls.cls)
-        vectors(JacDCls{vv.cls.cls, vv.cls.d, vv.cls.ncls, nullptr});
+        vectors(JacDCls<double>{vv.cls.cls, vv.cls.d, vv.cls.ncls, nullptr});
       else
-        vectors(JacD{pd->d_r});
+        vectors(JacD<double>{pd->d_r});
     } else {
       prec_launch(o, r, w, done);
       k_rw<kBlock><<<gV, kBlock, 0, stream()>>>(n, r, w, ctl, R1);

@@ -1,4 +1,4 @@
-"""PCG with the matrix as row classes (the default for large systems with few
+"""PCG and mixed-precision PCG with the matrix as row classes (the default for large systems with few
 distinct rows) against the CSR path: every product and sum is the same, so
 solutions, histories and flags are equal bit for bit.  Rows of 1 to 17 entries,
 few and too many classes, the first size that is encoded, ragged last row
@@ -37,7 +37,7 @@ def band(n, offs, weights=None, shift=0.05):
     return CSR(n, ia, cols[order].astype(np.int32), vals[order])
 
 
-def both(Ah, kind, b, maxit=40, d=None, x0=None, **opts):
+def both(Ah, kind, b, maxit=40, d=None, x0=None, solve=None, tol=0.0, **opts):
     A = S.DeviceCSR.from_csr(Ah)
     P = S.make_preconditioner(A, Ah, kind)
     if d is not None:
@@ -49,7 +49,7 @@ def both(Ah, kind, b, maxit=40, d=None, x0=None, **opts):
             prev = S.set_option("spmv_format", fmt)
             try:
                 kw = {} if x0 is None else {"x0": S.to_dev(x0)}
-                out.append(S.pcg(A, S.to_dev(b), P, tol=0.0, maxit=maxit, **kw))
+                out.append((solve or S.pcg)(A, S.to_dev(b), P, tol=tol, maxit=maxit, **kw))
             finally:
                 S.set_option("spmv_format", prev)
     finally:
@@ -121,3 +121,36 @@ def test_not_finite(bad):
     assert (r.iterations, r.flag) == (s.iterations, s.flag)
     assert np.array_equal(r.history, s.history, equal_nan=True)
     assert torch.equal(torch.isnan(r.x), torch.isnan(s.x))
+
+
+@pytest.mark.parametrize("name", ["first_encoded", "cube_odd", "plane", "diagonal", "row_9",
+                                  "row_15", "row_17", "mixed_classes", "too_many"])
+@pytest.mark.parametrize("vectors", [0, 1])
+def test_mixed_bitwise(name, vectors):
+    """Also through refinements; rows of 15 entries fill cls_inner's 16."""
+    Ah = CASES[name]()
+    b = np.random.default_rng(8).standard_normal(Ah.n)
+    r, s = both(Ah, "line_jacobi", b, maxit=60, solve=S.pcg_mixed, tol=1e-9,
+                mixed_vectors=vectors)
+    assert r.refinements == s.refinements and r.refinements > 0
+    same(r, s)
+
+
+@pytest.mark.parametrize("kind", ["none", "ichol"])
+def test_mixed_other_preconditioners(kind):
+    Ah = grid_laplacian([91, 73, 83], 1e-6)
+    b = np.random.default_rng(9).standard_normal(Ah.n)
+    same(*both(Ah, kind, b, maxit=25, solve=S.pcg_mixed, tol=1e-8))
+
+
+def test_mixed_rows_without_a_diagonal():
+    """Not positive definite, so few steps: rows of off-diagonals only, up to 16."""
+    Ah = band(MIN_ROWS + 3, [1, 2, 3, 4, 5, 6, 7, 900])
+    keep = np.ones(Ah.nnz, bool)
+    rows = np.repeat(np.arange(Ah.n), np.diff(Ah.ia))
+    keep[(rows == Ah.ja) & (rows % 2 == 0)] = False
+    keep[(rows == Ah.ja + 900) | (rows + 900 == Ah.ja)] = False
+    Bh = CSR(Ah.n, np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=Ah.n))])
+             .astype(np.int32), Ah.ja[keep], Ah.a[keep])
+    b = np.random.default_rng(10).standard_normal(Bh.n)
+    same(*both(Bh, "none", b, maxit=20, solve=S.pcg_mixed, tol=1e-9))
