@@ -489,11 +489,8 @@ int log2i(int k) {
 // (ia, ja, a, n, k, mode) -> chosen tile
 std::map<std::tuple<const void *, const void *, const void *, int, int, int>, int> g_tile;
 
-// The grid: spmm_wg_per_cu workgroups per CU, less what makes it a multiple of
-// 8 groups.  The group: as cls_group, the one with the fewest rows of P read by
-// several XCDs, from the plan's sample of column offsets (at most a 64th of the
-// row blocks, so that no XCD is left without work; a matrix without locality
-// has no better group than 1).
+// spmm_wg_per_cu workgroups per CU, dealt to the XCDs by the plan's sample of
+// column offsets (a matrix without locality has no better group than 1).
 SpmmShape spmm_shape(const SpmvPlan &A, int k) {
   const int per_cu = std::max(1, std::min(16, options().spmm_wg_per_cu));
   const int grid = std::max(8, per_cu * device_cus());
@@ -501,19 +498,9 @@ SpmmShape spmm_shape(const SpmvPlan &A, int k) {
   const long nblk = ((long)A.n + rows - 1) / rows;
   const auto known = A.spmm_shapes.find({rows, grid});
   if (known != A.spmm_shapes.end()) return {known->second.first, known->second.second};
-  SpmmShape best{(unsigned)grid, 1};
-  double least = 1e30;
-  for (int g = 1; g * 8 <= grid && (g == 1 || (long)g * 64 <= nblk); ++g) {
-    const int used = grid / (8 * g) * (8 * g);
-    if (used < 0.9 * grid) continue;
-    const double cost = xcd_cost(A.offsets, rows, g);
-    if (cost < 0.97 * least) {
-      least = cost;
-      best = {(unsigned)used, g};
-    }
-  }
-  A.spmm_shapes[{rows, grid}] = {best.grid, best.group};
-  return best;
+  const auto best = xcd_grid(A.offsets, rows, nblk, grid);
+  A.spmm_shapes[{rows, grid}] = best;
+  return {best.first, best.second};
 }
 
 unsigned vec_grid(size_t elems) {

@@ -230,6 +230,21 @@ double xcd_cost(const std::vector<int> &offsets, int rows, int group) {
   return cost;
 }
 
+std::pair<unsigned, int> xcd_grid(const std::vector<int> &offsets, int rows, long nblk, int most) {
+  std::pair<unsigned, int> best{(unsigned)most, 1};
+  double least = 1e30;
+  for (int g = 1; g * 8 <= most && (g == 1 || (long)g * 64 <= nblk); ++g) {
+    const int used = most / (8 * g) * (8 * g);
+    if (used < 0.9 * most) continue;
+    const double cost = xcd_cost(offsets, rows, g);
+    if (cost < 0.97 * least) {
+      least = cost;
+      best = {(unsigned)used, g};
+    }
+  }
+  return best;
+}
+
 int cls_group(const std::vector<int> &offsets, int rows, unsigned grid) {
   int best = 1;
   double least = 1e30;
@@ -244,7 +259,7 @@ int cls_group(const std::vector<int> &offsets, int rows, unsigned grid) {
 }
 
 ClsMat cls_encode(const char *tag, int n, int nnz, const int *ia, const int *ja, const double *a,
-                  const double *d_r, int max_row) {
+                  const double *d_r, int max_row, int least) {
   ClsMat m;
   if (n < 1 || nnz < 1 || max_row > kClsRow || lap_last_status() == LAP_ERR_HIP) return m;
   // what the host reads after the first pass and writes before the second, in
@@ -280,7 +295,7 @@ ClsMat cls_encode(const char *tag, int n, int nnz, const int *ia, const int *ja,
     h->reps[i] = found[i].second;
   }
   const std::string name = std::string("cls_") + tag;
-  const int width = std::max(8, (max_row + 7) / 8 * 8);
+  const int width = max_row <= least ? least : (max_row + 7) / 8 * 8;
   unsigned char *cls =
       reinterpret_cast<unsigned char *>(scratch_vec(name.c_str(), ((size_t)n + 7) / 8));
   double *val = scratch_vec((name + "_val").c_str(), (size_t)kClsMax * kClsRow);

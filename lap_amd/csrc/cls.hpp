@@ -54,17 +54,39 @@ __host__ __device__ __forceinline__ int cls_block(int wg, int group) {
 // How many of the column offsets lead to a row block of another XCD, for row
 // blocks of `rows` rows.
 double xcd_cost(const std::vector<int> &offsets, int rows, int group);
+// A grid of at most `most` workgroups (and at least 0.9 of it) for row blocks
+// of `rows` rows, and its group: the one with the least cost, at most a 64th of
+// the nblk row blocks, so that no XCD is left without work.
+std::pair<unsigned, int> xcd_grid(const std::vector<int> &offsets, int rows, long nblk, int most);
 // The group for row blocks of `rows` rows and a grid of `grid` workgroups: the
 // power of two with the fewest lines of x read by several XCDs, by the
 // matrix's column offsets.
 int cls_group(const std::vector<int> &offsets, int rows, unsigned grid);
 
+// The table's width is `least` (4, 8 or 16), or 8 or 16 where rows are longer.
 // Encodes the matrix (tag: names the buffers that hold the result until the
 // next encoding with the same tag).  d_r may be null.  Two passes over the
 // matrix; a matrix with too many distinct rows is noticed within a few
 // thousand rows.
 ClsMat cls_encode(const char *tag, int n, int nnz, const int *ia, const int *ja, const double *a,
-                  const double *d_r, int max_row);
+                  const double *d_r, int max_row, int least = 8);
+
+// The triangles (and A, for GS_it) of the sweep preconditioners as row classes
+// with d_r, and the grid of their sweeps; n == 0: not encoded.
+struct SweepCls {
+  int n = 0, group = 1;
+  unsigned grid = 1;
+  ClsMat L, U, A;
+};
+SweepCls sweep_encode(const SpmvPlan &L, const int *lia, const int *lja, const double *la,
+                      const SpmvPlan &U, const int *uia, const int *uja, const double *ua,
+                      const SpmvPlan *A, const int *ia, const int *ja, const double *a,
+                      const double *d_r);
+// The sweeps over classes (A: one of s's matrices).
+void sweep_one_launch(const SweepCls &s, const ClsMat &A, const double *x, const double *base,
+                      double *out, double *out2, int mode, bool first, const int *done);
+void sweep_pair_launch(const SweepCls &s, const double *x, const double *base, double *out,
+                       const int *done);
 
 // The mixed solver's inner operator of the same rows: per class first the
 // diagonal (with what rounding took from the row's off-diagonals), then the
@@ -101,12 +123,17 @@ struct ClsLds {
   // sum_j a_rj x_j in CSR order (the padding is left out: 0 * inf is not 0)
   template <class XT>
   __device__ __forceinline__ double sum(int c, const XT (&xv)[W]) const {
+    return sum_from(0.0, 1.0, c, xv);
+  }
+  // s + sum_j (alpha a_rj) x_j, term by term
+  template <class XT>
+  __device__ __forceinline__ double sum_from(double s, double alpha, int c,
+                                             const XT (&xv)[W]) const {
     const double *v = reinterpret_cast<const double *>(t + c * kRec);
     const int len = reinterpret_cast<const int *>(t + c * kRec + W * 12)[0];
-    double s = 0.0;
 #pragma unroll
     for (int i = 0; i < W; ++i) {
-      const double e = s + (1.0 * v[i]) * (double)xv[i];
+      const double e = s + (alpha * v[i]) * (double)xv[i];
       s = i < len ? e : s;
     }
     return s;

@@ -645,6 +645,7 @@ struct PrecOps {
   TriEll lell, uell;  // GS_std: the triangles packed for this solve (run_pcg)
   const IcPlan *ic = nullptr;
   double *aux1 = nullptr, *aux2 = nullptr, *aux3 = nullptr;
+  SweepCls sweep;  // the triangles as row classes (run_pcg)
 };
 
 static bool check_dev(const void *p, const char *what) {
@@ -755,16 +756,20 @@ static bool prec_fused(const PrecOps &o, const double *r, double *w, const int *
   const int n = o.n, K = o.k;
   lap_pdata *pd = o.pd;
   const double *dr = pd->d_r;
+  const bool cls = o.sweep.n > 0;
   auto pair = [&](const double *x, const double *base, double *out) {
+    if (cls) return sweep_pair_launch(o.sweep, x, base, out, done);
     sweep_pair_launch(*o.LU, pd->lia, pd->lja, pd->la, pd->uia, pd->uja, pd->ua, x, base, dr,
                       out, done);
   };
   auto one_l = [&](const double *x, const double *base, double *out, double *out2, int mode,
                    bool first) {
+    if (cls) return sweep_one_launch(o.sweep, o.sweep.L, x, base, out, out2, mode, first, done);
     sweep_one_launch(*o.Ls, pd->lia, pd->lja, pd->la, x, base, dr, out, out2, mode, first, done);
   };
   auto one_u = [&](const double *x, const double *base, double *out, double *out2, int mode,
                    bool first) {
+    if (cls) return sweep_one_launch(o.sweep, o.sweep.U, x, base, out, out2, mode, first, done);
     sweep_one_launch(*o.Us, pd->uia, pd->uja, pd->ua, x, base, dr, out, out2, mode, first, done);
   };
   if (o.kind == P_IT_JACOBI) {  // it_jacobi.c:4-32
@@ -781,7 +786,10 @@ static bool prec_fused(const PrecOps &o, const double *r, double *w, const int *
       if (j == 0)
         launch_vec_vec(n, r, dr, o.aux1, done);
       else {
-        sweep_one_launch(*o.A, o.ia, o.ja, o.a, w, r, dr, o.aux2, o.aux1, 2, false, done);
+        if (cls)
+          sweep_one_launch(o.sweep, o.sweep.A, w, r, o.aux2, o.aux1, 2, false, done);
+        else
+          sweep_one_launch(*o.A, o.ia, o.ja, o.a, w, r, dr, o.aux2, o.aux1, 2, false, done);
         base = o.aux2;
       }
       double *y = o.aux1, *alt = o.aux3;
@@ -1077,7 +1085,11 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
     for (long k = 0; k < max_batches + 1 && !finished; ++k) {
       if (k == 1 && classes && LAP_HIP(hipEventSynchronize(pe[0])) && !flags[0]) {
         vv.cls = cls_encode("a", n, nnz, ia, ja, a, jac ? pd->d_r : nullptr, A.max_row);
-        if (vv.cls.cls && !capture()) {
+        if (options().fuse_sweeps &&
+            (o.kind == P_IT_JACOBI || o.kind == P_GS_IT || o.kind == P_GS_IT2))
+          o.sweep = sweep_encode(*o.Ls, pd->lia, pd->lja, pd->la, *o.Us, pd->uia, pd->uja, pd->ua,
+                                 o.kind == P_GS_IT && o.m > 1 ? o.A : nullptr, ia, ja, a, pd->d_r);
+        if ((vv.cls.cls || o.sweep.n > 0) && !capture()) {
           status = LAP_ERR_HIP;
           break;
         }

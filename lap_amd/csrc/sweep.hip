@@ -20,6 +20,7 @@
 // L and U per block).
 #include <algorithm>
 
+#include "cls.hpp"
 #include "lap_core.hpp"
 #include "spmv_core.hpp"
 
@@ -139,6 +140,137 @@ __global__ __launch_bounds__(BS) void k_sweep_pair(
   }
 }
 
+// The same sweeps over row classes (cls.hpp): a byte per row for the matrix and
+// d_r, a lane per row, the sums in the same order, so every value is the CSR
+// sweep's bit for bit.  Bound by memory latency, so a workgroup has K row
+// blocks in flight; the blocks are dealt to the XCDs so that a row's neighbours
+// are mostly read through one L2.
+//
+// Measured at 121 x 93 x 140 (1.6M rows): the single sweep 21 -> 13 us (38 MB:
+// 3 TB/s with the launch), without d_r 19 -> 10, the pair 32 -> 14.  Taken from
+// the second batch of a large solve's iterations on, as in lap_pcg; matrices
+// with many distinct rows and small systems keep the CSR sweeps.
+struct ClsArg {
+  const unsigned char *cls;
+  int ncls;
+  const int *off;
+  const double *val;
+  const int *len;
+};
+enum { kStorePair = 4 };  // out = (base - (U x + L x)) * d_r: B is U, A is L
+
+template <int BS, int W, int MODE>
+__global__ __launch_bounds__(BS, 8) void k_sweep_cls(int n, ClsArg A, ClsArg B,
+                                                     const double *__restrict__ d,
+                                                     const double *__restrict__ x,
+                                                     const double *base, double *out,
+                                                     double *out2, int first, int group,
+                                                     const int *done) {
+  if (done && *done) return;
+  constexpr bool kPair = MODE == kStorePair;
+  constexpr int K = W <= 4 ? (kPair ? 2 : 4) : W <= 8 && !kPair ? 2 : 1;
+  extern __shared__ double sweep_mem[];
+  ClsLds<W> ta;
+  ClsLds<W> tb;
+  double *const dt = sweep_mem;  // d_r of each class of A
+  char *const at = reinterpret_cast<char *>(sweep_mem + (A.ncls + 1) / 2 * 2);
+  for (int i = threadIdx.x; i < A.ncls; i += BS) dt[i] = d[i];
+  const int t = threadIdx.x, nblk = (n - 1) / BS + 1;
+  int ca[K], cb[K];
+  auto ask = [&](int blk, int &a, int &b) {
+    const long long row = (long long)blk * BS + t;
+    a = row < n ? A.cls[row] : 0;
+    b = kPair && row < n ? B.cls[row] : 0;
+  };
+  const int me = cls_block(blockIdx.x, group), step = gridDim.x;
+#pragma unroll
+  for (int u = 0; u < K; ++u) ask(me + u * step, ca[u], cb[u]);
+  if (kPair) tb.init(at + A.ncls * ClsLds<W>::kRec, B.ncls, B.off, B.val, B.len);
+  ta.init(at, A.ncls, A.off, A.val, A.len);
+  for (int blk = me; blk < nblk; blk += K * step) {
+    double xa[K][W], xb[K][kPair ? W : 1], bv[K], ov[K];
+    int na[K], nb[K];
+#pragma unroll
+    for (int u = 0; u < K; ++u) ask(blk + (K + u) * step, na[u], nb[u]);
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      const long long row = (long long)(blk + u * step) * BS + t;
+      if (row >= n) continue;
+      ta.load(ca[u], x + row, xa[u]);
+      if constexpr (kPair) tb.load(cb[u], x + row, xb[u]);
+      bv[u] = base[row];
+      if (MODE == kStoreAccum) ov[u] = first ? 0.0 : out2[row];
+    }
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      const long long row = (long long)(blk + u * step) * BS + t;
+      if (row < n) {
+        const double dr = dt[ca[u]];
+        if constexpr (kPair) {
+          const double sl = ta.sum(ca[u], xa[u]), su = tb.sum(cb[u], xb[u]);
+          out[row] = (bv[u] - (su + sl)) * dr;
+        } else {
+          const double v = ta.sum_from(bv[u], -1.0, ca[u], xa[u]);
+          if constexpr (MODE == kStoreScaled) {
+            out[row] = v * dr;
+          } else if constexpr (MODE == kStorePlain) {
+            out[row] = v;
+          } else if constexpr (MODE == kStoreBoth) {
+            out[row] = v;
+            out2[row] = v * dr;
+          } else {
+            const double s = v * dr;
+            out2[row] = ov[u] + s;
+          }
+        }
+      }
+      ca[u] = na[u];
+      cb[u] = nb[u];
+    }
+  }
+}
+
+ClsArg cls_arg(const ClsMat &m) { return ClsArg{m.cls, m.ncls, m.off, m.val, m.len}; }
+
+template <int W>
+int sweep_lds(const ClsMat &A, const ClsMat &B) {
+  return (A.ncls + 1) / 2 * 16 + (A.ncls + B.ncls) * ClsLds<W>::kRec;
+}
+
+template <int W, int MODE>
+void sweep_cls_go(const SweepCls &s, const ClsMat &A, const ClsMat &B, const double *x,
+                  const double *base, double *out, double *out2, bool first, const int *done) {
+  k_sweep_cls<kBlock, W, MODE><<<s.grid, kBlock, sweep_lds<W>(A, B), stream()>>>(
+      s.n, cls_arg(A), cls_arg(B), A.d, x, base, out, out2, first ? 1 : 0, s.group, done);
+}
+
+template <int W>
+void sweep_cls_mode(const SweepCls &s, const ClsMat &A, const ClsMat &B, const double *x,
+                    const double *base, double *out, double *out2, int mode, bool first,
+                    const int *done) {
+  switch (mode) {
+    case kStoreScaled:
+      return sweep_cls_go<W, kStoreScaled>(s, A, B, x, base, out, out2, first, done);
+    case kStorePlain:
+      return sweep_cls_go<W, kStorePlain>(s, A, B, x, base, out, out2, first, done);
+    case kStoreBoth:
+      return sweep_cls_go<W, kStoreBoth>(s, A, B, x, base, out, out2, first, done);
+    case kStoreAccum:
+      return sweep_cls_go<W, kStoreAccum>(s, A, B, x, base, out, out2, first, done);
+    case kStorePair:
+      return sweep_cls_go<W, kStorePair>(s, A, B, x, base, out, out2, first, done);
+    default:
+      return;
+  }
+}
+
+void sweep_cls(const SweepCls &s, const ClsMat &A, const ClsMat &B, const double *x,
+               const double *base, double *out, double *out2, int mode, bool first,
+               const int *done) {
+  auto *f = A.width == 4 ? sweep_cls_mode<4> : A.width == 8 ? sweep_cls_mode<8> : sweep_cls_mode<16>;
+  f(s, A, B, x, base, out, out2, mode, first, done);
+}
+
 using PairKey = std::tuple<const int *, const int *, int, int, int, int>;
 std::map<PairKey, std::unique_ptr<PairPlan>> g_pair;
 
@@ -183,6 +315,45 @@ void forget_pair_plans(const void *p) {
   }
 }
 void release_pair_plans() { g_pair.clear(); }
+
+SweepCls sweep_encode(const SpmvPlan &L, const int *lia, const int *lja, const double *la,
+                      const SpmvPlan &U, const int *uia, const int *uja, const double *ua,
+                      const SpmvPlan *A, const int *ia, const int *ja, const double *a,
+                      const double *d_r) {
+  SweepCls s, none;
+  const int longest = std::max(L.max_row, U.max_row);
+  const int width = longest <= 4 ? 4 : (longest + 7) / 8 * 8;
+  s.n = L.n;
+  s.L = cls_encode("L", L.n, L.nnz, lia, lja, la, d_r, L.max_row, width);
+  if (!s.L.cls) return none;
+  s.U = cls_encode("U", U.n, U.nnz, uia, uja, ua, d_r, U.max_row, width);
+  if (!s.U.cls) return none;
+  if (A) {
+    s.A = cls_encode("S", A->n, A->nnz, ia, ja, a, d_r, A->max_row);
+    if (!s.A.cls) return none;
+  }
+  // (the pair's two tables: 64 KB of LDS at most)
+  if ((width == 4   ? sweep_lds<4>(s.L, s.U)
+       : width == 8 ? sweep_lds<8>(s.L, s.U)
+                    : sweep_lds<16>(s.L, s.U)) > 65536)
+    return none;
+  std::vector<int> offs = s.L.offsets;
+  offs.insert(offs.end(), s.U.offsets.begin(), s.U.offsets.end());
+  const auto g = xcd_grid(offs, kBlock, ((long)s.n - 1) / kBlock + 1, 8 * device_cus());
+  s.grid = g.first;
+  s.group = g.second;
+  return s;
+}
+
+void sweep_one_launch(const SweepCls &s, const ClsMat &A, const double *x, const double *base,
+                      double *out, double *out2, int mode, bool first, const int *done) {
+  sweep_cls(s, A, ClsMat(), x, base, out, out2, mode, first, done);
+}
+
+void sweep_pair_launch(const SweepCls &s, const double *x, const double *base, double *out,
+                       const int *done) {
+  sweep_cls(s, s.L, s.U, x, base, out, nullptr, kStorePair, false, done);
+}
 
 void sweep_one_launch(const SpmvPlan &p, const int *ia, const int *ja, const double *a,
                       const double *x, const double *base, const double *d_r, double *out,

@@ -37,9 +37,10 @@ def band(n, offs, weights=None, shift=0.05):
     return CSR(n, ia, cols[order].astype(np.int32), vals[order])
 
 
-def both(Ah, kind, b, maxit=40, d=None, x0=None, solve=None, tol=0.0, **opts):
+def both(Ah, kind, b, maxit=40, d=None, x0=None, solve=None, tol=0.0,
+         mk=(1, 1), **opts):
     A = S.DeviceCSR.from_csr(Ah)
-    P = S.make_preconditioner(A, Ah, kind)
+    P = S.make_preconditioner(A, Ah, kind, *mk)
     if d is not None:
         P.keep["d_r"].copy_(S.to_dev(d))
     out = []
@@ -154,3 +155,27 @@ def test_mixed_rows_without_a_diagonal():
              .astype(np.int32), Ah.ja[keep], Ah.a[keep])
     b = np.random.default_rng(10).standard_normal(Bh.n)
     same(*both(Bh, "none", b, maxit=20, solve=S.pcg_mixed, tol=1e-9))
+
+
+@pytest.mark.parametrize("kind,m,k", [("it_jacobi", 1, 1), ("it_jacobi", 1, 4), ("GS_it", 1, 1),
+                                      ("GS_it", 3, 2), ("GS_it2", 1, 1), ("GS_it2", 2, 3)])
+@pytest.mark.parametrize("name", ["first_encoded", "cube_odd", "row_9", "row_15", "row_17",
+                                  "mixed_classes", "one_sided", "too_many"])
+def test_sweeps(kind, m, k, name):
+    """Triangles of 2, 3, 4, 7 and 8 entries a row, and of 1 and 14 (so one
+    table is as wide as the other needs)."""
+    if name == "one_sided":
+        Ah = band(MIN_ROWS + 1, [1])
+        rows = np.repeat(np.arange(Ah.n), np.diff(Ah.ia))
+        ja = np.concatenate([Ah.ja] + [np.arange(Ah.n) - o for o in range(2, 15)])
+        rows = np.concatenate([rows, np.tile(np.arange(Ah.n), 13)])
+        a = np.concatenate([Ah.a, np.full(13 * Ah.n, -1e-3)])
+        keep = ja >= 0
+        rows, ja, a = rows[keep], ja[keep], a[keep]
+        order = np.lexsort((ja, rows))
+        Ah = CSR(Ah.n, np.concatenate([[0], np.cumsum(np.bincount(rows))]).astype(np.int32),
+                 ja[order].astype(np.int32), a[order])
+    else:
+        Ah = CASES[name]()
+    b = np.random.default_rng(11).standard_normal(Ah.n)
+    same(*both(Ah, kind, b, maxit=20, mk=(m, k)))
