@@ -4,22 +4,33 @@
 // (lap_adjacency_laplacian).
 //
 // COO -> CSR follows coo_to_csr (io_utils.c:141-235): rows are counted,
-// every entry (and, for a symmetric matrix, its mirror) is scattered into
-// its row, and each row is sorted by column.  The scatter uses atomics, so
-// the order inside a row is arbitrary; each entry therefore carries the key
-// (column << 32 | fill sequence), where the fill sequence is the position
-// the reference's serial fill gives it (2*i for COO entry i, 2*i+1 for its
-// mirror).  Keys are unique, so the sorted rows do not depend on timing and
-// equal a stable sort of the reference's fill, which is the reference's
-// result (glibc's qsort is a merge sort, and for distinct columns the order
-// is unique anyway).  Rows are sorted by length class:
-//   <= 32 entries      one thread per row, insertion sort;
+// every entry (and, for a symmetric matrix, its mirror) is put into its row,
+// and each row is sorted by column.  Atomics hand out the places in a row, so
+// the order inside it is arbitrary; what is put there (into ja, for the time) is the entry's fill sequence, the position the reference's serial
+// fill gives it (2*i for COO entry i, 2*i+1 for its mirror), and rows are
+// sorted by the key (column << 32 | fill sequence).  Keys are unique, so the
+// sorted rows do not depend on timing and equal a stable sort of the
+// reference's fill, which is the reference's result (glibc's qsort is a merge
+// sort, and for distinct columns the order is unique anyway).  Rows are sorted
+// by length class:
+//   <= 32 entries      in LDS, a lane per entry: its place is the number of
+//                      smaller keys in its row;
 //   <= 4096 entries    one workgroup per row, bitonic sort in LDS;
 //   longer             one workgroup per row: 4096-entry runs sorted in LDS,
 //                      then merged pairwise (merge path) through global
 //                      scratch.
-// Everything here is set-up work, run once per matrix; it is HBM- and
-// atomic-bound and makes no attempt at a roofline.
+//
+// Bound by atomics and by scattered writes.  Files list their entries by row or
+// by column, so neighbouring lanes mostly count for the same row: a run of
+// them takes one atomic.  One 4-byte word per CSR entry is scattered (the
+// column and value are gathered through it by the sort), by workgroups that
+// give each XCD one stretch of the file, so that the words of a line meet in
+// one L2.  150 x 160 x 170 (16.2M symmetric entries by row, 28.4M in CSR), the
+// size query and the conversion: 5.0 -> 0.8 ms (count 530 -> 78 us, twice;
+// placing 1590 -> 98; sorting 1160 -> 215, where its 450 MB take 92; scratch of
+// 16 bytes per CSR entry allocated before).  The same entries by column 4.7 ->
+// 1.2 ms; in random order, where each takes an atomic and a line of its own, 7.9
+// -> 5.7.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -31,7 +42,7 @@ namespace lap {
 namespace {
 
 constexpr int kShortRow = 32;
-constexpr int kLdsSort = 4096;  // entries per LDS sort (keys 32 KiB + index 8 KiB)
+constexpr int kLdsSort = 4096;  // entries per LDS sort (32 KiB of keys)
 
 // --------------------------------------------------------------- scans
 constexpr int kScanPer = 4;
@@ -142,37 +153,69 @@ __global__ void k_fill_int(long long n, int v, int *dst) {
 }
 
 // ---------------------------------------------------------- COO -> CSR
-__global__ void k_coo_count(long long nnz, int n, int m, const int *rows, const int *cols,
-                            int sym, int *cnt, int *err) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nnz;
-       i += (long long)gridDim.x * blockDim.x) {
-    const int r = rows[i], c = cols[i];
-    if (r < 0 || r >= n || c < 0 || c >= m) {
-      atomicOr(err, 1);
-      continue;
-    }
-    atomicAdd(&cnt[r], 1);
-    if (sym && r != c) atomicAdd(&cnt[c], 1);
+// Counts this lane's entry for row r (active lanes) and returns its place among
+// the row's: neighbouring lanes of one row take one atomic together.
+__device__ __forceinline__ int count_run(int *cnt, int r, bool active) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const unsigned long long on = __builtin_amdgcn_ballot_w64(active);
+  const int before = __shfl_up(r, 1, kWave);
+  const bool head = active && (lane == 0 || !((on >> (lane - 1)) & 1) || before != r);
+  const unsigned long long heads = __builtin_amdgcn_ballot_w64(head);
+  // the lanes up to this one that start a run; the first lane past this run
+  const unsigned long long upto = ~0ull >> (kWave - 1 - lane);
+  const int first = active ? kWave - 1 - __builtin_clzll(heads & upto) : lane;
+  const unsigned long long past = (heads | ~on) & ~upto;
+  int base = 0;
+  if (head) base = atomicAdd(&cnt[r], (past ? __builtin_ctzll(past) : kWave) - lane);
+  return __shfl(base, first, kWave) + (lane - first);
+}
+
+__global__ void __launch_bounds__(kBlock) k_coo_count(long long nnz, int n, int m,
+                                                      const int *__restrict__ rows,
+                                                      const int *__restrict__ cols, int sym,
+                                                      int *cnt, int *err) {
+  // (whole waves stay together)
+  for (long long i0 = (long long)blockIdx.x * kBlock; i0 < nnz;
+       i0 += (long long)gridDim.x * kBlock) {
+    const long long i = i0 + threadIdx.x;
+    const bool live = i < nnz;
+    const int r = live ? rows[i] : 0, c = live ? cols[i] : 0;
+    const bool ok = live && r >= 0 && r < n && c >= 0 && c < m;
+    if (live && !ok) atomicOr(err, 1);
+    count_run(cnt, r, ok);
+    if (sym) count_run(cnt, c, ok && r != c);
   }
 }
 
-__global__ void k_coo_scatter(long long nnz, const int *rows, const int *cols, const double *vals,
-                              int sym, int *fill, unsigned long long *key, double *tv) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nnz;
-       i += (long long)gridDim.x * blockDim.x) {
-    const int r = rows[i], c = cols[i];
-    const double v = vals[i];
-    const unsigned seq = (unsigned)(2 * i);
-    int pos = atomicAdd(&fill[r], 1);
-    key[pos] = ((unsigned long long)(unsigned)c << 32) | seq;
-    tv[pos] = v;
-    if (sym && r != c) {
-      pos = atomicAdd(&fill[c], 1);
-      key[pos] = ((unsigned long long)(unsigned)r << 32) | (seq + 1u);
-      tv[pos] = v;
-    }
+// fill: ia[0..n) at the start
+__global__ void __launch_bounds__(kBlock) k_coo_place(long long nnz, const int *__restrict__ rows,
+                                                      const int *__restrict__ cols, int sym,
+                                                      int *fill, unsigned *__restrict__ seq) {
+  // XCD x (workgroups x, x + 8, ..) takes the x-th eighth of the entries
+  const long long tiles = (nnz + kBlock - 1) / kBlock, per = (tiles + 7) / 8;
+  const long long t0 = (blockIdx.x & 7) * per, t1 = min(tiles, t0 + per);
+  for (long long t = t0 + (blockIdx.x >> 3); t < t1; t += gridDim.x >> 3) {
+    const long long i = t * kBlock + threadIdx.x;
+    const bool live = i < nnz;
+    const int r = live ? rows[i] : 0, c = live ? cols[i] : 0;
+    const int a = count_run(fill, r, live);
+    if (live) seq[a] = (unsigned)(2 * i);
+    if (!sym) continue;
+    const int b = count_run(fill, c, live && r != c);
+    if (live && r != c) seq[b] = (unsigned)(2 * i) + 1u;
   }
 }
+
+// What an entry's fill sequence stands for.
+struct CooSrc {
+  const int *rows, *cols;
+  const double *vals;
+  __device__ __forceinline__ unsigned long long key(unsigned q) const {
+    const int c = (q & 1) ? rows[q >> 1] : cols[q >> 1];
+    return ((unsigned long long)(unsigned)c << 32) | q;
+  }
+  __device__ __forceinline__ double val(unsigned q) const { return vals[q >> 1]; }
+};
 
 // Lists rows longer than kShortRow: medium (<= kLdsSort) and long rows,
 // long rows with a scratch offset.  cnt: [0] medium, [1] long; off: scratch
@@ -194,33 +237,90 @@ __global__ void k_row_classes(int n, const int *ia, int *med, int *lng, long lon
 
 __device__ __forceinline__ int col_of(unsigned long long k) { return (int)(k >> 32); }
 
-__global__ void k_sort_short(int n, const int *ia, unsigned long long *key, double *tv, int *ja,
-                             double *a) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int s = ia[i], len = ia[i + 1] - s;
-    if (len > kShortRow) continue;
-    for (int t = 1; t < len; ++t) {
-      const unsigned long long k = key[s + t];
-      const double v = tv[s + t];
-      int j = t - 1;
-      while (j >= 0 && key[s + j] > k) {
-        key[s + j + 1] = key[s + j];
-        tv[s + j + 1] = tv[s + j];
-        --j;
+// Rows of at most kShortRow entries, kSortRows of them by a workgroup, up to
+// kSortCap entries in LDS; counts the longer rows (ctr as k_row_classes).  seq
+// may be ja: a row's words are read before its columns are written.
+constexpr int kSortRows = 128, kSortCap = 2048;
+__global__ void __launch_bounds__(kBlock) k_sort_short(int n, const int *__restrict__ ia,
+                                                       const unsigned *seq, CooSrc src, int *ja,
+                                                       double *__restrict__ a, int *ctr,
+                                                       unsigned long long *off) {
+  constexpr int kPer = kSortCap / kBlock;
+  __shared__ unsigned long long key[kSortCap];
+  __shared__ __align__(16) unsigned char rowof[kSortCap];
+  __shared__ int st[kSortRows + 1];
+  const int tid = threadIdx.x;
+  for (long long r0 = (long long)blockIdx.x * kSortRows; r0 < n;
+       r0 += (long long)gridDim.x * kSortRows) {
+    const int nr = (int)min((long long)kSortRows, n - r0);
+    __syncthreads();  // (the last rows' keys are read)
+    for (int t = tid; t <= nr; t += kBlock) st[t] = ia[r0 + t];
+    __syncthreads();
+    const int e0 = st[0], cnt = st[nr] - e0;
+    if (tid < nr) {
+      const int len = st[tid + 1] - st[tid];
+      if (len > kLdsSort) {
+        atomicAdd(&ctr[1], 1);
+        atomicAdd(off, (unsigned long long)len);
+      } else if (len > kShortRow) {
+        atomicAdd(&ctr[0], 1);
       }
-      key[s + j + 1] = k;
-      tv[s + j + 1] = v;
     }
-    for (int t = 0; t < len; ++t) {
-      ja[s + t] = col_of(key[s + t]);
-      a[s + t] = tv[s + t];
+    if (cnt <= kSortCap) {
+      unsigned q[kPer];
+      unsigned long long k[kPer];
+      double v[kPer];
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) q[u] = u * kBlock + tid < cnt ? seq[e0 + u * kBlock + tid] : 0;
+#pragma unroll
+      for (int u = 0; u < kPer; ++u)
+        if (u * kBlock + tid < cnt) {
+          k[u] = src.key(q[u]);
+          v[u] = src.val(q[u]);
+        }
+      for (int t = tid * 16; t < cnt; t += kBlock * 16)
+        *reinterpret_cast<uint4 *>(rowof + t) = uint4{~0u, ~0u, ~0u, ~0u};
+      __syncthreads();
+      if (tid < nr) {
+        const int s = st[tid] - e0, len = st[tid + 1] - e0 - s;
+        if (len <= kShortRow)
+          for (int j = 0; j < len; ++j) rowof[s + j] = (unsigned char)tid;
+      }
+#pragma unroll
+      for (int u = 0; u < kPer; ++u)
+        if (u * kBlock + tid < cnt) key[u * kBlock + tid] = k[u];
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) {
+        if (u * kBlock + tid >= cnt) continue;
+        const int row = rowof[u * kBlock + tid];
+        if (row == 255) continue;  // of a longer row
+        const int s = st[row] - e0, len = st[row + 1] - e0 - s;
+        int rank = 0;
+        for (int j = 0; j < len; ++j) rank += key[s + j] < k[u];
+        ja[e0 + s + rank] = col_of(k[u]);
+        a[e0 + s + rank] = v[u];
+      }
+      continue;
+    }
+    // many entries, or long rows among them: a wave per short row
+    for (int row = threadIdx.x / kWave; row < nr; row += kBlock / kWave) {
+      const int s = st[row], len = st[row + 1] - s, lane = threadIdx.x & (kWave - 1);
+      if (len > kShortRow) continue;
+      const unsigned long long k = lane < len ? src.key(seq[s + lane]) : ~0ull;
+      int rank = 0;
+      for (int j = 0; j < len; ++j) rank += __shfl(k, j, kWave) < k;
+      if (lane < len) {
+        ja[s + rank] = col_of(k);
+        a[s + rank] = src.val((unsigned)k);
+      }
     }
   }
 }
 
-// Sorts k[0..P) ascending with its index array (P a power of two <=
-// kLdsSort), all threads of the workgroup.
-__device__ void lds_bitonic(unsigned long long *k, unsigned short *ix, int P) {
+// Sorts k[0..P) ascending (P a power of two <= kLdsSort), all threads of the
+// workgroup.
+__device__ void lds_bitonic(unsigned long long *k, int P) {
   for (int w = 2; w <= P; w <<= 1)
     for (int j = w >> 1; j > 0; j >>= 1) {
       for (int i = threadIdx.x; i < P; i += kBlock) {
@@ -231,9 +331,6 @@ __device__ void lds_bitonic(unsigned long long *k, unsigned short *ix, int P) {
           if ((x > y) == up) {
             k[i] = y;
             k[l] = x;
-            const unsigned short t = ix[i];
-            ix[i] = ix[l];
-            ix[l] = t;
           }
         }
       }
@@ -241,32 +338,27 @@ __device__ void lds_bitonic(unsigned long long *k, unsigned short *ix, int P) {
     }
 }
 
-// Loads key[s..s+len) (len <= kLdsSort) into LDS padded to a power of two
-// and sorts it.
-__device__ int lds_load_sort(const unsigned long long *key, long long s, int len,
-                             unsigned long long *k, unsigned short *ix) {
+// Loads the keys of seq[s..s+len) (len <= kLdsSort) into LDS padded to a
+// power of two and sorts them.
+__device__ void lds_load_sort(const unsigned *seq, const CooSrc &src, long long s, int len,
+                              unsigned long long *k) {
   int P = 1;
   while (P < len) P <<= 1;
-  for (int t = threadIdx.x; t < P; t += kBlock) {
-    k[t] = t < len ? key[s + t] : ~0ull;
-    ix[t] = (unsigned short)t;
-  }
+  for (int t = threadIdx.x; t < P; t += kBlock) k[t] = t < len ? src.key(seq[s + t]) : ~0ull;
   __syncthreads();
-  lds_bitonic(k, ix, P);
-  return P;
+  lds_bitonic(k, P);
 }
 
 __global__ void __launch_bounds__(kBlock) k_sort_medium(const int *rowlist, const int *ia,
-                                                        const unsigned long long *key,
-                                                        const double *tv, int *ja, double *a) {
+                                                        const unsigned *seq, CooSrc src, int *ja,
+                                                        double *a) {
   __shared__ unsigned long long k[kLdsSort];
-  __shared__ unsigned short ix[kLdsSort];
   const int row = rowlist[blockIdx.x];
   const int s = ia[row], len = ia[row + 1] - s;
-  lds_load_sort(key, s, len, k, ix);
+  lds_load_sort(seq, src, s, len, k);
   for (int t = threadIdx.x; t < len; t += kBlock) {
     ja[s + t] = col_of(k[t]);
-    a[s + t] = tv[s + ix[t]];
+    a[s + t] = src.val((unsigned)k[t]);
   }
 }
 
@@ -286,62 +378,45 @@ __device__ int merge_split(const unsigned long long *A, int la, const unsigned l
 }
 
 __global__ void __launch_bounds__(kBlock) k_sort_long(const int *rowlist, const long long *rowoff,
-                                                      const int *ia,
-                                                      const unsigned long long *key,
-                                                      const double *tv,
-                                                      unsigned long long *k0, int *i0,
-                                                      unsigned long long *k1, int *i1, int *ja,
+                                                      const int *ia, const unsigned *seq,
+                                                      CooSrc src, unsigned long long *k0,
+                                                      unsigned long long *k1, int *ja,
                                                       double *a) {
   __shared__ unsigned long long k[kLdsSort];
-  __shared__ unsigned short ix[kLdsSort];
   const int row = rowlist[blockIdx.x];
   const long long s = ia[row];
   const int len = ia[row + 1] - (int)s;
   const long long o = rowoff[blockIdx.x];
   unsigned long long *kb[2] = {k0 + o, k1 + o};
-  int *ib[2] = {i0 + o, i1 + o};
   // runs of kLdsSort sorted in LDS
   for (int c0 = 0; c0 < len; c0 += kLdsSort) {
     const int cl = min(kLdsSort, len - c0);
-    lds_load_sort(key, s + c0, cl, k, ix);
-    for (int t = threadIdx.x; t < cl; t += kBlock) {
-      kb[0][c0 + t] = k[t];
-      ib[0][c0 + t] = c0 + ix[t];
-    }
+    lds_load_sort(seq, src, s + c0, cl, k);
+    for (int t = threadIdx.x; t < cl; t += kBlock) kb[0][c0 + t] = k[t];
     __syncthreads();
   }
   // pairwise merges; each thread produces a contiguous slice of every merge
-  int src = 0;
+  int cur = 0;
   for (int w = kLdsSort; w < len; w <<= 1) {
     for (int lo = 0; lo < len; lo += 2 * w) {
       const int la = min(w, len - lo), lb = max(0, min(w, len - lo - w));
-      const unsigned long long *A = kb[src] + lo, *B = A + la;
-      const int *IA = ib[src] + lo, *IB = IA + la;
-      unsigned long long *O = kb[src ^ 1] + lo;
-      int *OI = ib[src ^ 1] + lo;
+      const unsigned long long *A = kb[cur] + lo, *B = A + la;
+      unsigned long long *O = kb[cur ^ 1] + lo;
       const int m = la + lb;
       const int d0 = (int)((long long)m * threadIdx.x / kBlock);
       const int d1 = (int)((long long)m * (threadIdx.x + 1) / kBlock);
       int x = merge_split(A, la, B, lb, d0), y = d0 - x;
       for (int d = d0; d < d1; ++d) {
         const bool takeA = y >= lb || (x < la && A[x] < B[y]);
-        if (takeA) {
-          O[d] = A[x];
-          OI[d] = IA[x];
-          ++x;
-        } else {
-          O[d] = B[y];
-          OI[d] = IB[y];
-          ++y;
-        }
+        O[d] = takeA ? A[x++] : B[y++];
       }
     }
     __syncthreads();
-    src ^= 1;
+    cur ^= 1;
   }
   for (int t = threadIdx.x; t < len; t += kBlock) {
-    ja[s + t] = col_of(kb[src][t]);
-    a[s + t] = tv[s + ib[src][t]];
+    ja[s + t] = col_of(kb[cur][t]);
+    a[s + t] = src.val((unsigned)kb[cur][t]);
   }
 }
 
@@ -432,6 +507,7 @@ int lap_coo_to_csr(int n, int m, int nnz, const int *rows, const int *cols, cons
     return LAP_ERR_ARG;
   DevBuf cnt(4 * ((size_t)n + 1) + 16), ws(scan_ws_bytes(n) + 16);
   int *c = cnt.as<int>();
+  if (!cnt.p || !ws.p) return lap_last_status();
   hipLaunchKernelGGL(k_fill_int, dim3(rows_grid(n + 1)), dim3(kBlock), 0, stream(),
                      (long long)n + 1, 0, c);
   if (nnz)
@@ -459,35 +535,40 @@ int lap_coo_to_csr(int n, int m, int nnz, const int *rows, const int *cols, cons
   if (total == 0) return LAP_OK;
   if (!check_device("coo_to_csr", {{ja, "ja", 4 * (size_t)total}, {a, "a", 8 * (size_t)total}}))
     return LAP_ERR_ARG;
-  // fill pointers, keyed scatter
+  DevBuf ctr(32);
+  if (!ctr.p) return lap_last_status();
+  unsigned *seq = reinterpret_cast<unsigned *>(ja);  // until the rows are sorted
+  const CooSrc src{rows, cols, vals};
   LAP_HIP(hipMemcpyAsync(c, ia, 4 * (size_t)n, hipMemcpyDeviceToDevice, stream()));
-  DevBuf key(8 * (size_t)total), tv(8 * (size_t)total);
-  hipLaunchKernelGGL(k_coo_scatter, dim3(rows_grid(nnz)), dim3(kBlock), 0, stream(),
-                     (long long)nnz, rows, cols, vals, symmetric, c, key.as<unsigned long long>(),
-                     tv.as<double>());
-  // row classes
-  DevBuf med(4 * (size_t)n + 16), lng(4 * (size_t)n + 16), lng_off(8 * (size_t)n + 16),
-      ctr(32);
+  hipLaunchKernelGGL(k_coo_place, dim3((rows_grid(nnz) + 7) / 8 * 8), dim3(kBlock), 0, stream(),
+                     (long long)nnz, rows, cols, symmetric, c, seq);
   hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, stream(), 8ll, 0, ctr.as<int>());
-  hipLaunchKernelGGL(k_row_classes, dim3(rows_grid(n)), dim3(kBlock), 0, stream(), n, ia,
-                     med.as<int>(), lng.as<int>(), lng_off.as<long long>(), ctr.as<int>(),
+  hipLaunchKernelGGL(k_sort_short, dim3(rows_grid(((long long)n + kSortRows - 1) / kSortRows * kBlock)),
+                     dim3(kBlock), 0, stream(), n, ia, seq, src, ja, a, ctr.as<int>(),
                      (unsigned long long *)(ctr.as<int>() + 2));
-  hipLaunchKernelGGL(k_sort_short, dim3(rows_grid(n)), dim3(kBlock), 0, stream(), n, ia,
-                     key.as<unsigned long long>(), tv.as<double>(), ja, a);
   int h[4] = {0, 0, 0, 0};
   LAP_HIP(hipMemcpyAsync(h, ctr.p, sizeof h, hipMemcpyDeviceToHost, stream()));
   sync();
   unsigned long long long_total;
   memcpy(&long_total, h + 2, sizeof long_total);
-  if (h[0])
-    hipLaunchKernelGGL(k_sort_medium, dim3(h[0]), dim3(kBlock), 0, stream(), med.as<int>(), ia,
-                       key.as<unsigned long long>(), tv.as<double>(), ja, a);
-  if (h[1]) {
-    DevBuf k0(8 * long_total), k1(8 * long_total), i0(4 * long_total), i1(4 * long_total);
-    hipLaunchKernelGGL(k_sort_long, dim3(h[1]), dim3(kBlock), 0, stream(), lng.as<int>(),
-                       lng_off.as<long long>(), ia, key.as<unsigned long long>(), tv.as<double>(),
-                       k0.as<unsigned long long>(), i0.as<int>(), k1.as<unsigned long long>(),
-                       i1.as<int>(), ja, a);
+  if (h[0] || h[1]) {
+    DevBuf med(4 * (size_t)h[0] + 16), lng(4 * (size_t)h[1] + 16), lng_off(8 * (size_t)h[1] + 16);
+    if (!med.p || !lng.p || !lng_off.p) return lap_last_status();
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, stream(), 8ll, 0, ctr.as<int>());
+    hipLaunchKernelGGL(k_row_classes, dim3(rows_grid(n)), dim3(kBlock), 0, stream(), n, ia,
+                       med.as<int>(), lng.as<int>(), lng_off.as<long long>(), ctr.as<int>(),
+                       (unsigned long long *)(ctr.as<int>() + 2));
+    if (h[0])
+      hipLaunchKernelGGL(k_sort_medium, dim3(h[0]), dim3(kBlock), 0, stream(), med.as<int>(), ia,
+                         seq, src, ja, a);
+    if (h[1]) {
+      DevBuf k0(8 * long_total), k1(8 * long_total);
+      if (!k0.p || !k1.p) return lap_last_status();
+      hipLaunchKernelGGL(k_sort_long, dim3(h[1]), dim3(kBlock), 0, stream(), lng.as<int>(),
+                         lng_off.as<long long>(), ia, seq, src, k0.as<unsigned long long>(),
+                         k1.as<unsigned long long>(), ja, a);
+      sync();
+    }
     sync();
   }
   sync();
