@@ -26,12 +26,12 @@ __device__ __forceinline__ void spmv_long_row(int r0, int e0, int e1, const int 
 
 // Row sums from the LDS products, in CSR order (row-sequential, as the
 // reference's simple_csr_matvec, simple_blas.c:24-44).
-template <int BS, class Epi>
+template <int BS, bool DEEP = false, class Epi>
 __device__ __forceinline__ void spmv_row_sums(int r0, int r1, int e0, const int *__restrict__ ia,
                                               const double *prod, Epi &epi) {
   for (int row = r0 + (int)threadIdx.x; row < r1; row += BS) {
     const int s0 = ia[row] - e0, s1 = ia[row + 1] - e0;
-    epi.store(row, lds_seq_sum(epi.init(row), prod, s0, s1));
+    epi.store(row, lds_seq_sum<false, DEEP>(epi.init(row), prod, s0, s1));
   }
 }
 
@@ -40,7 +40,7 @@ __device__ __forceinline__ void spmv_row_sums(int r0, int r1, int e0, const int 
 // order.  Block-uniform control flow.  Values (VT) and vectors (XT) may be
 // FP32; products and row sums are FP64.
 //  prod : __shared__ double[TILE], red : __shared__ double[BS/64].
-template <int BS, int TILE, class Epi, class VT = double, class XT = double>
+template <int BS, int TILE, class Epi, class VT = double, class XT = double, bool DEEP = false>
 __device__ __forceinline__ void spmv_block_rows(int b, const int *__restrict__ rowblk,
                                                 const int *__restrict__ ia,
                                                 const int *__restrict__ ja,
@@ -60,7 +60,7 @@ __device__ __forceinline__ void spmv_block_rows(int b, const int *__restrict__ r
     prod[k] = (alpha * (double)a[e]) * (double)x[ja[e]];
   }
   __syncthreads();
-  spmv_row_sums<BS>(r0, r1, e0, ia, prod, epi);
+  spmv_row_sums<BS, DEEP>(r0, r1, e0, ia, prod, epi);
   __syncthreads();
 }
 
