@@ -35,7 +35,12 @@ def ptr(t):
 
 
 def _sync():
-    torch.cuda.synchronize()
+    # torch.cuda.synchronize() without its device bookkeeping (2.8 -> 0.5 us
+    # when the device is idle)
+    if torch.cuda.is_initialized():
+        torch._C._cuda_synchronize()
+    else:
+        torch.cuda.synchronize()
 
 
 @dataclass
