@@ -7,7 +7,7 @@
 // CUs: 2^17 rows of 11 entries are 15 MB of matrix against 128 MiB of
 // registers.
 //
-// How: a workgroup of 1024 threads owns a contiguous range of rows, R rows per
+// How: a workgroup of 1024 (or 512) threads owns a contiguous range of rows, R per
 // thread, for the whole solve.  A thread keeps its rows' values, column slots,
 // x, r, p and 1/diag in registers; the LDS holds the p of the workgroup's rows
 // and of the other rows they refer to (its halo).  What crosses between
@@ -44,7 +44,6 @@ namespace lap {
 namespace {
 
 constexpr int kResThreads = 1024;
-constexpr int kResWaves = kResThreads / kWave;
 constexpr int kResHalo = 8192;     // halo entries of a workgroup at most
 constexpr int kResMaxWg = 256;     // workgroups at most (partials: one per thread of 4 waves)
 // Rows per workgroup at least: fewer workgroups have fewer partial sums to
@@ -53,6 +52,7 @@ constexpr int kResMaxWg = 256;     // workgroups at most (partials: one per thre
 // 3.89, 512^2 9.05 / 9.08 / 6.86, 40^3 7.15 / 6.66 / 6.70, 64^3 9.4 / 9.4 /
 // 11.1, 97 x 90 x 31 8.7 / 8.7 / 10.6: 2048 for rows of up to 5 entries.
 constexpr int kResRows = 1024, kResRowsShort = 2048, kResShort = 5;
+constexpr int kResBig = 1 << 16;   // rows of a large system
 constexpr int kResMaxN = 1 << 19;  // rows of a system at most (the analysis' bitmap in LDS)
 constexpr int kResMaxRows = 1 << 26;  // rows of all systems at most (box_w stays below 2^31 bytes)
 constexpr int kResIters = 8192;    // iterations per launch
@@ -113,11 +113,16 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {  // lane 63
   return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
 }
 
-// The launch.  R rows per thread, rows of at most L entries.
-template <int R, int L>
-__global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
+// The launch.  R rows per thread, rows of at most L entries, T threads.  512
+// threads add up as 1024 do, each what two of those would (the even and the odd
+// rows of its R), so x does not depend on T: two such workgroups share a CU and
+// one's waits are the other's time, but one by itself has its rows' work on half
+// the lanes.
+template <int R, int L, int T>
+__global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
+  constexpr int V = kResThreads / T, W = T / kWave, C = L % 4 ? L : 4;  // waves; entries in flight
   extern __shared__ double ps[];  // own rows, halo, a zero; the halo's rows
-  __shared__ double red[2][kResWaves], tot[2][4], one[2];
+  __shared__ double red[2][V * W], tot[2][4], one[2];
   __shared__ int dead;
   const int t = threadIdx.x, lane = t & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
@@ -126,8 +131,8 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
   const int base = wg.base, rows = wg.rows, team = wg.team, size = wg.size;
   ResState *const st = g.st + wg.sys;
   const int nh = g.hcnt[w];
-  double *const halo = ps + R * kResThreads;
-  const int zero = R * kResThreads + g.nhmax;
+  double *const halo = ps + R * T;
+  const int zero = R * T + g.nhmax;
   int *const hcol = reinterpret_cast<int *>(ps + zero + 1);  // the halo's rows
   const __amdgpu_buffer_rsrc_t box_a = fl_buffer(g.box_a, g.nwg * 16);
   const __amdgpu_buffer_rsrc_t box_b = fl_buffer(g.box_b, g.nwg * 32);
@@ -136,16 +141,16 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
     dead = 0;
     ps[zero] = 0.0;
   }
-  for (int h = t; h < nh; h += kResThreads) hcol[h] = g.hcol[(size_t)w * kResHalo + h];
+  for (int h = t; h < nh; h += T) hcol[h] = g.hcol[(size_t)w * kResHalo + h];
   __syncthreads();
   // the thread's rows
   double val[R][L], x[R], r[R], p[R], d[R];
-  unsigned slot[R][L / 2];
+  unsigned slot[R][(L + 1) / 2];
   bool have[R], sent[R];
   int longest[R];  // of the wave's rows
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    const int l = t + k * kResThreads, row = base + l;
+    const int l = t + k * T, row = base + l;
     have[k] = l < rows;
     const int e0 = have[k] ? g.ia[row] : 0, len = have[k] ? g.ia[row + 1] - e0 : 0;
 #pragma unroll
@@ -171,14 +176,14 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
     for (int k = 0; k < R; ++k) {
       s[k] = 0.0;
 #pragma unroll
-      for (int j = 0; j < L; j += 4) {
+      for (int j = 0; j < L; j += C) {
         if (j >= longest[k]) break;
-        double v[4];
+        double v[C];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < C; ++i)
           v[i] = ps[(i & 1) ? slot[k][(j + i) / 2] >> 16 : slot[k][(j + i) / 2] & 0xffffu];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[k] += val[k][j + i] * v[i];
+        for (int i = 0; i < C; ++i) s[k] += val[k][j + i] * v[i];
       }
     }
   };
@@ -198,20 +203,23 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
   };
   // Sums of v over the team (N = 1: box_a, 2: box_b), to every thread;
   // `between` runs while they are on their way.
-  auto all_sums = [&](auto &v, unsigned tag, auto &&between) {
-    constexpr int N = sizeof(v) / sizeof(v[0]);
+  auto all_sums = [&](auto &sum, auto &v, unsigned tag, auto &&between) {
+    constexpr int N = sizeof(sum) / sizeof(sum[0]);
     const __amdgpu_buffer_rsrc_t box = N == 1 ? box_a : box_b;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      const double s = wave_sum_dpp(v[i]);
-      if (lane == kWave - 1) red[i][wave] = s;
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        const double s = wave_sum_dpp(v[j][i]);
+        if (lane == kWave - 1) red[i][j * W + wave] = s;
+      }
     }
     __syncthreads();
     if (wave == 0) {
 #pragma unroll
       for (int i = 0; i < N; ++i) {
-        const double s = row_sum_dpp(lane < kResWaves ? red[i][lane] : 0.0);
-        if (lane == kResWaves - 1) {
+        const double s = row_sum_dpp(lane < V * W ? red[i][lane] : 0.0);
+        if (lane == V * W - 1) {
           if (size > 1)
             fl_put(box, w * N + i, tag, s);
           else
@@ -250,18 +258,18 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < N; ++i)
-      v[i] = size > 1 ? ((tot[i][0] + tot[i][1]) + tot[i][2]) + tot[i][3] : one[i];
+      sum[i] = size > 1 ? ((tot[i][0] + tot[i][1]) + tot[i][2]) + tot[i][3] : one[i];
   };
   // halo entries: p = w (first) or beta p + w, w as its owner sent it.  The
   // first entry of each thread is asked for ahead (halo_ask).
   FlBoxed<double> ahead;
   auto halo_ask = [&] { ahead.load(box_w, t < nh ? hcol[t] : 0); };
   auto halo_update = [&](unsigned tag, bool first, double beta) {
-    for (int h0 = wave * kWave; h0 < nh; h0 += kResThreads) {
+    for (int h0 = wave * kWave; h0 < nh; h0 += T) {
       const int h = h0 + lane;
       const int c = h < nh ? hcol[h] : 0;
       FlBoxed<double> f;
-      if (h0 < kResThreads)
+      if (h0 < T)
         f = ahead;
       else
         f.load(box_w, c);
@@ -276,7 +284,7 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
   };
   auto own_update = [&]() {
 #pragma unroll
-    for (int k = 0; k < R; ++k) ps[t + k * kResThreads] = p[k];
+    for (int k = 0; k < R; ++k) ps[t + k * T] = p[k];
   };
   auto nothing = [] {};
 
@@ -291,34 +299,34 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
     it = st->iter;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      const int row = base + t + k * kResThreads;
+      const int row = base + t + k * T;
       r[k] = have[k] ? g.r[row] : 0.0;
       p[k] = have[k] ? g.p[row] : 0.0;
     }
-    for (int h = t; h < nh; h += kResThreads) halo[h] = g.p[hcol[h]];
+    for (int h = t; h < nh; h += T) halo[h] = g.p[hcol[h]];
     own_update();
     __syncthreads();
   } else {
     // r = -(A x - b) (cg.c:48-55), w = d_r r, p = w
 #pragma unroll
-    for (int k = 0; k < R; ++k) ps[t + k * kResThreads] = x[k];
-    for (int h = t; h < nh; h += kResThreads) halo[h] = g.x[hcol[h]];
+    for (int k = 0; k < R; ++k) ps[t + k * T] = x[k];
+    for (int h = t; h < nh; h += T) halo[h] = g.x[hcol[h]];
     __syncthreads();
-    double s[R], v[2] = {0.0, 0.0};
+    double s[R], v[V][2] = {}, sum[2];
     row_sums(s);
     ++tag;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      const int row = base + t + k * kResThreads;
+      const int row = base + t + k * T;
       r[k] = have[k] ? -(s[k] - g.b[row]) : 0.0;
       p[k] = d[k] * r[k];
       if (sent[k]) fl_put(box_w, row, tag, p[k]);
-      v[0] += r[k] * p[k];
-      v[1] += r[k] * r[k];
+      v[k % V][0] += r[k] * p[k];
+      v[k % V][1] += r[k] * r[k];
     }
-    all_sums(v, tag, halo_ask);
-    rho = v[0];
-    res0 = res = sqrt(v[1]);
+    all_sums(sum, v, tag, halo_ask);
+    rho = sum[0];
+    res0 = res = sqrt(sum[1]);
     tolrel = g.tol * res0;
     it = 0;
     if (g.hist && w == 0 && t == 0) g.hist[0] = res0;
@@ -335,47 +343,47 @@ __global__ __launch_bounds__(kResThreads, 4) void k_resident(ResArgs g) {
   while (flag < 0 && it < stop && !__builtin_amdgcn_readfirstlane(dead)) {
     ++it;
     // q = A p, p.q, alpha
-    double q[R], v1[1] = {0.0};
+    double q[R], v1[V][1] = {}, pq[1];
     row_sums(q);
 #pragma unroll
-    for (int k = 0; k < R; ++k) v1[0] += p[k] * q[k];
-    all_sums(v1, ++tag, nothing);
-    const double alpha = rho / v1[0], nalpha = -1.0 * alpha;
+    for (int k = 0; k < R; ++k) v1[k % V][0] += p[k] * q[k];
+    all_sums(pq, v1, ++tag, nothing);
+    const double alpha = rho / pq[0], nalpha = -1.0 * alpha;
     // r -= alpha q, w = d_r r, r.w, r.r; x += alpha p on the way
-    double wv[R], v[2] = {0.0, 0.0};
+    double v[V][2] = {}, sum[2];
     ++tag;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
       r[k] = r[k] + nalpha * q[k];
-      wv[k] = d[k] * r[k];
-      if (sent[k]) fl_put(box_w, base + t + k * kResThreads, tag, wv[k]);
-      v[0] += r[k] * wv[k];
-      v[1] += r[k] * r[k];
+      const double wk = d[k] * r[k];
+      if (sent[k]) fl_put(box_w, base + t + k * T, tag, wk);
+      v[k % V][0] += r[k] * wk;
+      v[k % V][1] += r[k] * r[k];
     }
-    all_sums(v, tag, [&] {
+    all_sums(sum, v, tag, [&] {
 #pragma unroll
       for (int k = 0; k < R; ++k) x[k] += alpha * p[k];
       halo_ask();
     });
     // convergence test (cg.c:106-123) and beta
-    res = sqrt(v[1]);
+    res = sqrt(sum[1]);
     if (g.hist && w == 0 && t == 0) g.hist[it] = res;
     if (!isfinite(res)) flag = 2;
     else if (res < tolrel) flag = 0;
     else if (it > g.maxit) flag = 1;
     flag = __builtin_amdgcn_readfirstlane(flag);
     if (flag >= 0) break;
-    const double beta = v[0] / rho;
-    rho = v[0];
+    const double beta = sum[0] / rho;
+    rho = sum[0];
 #pragma unroll
-    for (int k = 0; k < R; ++k) p[k] = p[k] * beta + wv[k];
+    for (int k = 0; k < R; ++k) p[k] = p[k] * beta + d[k] * r[k];
     own_update();
     halo_update(tag, false, beta);
     __syncthreads();
   }
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    const int row = base + t + k * kResThreads;
+    const int row = base + t + k * T;
     if (!have[k]) continue;
     g.x[row] = x[k];
     if (flag < 0) {
@@ -464,21 +472,24 @@ __global__ void k_res_zero(long long n, unsigned *p) {
 
 using ResKernel = void (*)(ResArgs);
 struct ResShape {
-  int r, l;
+  int r, l, threads;
   ResKernel fn;
 };
 // A thread's registers hold R (2.5 L + 8) words beside the work of a row: 128
 // registers per thread at 1024 threads allow these.
-const ResShape kShapes[] = {{1, 8, k_resident<1, 8>},   {2, 8, k_resident<2, 8>},
-                            {1, 16, k_resident<1, 16>}, {1, 24, k_resident<1, 24>},
-                            {1, 32, k_resident<1, 32>}};
+const ResShape kShapes[] = {{4, 5, 512, k_resident<4, 5, 512>},
+                            {1, 8, 1024, k_resident<1, 8, 1024>},
+                            {2, 8, 1024, k_resident<2, 8, 1024>},
+                            {1, 16, 1024, k_resident<1, 16, 1024>},
+                            {1, 24, 1024, k_resident<1, 24, 1024>},
+                            {1, 32, 1024, k_resident<1, 32, 1024>}};
 
 }  // namespace
 
 struct ResPlan {
   bool ok = false;
   std::vector<int> off;
-  int nsys = 0, nwg = 0, nhmax = 0, lds = 0;
+  int nsys = 0, nwg = 0, nhmax = 0, lds = 0, threads = 0;
   ResKernel fn = nullptr;
   DevBufPtr wg, hcnt, hcol, sent, lcol, boxes, state, shared;
   size_t box_words = 0;
@@ -498,9 +509,21 @@ std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const 
   auto rows_per = [&](int rows) {
     return std::max(least, ((rows + cus - 1) / cus + kWave - 1) / kWave * kWave);
   };
+  long wgs_all = 0;
+  for (int q = 0; q < ns; ++q) {
+    const int rows = off[(size_t)q + 1] - off[(size_t)q];
+    wgs_all += rows ? (rows + rows_per(rows) - 1) / rows_per(rows) : 0;
+  }
+  // Two workgroups per CU for large systems and where there are half as many
+  // again as CUs.  With 1024 and 512 threads, us per iteration: 60 x 52 3.4 and
+  // 3.9, 128^2 4.0 and 4.2, 256^2 5.3 and 5.1, 512^2 7.1 and 7.0, 700^2 10.3 and
+  // 8.4; batches, ms: 160 grids of up to 150^2 (600 workgroups) 7.9 and 5.6, 60 of
+  // up to 400^2 132 and 89, 2000 of up to 20^2 1.3 and 1.0, but 300 of up to 60^2
+  // (340 workgroups) 1.57 and 1.79.
+  const bool half = A.max_row <= kResShort && (big >= kResBig || 2 * wgs_all > 3 * cus);
   for (const ResShape &c : kShapes) {
-    if (A.max_row > c.l) continue;
-    if (rows_per(big) <= c.r * kResThreads) {
+    if (A.max_row > c.l || half != (c.threads < kResThreads)) continue;
+    if (rows_per(big) <= c.r * c.threads) {
       s = &c;
       break;
     }
@@ -526,6 +549,7 @@ std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const 
   P->nsys = ns;
   P->nwg = (int)wgs.size();
   P->fn = s->fn;
+  P->threads = s->threads;
   P->wg = dev_upload(wgs);
   P->hcnt = dev_alloc(sizeof(int) * (size_t)P->nwg);
   P->hcol = dev_alloc(sizeof(int) * (size_t)P->nwg * kResHalo);
@@ -546,11 +570,11 @@ std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const 
   k_res_zero<<<256, kBlock, 0, stream()>>>(((long long)n + 3) / 4, P->sent->as<unsigned>());
   k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P->box_words, P->boxes->as<unsigned>());
   k_res_plan<<<P->nwg, kResThreads, plan_lds, stream()>>>(
-      P->wg->as<ResWg>(), s->r * kResThreads, ia, ja, P->hcnt->as<int>(), P->hcol->as<int>(),
+      P->wg->as<ResWg>(), s->r * s->threads, ia, ja, P->hcnt->as<int>(), P->hcol->as<int>(),
       P->sent->as<unsigned char>(), P->lcol->as<unsigned short>());
   for (int c : dev_download(P->hcnt->as<int>(), (size_t)P->nwg)) P->nhmax = std::max(P->nhmax, c);
   if (lap_last_status() == LAP_ERR_HIP || P->nhmax > kResHalo) return P;
-  P->lds = (int)sizeof(double) * (s->r * kResThreads + P->nhmax + 1) + 4 * P->nhmax;
+  P->lds = (int)sizeof(double) * (s->r * s->threads + P->nhmax + 1) + 4 * P->nhmax;
   if (!LAP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(P->fn),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, P->lds)))
     return P;
@@ -606,7 +630,7 @@ int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double
   for (long k = 0; k <= (long)(maxit + 1) / kResIters + 1; ++k) {
     g.resume = k > 0;
     g.tag0 = P.tag;
-    P.fn<<<P.nwg, kResThreads, P.lds, stream()>>>(g);
+    P.fn<<<P.nwg, P.threads, P.lds, stream()>>>(g);
     ResShared sh{};
     if (!LAP_HIP(hipGetLastError()) ||
         !LAP_HIP(hipMemcpyAsync(h.data(), g.st, sizeof(ResState) * h.size(),
