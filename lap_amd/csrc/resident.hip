@@ -52,11 +52,19 @@ constexpr int kResMaxWg = 256;     // workgroups at most (partials: one per thre
 // 3.89, 512^2 9.05 / 9.08 / 6.86, 40^3 7.15 / 6.66 / 6.70, 64^3 9.4 / 9.4 /
 // 11.1, 97 x 90 x 31 8.7 / 8.7 / 10.6: 2048 for rows of up to 5 entries.
 constexpr int kResRows = 1024, kResRowsShort = 2048, kResShort = 5;
-constexpr int kResBig = 1 << 16;   // rows of a large system
 constexpr int kResMaxN = 1 << 19;  // rows of a system at most (the analysis' bitmap in LDS)
 constexpr int kResMaxRows = 1 << 26;  // rows of all systems at most (box_w stays below 2^31 bytes)
 constexpr int kResIters = 8192;    // iterations per launch
 constexpr unsigned kResSpins = 1u << 22;
+// Every workgroup of a team reads every sum, through whichever XCD it is on and
+// past the caches: with many workgroups the few lines that hold the boxes are
+// what they wait for.  So a sum is sent in 8 copies and an XCD reads its own: us
+// per iteration with 1 and 8 copies, 128^2 (8 workgroups) 4.1 and 4.1, 256^2 5.2
+// and 4.4, 512^2 7.1 and 5.6, 40^3 6.6 and 5.7, 64^3 9.1 and 8.5, 97 x 90 x 31 8.2
+// and 7.5, a geometric graph of 150k nodes 8.2 and 7.4; the batch of 160 grids
+// 5.6 and 5.0 ms.
+constexpr int kResCopies = 8;
+constexpr int kResSkew = 256;  // places between the copies
 
 struct ResState {
   double rho, tolrel, res0, res;
@@ -87,7 +95,7 @@ struct ResArgs {
   unsigned tag0;
   double *hist;  // of a single system (may be null)
   void *box_a, *box_b, *box_w;
-  int n, nwg;
+  int n, stride;  // stride: places from a copy of the sums' boxes to the next
   ResState *st;  // per system
   ResShared *sh;
 };
@@ -113,6 +121,12 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {  // lane 63
   return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
 }
 
+__device__ __forceinline__ double readlane_f64(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  return fl_f64((unsigned)__builtin_amdgcn_readlane((int)b, l),
+                (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), l));
+}
+
 // The launch.  R rows per thread, rows of at most L entries, T threads.  512
 // threads add up as 1024 do, each what two of those would (the even and the odd
 // rows of its R), so x does not depend on T: two such workgroups share a CU and
@@ -134,8 +148,12 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
   double *const halo = ps + R * T;
   const int zero = R * T + g.nhmax;
   int *const hcol = reinterpret_cast<int *>(ps + zero + 1);  // the halo's rows
-  const __amdgpu_buffer_rsrc_t box_a = fl_buffer(g.box_a, g.nwg * 16);
-  const __amdgpu_buffer_rsrc_t box_b = fl_buffer(g.box_b, g.nwg * 32);
+  const __amdgpu_buffer_rsrc_t box_a = fl_buffer(g.box_a, kResCopies * g.stride * 16);
+  const __amdgpu_buffer_rsrc_t box_b = fl_buffer(g.box_b, kResCopies * g.stride * 32);
+  // the team's boxes in the copy that this workgroup reads
+  const size_t at = (size_t)((w & (kResCopies - 1)) * g.stride + team) * 16;
+  const __amdgpu_buffer_rsrc_t mine_a = fl_buffer(static_cast<char *>(g.box_a) + at, size * 16);
+  const __amdgpu_buffer_rsrc_t mine_b = fl_buffer(static_cast<char *>(g.box_b) + 2 * at, size * 32);
   const __amdgpu_buffer_rsrc_t box_w = fl_buffer(g.box_w, g.n * 16);
   if (t == 0) {
     dead = 0;
@@ -206,6 +224,7 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
   auto all_sums = [&](auto &sum, auto &v, unsigned tag, auto &&between) {
     constexpr int N = sizeof(sum) / sizeof(sum[0]);
     const __amdgpu_buffer_rsrc_t box = N == 1 ? box_a : box_b;
+    const __amdgpu_buffer_rsrc_t mine = N == 1 ? mine_a : mine_b;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
 #pragma unroll
@@ -219,12 +238,11 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         const double s = row_sum_dpp(lane < V * W ? red[i][lane] : 0.0);
-        if (lane == V * W - 1) {
-          if (size > 1)
-            fl_put(box, w * N + i, tag, s);
-          else
-            one[i] = s;
-        }
+        const double u = readlane_f64(s, V * W - 1);
+        if (size == 1)
+          one[i] = u;
+        else if (lane < kResCopies)
+          fl_put(box, (lane * g.stride + w) * N + i, tag, u);
       }
     }
     between();
@@ -236,7 +254,7 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
         for (;;) {
           bool ok = true;
 #pragma unroll
-          for (int i = 0; i < N; ++i) f[i].load(box, (team + t) * N + i);
+          for (int i = 0; i < N; ++i) f[i].load(mine, t * N + i);
 #pragma unroll
           for (int i = 0; i < N; ++i) ok = ok && f[i].is(tag);
           fl_fence();
@@ -489,7 +507,7 @@ const ResShape kShapes[] = {{4, 5, 512, k_resident<4, 5, 512>},
 struct ResPlan {
   bool ok = false;
   std::vector<int> off;
-  int nsys = 0, nwg = 0, nhmax = 0, lds = 0, threads = 0;
+  int nsys = 0, nwg = 0, stride = 0, nhmax = 0, lds = 0, threads = 0;
   ResKernel fn = nullptr;
   DevBufPtr wg, hcnt, hcol, sent, lcol, boxes, state, shared;
   size_t box_words = 0;
@@ -514,13 +532,12 @@ std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const 
     const int rows = off[(size_t)q + 1] - off[(size_t)q];
     wgs_all += rows ? (rows + rows_per(rows) - 1) / rows_per(rows) : 0;
   }
-  // Two workgroups per CU for large systems and where there are half as many
-  // again as CUs.  With 1024 and 512 threads, us per iteration: 60 x 52 3.4 and
-  // 3.9, 128^2 4.0 and 4.2, 256^2 5.3 and 5.1, 512^2 7.1 and 7.0, 700^2 10.3 and
-  // 8.4; batches, ms: 160 grids of up to 150^2 (600 workgroups) 7.9 and 5.6, 60 of
-  // up to 400^2 132 and 89, 2000 of up to 20^2 1.3 and 1.0, but 300 of up to 60^2
-  // (340 workgroups) 1.57 and 1.79.
-  const bool half = A.max_row <= kResShort && (big >= kResBig || 2 * wgs_all > 3 * cus);
+  // Two workgroups per CU where there are half as many again as CUs.  With 1024
+  // and 512 threads, ms: 160 grids of up to 150^2 (600 workgroups) 7.9 and 5.6, 60
+  // of up to 400^2 132 and 89, 2000 of up to 20^2 1.3 and 1.0, but 300 of up to
+  // 60^2 (340 workgroups) 1.57 and 1.79.  One system gains little (512^2 7.1 and
+  // 7.0 us per iteration, 128^2 4.0 and 4.2).
+  const bool half = A.max_row <= kResShort && 2 * wgs_all > 3 * cus;
   for (const ResShape &c : kShapes) {
     if (A.max_row > c.l || half != (c.threads < kResThreads)) continue;
     if (rows_per(big) <= c.r * c.threads) {
@@ -557,7 +574,8 @@ std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const 
   P->lcol = dev_alloc(sizeof(unsigned short) * (size_t)std::max(A.nnz, 1));
   P->state = dev_alloc(sizeof(ResState) * (size_t)ns);
   P->shared = dev_alloc(sizeof(ResShared));
-  P->box_words = 4 * ((size_t)n + 3 * (size_t)P->nwg);
+  P->stride = (P->nwg + 15) / 16 * 16 + kResSkew;
+  P->box_words = 4 * ((size_t)n + 3 * (size_t)kResCopies * P->stride);
   P->boxes = dev_alloc(sizeof(unsigned) * P->box_words);
   for (const DevBufPtr &b : {P->wg, P->hcnt, P->hcol, P->sent, P->lcol, P->state, P->shared,
                              P->boxes})
@@ -591,7 +609,7 @@ int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double
   char *box = P.boxes->as<char>();
   ResArgs g{};
   g.n = n;
-  g.nwg = P.nwg;
+  g.stride = P.stride;
   g.wg = P.wg->as<ResWg>();
   g.nhmax = P.nhmax;
   g.ia = ia;
@@ -612,8 +630,8 @@ int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double
   g.iters = P.nsys == 1 ? kResIters : 0x7fffffff;
   g.hist = hist;
   g.box_a = box;
-  g.box_b = box + 16 * (size_t)P.nwg;
-  g.box_w = box + 48 * (size_t)P.nwg;
+  g.box_b = box + 16 * (size_t)kResCopies * P.stride;
+  g.box_w = box + 48 * (size_t)kResCopies * P.stride;
   g.st = P.state->as<ResState>();
   g.sh = P.shared->as<ResShared>();
   std::vector<ResState> h((size_t)P.nsys);

@@ -1,6 +1,5 @@
-"""The resident solve with two workgroups per CU: the sizes at which it takes over
-(2^16 rows; a batch of many workgroups) and the rows (5 and 6 entries) where it
-stops.
+"""The resident solve of short rows: one to 240 workgroups, rows of 5 entries and
+more, and batches on either side of the rule for two workgroups per CU.
 
 Compared with the oracle after exactly as many iterations, as the smaller
 workgroups are: the dot products are summed in another order, relative 1e-16 per
