@@ -113,6 +113,31 @@ __global__ __launch_bounds__(kBlock) void k_cls_collect(int n, const int *__rest
   }
 }
 
+// one workgroup: *out = 1 when kClsProbe rows, evenly spread, have too many
+// hashes already
+constexpr int kClsProbe = 1024;
+__global__ __launch_bounds__(kClsProbe) void k_cls_probe(int n, const int *__restrict__ ia,
+                                                         const int *__restrict__ ja,
+                                                         const double *__restrict__ a,
+                                                         const double *__restrict__ d_r,
+                                                         int *out) {
+  __shared__ unsigned long long set[2 * kClsProbe];
+  __shared__ int count;
+  const int t = threadIdx.x;
+  set[t] = set[t + kClsProbe] = kClsEmpty;
+  if (t == 0) count = 0;
+  __syncthreads();
+  const unsigned long long k = cls_hash((int)((long long)t * n / kClsProbe), ia, ja, a, d_r);
+  unsigned h = (unsigned)(k >> 40) & (2 * kClsProbe - 1);
+  for (int probe = 0; probe < 2 * kClsProbe; ++probe, h = (h + 1) & (2 * kClsProbe - 1)) {
+    const unsigned long long prev = atomicCAS(&set[h], kClsEmpty, k);
+    if (prev == kClsEmpty) atomicAdd(&count, 1);
+    if (prev == kClsEmpty || prev == k) break;
+  }
+  __syncthreads();
+  if (t == 0) *out = count > kClsMax;
+}
+
 // one workgroup, a thread per class: the table from the class's row
 __global__ __launch_bounds__(kBlock) void k_cls_table(int ncls, int width,
                                                       const int *__restrict__ rep,
@@ -256,6 +281,15 @@ int cls_group(const std::vector<int> &offsets, int rows, unsigned grid) {
     }
   }
   return best;
+}
+
+bool cls_probe(int n, int nnz, const int *ia, const int *ja, const double *a, const double *d_r,
+               int max_row, int *host) {
+  if (n < 1 || nnz < 1 || max_row > kClsRow) return false;
+  int *out = reinterpret_cast<int *>(scratch_vec("cls_probe", 1));
+  if (!out) return false;
+  k_cls_probe<<<1, kClsProbe, 0, stream()>>>(n, ia, ja, a, d_r, out);
+  return LAP_HIP(hipMemcpyAsync(host, out, sizeof(int), hipMemcpyDeviceToHost, stream()));
 }
 
 ClsMat cls_encode(const char *tag, int n, int nnz, const int *ia, const int *ja, const double *a,

@@ -63,6 +63,13 @@ std::pair<unsigned, int> xcd_grid(const std::vector<int> &offsets, int rows, lon
 // matrix's column offsets.
 int cls_group(const std::vector<int> &offsets, int rows, unsigned grid);
 
+// Sends off a look at 1024 rows: *host (pinned) becomes 1 when they have too
+// many classes already, as a matrix of random weights has.  About 10 us on the
+// stream, where finding out in cls_encode takes 0.15 ms with the waits.  false:
+// the matrix cannot be encoded.
+bool cls_probe(int n, int nnz, const int *ia, const int *ja, const double *a, const double *d_r,
+               int max_row, int *host);
+
 // The table's width is `least` (4, 8 or 16), or 8 or 16 where rows are longer.
 // Encodes the matrix (tag: names the buffers that hold the result until the
 // next encoding with the same tag).  d_r may be null.  Two passes over the

@@ -1141,17 +1141,21 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
   };
   if (!capture()) status = LAP_ERR_HIP;
   // as in lap_pcg: a solve that ends in its first batch does not pay for them
-  const bool classes = options().spmv_format == 0 && n >= kClsMinRows;
+  bool classes = options().spmv_format == 0 && n >= kClsMinRows && maxit >= G;
   int *flags = pinned_flags();
   if (!flags) status = LAP_ERR_HIP;
   if (status == LAP_OK) {
     hipEvent_t pe[2];
     LAP_HIP(hipEventCreateWithFlags(&pe[0], hipEventDisableTiming));
     LAP_HIP(hipEventCreateWithFlags(&pe[1], hipEventDisableTiming));
+    if (classes)
+      classes = cls_probe(n, nnz, ia, ja, a, jac ? pd->d_r : nullptr, A64->max_row, flags + 2) &&
+                LAP_HIP(hipEventRecord(pe[1], stream()));
     const long max_batches = (long)(maxit + 1) / G + 3;
     bool finished = false;
     for (long k = 0; k < max_batches + 1 && !finished; ++k) {
-      if (k == 1 && classes && LAP_HIP(hipEventSynchronize(pe[0])) && !flags[0]) {
+      if (k == 1 && classes && LAP_HIP(hipEventSynchronize(pe[1])) && !flags[2] &&
+          LAP_HIP(hipEventSynchronize(pe[0])) && !flags[0]) {
         cls = cls_inner(cls_encode("a", n, nnz, ia, ja, a, jac ? pd->d_r : nullptr, A64->max_row),
                         A64->max_row);
         if (cls.cls && !capture()) {

@@ -1071,25 +1071,29 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
   };
   if (!capture()) status = LAP_ERR_HIP;
   // Row classes come in after the first batch of iterations: encoding (0.15 ms
-  // at 10^6 rows, 1.5 ms at 1.7 * 10^7, 0.08 ms to find too many) takes as long
-  // as 6 to 15 iterations win, which a solve that ends in the first batch would
-  // not get back.
-  const bool classes = options().spmv_format == 0 && n >= kClsMinRows;
+  // at 10^6 rows, 1.5 ms at 1.7 * 10^7) takes as long as 6 to 20 iterations win,
+  // which a solve that ends in the first batch would not get back.  The probe
+  // answers while that batch runs.
+  bool classes = options().spmv_format == 0 && n >= kClsMinRows && maxit >= G;
   if (status == LAP_OK) {
     hipEvent_t pe[2];
     LAP_HIP(hipEventCreateWithFlags(&pe[0], hipEventDisableTiming));
     LAP_HIP(hipEventCreateWithFlags(&pe[1], hipEventDisableTiming));
+    if (classes)
+      classes = cls_probe(n, nnz, ia, ja, a, jac ? pd->d_r : nullptr, A.max_row, flags + 2) &&
+                LAP_HIP(hipEventRecord(pe[1], stream()));
     // iter <= maxit + 1, so this many batches always reach done
     const long max_batches = (long)(maxit + 1) / G + 3;
     bool finished = false;
     for (long k = 0; k < max_batches + 1 && !finished; ++k) {
-      if (k == 1 && classes && LAP_HIP(hipEventSynchronize(pe[0])) && !flags[0]) {
+      if (k == 1 && classes && LAP_HIP(hipEventSynchronize(pe[1])) && !flags[2] &&
+          LAP_HIP(hipEventSynchronize(pe[0])) && !flags[0]) {
         vv.cls = cls_encode("a", n, nnz, ia, ja, a, jac ? pd->d_r : nullptr, A.max_row);
-        if (options().fuse_sweeps &&
+        if (vv.cls.cls && options().fuse_sweeps &&
             (o.kind == P_IT_JACOBI || o.kind == P_GS_IT || o.kind == P_GS_IT2))
           o.sweep = sweep_encode(*o.Ls, pd->lia, pd->lja, pd->la, *o.Us, pd->uia, pd->uja, pd->ua,
                                  o.kind == P_GS_IT && o.m > 1 ? o.A : nullptr, ia, ja, a, pd->d_r);
-        if ((vv.cls.cls || o.sweep.n > 0) && !capture()) {
+        if (vv.cls.cls && !capture()) {
           status = LAP_ERR_HIP;
           break;
         }

@@ -89,6 +89,18 @@ def test_bitwise_the_csr_solve(name):
     same(*both(Ah, "line_jacobi", b))
 
 
+def test_probe_passes_what_the_encoding_refuses():
+    """Few classes among the probed rows, many elsewhere."""
+    n = MIN_ROWS + 1024
+    at = np.arange(1024, dtype=np.int64) * n // 1024
+    far = np.ones(n, bool)
+    for o in range(-2, 3):
+        far[np.clip(at + o, 0, n - 1)] = False
+    Ah = band(n, [1], lambda i, k: np.where(far[i], 1.0 + i % 7919, 1.0))
+    b = np.random.default_rng(12).standard_normal(n)
+    same(*both(Ah, "line_jacobi", b))
+
+
 @pytest.mark.parametrize("kind", ["none", "it_jacobi", "GS_it2", "ichol"])
 def test_other_preconditioners(kind):
     Ah = grid_laplacian([91, 73, 83], 0.05)
