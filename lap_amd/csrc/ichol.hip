@@ -302,13 +302,15 @@ const IcPlan *ic_factor(int n, int nnzA, const int *ia, const int *ja, double *a
   return raw;
 }
 
-void ic_apply_launch(const IcPlan &p, const double *x, double *y, double *aux,
-                     const int *done) {
-  if (tri_solve_two_launch(*p.lplan, p.lell, *p.uplan, p.uell, p.comp, x, y, done)) return;
+bool ic_apply_launch(const IcPlan &p, const double *x, double *y, double *aux,
+                     const int *done, const TriTail *tail) {
+  if (tri_solve_two_launch(*p.lplan, p.lell, *p.uplan, p.uell, p.comp, x, y, done, tail))
+    return true;
   tri_solve_launch(*p.lplan, p.lia->as<int>(), p.lja->as<int>(), p.lval->as<double>(), nullptr,
                    x, aux, done, &p.lell);
   tri_solve_launch(*p.uplan, p.uia->as<int>(), p.uja->as<int>(), p.uval->as<double>(), nullptr,
                    aux, y, done, &p.uell);
+  return false;
 }
 
 }  // namespace lap

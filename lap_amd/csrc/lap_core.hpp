@@ -433,6 +433,18 @@ void tri_ell_build(const TriPlan &p, const int *ja, const double *a, TriEll &e);
 void tri_solve_launch(const TriPlan &p, const int *ia, const int *ja, const double *a,
                       const double *diag, const double *x, double *y, const int *ctl_done,
                       const TriEll *ell = nullptr);
+// What follows a chunked solve, done with its copy back to row order: y += the
+// solve (add), and the partial sums of r.y as k_rw with `grid` workgroups leaves
+// them (part != null).
+struct TriTail {
+  bool add = false;
+  const double *r = nullptr;
+  double *part = nullptr;
+  unsigned grid = 1;
+};
+// false: not a chunked solve, nothing was launched.
+bool tri_solve_tail_launch(const TriPlan &p, const double *x, double *y, const TriEll &ell,
+                           const TriTail &tail, const int *ctl_done);
 // The number of kernel launches tri_solve_launch makes for these arguments
 // (x == y: in place).
 int tri_launches(const TriPlan &p, const TriEll *ell, bool in_place);
@@ -457,7 +469,7 @@ int tri_launches32(const TriPlan &p, const TriChunks32 *c);
 DevBufPtr tri_compose(const TriPlan &first, const TriPlan &second);
 bool tri_solve_two_launch(const TriPlan &p1, const TriEll &e1, const TriPlan &p2,
                           const TriEll &e2, const DevBufPtr &comp, const double *x, double *y,
-                          const int *done);
+                          const int *done, const TriTail *tail = nullptr);
 bool tri_solve32_two_launch(const TriPlan &p1, const TriChunks32 &c1, const TriPlan &p2,
                             const TriChunks32 &c2, const DevBufPtr &comp, const float *x,
                             float *y, const int *done);
@@ -479,8 +491,9 @@ struct IcPlan {
 };
 const IcPlan *ic_plan_find(const double *vals);
 const IcPlan *ic_factor(int n, int nnzA, const int *ia, const int *ja, double *a);
-void ic_apply_launch(const IcPlan &p, const double *x, double *y, double *aux,
-                     const int *ctl_done);
+// true: `tail` (if any) is done too.
+bool ic_apply_launch(const IcPlan &p, const double *x, double *y, double *aux,
+                     const int *ctl_done, const TriTail *tail = nullptr);
 
 // ---------------------------------------------------- elementwise launches
 // `done` (device int*, may be null): the launch is a no-op once *done != 0.

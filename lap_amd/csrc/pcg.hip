@@ -831,11 +831,27 @@ static bool prec_fused(const PrecOps &o, const double *r, double *w, const int *
   return true;
 }
 
-// w = M^{-1} r, as launches on the library stream.
-static void prec_launch(const PrecOps &o, const double *r, double *w, const int *done) {
+// w = M^{-1} r, as launches on the library stream.  part: where k_rw with `grid`
+// workgroups would leave its sums of r.w; true: they are there.
+static bool prec_launch(const PrecOps &o, const double *r, double *w, const int *done,
+                        double *part = nullptr, unsigned grid = 1) {
   const int n = o.n;
   lap_pdata *pd = o.pd;
-  if (prec_fused(o, r, w, done)) return;
+  if (prec_fused(o, r, w, done)) return false;
+  bool dotted = false;
+  // aux2 = r - A w, then w += the triangle's solve of it
+  auto gs_step = [&](const TriPlan &t, const int *ia, const int *ja, const double *a,
+                     const double *diag, const TriEll &ell, bool last) {
+    sweep_one_launch(*o.A, o.ia, o.ja, o.a, w, r, nullptr, o.aux2, nullptr, 1, false, done);
+    TriTail tail{true, r, last ? part : nullptr, grid};
+    if (!part) tail.grid = vgrid(n);
+    if (tri_solve_tail_launch(t, o.aux2, w, ell, tail, done)) {
+      dotted = tail.part != nullptr;
+      return;
+    }
+    tri_solve_launch(t, ia, ja, a, diag, o.aux2, o.aux1, done, &ell);
+    launch_axpy(n, 1.0, o.aux1, w, done);
+  };
   switch (o.kind) {
     case P_NONE:
       launch_copy(n, r, w, done);
@@ -861,20 +877,11 @@ static void prec_launch(const PrecOps &o, const double *r, double *w, const int 
           // w = 0: r - A*0 == r and 0 + L^{-1} r == L^{-1} r, so solve directly
           tri_solve_launch(*o.Lt, pd->lia, pd->lja, pd->la, o.ldiag, r, w, done, &o.lell);
         } else {
-          launch_copy(n, r, o.aux2, done);
-          spmv_launch(*o.A, o.ia, o.ja, o.a, w, o.aux2, -1.0, 1.0, done);
-          tri_solve_launch(*o.Lt, pd->lia, pd->lja, pd->la, o.ldiag, o.aux2, o.aux1, done,
-                           &o.lell);
-          launch_axpy(n, 1.0, o.aux1, w, done);
+          gs_step(*o.Lt, pd->lia, pd->lja, pd->la, o.ldiag, o.lell, false);
         }
       }
-      for (int s = 0; s < o.k; ++s) {
-        launch_copy(n, r, o.aux2, done);
-        spmv_launch(*o.A, o.ia, o.ja, o.a, w, o.aux2, -1.0, 1.0, done);
-        tri_solve_launch(*o.Ut, pd->uia, pd->uja, pd->ua, o.udiag, o.aux2, o.aux1, done,
-                         &o.uell);
-        launch_axpy(n, 1.0, o.aux1, w, done);
-      }
+      for (int s = 0; s < o.k; ++s)
+        gs_step(*o.Ut, pd->uia, pd->uja, pd->ua, o.udiag, o.uell, s == o.k - 1);
       break;
     case P_GS_IT:  // GS.c:45-92
       launch_fill(n, 0.0, w, done);
@@ -923,11 +930,15 @@ static void prec_launch(const PrecOps &o, const double *r, double *w, const int 
       launch_copy(n, o.aux2, w, done);
       break;
     case P_ICHOL:  // simple_blas.c:184-223 order
-      ic_apply_launch(*o.ic, r, w, o.aux1, done);
+    {
+      const TriTail tail{false, r, part, grid};
+      dotted = ic_apply_launch(*o.ic, r, w, o.aux1, done, part ? &tail : nullptr) && part;
       break;
+    }
     default:
       break;
   }
+  return dotted;
 }
 
 // ------------------------------------------------------------- the solve
@@ -1027,8 +1038,8 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
       else
         vectors(JacD<double>{pd->d_r});
     } else {
-      prec_launch(o, r, w, done);
-      k_rw<kBlock><<<gV, kBlock, 0, stream()>>>(n, r, w, ctl, R1);
+      if (!prec_launch(o, r, w, done, R1, gV))
+        k_rw<kBlock><<<gV, kBlock, 0, stream()>>>(n, r, w, ctl, R1);
       k_pupd<kBlock><<<gV, kBlock, 0, stream()>>>(n, w, p, ctl, R1, (int)gV);
       launch_spmv_pq(gA, A, ia, ja, a, p, q, ctl, R2, vv);
       k_update<kBlock><<<gV, kBlock, 0, stream()>>>(n, x, r, p, q, ctl, R2, (int)gA, R3);

@@ -24,6 +24,7 @@
 #include <thread>
 
 #include "boxed.hpp"
+#include "cls.hpp"
 #include "lap_core.hpp"
 
 namespace lap {
@@ -749,6 +750,50 @@ __global__ __launch_bounds__(kBlock) void k_fl_spread(int n, const int *__restri
     st_nt(y + i, xc[ld_nt(pos + i)]);
 }
 
+// The same with what the caller does next in the same pass: y += the solve
+// (ADD), and partials of r.y (part != null).  Rows are walked and summed as
+// k_rw does it, so the partials are k_rw's bit for bit, in an order of the
+// workgroups that keeps an XCD on one run of rows per round.  Bound by the
+// gather, whose lines several XCDs read: at 97 x 110 x 83 the solve's copy back,
+// axpy and dot product took 7.6 + 5.5 + 4.6 us, this 10.7; at 128^3 the copy back
+// and dot product 14.0 + 8.8, this 20.4.
+template <bool ADD>
+__global__ __launch_bounds__(kBlock) void k_fl_tail(int n, const int *__restrict__ pos,
+                                                    const double *__restrict__ xc, double *y,
+                                                    const double *__restrict__ r, double *part,
+                                                    int group, const int *__restrict__ done) {
+  if (done && *done) return;
+  __shared__ double red[kBlock / kWave];
+  const int me = cls_block(blockIdx.x, group);
+  const size_t stride = (size_t)gridDim.x * kBlock;
+  double s = 0.0;
+  constexpr int U = 4;  // rows in flight
+  for (size_t i0 = (size_t)me * kBlock + threadIdx.x; i0 < (size_t)n; i0 += U * stride) {
+    int at[U];
+    double v[U], w[U], rv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t i = i0 + u * stride;
+      at[u] = i < (size_t)n ? ld_nt(pos + i) : 0;
+      w[u] = ADD && i < (size_t)n ? ld_nt(y + i) : 0.0;
+      rv[u] = part && i < (size_t)n ? ld_nt(r + i) : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = xc[at[u]];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t i = i0 + u * stride;
+      if (i >= (size_t)n) continue;
+      w[u] = ADD ? w[u] + 1.0 * v[u] : v[u];
+      st_nt(y + i, w[u]);
+      if (part) s += rv[u] * w[u];
+    }
+  }
+  if (!part) return;
+  const double t = block_sum<kBlock>(s, red);
+  if (threadIdx.x == 0) part[me] = t;
+}
+
 // comp[t] = pos[map[t]]: a schedule's right-hand sides taken from another
 // schedule's results.
 __global__ __launch_bounds__(kBlock) void k_fl_compose(int n, const int *__restrict__ map,
@@ -1435,6 +1480,13 @@ static void tri_fl_spread(const TriPlan &p, const DevBufPtr &xc, VT *y, const in
   k_fl_spread<VT><<<g, kBlock, 0, stream()>>>(p.n, p.ch.pos->as<int>(), xc->as<VT>(), y, done);
 }
 
+static void tri_fl_tail(const TriPlan &p, const DevBufPtr &xc, double *y, const TriTail &t,
+                        const int *done) {
+  auto *k = t.add ? k_fl_tail<true> : k_fl_tail<false>;
+  k<<<t.grid, kBlock, 0, stream()>>>(p.n, p.ch.pos->as<int>(), xc->as<double>(), y, t.r, t.part,
+                                     t.grid % 8 ? 1 : (int)t.grid / 8, done);
+}
+
 void tri_ell_build(const TriPlan &p, const int *ja, const double *a, TriEll &e) {
   e.w = 0;
   if (p.n <= 0 || p.max_row > 8) return;
@@ -1533,6 +1585,14 @@ void tri_solve_launch(const TriPlan &p, const int *ia, const int *ja, const doub
   tri_level_launch<double, double>(p, ja, a, diag, x, y, done);
 }
 
+bool tri_solve_tail_launch(const TriPlan &p, const double *x, double *y, const TriEll &ell,
+                           const TriTail &tail, const int *done) {
+  if (tri_path(p, &ell, x == y) != TRI_CHUNKS) return false;
+  tri_fl_launch<double, double>(p, ell.crec, ell.xc, x, p.ch.crow->as<int>(), done);
+  tri_fl_tail(p, ell.xc, y, tail, done);
+  return true;
+}
+
 DevBufPtr tri_compose(const TriPlan &first, const TriPlan &second) {
   if (first.ch.nchunks <= 0 || second.ch.nchunks <= 0) return nullptr;
   DevBufPtr m = dev_alloc(sizeof(int) * (size_t)second.ch.nrec);
@@ -1544,12 +1604,15 @@ DevBufPtr tri_compose(const TriPlan &first, const TriPlan &second) {
 
 bool tri_solve_two_launch(const TriPlan &p1, const TriEll &e1, const TriPlan &p2,
                           const TriEll &e2, const DevBufPtr &comp, const double *x, double *y,
-                          const int *done) {
+                          const int *done, const TriTail *tail) {
   if (!comp || tri_path(p1, &e1, false) != TRI_CHUNKS || tri_path(p2, &e2, false) != TRI_CHUNKS)
     return false;
   tri_fl_launch<double, double>(p1, e1.crec, e1.xc, x, p1.ch.crow->as<int>(), done);
   tri_fl_launch<double, double>(p2, e2.crec, e2.xc, e1.xc->as<double>(), comp->as<int>(), done);
-  tri_fl_spread(p2, e2.xc, y, done);
+  if (tail)
+    tri_fl_tail(p2, e2.xc, y, *tail, done);
+  else
+    tri_fl_spread(p2, e2.xc, y, done);
   return true;
 }
 
