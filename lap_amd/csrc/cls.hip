@@ -330,6 +330,9 @@ ClsMat cls_encode(const char *tag, int n, int nnz, const int *ia, const int *ja,
   }
   const std::string name = std::string("cls_") + tag;
   const int width = max_row <= least ? least : (max_row + 7) / 8 * 8;
+  // without the memory for a byte per row the solve keeps its matrix
+  size_t avail = 0, all = 0;
+  if (!LAP_HIP(hipMemGetInfo(&avail, &all)) || avail < (size_t)n + ((size_t)4 << 20)) return m;
   unsigned char *cls =
       reinterpret_cast<unsigned char *>(scratch_vec(name.c_str(), ((size_t)n + 7) / 8));
   double *val = scratch_vec((name + "_val").c_str(), (size_t)kClsMax * kClsRow);

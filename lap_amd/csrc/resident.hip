@@ -54,6 +54,8 @@ constexpr int kResMaxWg = 256;     // workgroups at most (partials: one per thre
 constexpr int kResRows = 1024, kResRowsShort = 2048, kResShort = 5;
 constexpr int kResMaxN = 1 << 19;  // rows of a system at most (the analysis' bitmap in LDS)
 constexpr int kResMaxRows = 1 << 26;  // rows of all systems at most (box_w stays below 2^31 bytes)
+// Workgroups of a batch at most: their halo lists take 32 KB each (1 GB).
+constexpr int kResMaxWgs = 1 << 15;
 constexpr int kResIters = 8192;    // iterations per launch
 constexpr unsigned kResSpins = 1u << 22;
 // Every workgroup of a team reads every sum, through whichever XCD it is on and
@@ -527,11 +529,12 @@ std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const 
   auto rows_per = [&](int rows) {
     return std::max(least, ((rows + cus - 1) / cus + kWave - 1) / kWave * kWave);
   };
-  long wgs_all = 0;
+  long wgs_all = 0;  // workgroups
   for (int q = 0; q < ns; ++q) {
     const int rows = off[(size_t)q + 1] - off[(size_t)q];
     wgs_all += rows ? (rows + rows_per(rows) - 1) / rows_per(rows) : 0;
   }
+  if (wgs_all > kResMaxWgs) return P;
   // Two workgroups per CU where there are half as many again as CUs.  With 1024
   // and 512 threads, ms: 160 grids of up to 150^2 (600 workgroups) 7.9 and 5.6, 60
   // of up to 400^2 132 and 89, 2000 of up to 20^2 1.3 and 1.0, but 300 of up to
@@ -568,14 +571,19 @@ std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const 
   P->fn = s->fn;
   P->threads = s->threads;
   P->wg = dev_upload(wgs);
+  P->stride = (P->nwg + 15) / 16 * 16 + kResSkew;
+  P->box_words = 4 * ((size_t)n + 3 * (size_t)kResCopies * P->stride);
+  // without the memory for it the solve goes by launches, as before
+  size_t avail = 0, all = 0;
+  const size_t need = sizeof(unsigned) * P->box_words + sizeof(int) * (size_t)P->nwg * kResHalo +
+                      sizeof(unsigned short) * (size_t)A.nnz + (size_t)n + ((size_t)64 << 20);
+  if (!LAP_HIP(hipMemGetInfo(&avail, &all)) || avail < need) return P;
   P->hcnt = dev_alloc(sizeof(int) * (size_t)P->nwg);
   P->hcol = dev_alloc(sizeof(int) * (size_t)P->nwg * kResHalo);
   P->sent = dev_alloc(((size_t)n + 3) / 4 * 4);
   P->lcol = dev_alloc(sizeof(unsigned short) * (size_t)std::max(A.nnz, 1));
   P->state = dev_alloc(sizeof(ResState) * (size_t)ns);
   P->shared = dev_alloc(sizeof(ResShared));
-  P->stride = (P->nwg + 15) / 16 * 16 + kResSkew;
-  P->box_words = 4 * ((size_t)n + 3 * (size_t)kResCopies * P->stride);
   P->boxes = dev_alloc(sizeof(unsigned) * P->box_words);
   for (const DevBufPtr &b : {P->wg, P->hcnt, P->hcol, P->sent, P->lcol, P->state, P->shared,
                              P->boxes})

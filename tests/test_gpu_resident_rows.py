@@ -62,3 +62,20 @@ def test_batch_equals_single_solves(systems):
         r = S.pcg(A, S.to_dev(rhs[s]), P, tol=1e-10)
         assert int(it[s]) == r.iterations
         assert torch.equal(B.split(x)[s], r.x)
+
+
+@pytest.mark.parametrize("systems", [32768, 32769])
+def test_batches_around_the_most_workgroups(systems):
+    """Past the limit the batch goes by launches: the same solutions (2 x 2 grids,
+    exact after 3 iterations)."""
+    A1 = grid_laplacian([2, 2], 0.5)
+    rng = np.random.default_rng(2)
+    rhs = rng.standard_normal((systems, 4))
+    B = S.Batch.from_systems([A1] * systems, list(rhs))
+    x, it, fl, *_ = S.pcg_batched(B, block=-1, tol=1e-12)
+    dense = np.zeros((4, 4))
+    for r in range(4):
+        dense[r, A1.ja[A1.ia[r]:A1.ia[r + 1]]] = A1.a[A1.ia[r]:A1.ia[r + 1]]
+    want = np.linalg.solve(dense, rhs.T).T.ravel()
+    assert not fl.any()
+    assert np.abs(x.cpu().numpy() - want).max() <= 1e-9 * np.abs(want).max()

@@ -71,8 +71,10 @@ def test_not_finite(orc):
     assert np.array_equal(S.spmm(A, S.to_dev(X)).cpu().numpy(), want, equal_nan=True)
 
 
-def test_operand_past_4_gb():
-    n, k = (1 << 23) + 77, 64
+@pytest.mark.parametrize("n", [(1 << 22) + (1 << 20), (1 << 23) - 1, (1 << 23) + 77])
+def test_operand_around_4_gb(n):
+    """2.7 GB, the last size within 32-bit offsets, and past it."""
+    k = 64
     i = np.arange(n, dtype=np.int64)
     ja = np.stack([np.maximum(i - 5, 0), i, np.minimum(i + 70000, n - 1)], axis=1)
     ja[:, 1] = np.where(ja[:, 0] == ja[:, 1], ja[:, 0], ja[:, 1])
