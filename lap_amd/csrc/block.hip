@@ -427,6 +427,17 @@ __global__ __launch_bounds__(BS) void k_blk_dir(int n, int k, int lk, double *__
   }
 }
 
+// col - row of the first kSampleLen entries of row t n / kBlock, kNoEntry past its end
+constexpr int kSampleLen = 32, kNoEntry = INT_MIN;
+__global__ __launch_bounds__(kBlock) void k_spmm_sample(int n, const int *__restrict__ ia,
+                                                        const int *__restrict__ ja,
+                                                        int *__restrict__ out) {
+  const int t = threadIdx.x, row = (int)((long long)t * n / kBlock);
+  const int e0 = ia[row], len = ia[row + 1] - e0;
+  for (int j = 0; j < kSampleLen; ++j)
+    out[t * kSampleLen + j] = j < len ? ja[e0 + j] - row : kNoEntry;
+}
+
 // The workgroups of an SpMM and how they are dealt to the XCDs (cls_block).
 struct SpmmShape {
   unsigned grid;
@@ -489,16 +500,25 @@ int log2i(int k) {
 // (ia, ja, a, n, k, mode) -> chosen tile
 std::map<std::tuple<const void *, const void *, const void *, int, int, int>, int> g_tile;
 
-// spmm_wg_per_cu workgroups per CU, dealt to the XCDs by the plan's sample of
-// column offsets (a matrix without locality has no better group than 1).
-SpmmShape spmm_shape(const SpmvPlan &A, int k) {
+// spmm_wg_per_cu workgroups per CU, dealt to the XCDs by a sample of the column
+// offsets, taken once per plan (a matrix without locality has no better group
+// than 1, nor has one of too few row blocks for two).
+SpmmShape spmm_shape(const SpmvPlan &A, const int *ia, const int *ja, int k) {
   const int per_cu = std::max(1, std::min(16, options().spmm_wg_per_cu));
   const int grid = std::max(8, per_cu * device_cus());
   const int rows = std::max(64 / k, 16) * (kBlock / kWave);
   const long nblk = ((long)A.n + rows - 1) / rows;
   const auto known = A.spmm_shapes.find({rows, grid});
   if (known != A.spmm_shapes.end()) return {known->second.first, known->second.second};
-  const auto best = xcd_grid(A.offsets, rows, nblk, grid);
+  std::vector<int> offsets;
+  if (nblk >= 2 * 64) {
+    DevBuf d(sizeof(int) * kBlock * kSampleLen);
+    if (!d.p) return {(unsigned)grid, 1};
+    k_spmm_sample<<<1, kBlock, 0, stream()>>>(A.n, ia, ja, d.as<int>());
+    for (int o : dev_download(d.as<int>(), (size_t)kBlock * kSampleLen))
+      if (o != kNoEntry) offsets.push_back(o);
+  }
+  const auto best = xcd_grid(offsets, rows, nblk, grid);
   A.spmm_shapes[{rows, grid}] = best;
   return {best.first, best.second};
 }
@@ -584,7 +604,7 @@ extern "C" int lap_csr_matmat(int n, int nnz, const int *ia, const int *ja, cons
   if (!check_device("csr_matmat", {{X, "X", nk}, {Y, "Y", nk}})) return lap_last_status();
   const SpmvPlan *A = spmv_plan(n, nnz, ia, ja);  // validates ia / ja
   if (!A) return lap_last_status();
-  const SpmmShape g = spmm_shape(*A, k);
+  const SpmmShape g = spmm_shape(*A, ia, ja, k);
   if (!tile) tile = pick_tile(g, n, ia, ja, a, k, X, Y);
   if (!tile) return LAP_ERR_HIP;
   spmm_for(k, tile)(g, n, ia, ja, a, X, Y, nullptr, nullptr, nullptr, 0);
@@ -613,7 +633,7 @@ extern "C" int lap_pcg_block(int n, int nnz, const int *ia, const int *ja, const
          *Q = scratch_vec("blk_q", (size_t)n * k);
   BlkCtl *ctl =
       reinterpret_cast<BlkCtl *>(scratch_vec("blk_ctl", sizeof(BlkCtl) / sizeof(double) + 1));
-  const SpmmShape g = spmm_shape(*A, k);
+  const SpmmShape g = spmm_shape(*A, ia, ja, k);
   const unsigned gv = vec_grid((size_t)n * k);
   double *part = scratch_vec("blk_part", (size_t)2 * kMaxK * std::max(g.grid, gv));
   const size_t hist_len = ((size_t)maxit + 2) * (size_t)k;

@@ -291,7 +291,6 @@ struct SpmvPlan {
   int nblocks = 0;        // row blocks
   DevBufPtr rowblk;       // int[nblocks + 1]: first row of each block
   int max_row = 0;
-  std::vector<int> offsets;  // col - row of the entries of some 256 rows (none below 4096 rows)
   // the SpMM's (grid, group) by (rows per block, most workgroups)
   mutable std::map<std::pair<int, int>, std::pair<unsigned, int>> spmm_shapes;
   // the resident Jacobi PCG's analyses of the same matrix, made at its first

@@ -118,11 +118,6 @@ const SpmvPlan *spmv_plan(int n, int nnz, const int *ia, const int *ja) {
                   h_ja[e], e);
         return nullptr;
       }
-    // (fewer rows are one group anyway: xcd_grid)
-    const int every = std::max(1, n / 256);
-    for (int row = every / 2; n >= 4096 && row < n; row += every)
-      for (int e = h_ia[row]; e < std::min(h_ia[row + 1], h_ia[row] + 32); ++e)
-        plan->offsets.push_back(h_ja[e] - row);
   }
   plan->nblocks = (int)starts.size() - 1;
   plan->max_row = max_row;
