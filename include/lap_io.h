@@ -79,7 +79,9 @@ int lap_csr_load(const char *path, int *ia, int *ja, double *a, int to_device);
  * entries before it), which is the order of a stable sort of that fill
  * (glibc's qsort is a merge sort).  cap is the length of ja and a;
  * *nnz_csr receives the number of CSR entries, and LAP_ERR_ARG is returned
- * without writing ja/a when cap is too small (call with cap = 0 to query). */
+ * without writing ja/a when cap is too small (call with cap = 0 to query).
+ * ja and a may share memory with rows, cols and vals (those entries are then
+ * copied first); ia may not. */
 int lap_coo_to_csr(int n, int m, int nnz, const int *rows, const int *cols, const double *vals,
                    int symmetric, int cap, int *ia, int *ja, double *a, int *nnz_csr);
 

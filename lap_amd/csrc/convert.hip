@@ -487,6 +487,10 @@ __global__ void k_adj_values(int n, const int *ia, const int *ja, double *a, con
 
 unsigned rows_grid(long long n) { return grid_for((size_t)std::max<long long>(n, 1), 1, kBlock, 65536); }
 
+bool overlap(const void *p, size_t pb, const void *q, size_t qb) {
+  return (const char *)p < (const char *)q + qb && (const char *)q < (const char *)p + pb;
+}
+
 }  // namespace
 }  // namespace lap
 
@@ -537,6 +541,21 @@ int lap_coo_to_csr(int n, int m, int nnz, const int *rows, const int *cols, cons
     return LAP_ERR_ARG;
   DevBuf ctr(32);
   if (!ctr.p) return lap_last_status();
+  // the entries are read until the last row is sorted, while ja and a are
+  // written: inputs that share memory with them are copied first
+  DevBufPtr held[3];
+  auto apart = [&](const void *in, size_t bytes, DevBufPtr &copy) {
+    if (!overlap(in, bytes, ja, 4 * (size_t)total) && !overlap(in, bytes, a, 8 * (size_t)total))
+      return in;
+    copy = dev_alloc(bytes);
+    if (copy->p)
+      LAP_HIP(hipMemcpyAsync(copy->p, in, bytes, hipMemcpyDeviceToDevice, stream()));
+    return (const void *)copy->p;
+  };
+  rows = static_cast<const int *>(apart(rows, 4 * (size_t)nnz, held[0]));
+  cols = static_cast<const int *>(apart(cols, 4 * (size_t)nnz, held[1]));
+  vals = static_cast<const double *>(apart(vals, 8 * (size_t)nnz, held[2]));
+  if (!rows || !cols || !vals) return lap_last_status();
   unsigned *seq = reinterpret_cast<unsigned *>(ja);  // until the rows are sorted
   const CooSrc src{rows, cols, vals};
   LAP_HIP(hipMemcpyAsync(c, ia, 4 * (size_t)n, hipMemcpyDeviceToDevice, stream()));
