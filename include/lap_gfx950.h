@@ -194,9 +194,11 @@ void lap_clear_error(void);
 
 /* Drops every cached analysis plan, factor and work buffer. */
 void lap_release_all(void);
-/* Plans (SpMV row blocks, triangular level sets, IC0 factors, the mixed-
- * precision copy, batch orders) are cached by the device addresses of the
- * arrays they were built from.  Call this when an address is about to hold a
+/* Plans (SpMV row blocks, the places of the columns in one-launch Jacobi
+ * solves, triangular level sets, IC0 factors, the mixed-precision copy, batch
+ * orders) are cached by the device addresses of the arrays they were built
+ * from.  (ja may be rewritten in place: a one-launch solve compares its places
+ * with it.)  Call this when an address is about to hold a
  * different matrix (e.g. after freeing and reallocating): every plan whose
  * key holds p is dropped.  analyze_spmv and
  * initialize_and_analyze_L_and_U_solve always rebuild their plans. */

@@ -590,28 +590,18 @@ LsPlan *ls_plan(Batch &B, const int *ia) {
   return B.ls.get();
 }
 
-// The batch through the resident solve; outputs as run_lockstep's.
-float run_resident(Batch &B, ResPlan &P, const int *ia, const double *a, const double *d_r, double *x,
-                   const double *b, double tol, int maxit) {
-  double *r = scratch_vec("bt_r", (size_t)B.n), *p = scratch_vec("bt_p", (size_t)B.n);
-  hipEvent_t e0, e1;
-  if (!r || !p || !LAP_HIP(hipEventCreate(&e0))) return -1.f;
-  if (!LAP_HIP(hipEventCreate(&e1))) {
-    (void)hipEventDestroy(e0);
-    return -1.f;
-  }
+// The batch through the resident solve; outputs as run_lockstep's.  0: it does
+// not go that way.
+int run_resident(Batch &B, const SpmvPlan &A, const int *ia, const int *ja, const double *a,
+                 const double *d_r, double *x, const double *b, double tol, int maxit, float *ms) {
+  double *r = scratch_vec("bt_r", (size_t)B.n), *p = scratch_vec("bt_p", (size_t)B.n),
+         *q = scratch_vec("bt_q", (size_t)B.n);
+  if (!r || !p || !q) return -1;
   const size_t ns = (size_t)B.nsys;
   std::vector<ResOut> out(ns);
-  LAP_HIP(hipEventRecord(e0, stream()));
-  const int st = pcg_resident(P, B.n, ia, a, d_r, x, b, tol, maxit, nullptr, r, p,
-                              out.data());
-  LAP_HIP(hipEventRecord(e1, stream()));
-  LAP_HIP(hipEventSynchronize(e1));
-  float ms = 0.f;
-  LAP_HIP(hipEventElapsedTime(&ms, e0, e1));
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  if (st < 0) return -1.f;
+  const int st = pcg_resident(A, A.res_batch, B.off, ia, ja, a, d_r, x, b, tol, maxit, nullptr, r,
+                              p, q, out.data(), ms);
+  if (st <= 0) return st;
   std::vector<int> it(ns), fl(ns);
   std::vector<double> r0(ns), rs(ns);
   for (size_t s = 0; s < ns; ++s) {
@@ -625,16 +615,16 @@ float run_resident(Batch &B, ResPlan &P, const int *ia, const double *a, const d
   B.flag_out->upload(fl.data(), sizeof(int) * ns);
   B.res0_out->upload(r0.data(), sizeof(double) * ns);
   B.res_out->upload(rs.data(), sizeof(double) * ns);
-  return ms;
+  return 1;
 }
 
 // One lockstep solve; outputs land in B's output arrays.  Returns the
 // device milliseconds (HIP events), or -1 on error.
 float run_lockstep(Batch &B, const SpmvPlan &A, const int *ia, const int *ja, const double *a,
                    const double *d_r, double *x, const double *b, double tol, int maxit) {
-  if (!A.res_batch || !res_plan_for(*A.res_batch, B.off))
-    A.res_batch = res_plan_build(A, ia, ja, B.off);
-  if (res_plan_ok(*A.res_batch)) return run_resident(B, *A.res_batch, ia, a, d_r, x, b, tol, maxit);
+  float res_ms = 0.f;
+  const int res = run_resident(B, A, ia, ja, a, d_r, x, b, tol, maxit, &res_ms);
+  if (res) return res < 0 ? -1.f : res_ms;
   LsPlan *P = ls_plan(B, ia);
   if (!P) return -1.f;
   const int nblk = P->nblk;

@@ -312,19 +312,17 @@ struct ResOut {
   int iterations, flag;
   double res0, res;
 };
-// Jacobi PCG solves as one launch with the systems in registers and LDS
-// (resident.hip).  off: the systems' row offsets within the block-diagonal
-// matrix A (0, n: one system).  The plan may turn out not to fit (res_plan_ok
-// false).
-std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const int *ja,
-                                        const std::vector<int> &off);
-bool res_plan_ok(const ResPlan &P);
-bool res_plan_for(const ResPlan &P, const std::vector<int> &off);  // built for these systems
-// Solves; out: one per system.  hist: device, maxit + 2 entries (one system;
-// null: none); r, p: n-vectors of scratch.  1: done, -1: an error was recorded.
-int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double *d_r, double *x,
+// Jacobi PCG of small and medium systems as one launch with the systems in
+// registers and LDS (resident.hip).  off: the systems' row offsets within the
+// block-diagonal matrix A (0, n: one system).  plan: A.res or A.res_batch, made
+// where there is none for these systems and columns.  out: one per system;
+// hist: device, maxit + 2 entries (one system; null: none); r, p, x0: n-vectors
+// of scratch; ms: the solve's device time.  1: done, 0: the systems do not go
+// this way and x is as it was, -1: an error was recorded.
+int pcg_resident(const SpmvPlan &A, std::shared_ptr<ResPlan> &plan, const std::vector<int> &off,
+                 const int *ia, const int *ja, const double *a, const double *d_r, double *x,
                  const double *b, double tol, int maxit, double *hist, double *r, double *p,
-                 ResOut *out);
+                 double *x0, ResOut *out, float *ms);
 
 // ------------------------------------------------- value-indexed CSR
 // Encodes a[0..nnz) as one-byte indices into a table of its distinct values

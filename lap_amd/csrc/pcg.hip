@@ -977,29 +977,22 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
   const int *done = &ctl->done;
   const SpmvPlan &A = *o.A;
   // small and medium systems: one launch (the analysis is kept with the plan)
-  if (o.kind == P_JACOBI && !A.res) A.res = res_plan_build(A, ia, ja, {0, n});
-  if (o.kind == P_JACOBI && res_plan_ok(*A.res)) {
-    hipEvent_t e0, e1;
-    LAP_HIP(hipEventCreate(&e0));
-    LAP_HIP(hipEventCreate(&e1));
-    LAP_HIP(hipEventRecord(e0, stream()));
+  if (o.kind == P_JACOBI) {
     ResOut ro{};
-    const int st = pcg_resident(*A.res, n, ia, a, pd->d_r, x, b, tol, maxit, hist, r, p, &ro);
-    LAP_HIP(hipEventRecord(e1, stream()));
-    LAP_HIP(hipEventSynchronize(e1));
     float ms = 0.f;
-    LAP_HIP(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    out.iterations = ro.iterations;
-    out.flag = st > 0 ? ro.flag : 2;
-    out.res0 = ro.res0;
-    out.res = ro.res;
-    out.gpu_ms = ms;
+    const int st = pcg_resident(A, A.res, {0, n}, ia, ja, a, pd->d_r, x, b, tol, maxit, hist, r, p,
+                                q, &ro, &ms);
     if (st < 0) return lap_last_status();
-    if (h_hist) LAP_HIP(hipMemcpy(h_hist, hist, sizeof(double) * (size_t)(ro.iterations + 1),
-                                  hipMemcpyDeviceToHost));
-    return lap_last_status() == LAP_ERR_HIP ? LAP_ERR_HIP : LAP_OK;
+    if (st > 0) {
+      out.iterations = ro.iterations;
+      out.flag = ro.flag;
+      out.res0 = ro.res0;
+      out.res = ro.res;
+      out.gpu_ms = ms;
+      if (h_hist) LAP_HIP(hipMemcpy(h_hist, hist, sizeof(double) * (size_t)(ro.iterations + 1),
+                                    hipMemcpyDeviceToHost));
+      return lap_last_status() == LAP_ERR_HIP ? LAP_ERR_HIP : LAP_OK;
+    }
   }
   const unsigned gA = spmv_grid(A), gV = vgrid(n);
 

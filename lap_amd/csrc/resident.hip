@@ -72,8 +72,9 @@ struct ResState {
   double rho, tolrel, res0, res;
   int iter, flag;  // flag: -1 not finished
 };
+enum { kResWait = 1, kResStale = 2 };
 struct ResShared {
-  int error;     // a wait ran out
+  int error;     // kResWait: a wait ran out; kResStale: the plan is of other columns
   unsigned tag;  // highest tag used
 };
 // A workgroup: its first row and row count, its team's first workgroup and
@@ -85,13 +86,13 @@ struct ResWg {
 struct ResArgs {
   int nhmax;
   const ResWg *wg;
-  const int *ia;
+  const int *ia, *ja;
   const double *a;
   const unsigned short *lcol;
   const int *hcnt, *hcol;
   const unsigned char *sent;
   const double *d_r, *b;
-  double *x, *r, *p;
+  double *x, *r, *p, *x0;  // x0: x at the start, kept for a solve that ends in an error
   double tol;
   int maxit, resume, iters;
   unsigned tag0;
@@ -168,6 +169,9 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
   unsigned slot[R][(L + 1) / 2];
   bool have[R], sent[R];
   int longest[R];  // of the wave's rows
+  // The slots were made from the columns that ja held at the first solve; where
+  // it has been rewritten since, the solve ends here and the host makes new ones
+  bool stale = false;
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     const int l = t + k * T, row = base + l;
@@ -177,6 +181,10 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
     for (int j = 0; j < L; ++j) {
       val[k][j] = j < len ? g.a[e0 + j] : 0.0;
       const unsigned s = j < len ? g.lcol[e0 + j] : (unsigned)zero;
+      if (j < len) {
+        const int c = g.ja[e0 + j], h = (int)s - R * T;
+        stale |= h < 0 ? (int)s >= rows || base + (int)s != c : h >= nh || hcol[h] != c;
+      }
       if (j & 1)
         slot[k][j / 2] |= s << 16;
       else
@@ -184,12 +192,19 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
     }
     d[k] = have[k] ? g.d_r[row] : 0.0;
     x[k] = have[k] ? g.x[row] : 0.0;
+    if (have[k] && !g.resume) g.x0[row] = x[k];
     r[k] = p[k] = 0.0;
+    stale |= len > L;
     sent[k] = have[k] && g.sent[row];
     int m = len;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
     longest[k] = __builtin_amdgcn_readfirstlane(m);
+  }
+  if (stale) {
+    dead = 1;  // (read after the barriers of the first sums)
+    __hip_atomic_fetch_max(&g.sh->error, (int)kResStale, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
   }
   auto row_sums = [&](double(&s)[R]) {  // CSR order; padding adds 0 * 0
 #pragma unroll
@@ -215,7 +230,8 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
                                                  __HIP_MEMORY_SCOPE_AGENT))) {
       if (lane == 0) {
         dead = 1;
-        __hip_atomic_store(&g.sh->error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_max(&g.sh->error, (int)kResWait, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
       }
       return false;
     }
@@ -516,8 +532,8 @@ struct ResPlan {
   unsigned tag = 0;
 };
 
-std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const int *ja,
-                                        const std::vector<int> &off) {
+static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const int *ja,
+                                               const std::vector<int> &off) {
   auto P = std::make_shared<ResPlan>();
   P->off = off;
   const int n = A.n, cus = std::min(device_cus(), kResMaxWg), ns = (int)off.size() - 1;
@@ -608,12 +624,11 @@ std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const 
   return P;
 }
 
-bool res_plan_ok(const ResPlan &P) { return P.ok; }
-bool res_plan_for(const ResPlan &P, const std::vector<int> &off) { return P.off == off; }
-
-int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double *d_r, double *x,
-                 const double *b, double tol, int maxit, double *hist, double *r, double *p,
-                 ResOut *out) {
+// Solves by the plan.  1: done, 0: the plan is of other columns than ja's, x is
+// as it was, -1: an error was recorded.
+static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double *a,
+                   const double *d_r, double *x, const double *b, double tol, int maxit,
+                   double *hist, double *r, double *p, double *x0, ResOut *out) {
   char *box = P.boxes->as<char>();
   ResArgs g{};
   g.n = n;
@@ -621,6 +636,7 @@ int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double
   g.wg = P.wg->as<ResWg>();
   g.nhmax = P.nhmax;
   g.ia = ia;
+  g.ja = ja;
   g.a = a;
   g.lcol = P.lcol->as<unsigned short>();
   g.hcnt = P.hcnt->as<int>();
@@ -631,6 +647,7 @@ int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double
   g.x = x;
   g.r = r;
   g.p = p;
+  g.x0 = x0;
   g.tol = tol;
   g.maxit = maxit;
   // one system: launches of kResIters iterations; several: one launch, so that
@@ -665,8 +682,13 @@ int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double
       return -1;
     sync();
     if (lap_last_status() == LAP_ERR_HIP) return -1;
-    if (sh.error) {  // start over with unused tags next time
-      clear_boxes();
+    if (sh.error) {
+      clear_boxes();  // start over with unused tags next time
+      if (!LAP_HIP(hipMemcpyAsync(x, x0, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice,
+                                  stream())))
+        return -1;
+      sync();
+      if (sh.error == kResStale) return 0;
       set_error(LAP_ERR_NUMERIC, "pcg: a wait between workgroups ran out");
       return -1;
     }
@@ -677,6 +699,31 @@ int pcg_resident(ResPlan &P, int n, const int *ia, const double *a, const double
     out[s] = ResOut{h[(size_t)s].iter, h[(size_t)s].flag < 0 ? 2 : h[(size_t)s].flag,
                     h[(size_t)s].res0, h[(size_t)s].res};
   return 1;
+}
+
+int pcg_resident(const SpmvPlan &A, std::shared_ptr<ResPlan> &plan, const std::vector<int> &off,
+                 const int *ia, const int *ja, const double *a, const double *d_r, double *x,
+                 const double *b, double tol, int maxit, double *hist, double *r, double *p,
+                 double *x0, ResOut *out, float *ms) {
+  int st = 0;
+  for (int tries = 0; tries < 2 && !st; ++tries) {
+    if (tries || !plan || plan->off != off) plan = res_plan_build(A, ia, ja, off);
+    if (!plan->ok) return 0;
+    hipEvent_t e0, e1;
+    if (!LAP_HIP(hipEventCreate(&e0))) return -1;
+    if (!LAP_HIP(hipEventCreate(&e1))) {
+      (void)hipEventDestroy(e0);
+      return -1;
+    }
+    LAP_HIP(hipEventRecord(e0, stream()));
+    st = res_run(*plan, A.n, ia, ja, a, d_r, x, b, tol, maxit, hist, r, p, x0, out);
+    LAP_HIP(hipEventRecord(e1, stream()));
+    LAP_HIP(hipEventSynchronize(e1));
+    LAP_HIP(hipEventElapsedTime(ms, e0, e1));
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+  }
+  return st;
 }
 
 }  // namespace lap
