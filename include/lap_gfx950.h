@@ -333,9 +333,11 @@ double lap_pcg_spmv_timed(int n, int nnz, const int *ia, const int *ja, const do
  * summed in a fixed tree order, rows of more than 1024 entries over several
  * workgroups), "fuse_sweeps", "spmv_format" (0 CSR, 1 value-indexed,
  * 2 delta-indexed), "mixed_vectors" (lap_pcg_mixed inner vectors: 0 FP32,
- * 1 FP64).  Results do not depend on them except vec_grid, spmv_walk and
- * spmv_wg_per_cu (the dot-product summation order), sptrsv_long and
- * mixed_vectors.  Returns the previous value, or -1 for an unknown name. */
+ * 1 FP64), "resident_polls" (one-launch Jacobi solves: looks at a value that
+ * another workgroup owes, each about 1 us, before the solve is started over by
+ * launches; 0: by launches at once).  Results do not depend on them except
+ * vec_grid, spmv_walk, spmv_wg_per_cu and resident_polls (the dot-product
+ * summation order), sptrsv_long and mixed_vectors.  Returns the previous value, or -1 for an unknown name. */
 int lap_set_option(const char *name, int value);
 
 /* No counterpart in the reference: hip_dot for callers that cannot allocate

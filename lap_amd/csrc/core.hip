@@ -165,6 +165,7 @@ int lap_set_option(const char *name, int value) {
   else if (!strcmp(name, "mixed_vectors")) slot = &o.mixed_vectors;
   else if (!strcmp(name, "sptrsv_long")) slot = &o.sptrsv_long;
   else if (!strcmp(name, "sptrsv_mode")) slot = &o.sptrsv_mode;
+  else if (!strcmp(name, "resident_polls")) slot = &o.resident_polls;
   else if (!strcmp(name, "spmm_wg_per_cu")) slot = &o.spmm_wg_per_cu;
   else if (!strcmp(name, "spmv_wg_per_cu")) slot = &o.spmv_wg_per_cu;
   if (!slot) return -1;
@@ -203,6 +204,10 @@ int lap_set_option(const char *name, int value) {
   }
   if (!strcmp(name, "graph_iters") && (value < 1 || value > 4096)) {
     set_error(LAP_ERR_ARG, "graph_iters must be in [1, 4096]");
+    return *slot;
+  }
+  if (!strcmp(name, "resident_polls") && (value < 0 || value > 1 << 30)) {
+    set_error(LAP_ERR_ARG, "resident_polls must be in [0, 2^30]");
     return *slot;
   }
   if (!strcmp(name, "use_graph") && (value < 0 || value > 1)) {

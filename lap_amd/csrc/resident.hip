@@ -30,8 +30,13 @@
 // team of consecutive workgroups of its own, the largest first: as teams end,
 // the next ones take their CUs.  A team waits for its own workgroups only, and
 // workgroups start in order, so the first team still running always has all of
-// its workgroups.  A team is at most one workgroup per CU.  Waits are bounded
-// and one that runs out ends every workgroup with an error.
+// its workgroups.  A team is at most one workgroup per CU.
+//
+// Nothing keeps other work off the GPU: another process' or stream's kernel can
+// hold CUs that a team's last workgroups wait for, and two one-launch solves of
+// two processes can each hold what the other waits for.  So waits are bounded
+// (option resident_polls); one that runs out ends every workgroup, x is put back
+// and the solve goes by launches, which need no two workgroups at once.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -57,7 +62,6 @@ constexpr int kResMaxRows = 1 << 26;  // rows of all systems at most (box_w stay
 // Workgroups of a batch at most: their halo lists take 32 KB each (1 GB).
 constexpr int kResMaxWgs = 1 << 15;
 constexpr int kResIters = 8192;    // iterations per launch
-constexpr unsigned kResSpins = 1u << 22;
 // Every workgroup of a team reads every sum, through whichever XCD it is on and
 // past the caches: with many workgroups the few lines that hold the boxes are
 // what they wait for.  So a sum is sent in 8 copies and an XCD reads its own: us
@@ -95,7 +99,7 @@ struct ResArgs {
   double *x, *r, *p, *x0;  // x0: x at the start, kept for a solve that ends in an error
   double tol;
   int maxit, resume, iters;
-  unsigned tag0;
+  unsigned tag0, polls;
   double *hist;  // of a single system (may be null)
   void *box_a, *box_b, *box_w;
   int n, stride;  // stride: places from a copy of the sums' boxes to the next
@@ -225,7 +229,7 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
   // One wait of this wave (every lane that still misses something): false
   // once it has to be given up.
   auto again = [&](unsigned &spins) {
-    if (++spins > kResSpins ||
+    if (++spins > g.polls ||
         ((spins & 63u) == 0 && __hip_atomic_load(&g.sh->error, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT))) {
       if (lane == 0) {
@@ -624,8 +628,10 @@ static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia,
   return P;
 }
 
-// Solves by the plan.  1: done, 0: the plan is of other columns than ja's, x is
-// as it was, -1: an error was recorded.
+// Solves by the plan.  kResDone, or x is as it was: kResWait: a wait ran out,
+// kResStale: the plan is of other columns than ja's, kResError: an error was
+// recorded.
+enum { kResDone = 0, kResError = -1 };
 static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double *a,
                    const double *d_r, double *x, const double *b, double tol, int maxit,
                    double *hist, double *r, double *p, double *x0, ResOut *out) {
@@ -650,6 +656,7 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
   g.x0 = x0;
   g.tol = tol;
   g.maxit = maxit;
+  g.polls = (unsigned)options().resident_polls;
   // one system: launches of kResIters iterations; several: one launch, so that
   // a team's CUs go to the next one when it ends
   g.iters = P.nsys == 1 ? kResIters : 0x7fffffff;
@@ -679,18 +686,16 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
         !LAP_HIP(hipMemcpyAsync(h.data(), g.st, sizeof(ResState) * h.size(),
                                 hipMemcpyDeviceToHost, stream())) ||
         !LAP_HIP(hipMemcpyAsync(&sh, g.sh, sizeof sh, hipMemcpyDeviceToHost, stream())))
-      return -1;
+      return kResError;
     sync();
-    if (lap_last_status() == LAP_ERR_HIP) return -1;
+    if (lap_last_status() == LAP_ERR_HIP) return kResError;
     if (sh.error) {
       clear_boxes();  // start over with unused tags next time
       if (!LAP_HIP(hipMemcpyAsync(x, x0, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice,
                                   stream())))
-        return -1;
+        return kResError;
       sync();
-      if (sh.error == kResStale) return 0;
-      set_error(LAP_ERR_NUMERIC, "pcg: a wait between workgroups ran out");
-      return -1;
+      return sh.error;
     }
     P.tag = sh.tag;
     if (P.nsys > 1 || h[0].flag >= 0) break;
@@ -698,15 +703,16 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
   for (int s = 0; s < P.nsys; ++s)
     out[s] = ResOut{h[(size_t)s].iter, h[(size_t)s].flag < 0 ? 2 : h[(size_t)s].flag,
                     h[(size_t)s].res0, h[(size_t)s].res};
-  return 1;
+  return kResDone;
 }
 
 int pcg_resident(const SpmvPlan &A, std::shared_ptr<ResPlan> &plan, const std::vector<int> &off,
                  const int *ia, const int *ja, const double *a, const double *d_r, double *x,
                  const double *b, double tol, int maxit, double *hist, double *r, double *p,
                  double *x0, ResOut *out, float *ms) {
-  int st = 0;
-  for (int tries = 0; tries < 2 && !st; ++tries) {
+  if (!options().resident_polls) return 0;
+  int st = kResStale;
+  for (int tries = 0; tries < 2 && st == kResStale; ++tries) {
     if (tries || !plan || plan->off != off) plan = res_plan_build(A, ia, ja, off);
     if (!plan->ok) return 0;
     hipEvent_t e0, e1;
@@ -723,7 +729,7 @@ int pcg_resident(const SpmvPlan &A, std::shared_ptr<ResPlan> &plan, const std::v
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
   }
-  return st;
+  return st == kResDone ? 1 : st == kResError ? -1 : 0;
 }
 
 }  // namespace lap
