@@ -334,7 +334,7 @@ double lap_pcg_spmv_timed(int n, int nnz, const int *ia, const int *ja, const do
  * workgroups), "fuse_sweeps", "spmv_format" (0 CSR, 1 value-indexed,
  * 2 delta-indexed), "mixed_vectors" (lap_pcg_mixed inner vectors: 0 FP32,
  * 1 FP64), "resident_polls" (one-launch Jacobi solves: looks at a value that
- * another workgroup owes, each about 1 us, before the solve is started over by
+ * another workgroup owes, each about 0.2 us, before the solve is started over by
  * launches; 0: by launches at once).  Results do not depend on them except
  * vec_grid, spmv_walk, spmv_wg_per_cu and resident_polls (the dot-product
  * summation order), sptrsv_long and mixed_vectors.  Returns the previous value, or -1 for an unknown name. */

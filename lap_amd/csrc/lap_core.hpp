@@ -260,8 +260,8 @@ struct Options {
   int mixed_vectors = 0;   // lap_pcg_mixed inner vectors: 0 FP32, 1 FP64
   int sptrsv_long = 0;     // level solves' rows > kTriLongRow entries: 0 summed
                            // in CSR order (bitwise), 1 as a workgroup tree
-  int resident_polls = 1 << 20;  // one-launch Jacobi solves: looks at a value of
-                                 // another workgroup, about 1 us each, before
+  int resident_polls = 1 << 23;  // one-launch Jacobi solves: looks at a value of
+                                 // another workgroup, about 0.2 us each, before
                                  // the solve goes by launches (0: at once)
   int spmv_format = 0;     // PCG SpMV: 0 CSR values, or row classes (cls.hpp) in
                            // large systems; 1 value-indexed when the

@@ -61,7 +61,12 @@ constexpr int kResMaxN = 1 << 19;  // rows of a system at most (the analysis' bi
 constexpr int kResMaxRows = 1 << 26;  // rows of all systems at most (box_w stays below 2^31 bytes)
 // Workgroups of a batch at most: their halo lists take 32 KB each (1 GB).
 constexpr int kResMaxWgs = 1 << 15;
-constexpr int kResIters = 8192;    // iterations per launch
+// Iterations of a system per launch.  A team that has only some of its workgroups
+// running waits for the CUs of systems ahead of it, and that wait counts against
+// resident_polls too: a launch of 8192 iterations holds a CU for at most 0.13 s
+// (15.7 us per iteration at 64 x 64 x 128), whatever maxit is, where a wait runs
+// out after 1 to 2 s (2^23 looks).
+constexpr int kResIters = 8192;
 // Every workgroup of a team reads every sum, through whichever XCD it is on and
 // past the caches: with many workgroups the few lines that hold the boxes are
 // what they wait for.  So a sum is sent in 8 copies and an XCD reads its own: us
@@ -151,6 +156,7 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
   const ResWg wg = g.wg[w];
   const int base = wg.base, rows = wg.rows, team = wg.team, size = wg.size;
   ResState *const st = g.st + wg.sys;
+  if (g.resume && st->flag >= 0) return;  // its system has ended (the whole team's)
   const int nh = g.hcnt[w];
   double *const halo = ps + R * T;
   const int zero = R * T + g.nhmax;
@@ -657,9 +663,7 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
   g.tol = tol;
   g.maxit = maxit;
   g.polls = (unsigned)options().resident_polls;
-  // one system: launches of kResIters iterations; several: one launch, so that
-  // a team's CUs go to the next one when it ends
-  g.iters = P.nsys == 1 ? kResIters : 0x7fffffff;
+  g.iters = kResIters;
   g.hist = hist;
   g.box_a = box;
   g.box_b = box + 16 * (size_t)kResCopies * P.stride;
@@ -667,17 +671,21 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
   g.st = P.state->as<ResState>();
   g.sh = P.shared->as<ResShared>();
   std::vector<ResState> h((size_t)P.nsys);
+  auto clear_shared = [&] {
+    k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResShared) / 4),
+                                          P.shared->as<unsigned>());
+  };
   auto clear_boxes = [&] {
     k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P.box_words, P.boxes->as<unsigned>());
+    clear_shared();
     P.tag = 0;
   };
-  if (P.tag > 0xf0000000u) clear_boxes();  // tags only grow
   k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResState) / 4 * P.nsys),
                                         P.state->as<unsigned>());
-  k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResShared) / 4),
-                                        P.shared->as<unsigned>());
+  clear_shared();
   // iter <= maxit + 1, so this many launches always finish
   for (long k = 0; k <= (long)(maxit + 1) / kResIters + 1; ++k) {
+    if (P.tag > 0xf0000000u) clear_boxes();  // tags only grow
     g.resume = k > 0;
     g.tag0 = P.tag;
     P.fn<<<P.nwg, P.threads, P.lds, stream()>>>(g);
@@ -698,7 +706,7 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
       return sh.error;
     }
     P.tag = sh.tag;
-    if (P.nsys > 1 || h[0].flag >= 0) break;
+    if (std::all_of(h.begin(), h.end(), [](const ResState &s) { return s.flag >= 0; })) break;
   }
   for (int s = 0; s < P.nsys; ++s)
     out[s] = ResOut{h[(size_t)s].iter, h[(size_t)s].flag < 0 ? 2 : h[(size_t)s].flag,

@@ -23,7 +23,7 @@ def polls():
 
 def test_option_range():
     start = S.set_option("resident_polls", 0)
-    assert start == 1 << 20
+    assert start == 1 << 23
     assert S.set_option("resident_polls", -1) == 0 and L.load().lap_last_status() != 0
     L.load().lap_clear_error()
     assert S.set_option("resident_polls", 1 << 30) == 0
@@ -39,7 +39,7 @@ def test_single_solve(dims, polls):
     rng = np.random.default_rng(5)
     b, x0 = S.to_dev(rng.standard_normal(Ah.n)), S.to_dev(rng.standard_normal(Ah.n))
     launches = S.pcg(A, b, P, tol=1e-10, x0=x0)
-    polls(1 << 20)
+    polls(1 << 23)
     resident = S.pcg(A, b, P, tol=1e-10, x0=x0)
     assert not np.array_equal(resident.history, launches.history)  # (two orders of the sums)
     polls(1)
@@ -47,7 +47,7 @@ def test_single_solve(dims, polls):
     assert L.load().lap_last_status() == 0
     assert (cut.iterations, cut.flag) == (launches.iterations, 0)
     assert torch.equal(cut.x, launches.x) and np.array_equal(cut.history, launches.history)
-    polls(1 << 20)
+    polls(1 << 23)
     again = S.pcg(A, b, P, tol=1e-10, x0=x0)
     assert torch.equal(again.x, resident.x) and np.array_equal(again.history, resident.history)
 
@@ -58,7 +58,7 @@ def test_batch(polls):
     B = S.Batch.from_systems(systems, [rng.standard_normal(A.n) for A in systems])
     x0 = S.to_dev(rng.standard_normal(B.A.n))
     launches = S.pcg_batched(B, tol=1e-10, block=-1, x0=x0)
-    polls(1 << 20)
+    polls(1 << 23)
     resident = S.pcg_batched(B, tol=1e-10, block=-1, x0=x0)
     polls(1)
     cut = S.pcg_batched(B, tol=1e-10, block=-1, x0=x0)
