@@ -626,9 +626,14 @@ static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia,
       P->sent->as<unsigned char>(), P->lcol->as<unsigned short>());
   for (int c : dev_download(P->hcnt->as<int>(), (size_t)P->nwg)) P->nhmax = std::max(P->nhmax, c);
   if (lap_last_status() == LAP_ERR_HIP || P->nhmax > kResHalo) return P;
-  P->lds = (int)sizeof(double) * (s->r * s->threads + P->nhmax + 1) + 4 * P->nhmax;
+  auto lds = [&](int halo) {
+    return (int)sizeof(double) * (s->r * s->threads + halo + 1) + 4 * halo;
+  };
+  P->lds = lds(P->nhmax);
+  // the limit belongs to the kernel, which other plans of the shape launch too:
+  // the same for all of them
   if (!LAP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(P->fn),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, P->lds)))
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds(kResHalo))))
     return P;
   P->ok = true;
   return P;
