@@ -542,6 +542,8 @@ struct ResPlan {
   unsigned tag = 0;
 };
 
+// The plan; not ok where the systems do not fit, null where there is no memory
+// for it now (the next solve looks again).
 static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const int *ja,
                                                const std::vector<int> &off) {
   auto P = std::make_shared<ResPlan>();
@@ -599,11 +601,10 @@ static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia,
   P->wg = dev_upload(wgs);
   P->stride = (P->nwg + 15) / 16 * 16 + kResSkew;
   P->box_words = 4 * ((size_t)n + 3 * (size_t)kResCopies * P->stride);
-  // without the memory for it the solve goes by launches, as before
   size_t avail = 0, all = 0;
   const size_t need = sizeof(unsigned) * P->box_words + sizeof(int) * (size_t)P->nwg * kResHalo +
                       sizeof(unsigned short) * (size_t)A.nnz + (size_t)n + ((size_t)64 << 20);
-  if (!LAP_HIP(hipMemGetInfo(&avail, &all)) || avail < need) return P;
+  if (!LAP_HIP(hipMemGetInfo(&avail, &all)) || avail < need) return nullptr;
   P->hcnt = dev_alloc(sizeof(int) * (size_t)P->nwg);
   P->hcol = dev_alloc(sizeof(int) * (size_t)P->nwg * kResHalo);
   P->sent = dev_alloc(((size_t)n + 3) / 4 * 4);
@@ -727,7 +728,7 @@ int pcg_resident(const SpmvPlan &A, std::shared_ptr<ResPlan> &plan, const std::v
   int st = kResStale;
   for (int tries = 0; tries < 2 && st == kResStale; ++tries) {
     if (tries || !plan || plan->off != off) plan = res_plan_build(A, ia, ja, off);
-    if (!plan->ok) return 0;
+    if (!plan || !plan->ok) return 0;
     hipEvent_t e0, e1;
     if (!LAP_HIP(hipEventCreate(&e0))) return -1;
     if (!LAP_HIP(hipEventCreate(&e1))) {
