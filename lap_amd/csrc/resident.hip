@@ -59,7 +59,7 @@ constexpr int kResMaxWg = 256;     // workgroups at most (partials: one per thre
 constexpr int kResRows = 1024, kResRowsShort = 2048, kResShort = 5;
 constexpr int kResMaxN = 1 << 19;  // rows of a system at most (the analysis' bitmap in LDS)
 constexpr int kResMaxRows = 1 << 26;  // rows of all systems at most (box_w stays below 2^31 bytes)
-// Workgroups of a batch at most: their halo lists take 32 KB each (1 GB).
+// Workgroups of a batch at most (their halo lists take up to 32 KB each: 1 GB).
 constexpr int kResMaxWgs = 1 << 15;
 // Iterations of a system per launch.  A team that has only some of its workgroups
 // running waits for the CUs of systems ahead of it, and that wait counts against
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
     dead = 0;
     ps[zero] = 0.0;
   }
-  for (int h = t; h < nh; h += T) hcol[h] = g.hcol[(size_t)w * kResHalo + h];
+  for (int h = t; h < nh; h += T) hcol[h] = g.hcol[(size_t)w * g.nhmax + h];
   __syncthreads();
   // the thread's rows
   double val[R][L], x[R], r[R], p[R], d[R];
@@ -445,10 +445,13 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
 
 // The analysis: workgroup w lists the rows outside its own that its rows refer
 // to (ascending), marks them as sent, and gives every nonzero its slot: own
-// rows first, then the halo.  cnt[w]: the halo's length (more than kResHalo, or
-// a column outside the system: nothing else is written).  Dynamic LDS: a bitmap
-// of the system's rows and the rank of each of its words.
+// rows first, then the halo.  Without FILL only cnt[w], the halo's length (more
+// than kResHalo also for a column outside the system); with FILL the rest, once
+// the longest halo, nhmax, is known.  Dynamic LDS: a bitmap of the system's rows
+// and the rank of each of its words.
+template <bool FILL>
 __global__ __launch_bounds__(kResThreads) void k_res_plan(const ResWg *__restrict__ wgs, int own,
+                                                          int nhmax,
                                                           const int *__restrict__ ia,
                                                           const int *__restrict__ ja,
                                                           int *__restrict__ cnt,
@@ -489,14 +492,14 @@ __global__ __launch_bounds__(kResThreads) void k_res_plan(const ResWg *__restric
     __syncthreads();
   }
   const int total = scan[kResThreads - 1];
-  if (t == 0) cnt[w] = bad ? kResHalo + 1 : total;
-  if (total > kResHalo || bad) return;
+  if (!FILL && t == 0) cnt[w] = bad ? kResHalo + 1 : total;
+  if (!FILL || bad || total > nhmax) return;
   int at = scan[t] - c;
   for (int i = i0; i < i1; ++i) {
     rank[i] = (unsigned short)at;
     for (unsigned m = bits[i]; m; m &= m - 1) {
       const int col = wg.s0 + i * 32 + __ffs((int)m) - 1;
-      hcol[(size_t)w * kResHalo + at++] = col;
+      hcol[(size_t)w * nhmax + at++] = col;
       sent[col] = 1;
     }
   }
@@ -598,35 +601,44 @@ static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia,
   P->nwg = (int)wgs.size();
   P->fn = s->fn;
   P->threads = s->threads;
-  P->wg = dev_upload(wgs);
   P->stride = (P->nwg + 15) / 16 * 16 + kResSkew;
   P->box_words = 4 * ((size_t)n + 3 * (size_t)kResCopies * P->stride);
+  const int words = (big + 31) / 32;
+  const int plan_lds = words * 4 + (words + 1) / 2 * 4;
+  for (auto *k : {k_res_plan<false>, k_res_plan<true>})
+    if (!LAP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, plan_lds)))
+      return P;
+  // the halos' lengths first: a plan that does not fit keeps no memory, one that
+  // does what its halos need
+  DevBufPtr wg = dev_upload(wgs), hcnt = dev_alloc(sizeof(int) * (size_t)P->nwg);
+  if (!wg->p || !hcnt->p) return P;
+  auto plan = [&](auto *k, int *hcol, unsigned char *sent, unsigned short *lcol) {
+    k<<<P->nwg, kResThreads, plan_lds, stream()>>>(wg->as<ResWg>(), s->r * s->threads, P->nhmax,
+                                                   ia, ja, hcnt->as<int>(), hcol, sent, lcol);
+  };
+  plan(k_res_plan<false>, nullptr, nullptr, nullptr);
+  for (int c : dev_download(hcnt->as<int>(), (size_t)P->nwg)) P->nhmax = std::max(P->nhmax, c);
+  if (lap_last_status() == LAP_ERR_HIP || P->nhmax > kResHalo) return P;
+  const size_t lists = sizeof(int) * (size_t)P->nwg * P->nhmax;
   size_t avail = 0, all = 0;
-  const size_t need = sizeof(unsigned) * P->box_words + sizeof(int) * (size_t)P->nwg * kResHalo +
+  const size_t need = sizeof(unsigned) * P->box_words + lists +
                       sizeof(unsigned short) * (size_t)A.nnz + (size_t)n + ((size_t)64 << 20);
   if (!LAP_HIP(hipMemGetInfo(&avail, &all)) || avail < need) return nullptr;
-  P->hcnt = dev_alloc(sizeof(int) * (size_t)P->nwg);
-  P->hcol = dev_alloc(sizeof(int) * (size_t)P->nwg * kResHalo);
+  P->wg = wg;
+  P->hcnt = hcnt;
+  P->hcol = dev_alloc(lists);
   P->sent = dev_alloc(((size_t)n + 3) / 4 * 4);
   P->lcol = dev_alloc(sizeof(unsigned short) * (size_t)std::max(A.nnz, 1));
   P->state = dev_alloc(sizeof(ResState) * (size_t)ns);
   P->shared = dev_alloc(sizeof(ResShared));
   P->boxes = dev_alloc(sizeof(unsigned) * P->box_words);
-  for (const DevBufPtr &b : {P->wg, P->hcnt, P->hcol, P->sent, P->lcol, P->state, P->shared,
-                             P->boxes})
+  for (const DevBufPtr &b : {P->hcol, P->sent, P->lcol, P->state, P->shared, P->boxes})
     if (!b->p) return P;
-  const int words = (big + 31) / 32;
-  const int plan_lds = words * 4 + (words + 1) / 2 * 4;
-  if (!LAP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_res_plan),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, plan_lds)))
-    return P;
   k_res_zero<<<256, kBlock, 0, stream()>>>(((long long)n + 3) / 4, P->sent->as<unsigned>());
   k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P->box_words, P->boxes->as<unsigned>());
-  k_res_plan<<<P->nwg, kResThreads, plan_lds, stream()>>>(
-      P->wg->as<ResWg>(), s->r * s->threads, ia, ja, P->hcnt->as<int>(), P->hcol->as<int>(),
-      P->sent->as<unsigned char>(), P->lcol->as<unsigned short>());
-  for (int c : dev_download(P->hcnt->as<int>(), (size_t)P->nwg)) P->nhmax = std::max(P->nhmax, c);
-  if (lap_last_status() == LAP_ERR_HIP || P->nhmax > kResHalo) return P;
+  plan(k_res_plan<true>, P->hcol->as<int>(), P->sent->as<unsigned char>(),
+       P->lcol->as<unsigned short>());
   auto lds = [&](int halo) {
     return (int)sizeof(double) * (s->r * s->threads + halo + 1) + 4 * halo;
   };
