@@ -706,9 +706,12 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
     if (P.tag > 0xf0000000u) clear_boxes();  // tags only grow
     g.resume = k > 0;
     g.tag0 = P.tag;
-    P.fn<<<P.nwg, P.threads, P.lds, stream()>>>(g);
+    // (this launch's own status: hipGetLastError would also give what an earlier
+    // call of the program left)
+    void *args[] = {&g};
     ResShared sh{};
-    if (!LAP_HIP(hipGetLastError()) ||
+    if (!LAP_HIP(hipLaunchKernel(reinterpret_cast<const void *>(P.fn), dim3((unsigned)P.nwg),
+                                 dim3((unsigned)P.threads), args, (size_t)P.lds, stream())) ||
         !LAP_HIP(hipMemcpyAsync(h.data(), g.st, sizeof(ResState) * h.size(),
                                 hipMemcpyDeviceToHost, stream())) ||
         !LAP_HIP(hipMemcpyAsync(&sh, g.sh, sizeof sh, hipMemcpyDeviceToHost, stream())))
