@@ -512,10 +512,10 @@ SpmmShape spmm_shape(const SpmvPlan &A, const int *ia, const int *ja, int k) {
   if (known != A.spmm_shapes.end()) return {known->second.first, known->second.second};
   std::vector<int> offsets;
   if (nblk >= 2 * 64) {
-    DevBuf d(sizeof(int) * kBlock * kSampleLen);
-    if (!d.p) return {(unsigned)grid, 1};
-    k_spmm_sample<<<1, kBlock, 0, stream()>>>(A.n, ia, ja, d.as<int>());
-    for (int o : dev_download(d.as<int>(), (size_t)kBlock * kSampleLen))
+    const DevBufPtr d = dev_try(sizeof(int) * kBlock * kSampleLen);
+    if (!d) return {(unsigned)grid, 1};
+    k_spmm_sample<<<1, kBlock, 0, stream()>>>(A.n, ia, ja, d->as<int>());
+    for (int o : dev_download(d->as<int>(), (size_t)kBlock * kSampleLen))
       if (o != kNoEntry) offsets.push_back(o);
   }
   const auto best = xcd_grid(offsets, rows, nblk, grid);

@@ -234,9 +234,9 @@ __global__ __launch_bounds__(kBlock) void k_cls_inner(int ncls, int width, int w
 ClsMat cls_inner(const ClsMat &A, int max_row) {
   ClsMat m = A;
   m.width = (max_row + 8) / 8 * 8;
-  double *val = scratch_vec("cls_inner_val", (size_t)kClsMax * kClsRow);
+  double *val = scratch_try("cls_inner_val", (size_t)kClsMax * kClsRow);
   int *off = reinterpret_cast<int *>(
-      scratch_vec("cls_inner_off", kClsMax * (kClsRow + 1) / 2 + 1));
+      scratch_try("cls_inner_off", kClsMax * (kClsRow + 1) / 2 + 1));
   if (!A.cls || m.width > kClsRow || !val || !off) return ClsMat();
   m.off = off;
   m.val = val;
@@ -286,7 +286,7 @@ int cls_group(const std::vector<int> &offsets, int rows, unsigned grid) {
 bool cls_probe(int n, int nnz, const int *ia, const int *ja, const double *a, const double *d_r,
                int max_row, int *host) {
   if (n < 1 || nnz < 1 || max_row > kClsRow) return false;
-  int *out = reinterpret_cast<int *>(scratch_vec("cls_probe", 1));
+  int *out = reinterpret_cast<int *>(scratch_try("cls_probe", 1));
   if (!out) return false;
   k_cls_probe<<<1, kClsProbe, 0, stream()>>>(n, ia, ja, a, d_r, out);
   return LAP_HIP(hipMemcpyAsync(host, out, sizeof(int), hipMemcpyDeviceToHost, stream()));
@@ -307,9 +307,9 @@ ClsMat cls_encode(const char *tag, int n, int nnz, const int *ia, const int *ja,
   };
   static DevBufPtr table;
   static Table *h = nullptr;
-  if (!table) table = dev_alloc(sizeof(Table));
-  if (!h && !LAP_HIP(hipHostMalloc((void **)&h, sizeof(Table), hipHostMallocDefault))) h = nullptr;
-  if (!table->p || !h) return m;
+  if (!table) table = dev_try(sizeof(Table));
+  if (!h && !hip_try(hipHostMalloc((void **)&h, sizeof(Table), hipHostMallocDefault))) h = nullptr;
+  if (!table || !h) return m;
   Table *t = table->as<Table>();
   k_cls_clear<<<4, kBlock, 0, stream()>>>(t->key, t->rep, &t->st);
   k_cls_collect<<<grid_for((size_t)n, 4, kBlock, 2048), kBlock, 0, stream()>>>(
@@ -332,14 +332,14 @@ ClsMat cls_encode(const char *tag, int n, int nnz, const int *ia, const int *ja,
   const int width = max_row <= least ? least : (max_row + 7) / 8 * 8;
   // without the memory for a byte per row the solve keeps its matrix
   size_t avail = 0, all = 0;
-  if (!LAP_HIP(hipMemGetInfo(&avail, &all)) || avail < (size_t)n + ((size_t)4 << 20)) return m;
+  if (!hip_try(hipMemGetInfo(&avail, &all)) || avail < (size_t)n + ((size_t)4 << 20)) return m;
   unsigned char *cls =
-      reinterpret_cast<unsigned char *>(scratch_vec(name.c_str(), ((size_t)n + 7) / 8));
-  double *val = scratch_vec((name + "_val").c_str(), (size_t)kClsMax * kClsRow);
+      reinterpret_cast<unsigned char *>(scratch_try(name.c_str(), ((size_t)n + 7) / 8));
+  double *val = scratch_try((name + "_val").c_str(), (size_t)kClsMax * kClsRow);
   int *off = reinterpret_cast<int *>(
-      scratch_vec((name + "_off").c_str(), kClsMax * (kClsRow + 1) / 2 + 1));
+      scratch_try((name + "_off").c_str(), kClsMax * (kClsRow + 1) / 2 + 1));
   int *len = off + kClsMax * kClsRow;
-  double *d = scratch_vec((name + "_d").c_str(), kClsMax + 1);
+  double *d = scratch_try((name + "_d").c_str(), kClsMax + 1);
   if (!cls || !val || !off || !d) return m;
   LAP_HIP(hipMemcpyAsync(t, h, offsetof(Table, key), hipMemcpyHostToDevice, stream()));
   k_cls_table<<<1, kBlock, 0, stream()>>>(nc, width, t->reps, ia, ja, a, d_r, off, len, val, d);

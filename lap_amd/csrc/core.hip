@@ -103,6 +103,11 @@ void DevBuf::upload(const void *src, size_t b, size_t off) {
   sync();
 }
 DevBufPtr dev_alloc(size_t bytes) { return std::make_shared<DevBuf>(bytes); }
+DevBufPtr dev_try(size_t bytes) {
+  auto b = std::make_shared<DevBuf>();
+  b->bytes = bytes;
+  return hip_try(hipMalloc(&b->p, bytes ? bytes : 16)) ? b : nullptr;
+}
 
 namespace {
 std::map<std::string, DevBufPtr> g_scratch;
@@ -121,6 +126,12 @@ double *scratch_vec(const char *tag, size_t n) {
   auto &slot = g_scratch[tag];
   if (!slot || slot->bytes < n * sizeof(double)) slot = dev_alloc(n * sizeof(double));
   return slot->as<double>();
+}
+
+double *scratch_try(const char *tag, size_t n) {
+  auto &slot = g_scratch[tag];
+  if (!slot || !slot->p || slot->bytes < n * sizeof(double)) slot = dev_try(n * sizeof(double));
+  return slot ? slot->as<double>() : nullptr;
 }
 
 ReduceWs &reduce_ws() {

@@ -65,6 +65,13 @@ struct DevBuf {
 };
 using DevBufPtr = std::shared_ptr<DevBuf>;
 DevBufPtr dev_alloc(size_t bytes);
+// For what a call can do without: a failure is not recorded as its error, and a
+// buffer that cannot be had is null.
+inline bool hip_try(hipError_t e) {
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e == hipSuccess;
+}
+DevBufPtr dev_try(size_t bytes);
 template <class T>
 DevBufPtr dev_upload(const std::vector<T> &v) {
   auto b = dev_alloc(v.size() * sizeof(T) + 16);
@@ -86,6 +93,7 @@ int *pinned_flags();
 
 // Cached n-vectors reused across solves (avoids hipMalloc in timed regions).
 double *scratch_vec(const char *tag, size_t n);
+double *scratch_try(const char *tag, size_t n);  // (by dev_try)
 
 // ------------------------------------------------------------ reductions
 // Fence-free deterministic reductions.  A producer kernel writes one partial

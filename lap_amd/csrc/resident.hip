@@ -546,7 +546,8 @@ struct ResPlan {
 };
 
 // The plan; not ok where the systems do not fit, null where there is no memory
-// for it now (the next solve looks again).
+// for it now (the next solve looks again).  Nothing here is an error of the
+// solve, which can go by launches.
 static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia, const int *ja,
                                                const std::vector<int> &off) {
   auto P = std::make_shared<ResPlan>();
@@ -603,57 +604,65 @@ static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia,
   P->threads = s->threads;
   P->stride = (P->nwg + 15) / 16 * 16 + kResSkew;
   P->box_words = 4 * ((size_t)n + 3 * (size_t)kResCopies * P->stride);
+  auto lds = [&](int halo) {
+    return (int)sizeof(double) * (s->r * s->threads + halo + 1) + 4 * halo;
+  };
+  // the limit belongs to the kernel, which other plans of the shape launch too:
+  // the same for all of them
+  if (!hip_try(hipFuncSetAttribute(reinterpret_cast<const void *>(P->fn),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds(kResHalo))))
+    return P;
   const int words = (big + 31) / 32;
   const int plan_lds = words * 4 + (words + 1) / 2 * 4;
   for (auto *k : {k_res_plan<false>, k_res_plan<true>})
-    if (!LAP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+    if (!hip_try(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, plan_lds)))
       return P;
   // the halos' lengths first: a plan that does not fit keeps no memory, one that
   // does what its halos need
-  DevBufPtr wg = dev_upload(wgs), hcnt = dev_alloc(sizeof(int) * (size_t)P->nwg);
-  if (!wg->p || !hcnt->p) return P;
+  const size_t wgs_bytes = sizeof(ResWg) * wgs.size();
+  DevBufPtr wg = dev_try(wgs_bytes), hcnt = dev_try(sizeof(int) * wgs.size());
+  if (!wg || !hcnt) return nullptr;
+  std::vector<int> cnt(wgs.size());
   auto plan = [&](auto *k, int *hcol, unsigned char *sent, unsigned short *lcol) {
     k<<<P->nwg, kResThreads, plan_lds, stream()>>>(wg->as<ResWg>(), s->r * s->threads, P->nhmax,
                                                    ia, ja, hcnt->as<int>(), hcol, sent, lcol);
   };
+  if (!hip_try(hipMemcpyAsync(wg->p, wgs.data(), wgs_bytes, hipMemcpyHostToDevice, stream())))
+    return nullptr;
   plan(k_res_plan<false>, nullptr, nullptr, nullptr);
-  for (int c : dev_download(hcnt->as<int>(), (size_t)P->nwg)) P->nhmax = std::max(P->nhmax, c);
-  if (lap_last_status() == LAP_ERR_HIP || P->nhmax > kResHalo) return P;
+  if (!hip_try(hipMemcpyAsync(cnt.data(), hcnt->p, sizeof(int) * cnt.size(), hipMemcpyDeviceToHost,
+                              stream())) ||
+      !hip_try(hipStreamSynchronize(stream())))
+    return nullptr;
+  P->nhmax = *std::max_element(cnt.begin(), cnt.end());
+  if (P->nhmax > kResHalo) return P;
   const size_t lists = sizeof(int) * (size_t)P->nwg * P->nhmax;
   size_t avail = 0, all = 0;
   const size_t need = sizeof(unsigned) * P->box_words + lists +
                       sizeof(unsigned short) * (size_t)A.nnz + (size_t)n + ((size_t)64 << 20);
-  if (!LAP_HIP(hipMemGetInfo(&avail, &all)) || avail < need) return nullptr;
+  if (!hip_try(hipMemGetInfo(&avail, &all)) || avail < need) return nullptr;
   P->wg = wg;
   P->hcnt = hcnt;
-  P->hcol = dev_alloc(lists);
-  P->sent = dev_alloc(((size_t)n + 3) / 4 * 4);
-  P->lcol = dev_alloc(sizeof(unsigned short) * (size_t)std::max(A.nnz, 1));
-  P->state = dev_alloc(sizeof(ResState) * (size_t)ns);
-  P->shared = dev_alloc(sizeof(ResShared));
-  P->boxes = dev_alloc(sizeof(unsigned) * P->box_words);
+  P->hcol = dev_try(lists);
+  P->sent = dev_try(((size_t)n + 3) / 4 * 4);
+  P->lcol = dev_try(sizeof(unsigned short) * (size_t)A.nnz);
+  P->state = dev_try(sizeof(ResState) * (size_t)ns);
+  P->shared = dev_try(sizeof(ResShared));
+  P->boxes = dev_try(sizeof(unsigned) * P->box_words);
   for (const DevBufPtr &b : {P->hcol, P->sent, P->lcol, P->state, P->shared, P->boxes})
-    if (!b->p) return P;
+    if (!b) return nullptr;
   k_res_zero<<<256, kBlock, 0, stream()>>>(((long long)n + 3) / 4, P->sent->as<unsigned>());
   k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P->box_words, P->boxes->as<unsigned>());
   plan(k_res_plan<true>, P->hcol->as<int>(), P->sent->as<unsigned char>(),
        P->lcol->as<unsigned short>());
-  auto lds = [&](int halo) {
-    return (int)sizeof(double) * (s->r * s->threads + halo + 1) + 4 * halo;
-  };
   P->lds = lds(P->nhmax);
-  // the limit belongs to the kernel, which other plans of the shape launch too:
-  // the same for all of them
-  if (!LAP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(P->fn),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds(kResHalo))))
-    return P;
   P->ok = true;
   return P;
 }
 
-// Solves by the plan.  kResDone, or x is as it was: kResWait: a wait ran out,
-// kResStale: the plan is of other columns than ja's, kResError: an error was
+// Solves by the plan.  kResDone, or x is as it was: kResWait: a wait ran out (or
+// the launch was refused), kResStale: the plan is of other columns than ja's, kResError: an error was
 // recorded.
 enum { kResDone = 0, kResError = -1 };
 static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double *a,
@@ -701,6 +710,11 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
   k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResState) / 4 * P.nsys),
                                         P.state->as<unsigned>());
   clear_shared();
+  auto restore = [&] {
+    return LAP_HIP(hipMemcpyAsync(x, x0, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice,
+                                  stream())) &&
+           LAP_HIP(hipStreamSynchronize(stream()));
+  };
   // iter <= maxit + 1, so this many launches always finish
   for (long k = 0; k <= (long)(maxit + 1) / kResIters + 1; ++k) {
     if (P.tag > 0xf0000000u) clear_boxes();  // tags only grow
@@ -710,21 +724,17 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
     // call of the program left)
     void *args[] = {&g};
     ResShared sh{};
-    if (!LAP_HIP(hipLaunchKernel(reinterpret_cast<const void *>(P.fn), dim3((unsigned)P.nwg),
-                                 dim3((unsigned)P.threads), args, (size_t)P.lds, stream())) ||
-        !LAP_HIP(hipMemcpyAsync(h.data(), g.st, sizeof(ResState) * h.size(),
+    if (!hip_try(hipLaunchKernel(reinterpret_cast<const void *>(P.fn), dim3((unsigned)P.nwg),
+                                 dim3((unsigned)P.threads), args, (size_t)P.lds, stream())))
+      return k == 0 || restore() ? kResWait : kResError;
+    if (!LAP_HIP(hipMemcpyAsync(h.data(), g.st, sizeof(ResState) * h.size(),
                                 hipMemcpyDeviceToHost, stream())) ||
-        !LAP_HIP(hipMemcpyAsync(&sh, g.sh, sizeof sh, hipMemcpyDeviceToHost, stream())))
+        !LAP_HIP(hipMemcpyAsync(&sh, g.sh, sizeof sh, hipMemcpyDeviceToHost, stream())) ||
+        !LAP_HIP(hipStreamSynchronize(stream())))
       return kResError;
-    sync();
-    if (lap_last_status() == LAP_ERR_HIP) return kResError;
     if (sh.error) {
       clear_boxes();  // start over with unused tags next time
-      if (!LAP_HIP(hipMemcpyAsync(x, x0, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice,
-                                  stream())))
-        return kResError;
-      sync();
-      return sh.error;
+      return restore() ? sh.error : kResError;
     }
     P.tag = sh.tag;
     if (std::all_of(h.begin(), h.end(), [](const ResState &s) { return s.flag >= 0; })) break;
