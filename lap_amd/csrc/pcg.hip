@@ -974,6 +974,7 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
   double *q = scratch_vec("pcg_q", (size_t)n);
   PcgCtl *ctl = reinterpret_cast<PcgCtl *>(scratch_vec("pcg_ctl", sizeof(PcgCtl) / 8 + 1));
   double *hist = scratch_vec("pcg_hist", (size_t)maxit + 2);
+  if (!r || !w || !p || !q || !ctl || !hist) return lap_last_status();
   const int *done = &ctl->done;
   const SpmvPlan &A = *o.A;
   // small and medium systems: one launch (the analysis is kept with the plan)

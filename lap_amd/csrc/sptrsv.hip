@@ -1443,15 +1443,16 @@ void tri_clear_error() {
 }
 
 // The chunked schedule's records for one set of values, and its right-hand
-// side buffer, each with kFlGroup steps of room past the end.
+// side buffer, each with kFlGroup steps of room past the end.  false: there is no
+// memory for them (the solve goes by levels).
 template <class AT, class VT>
 static bool tri_fl_pack(const TriPlan &p, const int *ja, const AT *a, DevBufPtr &rec,
                         DevBufPtr &xc) {
   const size_t steps = (size_t)p.ch.nrec / kWave + kFlGroup;
   const size_t rb = steps * FlRec<AT>::bytes, xb = steps * kWave * sizeof(VT);
-  if (!rec || rec->bytes < rb) rec = dev_alloc(rb);
-  if (!xc || xc->bytes < xb) xc = dev_alloc(xb);
-  if (!rec->p || !xc->p) return false;
+  if (!rec || rec->bytes < rb) rec = dev_try(rb);
+  if (!xc || xc->bytes < xb) xc = dev_try(xb);
+  if (!rec || !xc) return false;
   const unsigned g = grid_for((size_t)p.ch.nrec, 1, kBlock, 65536);
   k_fl_pack<AT, VT><<<g, kBlock, 0, stream()>>>(
       p.ch.nrec, p.ch.cmap->as<int>(), p.desc->as<int4>(), ja, a, p.ch.code->as<int2>(),
@@ -1491,9 +1492,9 @@ void tri_ell_build(const TriPlan &p, const int *ja, const double *a, TriEll &e) 
   e.w = 0;
   if (p.n <= 0 || p.max_row > 8) return;
   const int w = p.max_row <= 4 ? 4 : 8;
-  e.ja = dev_alloc(sizeof(int) * (size_t)p.n * w);
-  e.a = dev_alloc(sizeof(double) * (size_t)p.n * w);
-  if (!e.ja || !e.a || !e.ja->p || !e.a->p) return;
+  e.ja = dev_try(sizeof(int) * (size_t)p.n * w);
+  e.a = dev_try(sizeof(double) * (size_t)p.n * w);
+  if (!e.ja || !e.a) return;
   const unsigned g = grid_for((size_t)p.n, 1, kBlock, 65536);
   if (w == 4)
     k_ell_pack<4><<<g, kBlock, 0, stream()>>>(p.n, p.desc->as<int4>(), ja, a, e.ja->as<int>(),
@@ -1595,8 +1596,8 @@ bool tri_solve_tail_launch(const TriPlan &p, const double *x, double *y, const T
 
 DevBufPtr tri_compose(const TriPlan &first, const TriPlan &second) {
   if (first.ch.nchunks <= 0 || second.ch.nchunks <= 0) return nullptr;
-  DevBufPtr m = dev_alloc(sizeof(int) * (size_t)second.ch.nrec);
-  if (!m->p) return nullptr;
+  DevBufPtr m = dev_try(sizeof(int) * (size_t)second.ch.nrec);
+  if (!m) return nullptr;
   k_fl_compose<<<grid_for((size_t)second.ch.nrec, 4, kBlock, 4096), kBlock, 0, stream()>>>(
       second.ch.nrec, second.ch.crow->as<int>(), first.ch.pos->as<int>(), m->as<int>());
   return m;
