@@ -661,8 +661,8 @@ float run_lockstep(Batch &B, const SpmvPlan &A, const int *ia, const int *ja, co
   };
   // every system stops by iteration maxit + 1, so G * max_batches
   // iterations always reach all_done
-  const int G = std::max(1, std::min(options().graph_iters, maxit + 2));
-  const long max_batches = (long)(maxit + 1) / G + 3;
+  const int G = std::max(1, (int)std::min<long>(options().graph_iters, (long)maxit + 2));
+  const long max_batches = ((long)maxit + 1) / G + 3;
   bool ok = true;
   hipGraphExec_t gexec = nullptr;
   if (options().use_graph) {

@@ -675,8 +675,8 @@ extern "C" int lap_pcg_block(int n, int nnz, const int *ia, const int *ja, const
   };
   // iter <= maxit + 1 for every column, so G * max_batches iterations
   // always reach all_done
-  const int G = std::max(1, std::min(options().graph_iters, maxit + 2));
-  const long max_batches = (long)(maxit + 1) / G + 3;
+  const int G = std::max(1, (int)std::min<long>(options().graph_iters, (long)maxit + 2));
+  const long max_batches = ((long)maxit + 1) / G + 3;
   int status = LAP_OK;
   hipGraphExec_t gexec = nullptr;
   if (options().use_graph) {

@@ -1120,7 +1120,7 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
                           tri_launches(*icp->uplan, &icp->uell, false)
                     : tri_launches32(*icp->lplan, &M->lch) + tri_launches32(*icp->uplan, &M->uch);
   int G = std::max(1, std::min(options().graph_iters, 4096 / per_iter));
-  G = std::min(G, maxit + 2);
+  G = (int)std::min<long>(G, (long)maxit + 2);
 
   int status = LAP_OK;
   hipGraphExec_t gexec = nullptr;
@@ -1151,7 +1151,7 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
     if (classes)
       classes = cls_probe(n, nnz, ia, ja, a, jac ? pd->d_r : nullptr, A64->max_row, flags + 2) &&
                 LAP_HIP(hipEventRecord(pe[1], stream()));
-    const long max_batches = (long)(maxit + 1) / G + 3;
+    const long max_batches = ((long)maxit + 1) / G + 3;
     bool finished = false;
     for (long k = 0; k < max_batches + 1 && !finished; ++k) {
       if (k == 1 && classes && LAP_HIP(hipEventSynchronize(pe[1])) && !flags[2] &&

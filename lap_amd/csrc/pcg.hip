@@ -1053,7 +1053,7 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
   if (o.kind == P_IT_JACOBI || o.kind == P_GS_IT || o.kind == P_GS_IT2)
     per_iter += 8 * o.m * (o.k + 2);
   int G = std::max(1, std::min(options().graph_iters, 4096 / per_iter));
-  G = std::min(G, maxit + 2);
+  G = (int)std::min<long>(G, (long)maxit + 2);
 
   int status = LAP_OK;
   int *flags = pinned_flags();
@@ -1088,7 +1088,7 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
       classes = cls_probe(n, nnz, ia, ja, a, jac ? pd->d_r : nullptr, A.max_row, flags + 2) &&
                 LAP_HIP(hipEventRecord(pe[1], stream()));
     // iter <= maxit + 1, so this many batches always reach done
-    const long max_batches = (long)(maxit + 1) / G + 3;
+    const long max_batches = ((long)maxit + 1) / G + 3;
     bool finished = false;
     for (long k = 0; k < max_batches + 1 && !finished; ++k) {
       if (k == 1 && classes && LAP_HIP(hipEventSynchronize(pe[1])) && !flags[2] &&

@@ -716,7 +716,7 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
            LAP_HIP(hipStreamSynchronize(stream()));
   };
   // iter <= maxit + 1, so this many launches always finish
-  for (long k = 0; k <= (long)(maxit + 1) / kResIters + 1; ++k) {
+  for (long k = 0; k <= ((long)maxit + 1) / kResIters + 1; ++k) {
     if (P.tag > 0xf0000000u) clear_boxes();  // tags only grow
     g.resume = k > 0;
     g.tag0 = P.tag;
