@@ -19,7 +19,7 @@
 // themselves run in CSR order, one per column, which is the reference's
 // simple_csr_matvec sum (simple_blas.c:24-44) bit for bit whatever RU is.  RU
 // (1, 2, 4) is picked per (matrix, k) by timing the candidates once.  A chunk
-// with too many nonzeros for its LDS reads them from memory as it goes.
+// with too many nonzeros for its LDS reads them from memory as it goes (add_far).
 //
 // Workgroups are dealt to the 8 XCDs in turn, each with an L2 of its own, so
 // the chunks are handed out such that a row's neighbours are mostly worked on
@@ -69,11 +69,20 @@ struct BlkCtl {
 // ---------------------------------------------------------------- SpMM
 
 // The rows a wave works on at a time, and the nonzeros of them it has room for
-// (a lane's loads of each).
-template <int K>
+// (a lane's loads of each).  ONE: a row per lane group instead of 16 rows or
+// more.  16 rows in a row are one wave's serial work where they are long or hubs,
+// and few waves' where there are few.  Gain of k = 32 and 64 over a kernel
+// without chunks, 16 rows and ONE: power-law graph of 100,000 nodes (rows of up to
+// 10,676 entries) 0.96 / 0.32 and 3.7 / 3.0; 10,000 rows of 17 entries 1.11 / 0.89
+// and 1.16 / 0.98, 2000 of 101 0.76 / 0.46 and 1.58 / 1.32; but the 96^3 grid 2.17
+// / 1.39 and 1.24 / 0.82, 200,000 rows of 17 1.79 / 1.24 and 1.39 / 0.96.  So ONE
+// for up to one chunk of 16 rows per SIMD and for rows of more than the LDS of a
+// chunk; with k < 16, whose groups are more, it is not needed.
+constexpr int kOneK = 16, kOneRows = 16 * 1024, kOneLong = 256;
+template <int K, bool ONE>
 struct Chunk {
   static constexpr int G = 64 / K;
-  static constexpr int kRW = G > 16 ? G : 16;
+  static constexpr int kRW = ONE || G > 16 ? G : 16;
   static constexpr int kEPL = G > 16 ? 8 : 4;
   static constexpr int kCap = kEPL * 64;
 };
@@ -87,7 +96,7 @@ __device__ __forceinline__ void wave_sync() {
 // P.Q per column; 2: Q = -(A P - B) (initial residual) with partials of
 // Q.Q.  Partials: part[col * gridDim.x + blockIdx.x].
 // FAR: P has 4 GB or more, beyond the 32-bit offsets of a buffer load.
-template <int BS, int K, int RU, int EU, int MODE, bool FAR>
+template <int BS, int K, int RU, int EU, int MODE, bool FAR, bool ONE>
 __global__ __launch_bounds__(BS) void k_spmm(int n, const int *__restrict__ ia,
                                              const int *__restrict__ ja,
                                              const double *__restrict__ a,
@@ -95,7 +104,7 @@ __global__ __launch_bounds__(BS) void k_spmm(int n, const int *__restrict__ ia,
                                              const double *__restrict__ Bm, double *part,
                                              const BlkCtl *ctl, int group) {
   if (MODE == 1 && ctl->all_done) return;
-  using C = Chunk<K>;
+  using C = Chunk<K, ONE>;
   constexpr int G = C::G, RW = C::kRW, EPL = C::kEPL, NW = BS / 64;
   static_assert(RW % (G * RU) == 0 && RW <= 64, "whole steps per chunk");
   // a nonzero: its value and the byte offset (FAR: the number) of its row of P;
@@ -161,8 +170,9 @@ __global__ __launch_bounds__(BS) void k_spmm(int n, const int *__restrict__ ia,
     return e;
   };
   double acc = 0.0;
-  // the rows of a chunk; entry(e, end): its e-th nonzero, or none from end on
-  auto work = [&](int row0, auto entry) {
+  // the rows of a chunk; sum(e0, e1, s): the sums s of the group's rows, row j's
+  // nonzeros being e0[j] to e1[j] of the chunk's
+  auto rows = [&](int row0, auto sum) {
     for (int base = 0; base < RW && base < n - row0; base += G * RU) {
       int e0[RU], e1[RU];
       double s[RU], own[RU];
@@ -174,25 +184,7 @@ __global__ __launch_bounds__(BS) void k_spmm(int n, const int *__restrict__ ia,
         s[j] = 0.0;
         if (MODE == 1) own[j] = r < n - row0 ? P[(size_t)(row0 + r) * K + c] : 0.0;
       }
-      for (int off = 0;; off += EU) {
-        bool any = false;
-#pragma unroll
-        for (int j = 0; j < RU; ++j) any |= e0[j] + off < e1[j];
-        if (!any) break;
-        double av[RU][EU], v[RU][EU];
-#pragma unroll
-        for (int j = 0; j < RU; ++j)
-#pragma unroll
-          for (int t = 0; t < EU; ++t) {
-            const Nz x = entry(e0[j] + off + t, e1[j]);
-            av[j][t] = x.v;
-            v[j][t] = gather(x.at);
-          }
-#pragma unroll
-        for (int j = 0; j < RU; ++j)
-#pragma unroll
-          for (int t = 0; t < EU; ++t) s[j] += av[j][t] * v[j][t];
-      }
+      sum(e0, e1, s);
 #pragma unroll
       for (int j = 0; j < RU; ++j) {
         const int row = row0 + base + j * G + g;
@@ -207,6 +199,87 @@ __global__ __launch_bounds__(BS) void k_spmm(int n, const int *__restrict__ ia,
             if (MODE == 1) acc += own[j] * s[j];
           }
         }
+      }
+    }
+  };
+  // entry(e, end): a nonzero, or none from end on; no row has more than most
+  auto add = [&](const int(&e0)[RU], const int(&e1)[RU], int most, double(&s)[RU], auto entry) {
+    for (int off = 0; off < most; off += EU) {
+      bool any = false;
+#pragma unroll
+      for (int j = 0; j < RU; ++j) any |= e0[j] + off < e1[j];
+      if (!any) break;
+      double av[RU][EU], v[RU][EU];
+      unsigned at[RU][EU];
+#pragma unroll
+      for (int j = 0; j < RU; ++j)
+#pragma unroll
+        for (int t = 0; t < EU; ++t) {
+          const Nz x = entry(e0[j] + off + t, e1[j]);
+          av[j][t] = x.v;
+          at[j][t] = x.at;
+        }
+#pragma unroll
+      for (int j = 0; j < RU; ++j)
+#pragma unroll
+        for (int t = 0; t < EU; ++t) v[j][t] = gather(at[j][t]);
+#pragma unroll
+      for (int j = 0; j < RU; ++j)
+#pragma unroll
+        for (int t = 0; t < EU; ++t) s[j] += av[j][t] * v[j][t];
+    }
+  };
+  // a chunk with more nonzeros than its LDS holds: every lane reads its row's
+  // entries, EU of each of its rows at a time (the index is
+  // clamped: with a return past the row's end the loads wait for each other), or
+  // with 1 or 2 groups, whose lanes would all read the same few, the group's
+  // lanes read a window of each row together, the next one while this one is
+  // added.  us per call at 50,000 rows of 101 entries, k = 8, 32 and 64: 92, 262
+  // and 239 entry by entry, 73, 119 and 213 so
+  constexpr int WIN = C::kCap / (G * RU), WL = WIN >= K ? WIN / K : 1;
+  auto add_far = [&](int eb, const int(&e0)[RU], const int(&e1)[RU], double(&s)[RU]) {
+    if constexpr (K < 32) {
+      add(e0, e1, INT_MAX, s, [&](int i, int end) {
+        const int q = eb + (i < end ? i : 0);
+        const double v = a[q];
+        const unsigned at = (unsigned)ja[q] * kRowBytes;
+        return Nz{i < end ? v : 0.0, i < end ? at : kNone, 0};
+      });
+    } else {
+      int longest = 0;
+#pragma unroll
+      for (int j = 0; j < RU; ++j) longest = max(longest, e1[j] - e0[j]);
+      for (int off = K; off < 64; off <<= 1) longest = max(longest, __shfl_xor(longest, off));
+      longest = __builtin_amdgcn_readfirstlane(longest);
+      Nz win[RU][WL];
+      auto ask = [&](int w) {
+#pragma unroll
+        for (int j = 0; j < RU; ++j)
+#pragma unroll
+          for (int u = 0; u < WL; ++u) {
+            const int i = e0[j] + w + u * K + c;
+            const bool in = i < e1[j];
+            const double v = a[eb + (in ? i : 0)];
+            const unsigned at = (unsigned)ja[eb + (in ? i : 0)] * kRowBytes;
+            win[j][u] = Nz{in ? v : 0.0, in ? at : kNone, 0};
+          }
+      };
+      ask(0);
+      for (int w = 0; w < longest; w += WIN) {
+        wave_sync();  // (the last window's reads are done)
+#pragma unroll
+        for (int j = 0; j < RU; ++j)
+#pragma unroll
+          for (int u = 0; u < WL; ++u) nz[(j * G + g) * WIN + u * K + c] = win[j][u];
+        wave_sync();
+        ask(w + WIN);
+        int w0[RU], w1[RU];
+#pragma unroll
+        for (int j = 0; j < RU; ++j) {
+          w0[j] = (j * G + g) * WIN;
+          w1[j] = w0[j] + min(WIN, e1[j] - e0[j] - w);
+        }
+        add(w0, w1, WIN, s, [&](int i, int end) { return nz[i < end ? i : C::kCap]; });
       }
     }
   };
@@ -230,12 +303,11 @@ __global__ __launch_bounds__(BS) void k_spmm(int n, const int *__restrict__ ia,
     e = ask_ent(p);
     p = ask_ptr(blk + 2 * step);
     if (cnt <= C::kCap)
-      work(row0, [&](int i, int end) { return nz[i < end ? i : C::kCap]; });
-    else
-      work(row0, [&](int i, int end) {
-        if (i >= end) return Nz{0.0, kNone, 0};
-        return Nz{a[eb + i], (unsigned)ja[eb + i] * kRowBytes, 0};
+      rows(row0, [&](auto &e0, auto &e1, auto &s) {
+        add(e0, e1, INT_MAX, s, [&](int i, int end) { return nz[i < end ? i : C::kCap]; });
       });
+    else
+      rows(row0, [&](auto &e0, auto &e1, auto &s) { add_far(eb, e0, e1, s); });
   }
   if (MODE == 0) return;
   // fixed-order reduction: butterfly over the row groups of a wave, then
@@ -442,22 +514,23 @@ __global__ __launch_bounds__(kBlock) void k_spmm_sample(int n, const int *__rest
 struct SpmmShape {
   unsigned grid;
   int group;
+  bool one;
 };
 
 using SpmmFn = void (*)(SpmmShape, int, const int *, const int *, const double *, const double *,
                         double *, const double *, double *, const BlkCtl *, int);
 
-template <int K, int RU0>
+template <int K, int RU0, bool ONE>
 void spmm_launch(SpmmShape g, int n, const int *ia, const int *ja, const double *a,
                  const double *P, double *Q, const double *Bm, double *part, const BlkCtl *ctl,
                  int mode) {
-  constexpr int kMost = Chunk<K>::kRW / Chunk<K>::G;  // rows per group in a chunk
-  constexpr int RU = RU0 < kMost ? RU0 : kMost, EU = RU == 4 ? 4 : 8;
+  constexpr int kMost = Chunk<K, ONE>::kRW / Chunk<K, ONE>::G;  // rows per group in a chunk
+  constexpr int RU = RU0 < kMost ? RU0 : kMost, EU = ONE ? 16 : RU == 4 ? 4 : 8;
   auto pick = [&](auto far) {
     constexpr bool F = decltype(far)::value;
-    return mode == 2   ? k_spmm<kBlock, K, RU, EU, 2, F>
-           : mode == 1 ? k_spmm<kBlock, K, RU, EU, 1, F>
-                       : k_spmm<kBlock, K, RU, EU, 0, F>;
+    return mode == 2   ? k_spmm<kBlock, K, RU, EU, 2, F, ONE>
+           : mode == 1 ? k_spmm<kBlock, K, RU, EU, 1, F, ONE>
+                       : k_spmm<kBlock, K, RU, EU, 0, F, ONE>;
   };
   const bool far = (size_t)n * K * 8 > 0xfffffff0u;
   auto *f = far ? pick(std::true_type{}) : pick(std::false_type{});
@@ -465,23 +538,25 @@ void spmm_launch(SpmmShape g, int n, const int *ia, const int *ja, const double 
 }
 
 template <int K>
-SpmmFn spmm_for_k(int ru) {
+SpmmFn spmm_for_k(int ru, bool one) {
+  if constexpr (K >= kOneK)
+    if (one) return spmm_launch<K, 1, true>;
   switch (ru) {
-    case 1: return spmm_launch<K, 1>;
-    case 2: return spmm_launch<K, 2>;
-    default: return spmm_launch<K, 4>;
+    case 1: return spmm_launch<K, 1, false>;
+    case 2: return spmm_launch<K, 2, false>;
+    default: return spmm_launch<K, 4, false>;
   }
 }
 
-SpmmFn spmm_for(int k, int ru) {
+SpmmFn spmm_for(int k, int ru, bool one) {
   switch (k) {
-    case 1: return spmm_for_k<1>(ru);
-    case 2: return spmm_for_k<2>(ru);
-    case 4: return spmm_for_k<4>(ru);
-    case 8: return spmm_for_k<8>(ru);
-    case 16: return spmm_for_k<16>(ru);
-    case 32: return spmm_for_k<32>(ru);
-    case 64: return spmm_for_k<64>(ru);
+    case 1: return spmm_for_k<1>(ru, one);
+    case 2: return spmm_for_k<2>(ru, one);
+    case 4: return spmm_for_k<4>(ru, one);
+    case 8: return spmm_for_k<8>(ru, one);
+    case 16: return spmm_for_k<16>(ru, one);
+    case 32: return spmm_for_k<32>(ru, one);
+    case 64: return spmm_for_k<64>(ru, one);
     default: return nullptr;
   }
 }
@@ -506,21 +581,22 @@ std::map<std::tuple<const void *, const void *, const void *, int, int, int>, in
 SpmmShape spmm_shape(const SpmvPlan &A, const int *ia, const int *ja, int k) {
   const int per_cu = std::max(1, std::min(16, options().spmm_wg_per_cu));
   const int grid = std::max(8, per_cu * device_cus());
-  const int rows = std::max(64 / k, 16) * (kBlock / kWave);
+  const bool one = k >= kOneK && (A.n <= kOneRows || A.max_row > kOneLong);
+  const int rows = (one ? 64 / k : std::max(64 / k, 16)) * (kBlock / kWave);
   const long nblk = ((long)A.n + rows - 1) / rows;
   const auto known = A.spmm_shapes.find({rows, grid});
-  if (known != A.spmm_shapes.end()) return {known->second.first, known->second.second};
+  if (known != A.spmm_shapes.end()) return {known->second.first, known->second.second, one};
   std::vector<int> offsets;
   if (nblk >= 2 * 64) {
     const DevBufPtr d = dev_try(sizeof(int) * kBlock * kSampleLen);
-    if (!d) return {(unsigned)grid, 1};
+    if (!d) return {(unsigned)grid, 1, one};
     k_spmm_sample<<<1, kBlock, 0, stream()>>>(A.n, ia, ja, d->as<int>());
     for (int o : dev_download(d->as<int>(), (size_t)kBlock * kSampleLen))
       if (o != kNoEntry) offsets.push_back(o);
   }
   const auto best = xcd_grid(offsets, rows, nblk, grid);
   A.spmm_shapes[{rows, grid}] = best;
-  return {best.first, best.second};
+  return {best.first, best.second, one};
 }
 
 unsigned vec_grid(size_t elems) {
@@ -533,6 +609,7 @@ unsigned vec_grid(size_t elems) {
 int pick_tile(SpmmShape g, int n, const int *ia, const int *ja, const double *a, int k,
               const double *X, double *Y, int mode = 0, double *part = nullptr, const BlkCtl *ctl = nullptr) {
   auto key = std::make_tuple((const void *)ia, (const void *)ja, (const void *)a, n, k, mode);
+  if (g.one) return 1;  // (the tile says nothing)
   auto it = g_tile.find(key);
   if (it != g_tile.end()) return it->second;
   int best_ru = 0;
@@ -544,7 +621,7 @@ int pick_tile(SpmmShape g, int n, const int *ia, const int *ja, const double *a,
     return 0;
   }
   for (int ru = 1; ru <= 4; ru *= 2) {
-    SpmmFn fn = spmm_for(k, ru);
+    SpmmFn fn = spmm_for(k, ru, g.one);
     fn(g, n, ia, ja, a, X, Y, nullptr, part, ctl, mode);
     LAP_HIP(hipEventRecord(e0, stream()));
     for (int r = 0; r < 3; ++r) fn(g, n, ia, ja, a, X, Y, nullptr, part, ctl, mode);
@@ -607,7 +684,7 @@ extern "C" int lap_csr_matmat(int n, int nnz, const int *ia, const int *ja, cons
   const SpmmShape g = spmm_shape(*A, ia, ja, k);
   if (!tile) tile = pick_tile(g, n, ia, ja, a, k, X, Y);
   if (!tile) return LAP_ERR_HIP;
-  spmm_for(k, tile)(g, n, ia, ja, a, X, Y, nullptr, nullptr, nullptr, 0);
+  spmm_for(k, tile, g.one)(g, n, ia, ja, a, X, Y, nullptr, nullptr, nullptr, 0);
   if (!LAP_HIP(hipGetLastError())) return LAP_ERR_HIP;
   sync();
   return LAP_OK;
@@ -652,7 +729,7 @@ extern "C" int lap_pcg_block(int n, int nnz, const int *ia, const int *ja, const
   // timed in the solve's own mode (q = A p with the p.q epilogue)
   if (!tile) tile = pick_tile(g, n, ia, ja, a, k, Bm, Q, 1, part, ctl);
   if (!tile) return LAP_ERR_HIP;
-  SpmmFn spmm = spmm_for(k, tile);
+  SpmmFn spmm = spmm_for(k, tile, g.one);
   const int lk = log2i(k);
 
   hipEvent_t ev0, ev1;
