@@ -329,7 +329,7 @@ double lap_pcg_spmv_timed(int n, int nnz, const int *ia, const int *ja, const do
  * launch, 1..4096), "use_graph" (0 or 1), "spmm_wg_per_cu" (block CG SpMM
  * workgroups per CU), "sptrsv_mode" (triangular solves: 0 one launch per
  * level, 3, the default, one persistent launch over chunks of rows with
- * point-to-point waits), "sptrsv_long" (1: rows of more than 32 entries
+ * point-to-point waits where that is faster, 4 wherever the rows allow it), "sptrsv_long" (1: rows of more than 32 entries
  * summed in a fixed tree order, rows of more than 1024 entries over several
  * workgroups), "fuse_sweeps", "spmv_format" (0 CSR, 1 value-indexed,
  * 2 delta-indexed), "mixed_vectors" (lap_pcg_mixed inner vectors: 0 FP32,

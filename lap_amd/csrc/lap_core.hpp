@@ -263,7 +263,8 @@ struct Options {
   int spmm_wg_per_cu = 4;  // block CG SpMM grid: workgroups per CU
   int sptrsv_mode = 3;     // triangular solves: 0 one launch per level, 3 one
                            // persistent launch over chunks of rows with
-                           // point-to-point waits
+                           // point-to-point waits where that is faster, 4
+                           // wherever the rows allow it
   int fuse_sweeps = 1;     // it_jacobi / GS_it / GS_it2: one launch per sweep
   int mixed_vectors = 0;   // lap_pcg_mixed inner vectors: 0 FP32, 1 FP64
   int sptrsv_long = 0;     // level solves' rows > kTriLongRow entries: 0 summed
@@ -400,6 +401,8 @@ struct TriPlan {
   // chunk's inbox, filled by the chunk that solves the row.
   struct Chunks {
     int nchunks = 0, nrec = 0;  // nrec: 64 records per step, padding included
+    long long cost = 0;         // simulated length, in steps
+    mutable int taken = -1;     // 0: launches per level are faster (-1: not known yet)
     DevBufPtr cstep;  // int[nchunks + 1]: first step of each chunk
     DevBufPtr crow;   // int[nrec]: row of each record, -1: padding
     DevBufPtr pos;    // int[n]: record of each row

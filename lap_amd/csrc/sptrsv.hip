@@ -13,7 +13,8 @@
 // chunks of rows that are all resident, values between chunks passed as
 // tagged words through memory (k_tri_flow).  Same row arithmetic as the level
 // launches: bitwise identical.  Triangles whose rows do not fit a record keep
-// the level launches (option sptrsv_mode 0 forces them everywhere).  Measured
+// the level launches (option sptrsv_mode 0 forces them everywhere), and so do those
+// that are faster that way (tri_choose).  Measured
 // against the level launches and against one workgroup of 256-row steps per
 // chunk with progress counters, which it replaced, per IC0 / GS_std PCG
 // iteration (us): 128^3 434 / 480 against 1840 / 2100; 256^3 2100 / 2690
@@ -1271,6 +1272,7 @@ static void tri_chunks_build(TriPlan &p, const std::vector<int> &ia, const std::
     if (!b->p) return;
   ch.nrec = (int)T;
   ch.nchunks = G;
+  ch.cost = best.cost;
   if (getenv("LAP_SCHED_LOG"))
     fprintf(stderr, "[lapgfx] %s triangle n=%d: chunked schedule %zu of %zu, %d chunks, %d steps, "
             "%lld values between chunks, simulated length %lld (one launch per level: %d)\n",
@@ -1488,6 +1490,8 @@ static void tri_fl_tail(const TriPlan &p, const DevBufPtr &xc, double *y, const 
                                      t.grid % 8 ? 1 : (int)t.grid / 8, done);
 }
 
+static void tri_choose(const TriPlan &p, const TriEll &e);
+
 void tri_ell_build(const TriPlan &p, const int *ja, const double *a, TriEll &e) {
   e.w = 0;
   if (p.n <= 0 || p.max_row > 8) return;
@@ -1503,7 +1507,7 @@ void tri_ell_build(const TriPlan &p, const int *ja, const double *a, TriEll &e) 
     k_ell_pack<8><<<g, kBlock, 0, stream()>>>(p.n, p.desc->as<int4>(), ja, a, e.ja->as<int>(),
                                               e.a->as<double>());
   e.w = w;
-  if (p.ch.nchunks > 0) tri_fl_pack<double, double>(p, ja, a, e.crec, e.xc);
+  if (p.ch.nchunks > 0 && tri_fl_pack<double, double>(p, ja, a, e.crec, e.xc)) tri_choose(p, e);
 }
 
 void tri_ch_pack32(const TriPlan &p, const int *ja, const float *a, TriChunks32 &c) {
@@ -1537,12 +1541,35 @@ static void tri_level_launch(const TriPlan &p, const int *ja, const AT *a, const
   }
 }
 
+// One launch per level over the packed rows.
+static void tri_ell_launch(const TriPlan &p, const TriEll &ell, const double *diag,
+                           const double *x, double *y, const int *done) {
+  const int *order = p.order->as<int>();
+  for (int l = 0; l < p.nlevels; ++l) {
+    const int l0 = p.level_ptr[l], cnt = p.level_ptr[l + 1] - l0;
+    const unsigned g = (unsigned)((cnt + kBlock - 1) / kBlock);
+    const size_t off = (size_t)l0 * ell.w;
+    if (ell.w == 4)
+      k_tri_level_ell<4><<<g, kBlock, 0, stream()>>>(cnt, order + l0, ell.ja->as<int>() + off,
+                                                     ell.a->as<double>() + off, diag, x, y, done);
+    else
+      k_tri_level_ell<8><<<g, kBlock, 0, stream()>>>(cnt, order + l0, ell.ja->as<int>() + off,
+                                                     ell.a->as<double>() + off, diag, x, y, done);
+  }
+}
+
 // Which path tri_solve_launch takes.
 enum TriPath { TRI_CHUNKS, TRI_LEVELS_ELL, TRI_LEVELS };
 
-static TriPath tri_path(const TriPlan &p, const TriEll *ell, bool in_place) {
+// Whether the option asks for chunks: 4, or 3 and they are not known to be slower.
+static bool tri_mode_chunks(const TriPlan &p) {
   const int mode = options().sptrsv_mode;
-  if (mode == 3 && ell && ell->w && ell->crec && ell->xc && p.ch.nchunks > 0 && sf_state())
+  return mode == 4 || (mode == 3 && p.ch.taken != 0);
+}
+
+static TriPath tri_path(const TriPlan &p, const TriEll *ell, bool in_place) {
+  if (tri_mode_chunks(p) && ell && ell->w && ell->crec && ell->xc && p.ch.nchunks > 0 &&
+      sf_state())
     return TRI_CHUNKS;
   (void)in_place;  // the chunked kernel reads x from its own gathered copy
   if (ell && ell->w) return TRI_LEVELS_ELL;
@@ -1560,30 +1587,82 @@ void tri_solve_launch(const TriPlan &p, const int *ia, const int *ja, const doub
                       const double *diag, const double *x, double *y, const int *done,
                       const TriEll *ell) {
   (void)ia;  // the plan's descriptors carry every row's range
-  const int *order = p.order->as<int>();
   const TriPath path = tri_path(p, ell, x == y);
   if (path == TRI_CHUNKS) {
     tri_fl_launch<double, double>(p, ell->crec, ell->xc, x, p.ch.crow->as<int>(), done);
     tri_fl_spread(p, ell->xc, y, done);
     return;
   }
-  if (path == TRI_LEVELS_ELL) {
-    for (int l = 0; l < p.nlevels; ++l) {
-      const int l0 = p.level_ptr[l], cnt = p.level_ptr[l + 1] - l0;
-      const unsigned g = (unsigned)((cnt + kBlock - 1) / kBlock);
-      const size_t off = (size_t)l0 * ell->w;
-      if (ell->w == 4)
-        k_tri_level_ell<4><<<g, kBlock, 0, stream()>>>(cnt, order + l0, ell->ja->as<int>() + off,
-                                                       ell->a->as<double>() + off, diag, x, y,
-                                                       done);
-      else
-        k_tri_level_ell<8><<<g, kBlock, 0, stream()>>>(cnt, order + l0, ell->ja->as<int>() + off,
-                                                       ell->a->as<double>() + off, diag, x, y,
-                                                       done);
-    }
+  if (path == TRI_LEVELS_ELL) return tri_ell_launch(p, *ell, diag, x, y, done);
+  tri_level_launch<double, double>(p, ja, a, diag, x, y, done);
+}
+
+// Chunks or a launch per level, found out at a triangle's first values: both give
+// the same bits.  A triangle of wide levels without locality (nodes in random
+// order, far neighbours) has few levels, and chunks that wait for each other at
+// every step.  us per IC0 PCG iteration, chunks and levels: shuffled 100^2 grid (11
+// levels, simulated length 137) 247 and 102, 200^2 (13, 216) 101 and 125, 1200^2
+// (17, 345) 524 and 408, circulant of 500,000 rows with neighbours 23,000 and 70,000
+// away (22, 554) 351 and 201.  The simulated length does not tell these apart, so
+// where it is kTriSure times the levels or more the two are timed, once per plan;
+// below (grids: 1 to 2) a level costs its launch, 1.8 to 3 us, against 0.2 us a
+// step.  Up to 3 levels are no more launches than the chunks' three (100,000 rows
+// of one entry 85 and 61).  In a solve the chunks save some 4 us more, which the
+// timing does not see: two solves in a row skip a copy, the last copy does the axpy
+// or the dot product (circulant of 50,000 rows with neighbours 2300 and 7000 away,
+// 53 us either way alone, 134 and 170 an iteration).
+constexpr int kTriSure = 4, kTriFew = 3, kTriTimed = 8192;
+constexpr float kTriSaved = 4.f;
+static void tri_choose(const TriPlan &p, const TriEll &e) {
+  if (p.ch.taken >= 0 || options().sptrsv_mode != 3) return;
+  p.ch.taken = p.nlevels > kTriFew;
+  if (!p.ch.taken || p.ch.cost < (long long)kTriSure * p.nlevels || p.nlevels > kTriTimed) return;
+  double *x = scratch_try("tri_time_x", (size_t)p.n), *y = scratch_try("tri_time_y", (size_t)p.n);
+  hipEvent_t ev[2];
+  if (!x || !y || !hip_try(hipEventCreate(&ev[0]))) return;
+  if (!hip_try(hipEventCreate(&ev[1]))) {
+    (void)hipEventDestroy(ev[0]);
     return;
   }
-  tri_level_launch<double, double>(p, ja, a, diag, x, y, done);
+  launch_fill(p.n, 1.0, x);
+  const int solves = std::max(1, std::min(4, 2048 / p.nlevels));
+  float ms[2] = {0.f, 0.f};  // by levels, by chunks
+  bool ok = true;
+  for (int chunks = 0; ok && chunks < 2; ++chunks) {
+    // as the solves run them: several in a graph
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    ok = hip_try(hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal));
+    if (ok) {
+      // (the copy back to row order does what the levels leave to another launch:
+      // the next solve's gather, the axpy or the dot product)
+      for (int s = 0; s < solves; ++s)
+        if (chunks)
+          tri_fl_launch<double, double>(p, e.crec, e.xc, x, p.ch.crow->as<int>(), nullptr);
+        else
+          tri_ell_launch(p, e, nullptr, x, y, nullptr);
+      ok = hip_try(hipStreamEndCapture(stream(), &graph));
+    }
+    ok = ok && hip_try(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+    for (int rep = 0; ok && rep < 2; ++rep) {  // (the first one apart)
+      if (rep == 1) ok = hip_try(hipEventRecord(ev[0], stream()));
+      ok = ok && hip_try(hipGraphLaunch(exec, stream()));
+    }
+    ok = ok && hip_try(hipEventRecord(ev[1], stream())) && hip_try(hipEventSynchronize(ev[1])) &&
+         hip_try(hipEventElapsedTime(&ms[chunks], ev[0], ev[1]));
+    if (exec) (void)hipGraphExecDestroy(exec);
+    if (graph) (void)hipGraphDestroy(graph);
+  }
+  (void)hipEventDestroy(ev[0]);
+  (void)hipEventDestroy(ev[1]);
+  if (ok) p.ch.taken = ms[1] <= ms[0] + 1e-3f * solves * kTriSaved;
+  if (getenv("LAP_SCHED_LOG"))
+    fprintf(stderr, "[lapgfx] triangle n=%d: %.1f us by chunks, %.1f us by levels\n", p.n,
+            ms[1] * 1e3f / solves, ms[0] * 1e3f / solves);
+  if (tri_error()) {  // a wait ran out
+    tri_clear_error();
+    p.ch.taken = 0;
+  }
 }
 
 bool tri_solve_tail_launch(const TriPlan &p, const double *x, double *y, const TriEll &ell,
@@ -1624,7 +1703,7 @@ static void tri_mixed_launch(const TriPlan &p, const int *ja, const float *a, co
 }
 
 static bool tri_chunks32_ready(const TriPlan &p, const TriChunks32 *c) {
-  return c && c->ok && options().sptrsv_mode == 3 && p.ch.nchunks > 0 && sf_state();
+  return c && c->ok && tri_mode_chunks(p) && p.ch.nchunks > 0 && sf_state();
 }
 
 int tri_launches32(const TriPlan &p, const TriChunks32 *c) {
