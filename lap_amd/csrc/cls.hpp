@@ -21,6 +21,7 @@ namespace lap {
 
 constexpr int kClsMax = 255;   // classes
 constexpr int kClsRow = 16;    // entries of a row at most
+constexpr int kClsPair = 8;    // width of the triangles' tables at most for sweeps of both
 
 // Systems of fewer rows keep the CSR arrays: their matrix is in the Infinity
 // Cache and an iteration is mostly launches (at 10^6 rows of 7 entries an
@@ -79,7 +80,8 @@ ClsMat cls_encode(const char *tag, int n, int nnz, const int *ia, const int *ja,
                   const double *d_r, int max_row, int least = 8);
 
 // The triangles (and A, for GS_it) of the sweep preconditioners as row classes
-// with d_r, and the grid of their sweeps; n == 0: not encoded.
+// with d_r, and the grid of their sweeps; n == 0: not encoded.  pairs: the sweeps
+// will all be of L and U together.
 struct SweepCls {
   int n = 0, group = 1;
   unsigned grid = 1;
@@ -88,7 +90,7 @@ struct SweepCls {
 SweepCls sweep_encode(const SpmvPlan &L, const int *lia, const int *lja, const double *la,
                       const SpmvPlan &U, const int *uia, const int *uja, const double *ua,
                       const SpmvPlan *A, const int *ia, const int *ja, const double *a,
-                      const double *d_r);
+                      const double *d_r, bool pairs);
 // The sweeps over classes (A: one of s's matrices).
 void sweep_one_launch(const SweepCls &s, const ClsMat &A, const double *x, const double *base,
                       double *out, double *out2, int mode, bool first, const int *done);

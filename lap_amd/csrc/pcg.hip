@@ -758,7 +758,8 @@ static bool prec_fused(const PrecOps &o, const double *r, double *w, const int *
   const double *dr = pd->d_r;
   const bool cls = o.sweep.n > 0;
   auto pair = [&](const double *x, const double *base, double *out) {
-    if (cls) return sweep_pair_launch(o.sweep, x, base, out, done);
+    if (cls && o.sweep.L.width <= kClsPair)
+      return sweep_pair_launch(o.sweep, x, base, out, done);
     sweep_pair_launch(*o.LU, pd->lia, pd->lja, pd->la, pd->uia, pd->uja, pd->ua, x, base, dr,
                       out, done);
   };
@@ -1097,7 +1098,8 @@ static int run_pcg(int n, int nnz, const int *ia, const int *ja, const double *a
         if (vv.cls.cls && options().fuse_sweeps &&
             (o.kind == P_IT_JACOBI || o.kind == P_GS_IT || o.kind == P_GS_IT2))
           o.sweep = sweep_encode(*o.Ls, pd->lia, pd->lja, pd->la, *o.Us, pd->uia, pd->uja, pd->ua,
-                                 o.kind == P_GS_IT && o.m > 1 ? o.A : nullptr, ia, ja, a, pd->d_r);
+                                 o.kind == P_GS_IT && o.m > 1 ? o.A : nullptr, ia, ja, a, pd->d_r,
+                                 o.kind == P_IT_JACOBI);
         if (vv.cls.cls && !capture()) {
           status = LAP_ERR_HIP;
           break;

@@ -258,7 +258,8 @@ void sweep_cls_mode(const SweepCls &s, const ClsMat &A, const ClsMat &B, const d
     case kStoreAccum:
       return sweep_cls_go<W, kStoreAccum>(s, A, B, x, base, out, out2, first, done);
     case kStorePair:
-      return sweep_cls_go<W, kStorePair>(s, A, B, x, base, out, out2, first, done);
+      if constexpr (W <= kClsPair)
+        return sweep_cls_go<W, kStorePair>(s, A, B, x, base, out, out2, first, done);
     default:
       return;
   }
@@ -319,10 +320,16 @@ void release_pair_plans() { g_pair.clear(); }
 SweepCls sweep_encode(const SpmvPlan &L, const int *lia, const int *lja, const double *la,
                       const SpmvPlan &U, const int *uia, const int *uja, const double *ua,
                       const SpmvPlan *A, const int *ia, const int *ja, const double *a,
-                      const double *d_r) {
+                      const double *d_r, bool pairs) {
   SweepCls s, none;
   const int longest = std::max(L.max_row, U.max_row);
   const int width = longest <= 4 ? 4 : (longest + 7) / 8 * 8;
+  // Tables 16 wide: a pair would read 32 values of x for a row that has 15 of them
+  // at most, so pairs keep the CSR arrays.  us per iteration with classes and
+  // CSR pairs at 3 million rows of a ring (wide because its ends wrap round), 11,
+  // 13 and 15 entries a row: it_jacobi 295, 303, 312 and 231, 256, 286; GS_it2 (one
+  // pair an iteration) 497, 506, 514 and 436, 470, 498.
+  if (pairs && width > kClsPair) return none;
   s.n = L.n;
   s.L = cls_encode("L", L.n, L.nnz, lia, lja, la, d_r, L.max_row, width);
   if (!s.L.cls) return none;
