@@ -317,7 +317,8 @@ int lap_pcg_adjoint(int n, int nnz, const int *ia, const int *ja, const double *
 double lap_spmv_timed(int n, int nnz, const int *ia, const int *ja, const double *a,
                       const double *x, double *y, int reps);
 /* Same for the PCG's fused kernel q = A p with p.q and alpha in its
- * epilogue (the dominant kernel of a Jacobi PCG iteration). */
+ * epilogue, in the form that a long solve of the matrix runs (row classes for
+ * large systems with few distinct rows). */
 double lap_pcg_spmv_timed(int n, int nnz, const int *ia, const int *ja, const double *a,
                           const double *p, double *q, int reps);
 

@@ -1228,7 +1228,9 @@ double lap_pcg_spmv_timed(int n, int nnz, const int *ia, const int *ja, const do
   PcgCtl *ctl = reinterpret_cast<PcgCtl *>(scratch_vec("timed_ctl", sizeof(PcgCtl) / 8 + 1));
   LAP_HIP(hipMemcpyAsync(ctl, &h, sizeof h, hipMemcpyHostToDevice, stream()));
   const unsigned g = spmv_grid(*A);
-  const ViVals vv = vi_prepare(nnz, a, n, ia, ja);  // (format 0: the CSR kernel)
+  ViVals vv = vi_prepare(nnz, a, n, ia, ja);  // the kernel the solve would run
+  if (options().spmv_format == 0 && n >= kClsMinRows)
+    vv.cls = cls_encode("a", n, nnz, ia, ja, a, nullptr, A->max_row);
   auto launch = [&]() { launch_spmv_pq(g, *A, ia, ja, a, p, q, ctl, ws.partials + kR2, vv); };
   launch();
   hipEvent_t e0, e1;
