@@ -85,6 +85,7 @@ enum { kResWait = 1, kResStale = 2 };
 struct ResShared {
   int error;     // kResWait: a wait ran out; kResStale: the plan is of other columns
   unsigned tag;  // highest tag used
+  // (both stay from solve to solve; cleared with the boxes after an error)
 };
 // A workgroup: its first row and row count, its team's first workgroup and
 // workgroup count, its system and that system's rows.
@@ -95,13 +96,13 @@ struct ResWg {
 struct ResArgs {
   int nhmax;
   const ResWg *wg;
-  const int *ia, *ja;
+  const int *ia;
   const double *a;
   const unsigned short *lcol;
   const int *hcnt, *hcol;
   const unsigned char *sent;
   const double *d_r, *b;
-  double *x, *r, *p, *x0;  // x0: x at the start, kept for a solve that ends in an error
+  double *x, *r, *p;
   double tol;
   int maxit, resume, iters;
   unsigned tag0, polls;
@@ -169,19 +170,17 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
   const __amdgpu_buffer_rsrc_t mine_b = fl_buffer(static_cast<char *>(g.box_b) + 2 * at, size * 32);
   const __amdgpu_buffer_rsrc_t box_w = fl_buffer(g.box_w, g.n * 16);
   if (t == 0) {
-    dead = 0;
+    dead = g.sh->error;  // (k_res_prep's, or a wait's that ran out already)
     ps[zero] = 0.0;
   }
   for (int h = t; h < nh; h += T) hcol[h] = g.hcol[(size_t)w * g.nhmax + h];
   __syncthreads();
+  if (dead) return;  // (it changes behind the next barrier only)
   // the thread's rows
   double val[R][L], x[R], r[R], p[R], d[R];
   unsigned slot[R][(L + 1) / 2];
   bool have[R], sent[R];
   int longest[R];  // of the wave's rows
-  // The slots were made from the columns that ja held at the first solve; where
-  // it has been rewritten since, the solve ends here and the host makes new ones
-  bool stale = false;
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     const int l = t + k * T, row = base + l;
@@ -191,10 +190,6 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
     for (int j = 0; j < L; ++j) {
       val[k][j] = j < len ? g.a[e0 + j] : 0.0;
       const unsigned s = j < len ? g.lcol[e0 + j] : (unsigned)zero;
-      if (j < len) {
-        const int c = g.ja[e0 + j], h = (int)s - R * T;
-        stale |= h < 0 ? (int)s >= rows || base + (int)s != c : h >= nh || hcol[h] != c;
-      }
       if (j & 1)
         slot[k][j / 2] |= s << 16;
       else
@@ -202,19 +197,12 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
     }
     d[k] = have[k] ? g.d_r[row] : 0.0;
     x[k] = have[k] ? g.x[row] : 0.0;
-    if (have[k] && !g.resume) g.x0[row] = x[k];
     r[k] = p[k] = 0.0;
-    stale |= len > L;
     sent[k] = have[k] && g.sent[row];
     int m = len;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
     longest[k] = __builtin_amdgcn_readfirstlane(m);
-  }
-  if (stale) {
-    dead = 1;  // (read after the barriers of the first sums)
-    __hip_atomic_fetch_max(&g.sh->error, (int)kResStale, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
   }
   auto row_sums = [&](double(&s)[R]) {  // CSR order; padding adds 0 * 0
 #pragma unroll
@@ -443,6 +431,33 @@ __global__ __launch_bounds__(T, 4) void k_resident(ResArgs g) {
   }
 }
 
+// Before a solve: keeps x in x0 for one that ends in an error, clears the systems'
+// states, and compares every nonzero's slot with ja, from whose columns it was
+// made at the first solve: where ja has been rewritten since, the solve does not
+// begin (kResStale) and the host makes a new plan.  A workgroup per one of the
+// solve's; longest: entries of a row that the solve has room for.
+__global__ __launch_bounds__(kResThreads) void k_res_prep(
+    const ResWg *__restrict__ wgs, int own, int longest, int nhmax, const int *__restrict__ ia,
+    const int *__restrict__ ja, const unsigned short *__restrict__ lcol,
+    const int *__restrict__ hcnt, const int *__restrict__ hcol, const double *__restrict__ x,
+    double *__restrict__ x0, int nsys, ResState *st, ResShared *sh) {
+  const int w = blockIdx.x, t = threadIdx.x;
+  const ResWg wg = wgs[w];
+  const int nh = hcnt[w], *const halo = hcol + (size_t)w * nhmax;
+  bool stale = false;
+  for (int l = t; l < wg.rows; l += kResThreads) {
+    x0[wg.base + l] = x[wg.base + l];
+    stale |= ia[wg.base + l + 1] - ia[wg.base + l] > longest;
+  }
+  const int e1 = ia[wg.base + wg.rows];
+  for (int e = ia[wg.base] + t; e < e1; e += kResThreads) {
+    const int c = ja[e], s = lcol[e], h = s - own;
+    stale |= h < 0 ? s >= wg.rows || wg.base + s != c : h >= nh || halo[h] != c;
+  }
+  if (stale) atomicMax(&sh->error, (int)kResStale);
+  for (int s = w * kResThreads + t; s < nsys; s += (int)gridDim.x * kResThreads) st[s] = ResState{};
+}
+
 // The analysis: workgroup w lists the rows outside its own that its rows refer
 // to (ascending), marks them as sent, and gives every nonzero its slot: own
 // rows first, then the halo.  Without FILL only cnt[w], the halo's length (more
@@ -538,7 +553,7 @@ const ResShape kShapes[] = {{4, 5, 512, k_resident<4, 5, 512>},
 struct ResPlan {
   bool ok = false;
   std::vector<int> off;
-  int nsys = 0, nwg = 0, stride = 0, nhmax = 0, lds = 0, threads = 0;
+  int nsys = 0, nwg = 0, stride = 0, nhmax = 0, lds = 0, threads = 0, own = 0, longest = 0;
   ResKernel fn = nullptr;
   DevBufPtr wg, hcnt, hcol, sent, lcol, boxes, state, shared;
   size_t box_words = 0;
@@ -602,6 +617,8 @@ static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia,
   P->nwg = (int)wgs.size();
   P->fn = s->fn;
   P->threads = s->threads;
+  P->own = s->r * s->threads;
+  P->longest = s->l;
   P->stride = (P->nwg + 15) / 16 * 16 + kResSkew;
   P->box_words = 4 * ((size_t)n + 3 * (size_t)kResCopies * P->stride);
   auto lds = [&](int halo) {
@@ -654,6 +671,8 @@ static std::shared_ptr<ResPlan> res_plan_build(const SpmvPlan &A, const int *ia,
     if (!b) return nullptr;
   k_res_zero<<<256, kBlock, 0, stream()>>>(((long long)n + 3) / 4, P->sent->as<unsigned>());
   k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P->box_words, P->boxes->as<unsigned>());
+  k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResShared) / 4),
+                                        P->shared->as<unsigned>());
   plan(k_res_plan<true>, P->hcol->as<int>(), P->sent->as<unsigned char>(),
        P->lcol->as<unsigned short>());
   P->lds = lds(P->nhmax);
@@ -675,7 +694,6 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
   g.wg = P.wg->as<ResWg>();
   g.nhmax = P.nhmax;
   g.ia = ia;
-  g.ja = ja;
   g.a = a;
   g.lcol = P.lcol->as<unsigned short>();
   g.hcnt = P.hcnt->as<int>();
@@ -686,7 +704,6 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
   g.x = x;
   g.r = r;
   g.p = p;
-  g.x0 = x0;
   g.tol = tol;
   g.maxit = maxit;
   g.polls = (unsigned)options().resident_polls;
@@ -698,18 +715,14 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
   g.st = P.state->as<ResState>();
   g.sh = P.shared->as<ResShared>();
   std::vector<ResState> h((size_t)P.nsys);
-  auto clear_shared = [&] {
-    k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResShared) / 4),
-                                          P.shared->as<unsigned>());
-  };
   auto clear_boxes = [&] {
     k_res_zero<<<256, kBlock, 0, stream()>>>((long long)P.box_words, P.boxes->as<unsigned>());
-    clear_shared();
+    k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResShared) / 4),
+                                          P.shared->as<unsigned>());
     P.tag = 0;
   };
-  k_res_zero<<<1, kWave, 0, stream()>>>((long long)(sizeof(ResState) / 4 * P.nsys),
-                                        P.state->as<unsigned>());
-  clear_shared();
+  k_res_prep<<<P.nwg, kResThreads, 0, stream()>>>(g.wg, P.own, P.longest, P.nhmax, ia, ja, g.lcol,
+                                                  g.hcnt, g.hcol, x, x0, P.nsys, g.st, g.sh);
   auto restore = [&] {
     return LAP_HIP(hipMemcpyAsync(x, x0, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice,
                                   stream())) &&
@@ -725,8 +738,10 @@ static int res_run(ResPlan &P, int n, const int *ia, const int *ja, const double
     void *args[] = {&g};
     ResShared sh{};
     if (!hip_try(hipLaunchKernel(reinterpret_cast<const void *>(P.fn), dim3((unsigned)P.nwg),
-                                 dim3((unsigned)P.threads), args, (size_t)P.lds, stream())))
-      return k == 0 || restore() ? kResWait : kResError;
+                                 dim3((unsigned)P.threads), args, (size_t)P.lds, stream()))) {
+      clear_boxes();
+      return restore() ? kResWait : kResError;
+    }
     if (!LAP_HIP(hipMemcpyAsync(h.data(), g.st, sizeof(ResState) * h.size(),
                                 hipMemcpyDeviceToHost, stream())) ||
         !LAP_HIP(hipMemcpyAsync(&sh, g.sh, sizeof sh, hipMemcpyDeviceToHost, stream())) ||
