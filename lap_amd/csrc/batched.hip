@@ -23,11 +23,12 @@
 // system's convergence test and beta; p update) replayed from a HIP graph,
 // and the row blocks of systems that have stopped are skipped.  The
 // autotuner times it next to the persistent configurations.  Where every
-// system fits (rows of at most 32 entries, at most 2^19 rows), lockstep mode is
-// the resident solve instead (resident.hip): one launch, a team of workgroups
-// per system.  160 grids of 12 to 150 points a side: 55 ms with the best
-// persistent configuration, 60 ms in lockstep over the block-diagonal matrix,
-// 7.9 ms resident.
+// system fits, lockstep mode is the resident solve instead (resident.hip): one
+// launch, a team of workgroups per system.  A system fits with up to 2^19 rows of
+// up to 8 entries or 2^18 of up to 32, and with at most 8192 rows that a
+// workgroup's rows refer to outside its own.  160 grids of 12 to 150 points a
+// side: 55 ms with the best persistent configuration, 60 ms in lockstep over the
+// block-diagonal matrix, 5.1 ms resident.
 #include <algorithm>
 #include <cmath>
 #include <numeric>

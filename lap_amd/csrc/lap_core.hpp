@@ -394,7 +394,7 @@ struct TriPlan {
   std::vector<int> level_seg;  // host, nlevels + 1
   DevBufPtr segd, seg_part, seg_tick;
   bool has_diag = true;        // every row holds its pivot
-  // Chunked schedule (four chunks of rows per workgroup; built when every row
+  // Chunked schedule (two chunks of rows per workgroup; built when every row
   // holds at most 4 entries beside its pivot).  Chunk c runs its rows level by
   // level in steps of at most 64 rows, padded to that; a dependency on
   // another workgroup (or on a row too many steps back) is one entry of the

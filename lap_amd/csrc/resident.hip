@@ -57,7 +57,9 @@ constexpr int kResMaxWg = 256;     // workgroups at most (partials: one per thre
 // 3.89, 512^2 9.05 / 9.08 / 6.86, 40^3 7.15 / 6.66 / 6.70, 64^3 9.4 / 9.4 /
 // 11.1, 97 x 90 x 31 8.7 / 8.7 / 10.6: 2048 for rows of up to 5 entries.
 constexpr int kResRows = 1024, kResRowsShort = 2048, kResShort = 5;
-constexpr int kResMaxN = 1 << 19;  // rows of a system at most (the analysis' bitmap in LDS)
+// Rows of a system at most (the analysis' bitmap in LDS); of more than 8 entries,
+// which have a row per thread, 2^18 (256 workgroups of 1024).
+constexpr int kResMaxN = 1 << 19;
 constexpr int kResMaxRows = 1 << 26;  // rows of all systems at most (box_w stays below 2^31 bytes)
 // Workgroups of a batch at most (their halo lists take up to 32 KB each: 1 GB).
 constexpr int kResMaxWgs = 1 << 15;

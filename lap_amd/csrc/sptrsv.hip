@@ -888,7 +888,7 @@ void forget_tri_plans(const void *p) {
 
 // ------------------------------------------------ chunked schedule (host)
 //
-// A partition of the rows into at most kFlTeam chunks per CU is chosen among
+// A partition of the rows into at most kFlPerCu kFlTeam chunks per CU is chosen among
 // a few candidates by simulating the pipeline: every step of a chunk costs
 // one unit, a value from another chunk of the workgroup kSibCost more, one
 // from another workgroup kHopCost more (it goes through memory).  Candidates:
