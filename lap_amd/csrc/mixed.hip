@@ -988,6 +988,8 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
     return LAP_ERR_ARG;
   }
   const int walk = options().spmv_walk;
+  const bool chunked = ic && options().sptrsv_mode != 0;
+  if (chunked) tri_clear_error();
   // Deflation of the constant vector (generic path): when every row of A sums
   // to the same s > 0 and s is tiny against the diagonal (a graph Laplacian
   // plus a small shift), A 1 = s 1 is a near-null mode that the FP32
@@ -1204,6 +1206,11 @@ static int run_mixed(int n, int nnz, const int *ia, const int *ja, const double 
     LAP_HIP(hipMemcpy(h_hist, hist, sizeof(double) * (size_t)(h.last_iter + 1),
                       hipMemcpyDeviceToHost));
   if (status == LAP_OK && lap_last_status() == LAP_ERR_HIP) status = LAP_ERR_HIP;
+  if (chunked && tri_error()) {
+    set_error(LAP_ERR_NUMERIC, "pcg_mixed: a triangular-solve dependency wait ran out");
+    tri_clear_error();
+    if (status == LAP_OK) status = LAP_ERR_NUMERIC;
+  }
   return status;
 }
 
